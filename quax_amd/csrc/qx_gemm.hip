@@ -8,12 +8,17 @@
 // both operands are read "transposed", which the kernel does directly from
 // LDS tiles (no transposed copies).
 //
-// Kernel: 64 x 64 output tile per 256-thread workgroup (four 64-wide
-// wavefronts, 32 x 32 each as 2 x 2 tiles of v_mfma_f64_16x16x4f64), K in
-// steps of 32 staged through LDS.  MFMA operand layout (16x16x4, FP64,
+// Kernel: all of up to 128 rows of Y (MT tiles of 16, no padding beyond the
+// last one) x 128 columns per 256-thread workgroup, so X is read once: wave w
+// owns 32 columns and every row (MT x 2 tiles of v_mfma_f64_16x16x4f64).  K
+// goes in steps of 16 through two LDS buffers: the next step is loaded into
+// registers before the current one is multiplied and stored to the other
+// buffer after it, one barrier per step.  MFMA operand layout (16x16x4, FP64,
 // checked on gfx950 with a one-wavefront probe): lane l supplies
 // A[l % 16][l / 16] and B[l / 16][l % 16]; accumulator element r of lane l is
 // D[4 r + l / 16][l % 16] (rows interleaved across the four 16-lane groups).
+// Bound by the FP64 matrix rate (2 M flops per 8 bytes of X; 68-72 TFLOP/s
+// reached by a large product on this part).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -25,87 +30,121 @@ namespace {
 
 typedef double qx_dv4 __attribute__((ext_vector_type(4)));
 
-constexpr int GM_BM = 64, GM_BN = 64, GM_BK = 32, GM_THREADS = 256;
-constexpr int GM_PAD = 2;  // LDS row padding (doubles) against bank conflicts
+constexpr int GM_BK = 16, GM_THREADS = 256;
+constexpr int GM_BS = GM_BK + 2;  // B row stride: 16 rows x 4 k hit distinct LDS banks
 
-// out[i * ldo + j] = sum_k opA(i, k) opB(k, j), i < M, j < N, k < K, with
-// opA(i, k) = A[k * lda + i] (A stored K x M) and opB(k, j) = B[j * ldb + k]
-// (B stored N x K).  Grid: (ceil(N / 64), ceil(M / 64)).
+// out[i * ldo + j] = sum_k A[k * lda + i] B[j * ldb + k], i < M, j < N, k < K,
+// for the rows i0 = blockIdx.y * 16 MT onwards and NT * 64 columns.
+template <int MT, int NT>
 __global__ __launch_bounds__(GM_THREADS) void qx_dgemm_tt_kernel(int M, long long N, int K, const double* __restrict__ A,
                                                                   long long lda, const double* __restrict__ B,
                                                                   long long ldb, double* __restrict__ out,
                                                                   long long ldo) {
-  __shared__ double As[GM_BK][GM_BM + GM_PAD];
-  __shared__ double Bs[GM_BK][GM_BN + GM_PAD];
-  const int tid = threadIdx.x;
-  const int lane = tid & 63, wave = tid >> 6;
-  const int wr = wave >> 1, wc = wave & 1;  // wave's 32 x 32 quadrant
-  const long long i0 = (long long)blockIdx.y * GM_BM;
-  const long long j0 = (long long)blockIdx.x * GM_BN;
-  qx_dv4 acc[2][2];
+  constexpr int BM = 16 * MT, BN = 64 * NT;
+  constexpr int AS = BM + (MT % 2 ? 0 : 16);  // odd multiple of 16: the two k of a half wave hit distinct banks
+  constexpr int NA = (GM_BK * BM + GM_THREADS - 1) / GM_THREADS, NB = GM_BK * BN / GM_THREADS;
+  __shared__ double As[2][GM_BK * AS];
+  __shared__ double Bs[2][BN * GM_BS];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int i0 = (int)blockIdx.y * BM;
+  const long long j0 = (long long)blockIdx.x * BN;
+  qx_dv4 acc[MT][NT];
 #pragma unroll
-  for (int a = 0; a < 2; ++a)
+  for (int a = 0; a < MT; ++a)
 #pragma unroll
-    for (int b = 0; b < 2; ++b) acc[a][b] = qx_dv4{0.0, 0.0, 0.0, 0.0};
-  for (int k0 = 0; k0 < K; k0 += GM_BK) {
-    // A tile: rows k (32) x cols i (64), contiguous along i in memory
+    for (int b = 0; b < NT; ++b) acc[a][b] = qx_dv4{0.0, 0.0, 0.0, 0.0};
+  double ra[NA], rb[NB];
+  auto load = [&](int k0) {
 #pragma unroll
-    for (int r = 0; r < GM_BK * GM_BM / GM_THREADS; ++r) {
-      const int idx = tid + r * GM_THREADS;
-      const int k = idx / GM_BM, i = idx % GM_BM;
-      const long long gi = i0 + i;
-      const int gk = k0 + k;
-      As[k][i] = (gi < M && gk < K) ? A[(long long)gk * lda + gi] : 0.0;
+    for (int r = 0; r < NA; ++r) {
+      const int idx = tid + r * GM_THREADS, k = idx / BM, i = idx - k * BM;
+      ra[r] = k < GM_BK && i0 + i < M && k0 + k < K ? A[(long long)(k0 + k) * lda + i0 + i] : 0.0;
     }
-    // B tile: for each output column j, 32 consecutive k
 #pragma unroll
-    for (int r = 0; r < GM_BK * GM_BN / GM_THREADS; ++r) {
-      const int idx = tid + r * GM_THREADS;
-      const int j = idx / GM_BK, k = idx % GM_BK;
-      const long long gj = j0 + j;
-      const int gk = k0 + k;
-      Bs[k][j] = (gj < N && gk < K) ? B[gj * ldb + gk] : 0.0;
+    for (int r = 0; r < NB; ++r) {
+      const int idx = tid + r * GM_THREADS, j = idx / GM_BK, k = idx % GM_BK;
+      rb[r] = j0 + j < N && k0 + k < K ? B[(j0 + j) * ldb + k0 + k] : 0.0;
     }
-    __syncthreads();
+  };
+  auto store = [&](int buf) {
 #pragma unroll
-    for (int kk = 0; kk < GM_BK; kk += 4) {
+    for (int r = 0; r < NA; ++r) {
+      const int idx = tid + r * GM_THREADS, k = idx / BM, i = idx - k * BM;
+      if (k < GM_BK) As[buf][k * AS + i] = ra[r];
+    }
+#pragma unroll
+    for (int r = 0; r < NB; ++r) {
+      const int idx = tid + r * GM_THREADS, j = idx / GM_BK, k = idx % GM_BK;
+      Bs[buf][j * GM_BS + k] = rb[r];
+    }
+  };
+  load(0);
+  store(0);
+  __syncthreads();
+  int buf = 0;
+  for (int k0 = 0; k0 < K; k0 += GM_BK, buf ^= 1) {
+    const bool more = k0 + GM_BK < K;
+    if (more) load(k0 + GM_BK);
+    const int kc = min(GM_BK, K - k0);
+    for (int kk = 0; kk < kc; kk += 4) {  // block-uniform
       const int ka = kk + (lane >> 4);
-      double a[2], b[2];
+      double b[NT];
 #pragma unroll
-      for (int t = 0; t < 2; ++t) {
-        a[t] = As[ka][wr * 32 + t * 16 + (lane & 15)];
-        b[t] = Bs[ka][wc * 32 + t * 16 + (lane & 15)];
+      for (int t = 0; t < NT; ++t) b[t] = Bs[buf][(wave * 16 * NT + t * 16 + (lane & 15)) * GM_BS + ka];
+#pragma unroll
+      for (int t = 0; t < MT; ++t) {
+        const double a = As[buf][ka * AS + t * 16 + (lane & 15)];
+#pragma unroll
+        for (int u = 0; u < NT; ++u) acc[t][u] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, b[u], acc[t][u], 0, 0, 0);
       }
-#pragma unroll
-      for (int ta = 0; ta < 2; ++ta)
-#pragma unroll
-        for (int tb = 0; tb < 2; ++tb) acc[ta][tb] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[ta], b[tb], acc[ta][tb], 0, 0, 0);
     }
+    if (more) store(buf ^ 1);
     __syncthreads();
   }
 #pragma unroll
-  for (int ta = 0; ta < 2; ++ta)
+  for (int ta = 0; ta < MT; ++ta)
 #pragma unroll
-    for (int tb = 0; tb < 2; ++tb)
+    for (int tb = 0; tb < NT; ++tb)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const long long gi = i0 + wr * 32 + ta * 16 + 4 * r + (lane >> 4);
-        const long long gj = j0 + wc * 32 + tb * 16 + (lane & 15);
+        const long long gi = i0 + ta * 16 + 4 * r + (lane >> 4);
+        const long long gj = j0 + wave * 16 * NT + tb * 16 + (lane & 15);
         if (gi < M && gj < N) out[gi * ldo + gj] = acc[ta][tb][r];
       }
+}
+
+template <int MT>
+void gemm_launch(dim3 rows, int M, long long N, int K, const double* A, const double* B, double* out, hipStream_t s) {
+  // 128 columns per workgroup once that still gives every CU work, else 64
+  if (N >= 128 * 512) {
+    hipLaunchKernelGGL((qx_dgemm_tt_kernel<MT, 2>), dim3((unsigned)((N + 127) / 128), rows.y), dim3(GM_THREADS), 0, s, M, N,
+                       K, A, (long long)M, B, (long long)K, out, N);
+  } else {
+    hipLaunchKernelGGL((qx_dgemm_tt_kernel<MT, 1>), dim3((unsigned)((N + 63) / 64), rows.y), dim3(GM_THREADS), 0, s, M, N, K,
+                       A, (long long)M, B, (long long)K, out, N);
+  }
 }
 
 thread_local std::string g_gemm_error;
 
 int gemm_tt(int M, long long N, int K, const double* A, const double* B, double* out, hipStream_t s) {
   if (M <= 0 || N <= 0 || K <= 0) return QX_OK;
-  const long long gx = (N + GM_BN - 1) / GM_BN, gy = (M + GM_BM - 1) / GM_BM;
-  if (gy > 65535 || gx > 0x7fffffffLL) {
+  const int tiles = (M + 15) / 16, gy = (tiles + 7) / 8, mt = (tiles + gy - 1) / gy;  // equal shares of at most 8 tiles
+  if (gy > 65535 || (N + 63) / 64 > 0x7fffffffLL) {
     g_gemm_error = "tei transformation: tensor too large for one launch";
     return QX_EINVAL;
   }
-  hipLaunchKernelGGL(qx_dgemm_tt_kernel, dim3((unsigned)gx, (unsigned)gy), dim3(GM_THREADS), 0, s, M, N, K, A,
-                     (long long)M, B, (long long)K, out, N);
+  const dim3 rows(1, (unsigned)gy);
+  switch (mt) {
+    case 1: gemm_launch<1>(rows, M, N, K, A, B, out, s); break;
+    case 2: gemm_launch<2>(rows, M, N, K, A, B, out, s); break;
+    case 3: gemm_launch<3>(rows, M, N, K, A, B, out, s); break;
+    case 4: gemm_launch<4>(rows, M, N, K, A, B, out, s); break;
+    case 5: gemm_launch<5>(rows, M, N, K, A, B, out, s); break;
+    case 6: gemm_launch<6>(rows, M, N, K, A, B, out, s); break;
+    case 7: gemm_launch<7>(rows, M, N, K, A, B, out, s); break;
+    default: gemm_launch<8>(rows, M, N, K, A, B, out, s); break;
+  }
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) {
     g_gemm_error = std::string("tei transformation: ") + hipGetErrorString(e);
