@@ -37,7 +37,7 @@ FLAGS = ["-std=c++17", "-O3", f"--offload-arch={ARCH}", "-fPIC", "-munsafe-fp-at
          f"-I{os.path.join(ROOT, 'include')}", f"-I{HERE}"]
 
 RUNTIME_SOURCES = ["qx_runtime.hip", "qx_kernels.hip", "qx_gemm.hip", "qx_scf.hip"]
-HEADERS = ["qx_device.h", "qx_runtime.h"]
+HEADERS = ["qx_device.h", "qx_oei.h", "qx_runtime.h"]
 
 
 def _hash(paths, extra):
@@ -70,9 +70,11 @@ def _opt_flags(src):
 
 def _compile(src, force):
     if src.startswith(GEN):
-        # generated class kernels include only qx_device.h (the class tables
-        # in qx_classes.inc are compiled into qx_runtime.hip alone)
-        deps = [src, os.path.join(HERE, "qx_device.h")]
+        # generated class kernels include only qx_device.h, the one-electron
+        # ones also qx_oei.h and qx_runtime.h (the class tables in
+        # qx_classes.inc are compiled into qx_runtime.hip alone)
+        heads = HEADERS if os.path.basename(src).startswith("oei_") else ["qx_device.h"]
+        deps = [src] + [os.path.join(HERE, h) for h in heads]
     else:
         deps = [src] + [os.path.join(HERE, h) for h in HEADERS] + [os.path.join(ROOT, "include", "quax_amd.h"),
                                                                    os.path.join(GEN, "qx_classes.inc")]

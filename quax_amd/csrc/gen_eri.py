@@ -726,6 +726,88 @@ def emit_class_files(cls, outdir, fp32):
     return files, stats, len(parts), groups, len(tparts)
 
 
+def emit_oei(la, lb, outdir):
+    """oei_<la><lb>.hip: the attraction recurrences of one shell-pair class
+    (the ERI bra recurrence with W - P = C - P and the (ss|ss) integrals
+    replaced by the (s|1/r_C|s) ones) and its kernels (qx_oei.h)."""
+    nm = f"{la}{lb}"
+    A, B = comps(la), comps(lb)
+
+    def head(L, v, PA="PA", PC="PC", nb=0):
+        used = "\n".join(v.lines)
+        for i, ax in enumerate(AX):
+            if f"PA{ax}" in used:
+                L.append(f"  const R PA{ax} = {PA}[{i}], WP{ax} = -{PC}[{i}];")
+        if " rp " in used:
+            L.append("  const double rp = 1.0;")
+        for m in range(nb + 1):
+            L.append(f"  const R b{m} = F[{m}];")
+        L.extend("  " + x for x in v.lines)
+
+    h, v, vn, outs, _ = build_dag([(a, b, Z3, Z3) for a in A for b in B])
+    L = []
+    L.append(f"#define NA_{nm} {len(A)}")
+    L.append(f"#define NB_{nm} {len(B)}")
+    L.append(f"template <typename R>\n__device__ __forceinline__ void qx_ov_{nm}(const R (&PA)[3], const R (&PC)[3], "
+             f"double oo2p, const R (&F)[{la + lb + 1}], R (&s)[{len(vn)}]) {{")
+    head(L, v, nb=la + lb)
+    for k, (_, name) in enumerate(sorted(vn.items())):
+        L.append(f"  s[{k}] += {name};")
+    L.append("}")
+
+    def hrr_in(L, vn, src=None):
+        for k, ((a, c), name) in enumerate(sorted(vn.items())):
+            L.append(f"  const R s_{a[0]}{a[1]}{a[2]}_000 = {f'{src}[{k}]' if src else name};")
+
+    L.append(f"template <typename R>\n__device__ __forceinline__ void qx_ovh_{nm}(const R (&AB)[3], "
+             f"const R (&s)[{len(vn)}], R (&o)[{len(A) * len(B)}]) {{")
+    L.append("  const R ABx = AB[0], ABy = AB[1], ABz = AB[2];")
+    hrr_in(L, vn, "s")
+    L += ["  " + x for x in h.lines]
+    L += [f"  o[{k}] = {x};" for k, x in enumerate(outs)]
+    L.append("}")
+    ns = len(vn)
+    # derivative: d/dA and d/dB of every (a|b), contracted with the density block
+    combos = [(c, x) for c in "AB" for x in range(3)]
+    T, plan = [], []
+    for i, a in enumerate(A):
+        for j, b in enumerate(B):
+            for ci, (cen, x) in enumerate(combos):
+                q = [a, b]
+                k = "AB".index(cen)
+                up = list(q)
+                up[k] = inc(q[k], x)
+                T.append((up[0], up[1], Z3, Z3))
+                n = q[k][x]
+                if n > 0:
+                    dn = list(q)
+                    dn[k] = inc(q[k], x, -1)
+                    T.append((dn[0], dn[1], Z3, Z3))
+                plan.append((i * len(B) + j, ci, cen, n))
+    h, v, vn, outs, pos = build_dag(T)
+    L.append(f"template <typename R>\n__device__ __forceinline__ void qx_ovg_{nm}(const R (&PA)[3], const R (&PC)[3], "
+             f"double oo2p, const R (&F)[{la + lb + 2}], const R (&AB)[3], double wA, double wB, "
+             f"const double (&pd)[{len(A) * len(B)}], double (&g)[6]) {{")
+    L.append("  const R ABx = AB[0], ABy = AB[1], ABz = AB[2];")
+    head(L, v, nb=la + lb + 1)
+    hrr_in(L, vn)
+    groups, t = [], 0
+    for (e, ci, cen, n) in plan:
+        last, ex = pos[t], f"w{cen} * {outs[t]}"
+        t += 1
+        if n > 0:
+            last, ex = max(last, pos[t]), ex + f" - double({n}) * {outs[t]}"
+            t += 1
+        groups.append((max(last, groups[-1][0] if groups else 0), [f"  g[{ci}] += pd[{e}] * oei_out({ex});"]))
+    L += ["  " + x if not x.startswith("  ") else x for x in interleave(h.lines, groups)]
+    L.append("}")
+    L += ["", f"QX_DEFINE_OEI({nm}, {la}, {lb}, {ns})"]
+    path = os.path.join(outdir, f"oei_{nm}.hip")
+    with open(path, "w") as fh:
+        fh.write("\n".join(['#include "../qx_oei.h"', ""] + L + [""]))
+    return path
+
+
 def main():
     outdir = sys.argv[1]
     lmax = int(sys.argv[2]) if len(sys.argv) > 2 else 2
@@ -742,6 +824,8 @@ def main():
         groups[cls] = grp
         jkf[cls] = s[0][2]["jk_flops"]
         flops[cls] = (s[0][2]["flops"], [st["flops"] for _, _, st in s[1:]], [st["ncomb"] for _, _, st in s[1:]])
+    pairs = [(a, b) for a in range(lmax + 1) for b in range(a + 1)]
+    files += [emit_oei(a, b, outdir) for a, b in pairs]
     D = ["// generated: kernel launch tables indexed by canonical class id", "#pragma once",
          f"#define QX_GEN_LMAX {lmax}", f"#define QX_NUM_CLASSES {len(classes)}",
          f"#define QX_MAX_DPARTS {max(nparts.values())}",
@@ -796,6 +880,10 @@ def main():
     for cls in classes:
         D.append(f"  {{{TILES['jk'].get(cls, 128)}, {TILES['grad'].get(cls, 128)}}},")
     D.append("};")
+    D.append("// one-electron kernels per shell-pair class")
+    D += [f'extern "C" int qx_launch_oei_{a}{b}(const QxOei*, int, hipStream_t);' for a, b in pairs]
+    D.append(f"static int (*const qx_oei_table[{len(pairs)}])(const QxOei*, int, hipStream_t) = {{"
+             + ", ".join(f"qx_launch_oei_{a}{b}" for a, b in pairs) + "};")
     with open(os.path.join(outdir, "qx_classes.inc"), "w") as fh:
         fh.write("\n".join(D) + "\n")
     with open(os.path.join(outdir, "stats.txt"), "w") as fh:

@@ -57,6 +57,8 @@ struct qx_ctx {
   std::vector<void*> allocs;
   double* d_boys = nullptr;
   QxShellsDev shells{};
+  int* d_shell_by_l = nullptr;           // shells grouped by l; group l is [l_off[l], l_off[l + 1])
+  int l_off[QX_LMAX_SUPPORTED + 2] = {};
   // screened pairs + pseudo pairs (sorted)
   QxPairsDev pr{};
   QxPrimPairsDev pp{};
@@ -171,10 +173,6 @@ int qxk_cart_to_ao_mat(const QxShellsDev* sh, const double* in, double* out, hip
 int qxk_ao_to_cart_mat(const QxShellsDev* sh, const double* in, double* out, hipStream_t s);   // T^T X T
 int qxk_cart_to_ao_axis(const QxShellsDev* sh, const double* in, double* out, long long outer, int axis_len_in,
                         int axis_len_out, long long inner, hipStream_t s);
-int qxk_oei(const QxShellsDev* sh, double* S, double* T, double* V, hipStream_t s);
-int qxk_oei_deriv(const QxShellsDev* sh, const double* Pd, const double* Wd, double* grad, double* dS, double* dT,
-                  double* dV, hipStream_t s);
+int qxk_oei_deriv(const QxShellsDev* sh, double* dS, double* dT, double* dV, hipStream_t s);
 // grad += Pd . d/dtv d(T+V)/dR + Wd . d/dtv dS/dR (Cartesian Pd, Wd)
-int qxk_oei_hess_dir(const QxShellsDev* sh, const double* Pd, const double* Wd, const double* tv, double* grad,
-                     hipStream_t s);
 }

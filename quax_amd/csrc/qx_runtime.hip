@@ -19,6 +19,7 @@
 
 #include "quax_amd.h"
 #include "qx_runtime.h"
+#include "qx_oei.h"
 #include "qx_classes.inc"  // generated; in the build's generated-source directory
 
 static_assert(QX_GEN_LMAX == QX_LMAX_SUPPORTED, "generated kernels and runtime disagree on lmax");
@@ -651,6 +652,15 @@ void setup_shell_tables(qx_ctx* c) {
       }
     for (int k = 0; k < nsph(l, c->pure); ++k) as.push_back(sh);
   }
+  // shells grouped by angular momentum (one-electron pair classes)
+  std::vector<int> by_l;
+  for (int l = 0; l <= QX_LMAX_SUPPORTED; ++l) {
+    c->l_off[l] = (int)by_l.size();
+    for (int sh = 0; sh < c->nshell; ++sh)
+      if (c->l[sh] == l) by_l.push_back(sh);
+  }
+  c->l_off[QX_LMAX_SUPPORTED + 1] = (int)by_l.size();
+  c->d_shell_by_l = dupload(c, by_l);
   s.f_shell = dupload(c, fs); s.f_comp = dupload(c, fc); s.ao_shell = dupload(c, as);
   // transform blocks: identity for l < 2 (stored for uniform access), solid harmonics for d
   std::vector<double> blk;
@@ -1380,24 +1390,60 @@ int qx_jk_deriv_dir(qx_ctx* c, const double* D, const double* v, double* J, doub
   });
 }
 
+// Every shell-pair class of a one-electron pass.
+static void run_oei(qx_ctx* c, QxOei& a, int mode, hipStream_t s, const char* what) {
+  a.sh = c->shells;
+  a.boys = c->d_boys;
+  for (int la = 0, X = 0; la <= QX_LMAX_SUPPORTED; ++la)
+    for (int lb = 0; lb <= la; ++lb, ++X) {
+      a.la = c->d_shell_by_l + c->l_off[la]; a.nla = c->l_off[la + 1] - c->l_off[la];
+      a.lb = c->d_shell_by_l + c->l_off[lb]; a.nlb = c->l_off[lb + 1] - c->l_off[lb];
+      const long long np = la == lb ? (long long)a.nla * (a.nla + 1) / 2 : (long long)a.nla * a.nlb;
+      QX_REQUIRE(np <= 0x7fffffff, QX_EUNSUPPORTED, "too many shell pairs for a one-electron pass");
+      a.npair = (int)np;
+      check_launch(qx_oei_table[X](&a, mode, s), what);
+    }
+}
+
 int qx_oei(qx_ctx* c, double* S, double* T, double* V, void* stream) {
   if (!c || !S || !T || !V) return QX_EINVAL;
   return guarded(c, [&]() -> int {
     QX_HIP(hipSetDevice(c->device));
     hipStream_t s = (hipStream_t)stream;
-    const size_t nc = c->ncart;
+    const size_t n2 = (size_t)c->ncart * c->ncart;
+    QxOei a{};
+    a.S = S; a.T = T; a.V = V;
     if (!c->pure) {
-      check_launch(qxk_oei(&c->shells, S, T, V, s), "oei");
+      run_oei(c, a, 0, s, "oei");
     } else {
-      DevBuf a(nc * nc * 8), b(nc * nc * 8), d(nc * nc * 8);
-      check_launch(qxk_oei(&c->shells, a.d(), b.d(), d.d(), s), "oei");
-      check_launch(qxk_cart_to_ao_mat(&c->shells, a.d(), S, s), "cart_to_ao");
-      check_launch(qxk_cart_to_ao_mat(&c->shells, b.d(), T, s), "cart_to_ao");
-      check_launch(qxk_cart_to_ao_mat(&c->shells, d.d(), V, s), "cart_to_ao");
+      DevBuf w(3 * n2 * 8);
+      a.S = w.d(); a.T = a.S + n2; a.V = a.T + n2;
+      run_oei(c, a, 0, s, "oei");
+      check_launch(qxk_cart_to_ao_mat(&c->shells, a.S, S, s), "cart_to_ao");
+      check_launch(qxk_cart_to_ao_mat(&c->shells, a.T, T, s), "cart_to_ao");
+      check_launch(qxk_cart_to_ao_mat(&c->shells, a.V, V, s), "cart_to_ao");
       QX_HIP(hipStreamSynchronize(s));
     }
     return QX_OK;
   });
+}
+
+// grad += Pd . d(T+V)/dR + Wd . dS/dR, or (v) its derivative along v.
+static void oei_contract(qx_ctx* c, const double* Pd, const double* Wd, const double* v, double* grad, hipStream_t s,
+                         const char* what) {
+  const size_t n2 = (size_t)c->ncart * c->ncart;
+  QxOei a{};
+  a.Pd = Pd; a.Wd = Wd; a.grad = grad; a.tv = v;
+  if (!c->pure) {
+    run_oei(c, a, v ? 2 : 1, s, what);
+  } else {
+    DevBuf w(2 * n2 * 8);
+    check_launch(qxk_ao_to_cart_mat(&c->shells, Pd, w.d(), s), "ao_to_cart");
+    check_launch(qxk_ao_to_cart_mat(&c->shells, Wd, w.d() + n2, s), "ao_to_cart");
+    a.Pd = w.d(); a.Wd = a.Pd + n2;
+    run_oei(c, a, v ? 2 : 1, s, what);
+    QX_HIP(hipStreamSynchronize(s));
+  }
 }
 
 int qx_oei_grad(qx_ctx* c, const double* Pd, const double* Wd, double* grad, void* stream) {
@@ -1405,16 +1451,7 @@ int qx_oei_grad(qx_ctx* c, const double* Pd, const double* Wd, double* grad, voi
   return guarded(c, [&]() -> int {
     QX_HIP(hipSetDevice(c->device));
     hipStream_t s = (hipStream_t)stream;
-    const size_t nc = c->ncart;
-    if (!c->pure) {
-      check_launch(qxk_oei_deriv(&c->shells, Pd, Wd, grad, nullptr, nullptr, nullptr, s), "oei_grad");
-    } else {
-      DevBuf a(nc * nc * 8), b(nc * nc * 8);
-      check_launch(qxk_ao_to_cart_mat(&c->shells, Pd, a.d(), s), "ao_to_cart");
-      check_launch(qxk_ao_to_cart_mat(&c->shells, Wd, b.d(), s), "ao_to_cart");
-      check_launch(qxk_oei_deriv(&c->shells, a.d(), b.d(), grad, nullptr, nullptr, nullptr, s), "oei_grad");
-      QX_HIP(hipStreamSynchronize(s));
-    }
+    oei_contract(c, Pd, Wd, nullptr, grad, s, "oei_grad");
     return QX_OK;
   });
 }
@@ -1427,16 +1464,7 @@ int qx_oei_hess_dir(qx_ctx* c, const double* Pd, const double* Wd, const double*
   return guarded(c, [&]() -> int {
     QX_HIP(hipSetDevice(c->device));
     hipStream_t s = (hipStream_t)stream;
-    const size_t nc = c->ncart;
-    if (!c->pure) {
-      check_launch(qxk_oei_hess_dir(&c->shells, Pd, Wd, v, grad, s), "oei_hess_dir");
-    } else {
-      DevBuf a(nc * nc * 8), b(nc * nc * 8);
-      check_launch(qxk_ao_to_cart_mat(&c->shells, Pd, a.d(), s), "ao_to_cart");
-      check_launch(qxk_ao_to_cart_mat(&c->shells, Wd, b.d(), s), "ao_to_cart");
-      check_launch(qxk_oei_hess_dir(&c->shells, a.d(), b.d(), v, grad, s), "oei_hess_dir");
-      QX_HIP(hipStreamSynchronize(s));
-    }
+    oei_contract(c, Pd, Wd, v, grad, s, "oei_hess_dir");
     return QX_OK;
   });
 }
@@ -1454,7 +1482,7 @@ int qx_oei_deriv(qx_ctx* c, double* dS, double* dT, double* dV, void* stream) {
     check_launch(qxk_fill(cS, m * nc2, 0.0, s), "fill");
     check_launch(qxk_fill(cT, m * nc2, 0.0, s), "fill");
     check_launch(qxk_fill(cV, m * nc2, 0.0, s), "fill");
-    check_launch(qxk_oei_deriv(&c->shells, nullptr, nullptr, nullptr, cS, cT, cV, s), "oei_deriv");
+    check_launch(qxk_oei_deriv(&c->shells, cS, cT, cV, s), "oei_deriv");
     if (c->pure) {
       // every coordinate slice Cartesian -> AO
       for (long long x = 0; x < m; ++x) {
