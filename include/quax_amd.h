@@ -317,6 +317,13 @@ int qx_jk_build_masked(qx_ctx* ctx, const double* D, double* J, double* K, int p
  * of default priority that join back into it before the call returns. */
 int qx_set_streams(qx_ctx* ctx, int nstreams);
 
+/* Most device memory (bytes; 0 = what the device has) that the tensor entry
+ * points (compute_2e_int, eri_deriv_core(1), compute_2e_deriv of order 0 and
+ * 1) take for their function-pair matrices; a tighter limit makes them work
+ * through fewer derivative slices at a time and then through row panels, with
+ * the same result. */
+int qx_set_tensor_limit(qx_ctx* ctx, long long bytes);
+
 /* Measurement support (no reference counterpart).
  * qx_class_quartets: canonical screened quartets per kernel class (eri[]) and
  * those not on a single atom (deri[], the derivative work); arrays of

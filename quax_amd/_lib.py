@@ -76,6 +76,7 @@ SIGNATURES = {
     "qx_set_fp32_classes": (_i, [_vp, _i, _vp]),
     "qx_get_fp32_classes": (_i, [_vp, _i, _vp]),
     "qx_set_streams": (_i, [_vp, _i]),
+    "qx_set_tensor_limit": (_i, [_vp, _ll]),
     "qx_set_class_tiles": (_i, [_vp, _i, _vp]),
     "qx_set_grad_wave_reduce": (_i, [_vp, _vp]),
     "qx_set_grad_copies": (_i, [_vp, _vp]),

@@ -36,8 +36,12 @@ FLAGS = ["-std=c++17", "-O3", f"--offload-arch={ARCH}", "-fPIC", "-munsafe-fp-at
          "-Wno-unused-variable", "-Wno-unused-but-set-variable",
          f"-I{os.path.join(ROOT, 'include')}", f"-I{HERE}"]
 
-RUNTIME_SOURCES = ["qx_runtime.hip", "qx_kernels.hip", "qx_gemm.hip", "qx_scf.hip"]
-HEADERS = ["qx_device.h", "qx_oei.h", "qx_runtime.h"]
+RUNTIME_SOURCES = ["qx_runtime.hip", "qx_kernels.hip", "qx_jk.hip", "qx_gemm.hip", "qx_scf.hip"]
+HEADERS = ["qx_device.h", "qx_pairm.h", "qx_jk.h", "qx_grad.h", "qx_rys.h", "qx_oei.h", "qx_runtime.h"]
+# what each header of the generated sources stands for, besides qx_device.h
+INCLUDES = {"qx_device.h": [], "qx_pairm.h": ["qx_pairm.h"], "qx_jk.h": ["qx_jk.h"], "qx_grad.h": ["qx_grad.h", "qx_jk.h"],
+            "qx_rys.h": ["qx_rys.h", "qx_grad.h", "qx_jk.h", "qx_pairm.h"],
+            "qx_oei.h": ["qx_oei.h", "qx_runtime.h", "qx_pairm.h", "qx_jk.h"]}
 
 
 def _hash(paths, extra):
@@ -53,28 +57,19 @@ def _flags(src):
     """Compiler flags of one translation unit: the runtime sources also see
     the generated class tables (qx_classes.inc in GEN)."""
     if not src.startswith(GEN):
-        return _opt_flags(src) + [f"-I{GEN}"]
-    return _opt_flags(src)
-
-
-def _opt_flags(src):
-    """Tangent (second-derivative) kernels build at -O2: at -O3 the gfx950
-    compiler returned a wrong value for one element of the inlined (dd|ps)
-    tangent part (cls_2210_t3: (d_yy d_zz | p_j s), checked against the same
-    source built with g++ on the host, evaluated in Python, built with the
-    core not inlined, and built at -O2 -- all four agree with the oracle)."""
-    if os.path.basename(src).split("_")[-1].startswith("t"):
-        return [f if f != "-O3" else "-O2" for f in FLAGS]
+        return FLAGS + [f"-I{GEN}"]
     return FLAGS
 
 
 def _compile(src, force):
     if src.startswith(GEN):
-        # generated class kernels include only qx_device.h, the one-electron
-        # ones also qx_oei.h and qx_runtime.h (the class tables in
-        # qx_classes.inc are compiled into qx_runtime.hip alone)
-        heads = HEADERS if os.path.basename(src).startswith("oei_") else ["qx_device.h"]
-        deps = [src] + [os.path.join(HERE, h) for h in heads]
+        # generated class kernels depend on the header they include and on
+        # qx_device.h (the class tables in qx_classes.inc are compiled into
+        # qx_runtime.hip alone)
+        with open(src) as fh:
+            first = re.match(r'#include "\.\./(\w+\.h)"', fh.readline())
+        heads = {"qx_device.h"} | set(INCLUDES[first.group(1)])
+        deps = [src] + sorted(os.path.join(HERE, h) for h in heads)
     else:
         deps = [src] + [os.path.join(HERE, h) for h in HEADERS] + [os.path.join(ROOT, "include", "quax_amd.h"),
                                                                    os.path.join(GEN, "qx_classes.inc")]

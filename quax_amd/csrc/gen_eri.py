@@ -10,8 +10,8 @@ the epilogue), as straight-line code:
      dependency order (bra side first, then transferred to the ket),
   3. Head-Gordon-Pople horizontal recurrence to (ab|cd), choosing the cheaper
      of bra-first / ket-first per class,
-  4. an epilogue selected at run time (store, full-tensor scatter, Schwarz
-     diagonal, direct J/K).
+  4. an epilogue selected at run time (pair matrix, store, Schwarz diagonal) or
+     the contraction of a K kernel.
 
 Derivative kernels build d/dX_i (ab|cd) from d/dA_i phi_a = 2 alpha
 phi_{a+1_i} - a_i phi_{a-1_i}.  Every kernel forms d/dA, d/dB, d/dC and
@@ -21,8 +21,8 @@ its node budget is split into parts over the Cartesian components of a
 (a, b, c, d) in its ranges.  A part recomputes the recurrence
 nodes it shares with the others, but its live set fits the register file
 (the unsplit heavy bodies spill several KB per lane to scratch, and scratch
-latency, not arithmetic, then bounds them).  Epilogues: full-tensor scatter
-or the adjoint gradient.
+latency, not arithmetic, then bounds them).  The heavy classes, and every
+derivative tensor, use the quadrature kernels of qx_rys.h instead.
 
 Usage: python gen_eri.py OUTDIR [LMAX] [--no-fp32]
 """
@@ -303,36 +303,16 @@ def deriv_targets(l, part):
     return T
 
 
-# streaming J/K bodies of classes with at least this many integrals read each
-# density value where it is used instead of preloading the six blocks (the
-# (dd|dp) blocks alone are 162 doubles, i.e. 324 of the 512 registers)
-JK_LAZY_D_MIN = int(os.environ.get("QX_JK_LAZY_D_MIN", "324"))
-
-# largest SSA node count of one streaming J/K body; above it the class is
-# split over ranges of a components (as the derivative parts are).  Measured
-# on cluster10: splitting (dd|dp) into 3 and (dd|dd) into 6 parts made their
-# J/K kernels 1.2x and 1.8x slower (recomputed recurrences cost more than
-# the 5-11 KB of spills saved).  The unsplit (dd|dd) body (7614 nodes) needs
-# 9.2 KB of scratch per lane, and the HSA runtime has refused to provide
-# scratch above ~8 KB per lane for some dispatches (the queue aborts with
-# HSA_STATUS_ERROR_OUT_OF_RESOURCES), so (dd|dd) alone is split in two.
-JK_NODES = 7000
+def _classes(var, default):
+    """Class set of a quadrature path; the environment overrides it (tuning builds)."""
+    return set(os.environ.get(var, default).replace(",", " ").split())
 
 
-def jk_parts(l, budget=None):
-    budget = budget or JK_NODES
-    la, lb, lc, ld = l
-    NA = ncart(la)
-
-    def nodes(a0, a1):
-        T = [(a, b, c, d) for a in comps(la)[a0:a1] for b in comps(lb) for c in comps(lc) for d in comps(ld)]
-        h, v, _, _, _ = build_dag(T)
-        return len(h.lines) + len(v.lines)
-
-    for k in range(1, NA + 1):
-        rs = _ranges(NA, k)
-        if k == NA or all(nodes(*r) <= budget for r in rs):
-            return rs
+# classes whose K, adjoint gradient and (stored) integrals come from the
+# Rys-quadrature kernels (qx_rys.h) instead of the one-lane-per-quartet bodies
+RYS_K = _classes("QX_RYS_K", "2121 2211 2221 2222")
+RYS_G = _classes("QX_RYS_G", "2111 2120 2121 2210 2211 2220 2221 2222")
+RYS_E = _classes("QX_RYS_E", "2111 2120 2121 2211 2220 2221 2222")
 
 
 def _ranges(n, k):
@@ -376,54 +356,6 @@ def deriv_parts(l, budget=None):
     # as the class's csplit allows (1 keeps the (a, b) parts)
     kc = min(deriv_csplit(l), NC)
     return [part((a, a + 1), (b, b + 1), r) for a in range(NA) for b in range(NB) for r in _ranges(NC, kc)]
-
-
-# Largest SSA node count of one tangent (forward-mode) derivative part.  Dual
-# values double the live set: a (dd|dd) part over one (a, b) pair and all c
-# (3727 nodes) needs 14.3 KB of scratch per lane, which the runtime refused
-# to provide (HSA_STATUS_ERROR_OUT_OF_RESOURCES at dispatch); one c component
-# per part (1860 nodes) needs 7.2 KB, no more than the plain derivative
-# kernels that run.  Parts above this cap are split over single c components.
-TANGENT_NODES = 2000
-
-
-def tangent_parts(l):
-    """Derivative parts for the tangent kernels: the class's derivative parts,
-    each still above TANGENT_NODES split into one part per c component."""
-    out = []
-    for part in deriv_parts(l):
-        h, v, _, _, _ = build_dag(deriv_targets(l, part))
-        c0, c1 = part.get("c", (0, ncart(l[2])))
-        if len(h.lines) + len(v.lines) <= TANGENT_NODES or c1 - c0 == 1:
-            out.append(part)
-        else:
-            out += [dict(part, c=(c, c + 1)) for c in range(c0, c1)]
-    return out
-
-
-def emit_setup_tangent(L, Lt):
-    """Set-up of a tangent body: every geometric quantity is a qx_dual whose
-    derivative part follows the atoms along A_.e.tv (exponents are fixed)."""
-    L.append("  const double p = A_.pp.p[u1], q = A_.pp.p[u2];")
-    L.append("  const QxTanPair tb_ = qx_tan_pair(A_, P1, u1), tk_ = qx_tan_pair(A_, P2, u2);")
-    L.append("  const qx_dual Kab = tb_.K, Kcd = tk_.K;")
-    L.append("  const qx_dual Px = tb_.P[0], Py = tb_.P[1], Pz = tb_.P[2];")
-    L.append("  const qx_dual Qx = tk_.P[0], Qy = tk_.P[1], Qz = tk_.P[2];")
-    L.append("  const qx_dual Ax = tb_.A[0], Ay = tb_.A[1], Az = tb_.A[2];")
-    L.append("  const qx_dual Cx = tk_.A[0], Cy = tk_.A[1], Cz = tk_.A[2];")
-    L.append("  const R ABx = tb_.AB[0], ABy = tb_.AB[1], ABz = tb_.AB[2];")
-    L.append("  const R CDx = tk_.AB[0], CDy = tk_.AB[1], CDz = tk_.AB[2];")
-    L.append("  const double pq = p + q, opq = 1.0 / pq;")
-    L.append("  const qx_dual Wx = (p * Px + q * Qx) * opq, Wy = (p * Py + q * Qy) * opq, "
-             "Wz = (p * Pz + q * Qz) * opq;")
-    L.append("  const qx_dual PQx = Px - Qx, PQy = Py - Qy, PQz = Pz - Qz;")
-    L.append("  const double rho = p * q * opq;")
-    L.append("  const qx_dual T = rho * (PQx * PQx + PQy * PQy + PQz * PQz);")
-    L.append(f"  qx_dual F[{Lt + 1}];")
-    L.append(f"  qx_boys_tan<{Lt}>(T, A_.boys, F);")
-    L.append("  const qx_dual pref = (QX_TWO_PI_5_2 / (p * q * sqrt(pq))) * (Kab * Kcd);")
-    for m in range(Lt + 1):
-        L.append(f"  const R b{m} = pref * F[{m}];")
 
 
 def emit_setup(L, Lt, deriv_w):
@@ -470,15 +402,10 @@ def emit_vrr_consts(L, vrr_lines):
         L.append("  const R rq = (R)(p * opq);")
 
 
-def _head(L, fn, sig, Lt, v, vn, ret="void", inline="__forceinline__", tangent=False):
-    if tangent:
-        L.append(f"__device__ {inline} {ret} {fn}(const QxArgs& A_, int P1, int P2, int u1, int u2{sig}) {{")
-        L.append("  using R = qx_dual;")
-        emit_setup_tangent(L, Lt)
-    else:
-        L.append(f"template <typename R>\n__device__ {inline} {ret} {fn}(const QxArgs& A_, int P1, int P2, "
-                 f"int u1, int u2{sig}) {{")
-        emit_setup(L, Lt, False)
+def _head(L, fn, sig, Lt, v, vn, ret="void", inline="__forceinline__"):
+    L.append(f"template <typename R>\n__device__ {inline} {ret} {fn}(const QxArgs& A_, int P1, int P2, "
+             f"int u1, int u2{sig}) {{")
+    emit_setup(L, Lt, False)
     emit_vrr_consts(L, v.lines)
     L += ["  " + x for x in v.lines]
     for (a, c), name in sorted(vn.items()):
@@ -486,9 +413,10 @@ def _head(L, fn, sig, Lt, v, vn, ret="void", inline="__forceinline__", tangent=F
 
 
 def emit_eri_core(l):
-    """Two bodies per class: qx_core_e* writes the integrals to an array (the
-    store / tensor-scatter / Schwarz epilogues), qx_jk_e* contracts each
-    integral into the J' and K' accumulators as soon as it is formed."""
+    """Two bodies per class: qx_core_e* adds the integrals to an array (the
+    pair-matrix / store / Schwarz epilogues), qx_kb_e* sums the primitive
+    quartets of a contracted one and contracts each integral into the K'
+    accumulators as soon as it is formed."""
     la, lb, lc, ld = l
     nn = (ncart(la), ncart(lb), ncart(lc), ncart(ld))
     NA, NB, NC, ND = nn
@@ -500,58 +428,50 @@ def emit_eri_core(l):
     # array form
     L = []
     _head(L, f"qx_core_e{nm}", f", R (&o)[{N}]", Lt, v, vn)
-    groups = [(pos[k], [f"  o[{k}] = {outs[k]};"]) for k in range(N)]
+    groups = [(pos[k], [f"  o[{k}] += {outs[k]};"]) for k in range(N)]
     L += ["  " + x if not x.startswith("  ") else x for x in interleave(h.lines, groups)]
     L.append("}")
     stats = dict(vrr=len(v.lines), vrr_flops=v.nflop, hrr=len(h.lines), hrr_flops=h.nflop, L=Lt, N=N,
                  flops=core_flops(Lt, v.nflop, h.nflop))
-    # streaming J/K form, one body per range of a components
-    jks = []
-    for pi, (a0, a1) in enumerate(jk_parts(l)):
-        Tp = [t for t in T if comps(la).index(t[0]) in range(a0, a1)]
-        hp, vp, vnp, outp, posp = build_dag(Tp)
-        J = []
-        _head(J, f"qx_jk_e{nm}_{pi}", ", double (&jab)[%d], double (&jcd)[%d], double (&kac)[%d], double (&kad)[%d], "
-              "double (&kbc)[%d], double (&kbd)[%d]" % (NA * NB, NC * ND, NA * NC, NA * ND, NB * NC, NB * ND),
-              Lt, vp, vnp)
-        lazy = N >= JK_LAZY_D_MIN
-        emit_dblocks(J, nn, arrays=not lazy)
-
-        def dv(blk, r, c):
-            """density value: a preloaded block entry, or a load at the use"""
-            if not lazy:
-                nc_ = {"Dab": NB, "Dcd": ND, "Dac": NC, "Dad": ND, "Dbc": NC, "Dbd": ND}[blk]
-                return f"{blk}[{r * nc_ + c}]"
-            row, col = {"Dab": ("ia_", "ib_"), "Dcd": ("ic_", "id_"), "Dac": ("ia_", "ic_"),
-                        "Dad": ("ia_", "id_"), "Dbc": ("ib_", "ic_"), "Dbd": ("ib_", "id_")}[blk]
-            return f"Dm_[(size_t)({row} + {r}) * n_ + {col} + {c}]"
-
-        groups = []
-        k = 0
-        for i in range(a0, a1):
-            for j in range(NB):
-                for kk in range(NC):
-                    for ll in range(ND):
-                        ij, kl, ik, il, jk, jl = (i * NB + j, kk * ND + ll, i * NC + kk, i * ND + ll, j * NC + kk,
-                                                  j * ND + ll)
-                        groups.append((posp[k], [
-                            f"  {{ const double v_ = (double){outp[k]};",
-                            f"    jab[{ij}] += v_ * {dv('Dcd', kk, ll)}; jcd[{kl}] += v_ * {dv('Dab', i, j)};",
-                            f"    kac[{ik}] += v_ * {dv('Dbd', j, ll)}; kad[{il}] += v_ * {dv('Dbc', j, kk)};",
-                            f"    kbc[{jk}] += v_ * {dv('Dad', i, ll)}; kbd[{jl}] += v_ * {dv('Dac', i, kk)}; }}"]))
-                        k += 1
-        J += ["  " + x if not x.startswith("  ") else x for x in interleave(hp.lines, groups)]
-        J.append("}")
-        # J/K epilogue: 6 fused multiply-adds per integral
-        jks.append(("\n".join(J), (a0, a1), core_flops(Lt, vp.nflop, hp.nflop) + 12 * k))
-    return "\n".join(L), jks, stats
+    # K form: the integrals of all primitives are summed as [e0|f0], then
+    # transferred and contracted with the density blocks one by one
+    K = [f"template <typename R>\n__device__ __forceinline__ void qx_kb_e{nm}_0(const QxArgs& A_, int P1, int P2, int s_, int ns_, "
+         f"const double (&Dac)[{NA * NC}], const double (&Dad)[{NA * ND}], const double (&Dbc)[{NB * NC}], "
+         f"const double (&Dbd)[{NB * ND}], double (&kac)[{NA * NC}], double (&kad)[{NA * ND}], "
+         f"double (&kbc)[{NB * NC}], double (&kbd)[{NB * ND}]) {{"]
+    names = {ac: f"s_{ac[0][0]}{ac[0][1]}{ac[0][2]}_{ac[1][0]}{ac[1][1]}{ac[1][2]}" for ac in sorted(vn)}
+    K += [f"  R {x}(0);" for x in names.values()]
+    K.append("  const int v1_ = A_.pr.pp_first[P1], v2_ = A_.pr.pp_first[P2], n2_ = A_.pr.pp_n[P2];")
+    K.append("  for (int k_ = s_; k_ < A_.pr.pp_n[P1] * n2_; k_ += ns_) {")
+    K.append("  const int u1 = v1_ + k_ / n2_, u2 = v2_ + k_ % n2_;")
+    body = []
+    emit_setup(body, Lt, False)
+    transfer = [x for x in body if x.startswith("  const R ABx") or x.startswith("  const R CDx")]
+    body = [x for x in body if x not in transfer]
+    emit_vrr_consts(body, v.lines)
+    body += ["  " + x for x in v.lines]
+    body += [f"  {names[ac]} += {vn[ac]};" for ac in sorted(vn)]
+    K += ["  " + x for x in body] + ["  }"] + transfer
+    groups = []
+    for k in range(N):
+        i, rem = divmod(k, NB * NC * ND)
+        j, rem = divmod(rem, NC * ND)
+        kk, ll = divmod(rem, ND)
+        ik, il, jk, jl = i * NC + kk, i * ND + ll, j * NC + kk, j * ND + ll
+        groups.append((pos[k], [
+            f"  {{ const double v_ = qx_value({outs[k]});",
+            f"    kac[{ik}] += v_ * Dbd[{jl}]; kad[{il}] += v_ * Dbc[{jk}];",
+            f"    kbc[{jk}] += v_ * Dad[{il}]; kbd[{jl}] += v_ * Dac[{ik}]; }}"]))
+    K += ["  " + x if not x.startswith("  ") else x for x in interleave(h.lines, groups)]
+    K.append("}")
+    # K epilogue: 4 fused multiply-adds per integral
+    return "\n".join(L), ["\n".join(K)], dict(stats, jk_flops=[core_flops(Lt, v.nflop, h.nflop) + 8 * N])
 
 
 def emit_deriv_core(l, pi, part):
-    """Two bodies per derivative part: qx_core_d* writes every derivative
-    block to an array (tensor scatter), qx_gr_d* contracts each derivative
-    integral with the density pair product as soon as it is formed (the
-    adjoint gradient), so no derivative block is ever held whole."""
+    """One derivative part: qx_gr_d* contracts each derivative integral with
+    the density pair product as soon as it is formed (the adjoint gradient),
+    so no derivative block is ever held whole."""
     la, lb, lc, ld = l
     nn = (ncart(la), ncart(lb), ncart(lc), ncart(ld))
     NA, NB, NC_, ND = nn
@@ -592,24 +512,6 @@ def emit_deriv_core(l, pi, part):
                             ti += 1
                         exprs.append(f"w{cn} * {up}" + (f" - R({n}) * {dn}" if dn else ""))
                     elems.append((e, le, last, exprs))
-    # array form: dv holds only this part's elements (local index le)
-    NEL = len(elems)
-    L = []
-    _head(L, f"qx_core_d{nm}_{pi}", f", R (&dv)[{NC * NEL}]", Lt, v, vn)
-    L += wdecl
-    groups = [(last, [f"  dv[{ci * NEL + le}] = {ex};" for ci, ex in enumerate(exprs)])
-              for (e, le, last, exprs) in elems]
-    L += ["  " + x if not x.startswith("  ") else x for x in interleave(h.lines, groups)]
-    L.append("}")
-    # tangent array form: the derivative part of each dual value, i.e. the
-    # second derivative along A_.e.tv
-    Tn = []
-    _head(Tn, f"qx_core_t{nm}_{pi}", f", double (&dv)[{NC * NEL}]", Lt, v, vn, tangent=True)
-    Tn += wdecl
-    groups = [(last, [f"  dv[{ci * NEL + le}] = qx_tan({ex});" for ci, ex in enumerate(exprs)])
-              for (e, le, last, exprs) in elems]
-    Tn += ["  " + x if not x.startswith("  ") else x for x in interleave(h.lines, groups)]
-    Tn.append("}")
     # streaming adjoint form
     G = []
     _head(G, f"qx_gr_d{nm}_{pi}", f", double (&g)[{NC}]", Lt, v, vn)
@@ -634,96 +536,58 @@ def emit_deriv_core(l, pi, part):
     stats = dict(part=pi, a=part["a"], b=part["b"], c=(c0, c1), dinv=dinv, vrr=len(v.lines), vrr_flops=v.nflop,
                  hrr=len(h.lines), hrr_flops=h.nflop, L=Lt, N=N, nel=nel, ncomb=NC,
                  flops=core_flops(Lt, v.nflop, h.nflop) + nel * (8 + 5 * NC))
-    return "\n".join(L), "\n".join(G), "\n".join(Tn), stats, (cmask, xmask, dinv, NC, a0, a1, b0, b1, c0, c1)
+    return "\n".join(G), stats, (cmask, xmask, dinv, NC)
 
 
-def core_flops(L, vrr_flops, hrr_flops):
-    """Algorithmic FP operations of one primitive-quartet body (mul and add
-    count 1, fused multiply-add 2): 30 for the pair/quartet setup, 12 + 4L
-    for the Boys function (Taylor step plus downward recursion), then the
-    recurrences as emitted."""
-    return 30 + 12 + 4 * L + vrr_flops + hrr_flops
+def herm(L):
+    """Hermite indices t + u + v <= L, v fastest (qx_herm's order)."""
+    return [(t, u, v) for t in range(L + 1) for u in range(L + 1 - t) for v in range(L + 1 - t - u)]
 
 
-def canonical_classes(lmax):
-    pairs = [(a, b) for a in range(lmax + 1) for b in range(a + 1)]
+def emit_j(L1, outdir, lmax, fp32):
+    """jeng_<L1>.hip: the J kernel of bra pairs of total angular momentum L1:
+    per ket order L2 a body that runs the Hermite Coulomb recursion
+    R^n_{t+1} = t R^{n+1}_{t-1} + X R^{n+1}_t and contracts it with the ket's
+    Hermite density."""
     out = []
-    for i, (la, lb) in enumerate(pairs):
-        for j, (lc, ld) in enumerate(pairs):
-            if j <= i:
-                out.append((la, lb, lc, ld))
-    return pairs, out
+    for L2 in range(2 * lmax + 1):
+        L = L1 + L2
+        H1, H2 = herm(L1), herm(L2)
+        S = [f"template <typename G, typename R>\n__device__ __forceinline__ void qx_jc_{L1}{L2}(R X, R Y, R Z, "
+             f"const R (&b)[{L + 1}], const G (&h)[{len(H2)}], G (&j)[{len(H1)}]) {{"]
+        memo = {}
 
+        def r(t, n):
+            if (t, n) in memo:
+                return memo[(t, n)]
+            if tot(t) == 0:
+                name = f"b[{n}]"
+            else:
+                i = first_axis(t)
+                t1 = inc(t, i, -1)
+                ex = f"{'XYZ'[i]} * {r(t1, n + 1)}"
+                if t1[i] > 0:
+                    ex += f" + R({t1[i]}) * {r(inc(t1, i, -1), n + 1)}"
+                name = f"r{len(memo)}"
+                S.append(f"  const R {name} = {ex};")
+            memo[(t, n)] = name
+            return name
 
-# most derivative parts one adjoint-gradient launch (and source file) covers.
-# Grouping several parts under blockIdx.y would fill the GPU for classes with
-# few quartets, but hipcc's time on such a file grows far faster than the
-# number of parts (12 (dd|dd) parts: 24 minutes inlined, 12 minutes as
-# separate functions, against ~7 s per part alone), so every part keeps its
-# own kernel (the launch table and ABI still speak of groups of one).
-GROUP_PARTS = 1
-
-
-def part_groups(nparts):
-    """Contiguous, nearly equal groups of at most GROUP_PARTS parts."""
-    ng = -(-nparts // GROUP_PARTS)
-    return [list(range(i * nparts // ng, (i + 1) * nparts // ng)) for i in range(ng)]
-
-
-def emit_class_files(cls, outdir, fp32):
-    """Writes, per class: cls_<l>_e.hip (array-form ERI kernel),
-    cls_<l>_j<k>.hip (streaming J/K kernel per range of a), per derivative part
-    cls_<l>_d<k>.hip (array form) and cls_<l>_t<k>.hip (tangent array form,
-    second derivatives) and, per group of parts, cls_<l>_g<k>.hip
-    (streaming adjoint kernel, blockIdx.y = part within the group)."""
-    la, lb, lc, ld = cls
-    nm = "".join(map(str, cls))
-    dims = f"{ncart(la)}, {ncart(lb)}, {ncart(lc)}, {ncart(ld)}"
-    N = ncart(la) * ncart(lb) * ncart(lc) * ncart(ld)
-    files, stats = [], []
-
-    def write(name, body):
-        path = os.path.join(outdir, name)
-        with open(path, "w") as fh:
-            fh.write("\n".join(['#include "../qx_device.h"', ""] + body + [""]))
-        files.append(path)
-
-    src_e, jks, st = emit_eri_core(cls)
-    write(f"cls_{nm}_e.hip", [src_e, "", f"QX_DEFINE_ERI_KERNEL(e{nm}, {N}, {dims})"])
-    for pi, (src_j, (a0, a1), _) in enumerate(jks):
-        write(f"cls_{nm}_j{pi}.hip", [src_j, "", f"QX_DEFINE_JK_KERNEL(e{nm}_{pi}, {dims}, {1 if fp32 else 0}, "
-                                                  f"{a0}, {a1})"])
-    st["jk_flops"] = [f for _, _, f in jks]
-    stats.append((cls, "eri", st))
-    parts = deriv_parts(cls)
-    gsrc = []
-    for pi, part in enumerate(parts):
-        src_d, src_g, _, st, (cmask, xmask, dinv, NC, a0, a1, b0, b1, c0, c1) = emit_deriv_core(cls, pi, part)
-        assert (cmask, xmask, dinv, NC) == (7, 7, True, 9)
-        args = f"{N}, {dims}, {cmask}, {xmask}, {1 if dinv else 0}, {NC}"
-        write(f"cls_{nm}_d{pi}.hip", [src_d, "", f"QX_DEFINE_DERI_KERNEL(d{nm}_{pi}, {args}, {a0}, {a1}, {b0}, {b1}, "
-                                                  f"{c0}, {c1})"])
-        gsrc.append(src_g)
-        stats.append((cls, f"deriv{pi}", st))
-    tparts = tangent_parts(cls)
-    for pi, part in enumerate(tparts):
-        _, _, src_t, _, (cmask, xmask, dinv, NC, a0, a1, b0, b1, c0, c1) = emit_deriv_core(cls, pi, part)
-        args = f"{N}, {dims}, {cmask}, {xmask}, {1 if dinv else 0}, {NC}"
-        write(f"cls_{nm}_t{pi}.hip", [src_t, "", f"QX_DEFINE_DERT_KERNEL(t{nm}_{pi}, {args}, {a0}, {a1}, {b0}, {b1}, "
-                                                  f"{c0}, {c1})"])
-    groups = part_groups(len(parts))
-    for gi, members in enumerate(groups):
-        (pi,) = members
-        w = deriv_waves(cls)
-        attr = f" __attribute__((amdgpu_waves_per_eu({w}, {w})))" if w > 0 else ""
-        kern = ["template <typename R>",
-                f"__global__ __launch_bounds__(QX_BLOCK_MAX){attr} void qx_kg_d{nm}_g{gi}(QxArgs A_) {{",
-                "  __shared__ double sg[QX_GRAD_LDS];",
-                "  qx_grad_body(A_, sg, [&](int P1, int P2, int u1, int u2, double (&g)[QX_GRAD_NCOMB]) {",
-                f"    qx_gr_d{nm}_{pi}<R>(A_, P1, P2, u1, u2, g);", "  });", "}",
-                f"QX_DEFINE_GRAD_LAUNCHER(d{nm}_g{gi}, {len(members)}, {1 if fp32 else 0})"]
-        write(f"cls_{nm}_g{gi}.hip", [gsrc[pi] for pi in members] + [""] + kern)
-    return files, stats, len(parts), groups, len(tparts)
+        for k, tau in enumerate(H2):
+            for m, t in enumerate(H1):
+                s = tuple(x + y for x, y in zip(t, tau))
+                v = r(s, 0)
+                if not v.startswith("b") and (s, "g") not in memo:
+                    memo[(s, "g")] = v
+                S.append(f"  j[{m}] += h[{k}] * G({v});")
+        S.append("}")
+        out += S + [""]
+    cases = " ".join(f"QX_J_CASE({L1}, {L2})" for L2 in range(2 * lmax + 1))
+    out.append(f"QX_DEFINE_J_KERNEL({L1}, {1 if fp32 else 0}, {cases})")
+    path = os.path.join(outdir, f"jeng_{L1}.hip")
+    with open(path, "w") as fh:
+        fh.write("\n".join(['#include "../qx_jk.h"', ""] + out + [""]))
+    return path
 
 
 def emit_oei(la, lb, outdir):
@@ -808,16 +672,181 @@ def emit_oei(la, lb, outdir):
     return path
 
 
+# Rys tables: must agree with qx_rys.h
+RYS_TMAX, RYS_DEG, RYS_MAXN = 72, 12, 6
+
+
+def rys_tables():
+    """Roots and weights of exp(-T t^2) on [0, 1] in u = t^2, per order N <=
+    RYS_MAXN and unit interval of T: degree-RYS_DEG polynomials in x in [-1, 1]
+    (interpolation at Chebyshev nodes, monomial coefficients), then the
+    half-range Hermite values that T scales for T >= RYS_TMAX.  The orthogonal
+    polynomials come from Stieltjes' procedure on a 96-point Gauss-Legendre
+    rule (Gautschi 1982), in long double throughout."""
+    import numpy as np
+    LD = np.longdouble
+    one = LD(1)
+
+    def legendre(n):
+        x = np.polynomial.legendre.leggauss(n)[0].astype(LD)
+        for last in (0, 0, 0, 1):
+            p0, p1 = np.ones_like(x), x.copy()
+            for k in range(2, n + 1):
+                p0, p1 = p1, ((2 * k - 1) * x * p1 - (k - 1) * p0) / k
+            d = n * (x * p1 - p0) / (x * x - one)
+            if not last:
+                x = x - p1 / d
+        return (x + one) / 2, one / ((one - x * x) * d * d)
+
+    def gauss(u, w, N):
+        """N-point Gauss rule of the discrete measure (u, w)."""
+        a, b, nrm = [], [w.sum()], w.sum()
+        pm, p = np.zeros_like(u), np.ones_like(u)
+        for k in range(N):
+            a.append((w * u * p * p).sum() / nrm)
+            pm, p = p, (u - a[k]) * p - (b[k] * pm if k else 0)
+            n2 = (w * p * p).sum()
+            b.append(n2 / nrm)
+            nrm = n2
+        s = np.sqrt(np.array(b[1:N], float))
+        r = np.linalg.eigvalsh(np.diag(np.array(a, float)) + np.diag(s, 1) + np.diag(s, -1)).astype(LD)
+        for last in (0, 0, 0, 1):
+            p0, p1 = np.zeros_like(r), np.ones_like(r)
+            d0, d1 = np.zeros_like(r), np.zeros_like(r)
+            S, nr = np.zeros_like(r), b[0]
+            for k in range(N):
+                S = S + p1 * p1 / nr
+                nr = nr * b[k + 1]
+                p0, p1, d0, d1 = (p1, (r - a[k]) * p1 - (b[k] * p0 if k else 0),
+                                  d1, p1 + (r - a[k]) * d1 - (b[k] * d0 if k else 0))
+            if not last:
+                r = r - p1 / d1
+        return np.concatenate([r, one / S])
+
+    X, W = legendre(96)
+    n = RYS_DEG + 1
+    pi = LD("3.14159265358979323846264338327950288")
+    th = (np.arange(n).astype(LD) + LD("0.5")) * pi / n
+    # interpolation matrix: node values -> Chebyshev -> monomial coefficients
+    cheb = np.array([[(one if j == 0 else LD(2)) / n * np.cos(j * t) for t in th] for j in range(n)])
+    mono = np.zeros((n, n), LD)
+    mono[0, 0] = mono[1, 1] = one
+    for j in range(2, n):
+        mono[j, 1:] = 2 * mono[j - 1, :-1]
+        mono[j] -= mono[j - 2]
+    M = mono.T @ cheb
+    out = []
+    for N in range(1, RYS_MAXN + 1):
+        for iv in range(RYS_TMAX):
+            F = np.array([gauss(X * X, W * np.exp(-(iv + (np.cos(t) + one) / 2) * X * X), N) for t in th])
+            out += [(M @ F[:, f]) for f in range(2 * N)]
+        # half-range Hermite: x^2 of exp(-x^2) on [0, inf) by mapping [0, 9]
+        x, w = legendre(160)
+        g = gauss((9 * x) ** 2, 9 * w * np.exp(-(9 * x) ** 2), N)
+        out.append(g)
+    flat = [v for c in out for v in c]
+    return "// generated: Rys roots and weights\n" + ",\n".join(
+        ", ".join(repr(float(v)) for v in flat[i:i + 8]) for i in range(0, len(flat), 8)) + "\n"
+
+
+def core_flops(L, vrr_flops, hrr_flops):
+    """Algorithmic FP operations of one primitive-quartet body (mul and add
+    count 1, fused multiply-add 2): 30 for the pair/quartet setup, 12 + 4L
+    for the Boys function (Taylor step plus downward recursion), then the
+    recurrences as emitted."""
+    return 30 + 12 + 4 * L + vrr_flops + hrr_flops
+
+
+def canonical_classes(lmax):
+    pairs = [(a, b) for a in range(lmax + 1) for b in range(a + 1)]
+    out = []
+    for i, (la, lb) in enumerate(pairs):
+        for j, (lc, ld) in enumerate(pairs):
+            if j <= i:
+                out.append((la, lb, lc, ld))
+    return pairs, out
+
+
+# most derivative parts one adjoint-gradient launch (and source file) covers.
+# Grouping several parts under blockIdx.y would fill the GPU for classes with
+# few quartets, but hipcc's time on such a file grows far faster than the
+# number of parts (12 (dd|dd) parts: 24 minutes inlined, 12 minutes as
+# separate functions, against ~7 s per part alone), so every part keeps its
+# own kernel (the launch table and ABI still speak of groups of one).
+GROUP_PARTS = 1
+
+
+def part_groups(nparts):
+    """Contiguous, nearly equal groups of at most GROUP_PARTS parts."""
+    ng = -(-nparts // GROUP_PARTS)
+    return [list(range(i * nparts // ng, (i + 1) * nparts // ng)) for i in range(ng)]
+
+
+def emit_class_files(cls, outdir, fp32):
+    """Writes, per class: cls_<l>_e.hip (array-form ERI kernel), cls_<l>_j0.hip
+    (K), cls_<l>_r0.hip (integrals into the pair matrix by quadrature, heavy
+    classes), cls_<l>_d0.hip (derivative slices), cls_<l>_v0.hip (directional
+    derivatives of K and of the adjoint gradient) and cls_<l>_g<k>.hip (adjoint
+    gradient: one kernel by quadrature, or one per derivative part)."""
+    la, lb, lc, ld = cls
+    nm = "".join(map(str, cls))
+    dims = f"{ncart(la)}, {ncart(lb)}, {ncart(lc)}, {ncart(ld)}"
+    N = ncart(la) * ncart(lb) * ncart(lc) * ncart(ld)
+    files, stats = [], []
+
+    def write(name, body, header="qx_device.h"):
+        path = os.path.join(outdir, name)
+        with open(path, "w") as fh:
+            fh.write("\n".join([f'#include "../{header}"', ""] + body + [""]))
+        files.append(path)
+
+    src_e, jks, st = emit_eri_core(cls)
+    write(f"cls_{nm}_e.hip", [src_e, "", f"QX_DEFINE_ERI_KERNEL(e{nm}, {N}, {dims})"], "qx_pairm.h")
+    if nm in RYS_K:
+        write(f"cls_{nm}_j0.hip", [f"QX_DEFINE_RYS_K(e{nm}_0, {la}, {lb}, {lc}, {ld}, {1 if fp32 else 0})"], "qx_rys.h")
+    else:
+        write(f"cls_{nm}_j0.hip", [jks[0], "", f"QX_DEFINE_K_KERNEL(e{nm}_0, {dims}, {1 if fp32 else 0})"], "qx_jk.h")
+    stats.append((cls, "eri", st))
+    if nm in RYS_E:
+        write(f"cls_{nm}_r0.hip", [f"QX_DEFINE_RYS_E(e{nm}, {la}, {lb}, {lc}, {ld})"], "qx_rys.h")
+    write(f"cls_{nm}_d0.hip", [f"QX_DEFINE_RYS_D(d{nm}, {la}, {lb}, {lc}, {ld})"], "qx_rys.h")
+    write(f"cls_{nm}_v0.hip", [f"QX_DEFINE_RYS_KV(e{nm}, {la}, {lb}, {lc}, {ld})",
+                               f"QX_DEFINE_RYS_H(d{nm}, {la}, {lb}, {lc}, {ld})"], "qx_rys.h")
+    parts = deriv_parts(cls)
+    gsrc = []
+    for pi, part in enumerate(parts):
+        src_g, st, (cmask, xmask, dinv, NC) = emit_deriv_core(cls, pi, part)
+        assert (cmask, xmask, dinv, NC) == (7, 7, True, 9)
+        gsrc.append(src_g)
+        stats.append((cls, f"deriv{pi}", st))
+    if nm in RYS_G:  # one kernel for the whole class
+        groups = [list(range(len(parts)))]
+        write(f"cls_{nm}_g0.hip", [f"QX_DEFINE_RYS_G(d{nm}_g0, {la}, {lb}, {lc}, {ld}, {1 if fp32 else 0})"], "qx_rys.h")
+        return files, stats, len(parts), groups
+    groups = part_groups(len(parts))
+    for gi, members in enumerate(groups):
+        (pi,) = members
+        w = deriv_waves(cls)
+        attr = f" __attribute__((amdgpu_waves_per_eu({w}, {w})))" if w > 0 else ""
+        kern = ["template <typename R>",
+                f"__global__ __launch_bounds__(QX_BLOCK_MAX){attr} void qx_kg_d{nm}_g{gi}(QxArgs A_, QxKList kl) {{",
+                "  __shared__ double sg[QX_GRAD_LDS];",
+                "  qx_grad_block(A_, kl, sg, [&](int P1, int P2, int u1, int u2, double (&g)[QX_GRAD_NCOMB]) {",
+                f"    qx_gr_d{nm}_{pi}<R>(A_, P1, P2, u1, u2, g);", "  });", "}",
+                f"QX_DEFINE_GRAD_LAUNCHER(d{nm}_g{gi}, {1 if fp32 else 0})"]
+        write(f"cls_{nm}_g{gi}.hip", [gsrc[pi] for pi in members] + [""] + kern, "qx_grad.h")
+    return files, stats, len(parts), groups
+
+
 def main():
     outdir = sys.argv[1]
     lmax = int(sys.argv[2]) if len(sys.argv) > 2 else 2
     fp32 = "--no-fp32" not in sys.argv
     os.makedirs(outdir, exist_ok=True)
     _, classes = canonical_classes(lmax)
-    files, allstats, nparts, flops, groups, jkf, ntparts = [], [], {}, {}, {}, {}, {}
+    files, allstats, nparts, flops, groups, jkf = [], [], {}, {}, {}, {}
     for cls in classes:
-        f, s, np_, grp, ntp = emit_class_files(cls, outdir, fp32)
-        ntparts[cls] = ntp
+        f, s, np_, grp = emit_class_files(cls, outdir, fp32)
         files += f
         allstats += s
         nparts[cls] = np_
@@ -826,30 +855,28 @@ def main():
         flops[cls] = (s[0][2]["flops"], [st["flops"] for _, _, st in s[1:]], [st["ncomb"] for _, _, st in s[1:]])
     pairs = [(a, b) for a in range(lmax + 1) for b in range(a + 1)]
     files += [emit_oei(a, b, outdir) for a, b in pairs]
+    files += [emit_j(L, outdir, lmax, fp32) for L in range(2 * lmax + 1)]
+    with open(os.path.join(outdir, "qx_rys.inc"), "w") as fh:
+        fh.write(rys_tables())
     D = ["// generated: kernel launch tables indexed by canonical class id", "#pragma once",
          f"#define QX_GEN_LMAX {lmax}", f"#define QX_NUM_CLASSES {len(classes)}",
          f"#define QX_MAX_DPARTS {max(nparts.values())}",
          f"#define QX_MAX_JKPARTS {max(len(v) for v in jkf.values())}",
          "static_assert(QX_MAX_JKPARTS <= QX_JKPARTS_CAP, \"J/K part table too small\");",
-         "static_assert(QX_MAX_DPARTS <= QX_DPARTS_CAP, \"derivative part table too small\");",
-         f"static_assert({max(ntparts.values())} <= QX_TPARTS_CAP, \"tangent part table too small\");", ""]
+         "static_assert(QX_MAX_DPARTS <= QX_DPARTS_CAP, \"derivative part table too small\");", ""]
     for cls in classes:
         nm = "".join(map(str, cls))
         D.append(f'extern "C" int qx_launch_e{nm}(const QxArgs*, const QxLaunch*);')
         for pi in range(len(jkf[cls])):
             D.append(f'extern "C" int qx_launchj_e{nm}_{pi}(const QxArgs*, const QxLaunch*);')
-        for pi in range(nparts[cls]):
-            D.append(f'extern "C" int qx_launch_d{nm}_{pi}(const QxArgs*, const QxLaunch*);')
-        for pi in range(ntparts[cls]):
-            D.append(f'extern "C" int qx_launcht_t{nm}_{pi}(const QxArgs*, const QxLaunch*);')
+        names = [f"qx_launch_d{nm}", f"qx_launchv_e{nm}", f"qx_launchh_d{nm}"] + ([f"qx_launchr_e{nm}"] if nm in RYS_E else [])
+        D += [f'extern "C" int {x}(const QxArgs*, const QxLaunch*);' for x in names]
         for gi in range(len(groups[cls])):
             D.append(f'extern "C" int qx_launchg_d{nm}_g{gi}(const QxArgs*, const QxLaunch*);')
     D.append("")
     D.append("static const QxClassEntry qx_class_table[QX_NUM_CLASSES] = {")
     for cls in classes:
         nm = "".join(map(str, cls))
-        dl = ", ".join(f"qx_launch_d{nm}_{pi}" for pi in range(nparts[cls]))
-        tl = ", ".join(f"qx_launcht_t{nm}_{pi}" for pi in range(ntparts[cls]))
         gl = ", ".join(f"qx_launchg_d{nm}_g{gi}" for gi in range(len(groups[cls])))
         ef, pf, pc = flops[cls]
         pfs = ", ".join(f"{x:.1f}" for x in pf)
@@ -858,9 +885,10 @@ def main():
         gps = ", ".join(str(len(g)) for g in groups[cls])
         jl = ", ".join(f"qx_launchj_e{nm}_{pi}" for pi in range(len(jkf[cls])))
         jfs = ", ".join(f"{x:.1f}" for x in jkf[cls])
-        D.append(f"  {{{cls[0]}, {cls[1]}, {cls[2]}, {cls[3]}, qx_launch_e{nm}, {len(jkf[cls])}, {{{jl}}}, {{{jfs}}}, "
-                 f"{nparts[cls]}, {{{dl}}}, {ntparts[cls]}, {{{tl}}}, {len(groups[cls])}, {{{gl}}}, {ef:.1f}, {{{pfs}}}, {{{pcs}}}, {{{gfs}}}, "
-                 f"{{{gps}}}}},")
+        re = f"qx_launchr_e{nm}" if nm in RYS_E else "nullptr"
+        D.append(f"  {{{cls[0]}, {cls[1]}, {cls[2]}, {cls[3]}, qx_launch_e{nm}, {re}, qx_launch_d{nm}, qx_launchv_e{nm}, "
+                 f"qx_launchh_d{nm}, {len(jkf[cls])}, {{{jl}}}, {{{jfs}}}, {nparts[cls]}, {len(groups[cls])}, {{{gl}}}, "
+                 f"{ef:.1f}, {{{pfs}}}, {{{pcs}}}, {{{gfs}}}, {{{gps}}}}},")
     D.append("};")
     D.append("// per class: mixed-precision J/K and gradient passes may use FP32")
     D.append("static const unsigned char qx_fp32_default[QX_NUM_CLASSES][2] = {")
@@ -880,6 +908,16 @@ def main():
     for cls in classes:
         D.append(f"  {{{TILES['jk'].get(cls, 128)}, {TILES['grad'].get(cls, 128)}}},")
     D.append("};")
+    D.append("// J kernels per bra pair angular momentum")
+    D += [f'extern "C" int qx_launch_jeng_{L}(const QxArgs*, const QxJList*, int, int, int, hipStream_t);'
+          for L in range(2 * lmax + 1)]
+    D.append(f"static int (*const qx_j_table[{2 * lmax + 1}])(const QxArgs*, const QxJList*, int, int, int, hipStream_t) = {{"
+             + ", ".join(f"qx_launch_jeng_{L}" for L in range(2 * lmax + 1)) + "};")
+    for name, table in (("k", RYS_K), ("g", RYS_G)):
+        D.append(f"// per class: {'K' if name == 'k' else 'the adjoint gradient'} by Rys quadrature")
+        D.append(f"static const unsigned char qx_rys_{name}[QX_NUM_CLASSES] = {{")
+        D.append("  " + ", ".join(str(int("".join(map(str, cls)) in table)) for cls in classes))
+        D.append("};")
     D.append("// one-electron kernels per shell-pair class")
     D += [f'extern "C" int qx_launch_oei_{a}{b}(const QxOei*, int, hipStream_t);' for a, b in pairs]
     D.append(f"static int (*const qx_oei_table[{len(pairs)}])(const QxOei*, int, hipStream_t) = {{"

@@ -13,9 +13,17 @@
 
 namespace {
 
-__global__ void k_fill(double* p, long long n, double v) {
-  for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long long)gridDim.x * blockDim.x)
-    p[i] = v;
+// 16-byte stores where p allows, a few per lane: the 0.43 GB pair matrix of a
+// 112-function tensor takes 0.08 ms (8-byte stores, one per lane: 0.39 ms).
+__global__ __launch_bounds__(256) void k_fill(double* p, long long n, double v) {
+  const long long step = (long long)gridDim.x * blockDim.x, i0 = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+  if ((reinterpret_cast<size_t>(p) & 15) == 0) {
+    double2* q = reinterpret_cast<double2*>(p);
+    for (long long i = i0; i < n / 2; i += step) q[i] = make_double2(v, v);
+    if (i0 == 0 && (n & 1)) p[n - 1] = v;
+  } else {
+    for (long long i = i0; i < n; i += step) p[i] = v;
+  }
 }
 
 // out[i] += sum_c copies[c * n + i]
@@ -27,13 +35,6 @@ __global__ void k_add_copies(const double* copies, int ncopy, int n, double* out
   out[i] += v;
 }
 
-__global__ void k_sym_half(const double* in, double* out, int n) {
-  const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= (long long)n * n) return;
-  const int i = (int)(t / n), j = (int)(t % n);
-  out[t] = 0.5 * (in[(size_t)i * n + j] + in[(size_t)j * n + i]);
-}
-
 // AO function k of shell s: row of the transform block; Cartesian function p
 // of the same shell: column.
 __device__ __forceinline__ double tcoef(const QxShellsDev& sh, int s, int row, int col) {
@@ -43,7 +44,7 @@ __device__ __forceinline__ double tcoef(const QxShellsDev& sh, int s, int row, i
 }
 
 // out[i][j] = sum_{p in shell(i), q in shell(j)} T[i][p] X[p][q] T[j][q]
-__global__ void k_cart_to_ao_mat(QxShellsDev sh, const double* X, double* out) {
+__device__ __forceinline__ void cart_to_ao_at(const QxShellsDev& sh, const double* X, double* out) {
   const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
   const int nb = sh.nbf, nc = sh.ncart;
   if (t >= (long long)nb * nb) return;
@@ -62,7 +63,7 @@ __global__ void k_cart_to_ao_mat(QxShellsDev sh, const double* X, double* out) {
 }
 
 // out[p][q] = sum_{i in shell(p), j in shell(q)} T[i][p] X[i][j] T[j][q]
-__global__ void k_ao_to_cart_mat(QxShellsDev sh, const double* X, double* out) {
+__device__ __forceinline__ void ao_to_cart_at(const QxShellsDev& sh, const double* X, double* out) {
   const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
   const int nb = sh.nbf, nc = sh.ncart;
   if (t >= (long long)nc * nc) return;
@@ -80,26 +81,205 @@ __global__ void k_ao_to_cart_mat(QxShellsDev sh, const double* X, double* out) {
   out[t] = acc;
 }
 
-// out[o][i][r] = sum_{p in shell(i)} T[i][p] in[o][p][r]
-__global__ void k_cart_to_ao_axis(QxShellsDev sh, const double* in, double* out, long long outer, int lin, int lout,
-                                  long long inner) {
-  const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  const long long total = outer * lout * inner;
-  if (t >= total) return;
-  const long long r = t % inner;
-  const long long rest = t / inner;
-  const int i = (int)(rest % lout);
-  const long long o = rest / lout;
-  const int s = sh.ao_shell[i];
-  const int ri = i - sh.bfs[s];
-  const int l = sh.l[s];
-  const int nc = (l + 1) * (l + 2) / 2;
-  double acc = 0.0;
+// Up to three matrices at once (grid row y): the kernels' arithmetic is that of
+// the single forms above.
+struct MatPtrs {
+  const double* in[3];
+  double* out[3];
+};
+__global__ void k_cart_to_ao_mats(QxShellsDev sh, MatPtrs m) { cart_to_ao_at(sh, m.in[blockIdx.y], m.out[blockIdx.y]); }
+__global__ void k_ao_to_cart_mats(QxShellsDev sh, MatPtrs m) { ao_to_cart_at(sh, m.in[blockIdx.y], m.out[blockIdx.y]); }
+
+// ---------------------------------------------------------------- pair matrix
+__global__ void k_fill_int(int* p, long long n, int v) {
+  for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long long)gridDim.x * blockDim.x)
+    p[i] = v;
+}
+
+// One thread per screened shell pair: its function pairs' rows.
+__global__ void k_pairm_index(QxShellsDev sh, QxPairsDev pr, int npairs, QxPairIndex ix, int* index, int* fn) {
+  const int P = blockIdx.x * blockDim.x + threadIdx.x;
+  if (P >= npairs) return;
+  const int la = sh.l[pr.sa[P]], lb = sh.l[pr.sb[P]];
+  const int na = (la + 1) * (la + 2) / 2, nb = (lb + 1) * (lb + 2) / 2, n = sh.ncart;
+  int X = la * (la + 1) / 2 + lb, off = 0;
+  for (int k = 0; k < X; ++k) off += ix.cnt[k];
+  const bool diag = pr.sa[P] == pr.sb[P];  // both orders are components of the block
+  for (int i = 0; i < na; ++i)
+    for (int j = 0; j < nb; ++j) {
+      const int row = ix.base[X] + (i * nb + j) * ix.cnt[X] + (P - off);
+      index[(size_t)(pr.bfa[P] + i) * n + pr.bfb[P] + j] = row;
+      fn[row] = (pr.bfa[P] + i) * n + pr.bfb[P] + j;
+      if (!diag) index[(size_t)(pr.bfb[P] + j) * n + pr.bfa[P] + i] = row;
+    }
+}
+
+// One thread per AO function: its Cartesian terms.
+__global__ void k_ao_terms(QxShellsDev sh, QxAoTerms* ao) {
+  const int r = blockIdx.x * blockDim.x + threadIdx.x;
+  if (r >= sh.nbf) return;
+  const int s = sh.ao_shell[r], l = sh.l[s], nc = (l + 1) * (l + 2) / 2;
+  QxAoTerms t{};
   for (int p = 0; p < nc; ++p) {
-    const double tp = tcoef(sh, s, ri, p);
-    if (tp != 0.0) acc += tp * in[(o * lin + sh.bfc[s] + p) * inner + r];
+    const double c = tcoef(sh, s, r - sh.bfs[s], p);
+    if (c == 0.0 || t.n == 3) continue;
+    t.f[t.n] = sh.bfc[s] + p;
+    t.c[t.n++] = c;
   }
-  out[t] = acc;
+  ao[r] = t;
+}
+
+// Class and pair position of row r.
+__device__ __forceinline__ void pairm_row(const QxPairIndex& ix, int r, int& X, int& pos) {
+  X = 0;
+#pragma unroll
+  for (int k = 1; k < 6; ++k) X = r >= ix.base[k] ? k : X;
+  pos = (r - ix.base[X]) % max(ix.cnt[X], 1);
+}
+
+// The quartet kernels store (row, column) for bra class > ket class, or bra
+// position >= ket position within a class; the other elements are the
+// transposed ones.  A workgroup owns the 64 x 64 tile (tr, tc) and its mirror
+// image, so it reads both before it writes either.  Bound by HBM: half of M
+// read and written.
+#define PM_TILE 64
+#define PM_LDS_MAX (140 * 1024)  // a staged row; the rest of a workgroup's 160 KB holds the term lists
+#define PM_AO_MAX 384            // AO functions whose term lists are kept in LDS
+__global__ __launch_bounds__(256) void k_pairm_sym(double* M, long long ld, long long slice, QxPairIndex ix) {
+  __shared__ double a[PM_TILE][PM_TILE + 1], b[PM_TILE][PM_TILE + 1];
+  M += (long long)blockIdx.y * slice;
+  const long long t = blockIdx.x;
+  int tr = (int)((sqrt(8.0 * (double)t + 1.0) - 1.0) * 0.5);
+  while ((long long)(tr + 1) * (tr + 2) / 2 <= t) ++tr;
+  while ((long long)tr * (tr + 1) / 2 > t) --tr;
+  const int tc = (int)(t - (long long)tr * (tr + 1) / 2);
+  const int r0 = tr * PM_TILE, c0 = tc * PM_TILE;
+  const int lx = threadIdx.x & 63, ly = threadIdx.x >> 6;
+  for (int y = ly; y < PM_TILE; y += 4) {
+    a[y][lx] = r0 + y < ld && c0 + lx < ld ? M[(long long)(r0 + y) * ld + c0 + lx] : 0.0;
+    b[y][lx] = c0 + y < ld && r0 + lx < ld ? M[(long long)(c0 + y) * ld + r0 + lx] : 0.0;
+  }
+  __syncthreads();
+  for (int y = ly; y < PM_TILE; y += 4) {
+    int Xr, Xc, pr, pc;
+    if (r0 + y < ld && c0 + lx < ld) {          // element (r0 + y, c0 + lx)
+      pairm_row(ix, r0 + y, Xr, pr);
+      pairm_row(ix, c0 + lx, Xc, pc);
+      const bool there = Xr > Xc || (Xr == Xc && pr >= pc);
+      if (!there) M[(long long)(r0 + y) * ld + c0 + lx] = b[lx][y];
+    }
+    if (c0 + y < ld && r0 + lx < ld && tr != tc) {  // element (c0 + y, r0 + lx)
+      pairm_row(ix, c0 + y, Xr, pr);
+      pairm_row(ix, r0 + lx, Xc, pc);
+      const bool there = Xr > Xc || (Xr == Xc && pr >= pc);
+      if (!there) M[(long long)(c0 + y) * ld + r0 + lx] = a[lx][y];
+    }
+  }
+}
+
+// The elements of a panel of rows (pairs [i0, i0 + cnt) of class X, ncomp
+// components) to all their places in a Cartesian tensor: eight scattered
+// stores per element, used only when no whole pair matrix fits in memory.
+__global__ void k_pairm_scatter(int nc, const double* M, long long ld, long long slice, QxPairIndex ix, const int* fn,
+                                int X, int ncomp, int i0, int cnt, double* out) {
+  const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+  const int rows = ncomp * cnt, cols = ix.base[X + 1];  // kets of class X and below
+  if (t >= (long long)rows * cols) return;
+  const int pr = (int)(t / cols), col = (int)(t - (long long)pr * cols);
+  int Y, j;
+  pairm_row(ix, col, Y, j);
+  const int k = pr / cnt, i = i0 + (pr - k * cnt);
+  if (Y > X || (Y == X && j > i)) return;
+  const double v = M[(long long)blockIdx.y * slice + (long long)pr * ld + col];
+  const int pq = fn[ix.base[X] + k * ix.cnt[X] + i], rs = fn[col];
+  const size_t n = nc, p = pq / nc, q = pq % nc, r = rs / nc, u = rs % nc;
+  double* o = out + (size_t)blockIdx.y * n * n * n * n;
+  o[((p * n + q) * n + r) * n + u] = v;
+  o[((q * n + p) * n + r) * n + u] = v;
+  o[((p * n + q) * n + u) * n + r] = v;
+  o[((q * n + p) * n + u) * n + r] = v;
+  o[((r * n + u) * n + p) * n + q] = v;
+  o[((u * n + r) * n + p) * n + q] = v;
+  o[((r * n + u) * n + q) * n + p] = v;
+  o[((u * n + r) * n + q) * n + p] = v;
+}
+
+// One workgroup per AO function pair p >= q (and slice): the row of (p, q),
+// transformed to AO on its two bra indices, is staged in LDS (or read in
+// place when it does not fit, STAGE = false), then written to out[p][q] and
+// out[q][p] with the ket transform applied: consecutive lanes write
+// consecutive doubles.  Bound by the tensor's HBM writes.
+template <bool PURE, bool STAGE>
+__global__ __launch_bounds__(256) void k_pairm_expand(int n, int nc, const double* M, long long ld, long long slice,
+                                                      const int* index, const QxAoTerms* ao, double* out) {
+  HIP_DYNAMIC_SHARED(double, row)
+  __shared__ QxAoTerms terms[PURE ? PM_AO_MAX : 1];  // AO terms, where they fit
+  __shared__ long long src[9];
+  __shared__ double coef[9];
+  __shared__ int nsrc;
+  const long long t = blockIdx.x;
+  int p = (int)((sqrt(8.0 * (double)t + 1.0) - 1.0) * 0.5);
+  while ((long long)(p + 1) * (p + 2) / 2 <= t) ++p;
+  while ((long long)p * (p + 1) / 2 > t) --p;
+  const int q = (int)(t - (long long)p * (p + 1) / 2);
+  M += (long long)blockIdx.y * slice;
+  if (threadIdx.x == 0) {
+    int k = 0;
+    if (PURE) {
+      const QxAoTerms tp = ao[p], tq = ao[q];
+      for (int i = 0; i < tp.n; ++i)
+        for (int j = 0; j < tq.n; ++j) {
+          const int r = index[(size_t)tp.f[i] * nc + tq.f[j]];
+          if (r >= 0) { src[k] = r * ld; coef[k++] = tp.c[i] * tq.c[j]; }
+        }
+    } else {
+      const int r = index[(size_t)p * nc + q];
+      if (r >= 0) { src[k] = r * ld; coef[k++] = 1.0; }
+    }
+    nsrc = k;
+  }
+  const bool near = PURE && n <= PM_AO_MAX;
+  if (near)
+    for (int i = threadIdx.x; i < n; i += blockDim.x) terms[i] = ao[i];
+  __syncthreads();
+  const int ns = nsrc;
+  if (STAGE) {
+    for (int c = threadIdx.x; c < ld; c += blockDim.x) {
+      double v = 0.0;
+      for (int k = 0; k < ns; ++k) v += coef[k] * M[src[k] + c];
+      row[c] = v;
+    }
+    __syncthreads();
+  }
+  auto at = [&](int c) -> double {
+    if (c < 0) return 0.0;
+    if (STAGE) return row[c];
+    double v = 0.0;
+    for (int k = 0; k < ns; ++k) v += coef[k] * M[src[k] + c];
+    return v;
+  };
+  const long long nn = (long long)n * n;
+  double* o1 = out + (long long)blockIdx.y * nn * nn + ((long long)p * n + q) * nn;
+  double* o2 = out + (long long)blockIdx.y * nn * nn + ((long long)q * n + p) * nn;
+  for (int i = threadIdx.x; i < nn; i += blockDim.x) {
+    double v;
+    if (PURE) {
+      const int r = i / n, u = i - r * n;
+      const QxAoTerms* tr = near ? &terms[r] : ao + r;
+      const QxAoTerms* tu = near ? &terms[u] : ao + u;
+      const int nr = tr->n, nu = tu->n;
+      v = 0.0;
+      for (int x = 0; x < nr; ++x) {
+        const int* ix = index + (size_t)tr->f[x] * nc;
+        const double cx = tr->c[x];
+        for (int y = 0; y < nu; ++y) v += cx * tu->c[y] * at(ix[tu->f[y]]);
+      }
+    } else {
+      v = at(index[i]);
+    }
+    o1[i] = v;
+    if (p != q) o2[i] = v;
+  }
 }
 
 // ---------------------------------------------------------------- OEI
@@ -330,7 +510,7 @@ extern "C" {
 
 int qxk_fill(double* p, long long n, double v, hipStream_t s) {
   if (n <= 0) return 0;
-  const long long blocks = std::min<long long>((n + 255) / 256, 1 << 20);
+  const long long blocks = std::min<long long>((n + 511) / 512, 8192);
   hipLaunchKernelGGL(k_fill, dim3((unsigned)blocks), dim3(256), 0, s, p, n, v);
   return (int)hipGetLastError();
 }
@@ -341,27 +521,72 @@ int qxk_add_copies(const double* copies, int ncopy, int n, double* out, hipStrea
   return (int)hipGetLastError();
 }
 
-int qxk_sym_half(const double* in, double* out, int n, hipStream_t s) {
-  hipLaunchKernelGGL(k_sym_half, dim3(nblk((long long)n * n, 256)), dim3(256), 0, s, in, out, n);
+int qxk_cart_to_ao_mats(const QxShellsDev* sh, const double* in, size_t stride, double* const* out, int count,
+                        hipStream_t s) {
+  MatPtrs m{};
+  for (int k = 0; k < count; ++k) { m.in[k] = in + k * stride; m.out[k] = out[k]; }
+  hipLaunchKernelGGL(k_cart_to_ao_mats, dim3(nblk((long long)sh->nbf * sh->nbf, 256), (unsigned)count), dim3(256), 0, s,
+                     *sh, m);
+  return (int)hipGetLastError();
+}
+
+int qxk_ao_to_cart_mats(const QxShellsDev* sh, const double* const* in, double* out, size_t stride, int count,
+                        hipStream_t s) {
+  MatPtrs m{};
+  for (int k = 0; k < count; ++k) { m.in[k] = in[k]; m.out[k] = out + k * stride; }
+  hipLaunchKernelGGL(k_ao_to_cart_mats, dim3(nblk((long long)sh->ncart * sh->ncart, 256), (unsigned)count), dim3(256), 0,
+                     s, *sh, m);
   return (int)hipGetLastError();
 }
 
 int qxk_cart_to_ao_mat(const QxShellsDev* sh, const double* in, double* out, hipStream_t s) {
-  hipLaunchKernelGGL(k_cart_to_ao_mat, dim3(nblk((long long)sh->nbf * sh->nbf, 256)), dim3(256), 0, s, *sh, in, out);
-  return (int)hipGetLastError();
+  return qxk_cart_to_ao_mats(sh, in, 0, &out, 1, s);
 }
 
 int qxk_ao_to_cart_mat(const QxShellsDev* sh, const double* in, double* out, hipStream_t s) {
-  hipLaunchKernelGGL(k_ao_to_cart_mat, dim3(nblk((long long)sh->ncart * sh->ncart, 256)), dim3(256), 0, s, *sh, in,
-                     out);
+  return qxk_ao_to_cart_mats(sh, &in, out, 0, 1, s);
+}
+
+int qxk_pairm_tables(const QxShellsDev* sh, const QxPairsDev* pr, int npairs, const QxPairIndex* ix, int* index,
+                     int* fn, QxAoTerms* ao, hipStream_t s) {
+  const long long n2 = (long long)sh->ncart * sh->ncart;
+  hipLaunchKernelGGL(k_fill_int, dim3(std::min(nblk(n2, 256), 4096u)), dim3(256), 0, s, index, n2, -1);
+  if (npairs > 0)
+    hipLaunchKernelGGL(k_pairm_index, dim3(nblk(npairs, 128)), dim3(128), 0, s, *sh, *pr, npairs, *ix, index, fn);
+  if (sh->pure) hipLaunchKernelGGL(k_ao_terms, dim3(nblk(sh->nbf, 128)), dim3(128), 0, s, *sh, ao);
   return (int)hipGetLastError();
 }
 
-int qxk_cart_to_ao_axis(const QxShellsDev* sh, const double* in, double* out, long long outer, int lin, int lout,
-                        long long inner, hipStream_t s) {
-  const long long total = outer * lout * inner;
-  hipLaunchKernelGGL(k_cart_to_ao_axis, dim3(nblk(total, 256)), dim3(256), 0, s, *sh, in, out, outer, lin, lout,
-                     inner);
+int qxk_pairm_sym(double* M, long long ld, long long slice, int nslice, const QxPairIndex* ix, hipStream_t s) {
+  const long long T = (ld + PM_TILE - 1) / PM_TILE, tiles = T * (T + 1) / 2;
+  if (tiles <= 0 || nslice <= 0) return 0;
+  if (tiles > 0x7fffffffLL || nslice > 65535) return (int)hipErrorInvalidValue;
+  hipLaunchKernelGGL(k_pairm_sym, dim3((unsigned)tiles, (unsigned)nslice), dim3(256), 0, s, M, ld, slice, *ix);
+  return (int)hipGetLastError();
+}
+
+int qxk_pairm_scatter(int ncart, const double* M, long long ld, long long slice, int nslice, const QxPairIndex* ix,
+                      const int* fn, int X, int ncomp, int i0, int cnt, double* out, hipStream_t s) {
+  const long long total = (long long)ncomp * cnt * ix->base[X + 1];
+  if (total <= 0 || nslice <= 0) return 0;
+  if ((total + 255) / 256 > 0x7fffffffLL || nslice > 65535) return (int)hipErrorInvalidValue;
+  hipLaunchKernelGGL(k_pairm_scatter, dim3(nblk(total, 256), (unsigned)nslice), dim3(256), 0, s, ncart, M, ld, slice,
+                     *ix, fn, X, ncomp, i0, cnt, out);
+  return (int)hipGetLastError();
+}
+
+int qxk_pairm_expand(const QxShellsDev* sh, const double* M, long long ld, long long slice, int nslice,
+                     const int* index, const QxAoTerms* ao, double* out, hipStream_t s) {
+  const int n = sh->nbf;
+  const dim3 grid((unsigned)((long long)n * (n + 1) / 2), (unsigned)nslice);
+  if (nslice <= 0) return 0;
+  if (nslice > 65535) return (int)hipErrorInvalidValue;
+  const size_t bytes = (size_t)ld * sizeof(double);
+  const bool stage = bytes <= PM_LDS_MAX;
+#define PM_GO(P, S) hipLaunchKernelGGL((k_pairm_expand<P, S>), grid, dim3(256), (S) ? bytes : 0, s, n, sh->ncart, M, ld, slice, index, ao, out)
+  if (sh->pure) { if (stage) PM_GO(true, true); else PM_GO(true, false); }
+  else { if (stage) PM_GO(false, true); else PM_GO(false, false); }
+#undef PM_GO
   return (int)hipGetLastError();
 }
 

@@ -1,0 +1,102 @@
+// Pair-matrix form of the integral and derivative tensors.
+//
+// The (n, n, n, n) tensor holds every integral up to eight times.  Writing
+// those eight places from the lane that computed it costs eight scattered
+// 8-byte stores (atomic ones for derivatives and contracted shells), and the
+// lanes of a wavefront hold kets sorted by Schwarz bound, so no two of them
+// share a cache line.  Instead a quartet's block goes to a matrix M over
+// Cartesian function pairs, M[row of (a, b)][column of (c, d)], whose index is
+//   class base + component * (pairs of the class) + (pair position):
+// consecutive lanes (consecutive ket pairs) write consecutive doubles, each
+// element once and without atomics, also for contracted shells, because one
+// lane sums all primitive quartets of its contracted quartet.  A quarter of
+// the tensor's bytes is written this way; the runtime then mirrors M
+// (qxk_pairm_sym) and expands it row by row into the tensor with coalesced
+// stores, applying the Cartesian -> spherical transform on the way
+// (qxk_pairm_expand).
+#pragma once
+#include "qx_device.h"
+
+struct QxPairM {
+  double* M;                 // slice y starts at M + y * slice
+  long long ld, slice;
+  int row0, rown, rowp;      // bra class: first row, pairs, first sorted pair
+  int col0, coln, colp;      // ket class
+  const long long* prefix;   // running contracted-quartet counts over the bra pairs (nbra + 1)
+  const int* kstart;         // per bra pair: first admissible ket pair (null = 0)
+  int nbra;
+  long long nquart;          // contracted quartets
+  long long t0;              // number of the first one (a panel of bra pairs starts inside the list)
+};
+
+// Contracted quartet t of the list: its bra and ket pairs.
+__device__ __forceinline__ void qx_locate_pairs(const QxPairM& pm, long long t, int& P1, int& P2) {
+  t += pm.t0;
+  int lo = 0, hi = pm.nbra;  // prefix[lo] <= t < prefix[hi]
+  while (hi - lo > 1) {
+    const int mid = (lo + hi) >> 1;
+    if (pm.prefix[mid] <= t) lo = mid; else hi = mid;
+  }
+  P1 = pm.rowp + lo;
+  P2 = pm.colp + (pm.kstart ? pm.kstart[lo] : 0) + (int)(t - pm.prefix[lo]);
+}
+
+template <int NAB, int NCD, typename R>
+__device__ __forceinline__ void qx_pairm_eri(const QxPairM& pm, int P1, int P2, const R (&o)[NAB * NCD]) {
+  double* m = pm.M + (long long)(pm.row0 + P1 - pm.rowp) * pm.ld + pm.col0 + (P2 - pm.colp);
+#pragma unroll
+  for (int ij = 0; ij < NAB; ++ij)
+#pragma unroll
+    for (int kl = 0; kl < NCD; ++kl) m[(long long)ij * pm.rown * pm.ld + (long long)kl * pm.coln] = (double)o[ij * NCD + kl];
+}
+
+// ---- array-form kernels ---------------------------------------------------
+// The integral cores add to their output array, so that a PAIRM launch (one
+// lane per contracted quartet) sums its primitive quartets in place; the
+// other epilogues run one lane per primitive quartet.
+struct QxArrayQuartet {
+  int P1, P2, u1, u2, n1, n2;
+};
+__device__ __forceinline__ bool qx_array_quartet(const QxArgs& A_, const QxPairM& pm, long long t, QxArrayQuartet& q) {
+  if (A_.e.epi == QX_EPI_PAIRM) {
+    if (t >= pm.nquart) return false;
+    qx_locate_pairs(pm, t, q.P1, q.P2);
+    q.u1 = A_.pr.pp_first[q.P1];
+    q.u2 = A_.pr.pp_first[q.P2];
+    q.n1 = A_.pr.pp_n[q.P1];
+    q.n2 = A_.pr.pp_n[q.P2];
+  } else {
+    if (t >= A_.w.nquart) return false;
+    qx_locate(A_, t, q.u1, q.u2, q.P1, q.P2);
+    q.n1 = q.n2 = 1;
+  }
+  return true;
+}
+
+static inline dim3 qx_array_grid(const QxArgs* a, const QxLaunch* L, long long& nq) {
+  nq = a->e.epi == QX_EPI_PAIRM ? (L->pm ? L->pm->nquart : 0) : a->w.nquart;
+  return dim3((unsigned)((nq + QX_BLOCK - 1) / QX_BLOCK));
+}
+
+// Array-form ERI kernel: pair-matrix / store / Schwarz epilogues.
+#define QX_DEFINE_ERI_KERNEL(NAME, N, NA, NB, NC, ND)                                             \
+  __global__ __launch_bounds__(QX_BLOCK) void qx_k_##NAME(QxArgs A_, QxPairM pm) {                \
+    const long long t = (long long)blockIdx.x * QX_BLOCK + threadIdx.x;                          \
+    QxArrayQuartet q;                                                                             \
+    if (!qx_array_quartet(A_, pm, t, q)) return;                                                  \
+    if (A_.e.skip_single && qx_single_atom(A_, q.P1, q.P2)) return;                               \
+    double o[N] = {};                                                                             \
+    for (int i = 0; i < q.n1; ++i)                                                                \
+      for (int j = 0; j < q.n2; ++j) qx_core_##NAME<double>(A_, q.P1, q.P2, q.u1 + i, q.u2 + j, o); \
+    if (A_.e.epi == QX_EPI_PAIRM) qx_pairm_eri<NA * NB, NC * ND, double>(pm, q.P1, q.P2, o);      \
+    else qx_epi_eri<NA, NB, NC, ND, double>(A_, t, q.P1, q.P2, o, true);                          \
+  }                                                                                               \
+  extern "C" int qx_launch_##NAME(const QxArgs* a, const QxLaunch* L) {                           \
+    long long nq;                                                                                 \
+    const dim3 grid = qx_array_grid(a, L, nq);                                                    \
+    if (nq <= 0) return 0;                                                                        \
+    if (L->fp32 || a->e.epi == QX_EPI_JK) return -1;                                              \
+    const QxPairM pm = L->pm ? *L->pm : QxPairM{};                                                \
+    hipLaunchKernelGGL(qx_k_##NAME, grid, dim3(QX_BLOCK), 0, L->stream, *a, pm);                  \
+    return (int)hipGetLastError();                                                                \
+  }

@@ -7,6 +7,8 @@
 #include <vector>
 
 #include "qx_device.h"
+#include "qx_jk.h"
+#include "qx_pairm.h"
 
 #define QX_LMAX_SUPPORTED 2
 
@@ -33,6 +35,18 @@ struct QxWorkHost {
   int bra_class, ket_class;
   QxWorkDev w;             // device view (prefix/kstart point into ctx buffers)
   long long prefix_off;    // offset of this list's prefix in ctx->d_prefix
+  // the same list over contracted pairs: running counts per bra pair in
+  // ctx->d_cprefix and (fragmented contexts) first kets in ctx->d_ckstart
+  long long cprefix_off;
+  long long ncq;           // contracted quartets
+  int maxket;              // most kets of one bra pair
+};
+
+// Row/column index of the pair matrix (qx_pairm.h): pair class X holds
+// rows base[X] + component * cnt[X] + (pair position in X).
+struct QxPairIndex {
+  int base[7];
+  int cnt[6];
 };
 
 #define QX_NUM_CLASSES_MAX 21  // canonical classes with l <= 2
@@ -75,9 +89,25 @@ struct qx_ctx {
   std::vector<QxWorkHost> work;
   long long* d_prefix = nullptr;
   int* d_kstart = nullptr;               // per bra pseudo pair, fragmented contexts only
+  long long* d_cprefix = nullptr;        // running contracted quartet counts per bra pair of every list
+  int* d_ckstart = nullptr;              // per bra pair (d_cprefix's offsets), fragmented contexts only
+  // J kernels: admissible pseudo kets of every pair in every class, the
+  // Hermite densities and potentials (value and derivative parts: 4 arrays of
+  // nherm doubles) and their layout; Rys tables of the K kernels
+  QxRange* d_range = nullptr;
+  QxJList jlist{};
+  double* d_herm = nullptr;
+  long long nherm = 0;
+  double* d_rys = nullptr;
+  // pair-matrix workspace of the tensor entry points, kept up to
+  // QX_PAIRM_KEEP bytes; passes that use it are ordered like those on ws
+  double* pairm = nullptr;
+  size_t pairm_bytes = 0;
+  size_t pairm_limit = 0;                // most bytes of pair matrices per pass (0: what the device has)
   // host copies of the list arrays (quartet -> pair maps for callers that
   // read the stored integrals) and of the pseudo pair -> pair map
   std::vector<long long> h_prefix;
+  std::vector<long long> h_cprefix;
   std::vector<int> h_kstart;             // per bra pseudo pair of every list
   std::vector<long long> h_kstart_off;   // per list: offset into h_kstart
   std::vector<int> h_ppair;
@@ -139,6 +169,7 @@ struct qx_ctx {
   // fragmented contexts: first Cartesian function of each fragment id's range
   // and the widest range (the width of the J/K kernels' LDS K' rows)
   int* d_frag_col0 = nullptr;
+  int* d_frag_atoms = nullptr;           // lowest atom and window width of each fragment id
   int kcols = 0;
   // mixed precision: per class and pass (0 J/K, 1 gradient) whether quartets
   // below the threshold run in FP32 (classes whose FP32 kernels are faster)
@@ -148,10 +179,10 @@ struct qx_ctx {
   // are its first nk64 kets)
   struct Split {
     double thr = -1.0;
-    std::vector<QxWorkHost> wm;          // c->work with w.nk64 set
     std::vector<long long> pq64, pq32;   // per list: pseudo-pair quartets above / below thr
     std::vector<long long> cq64, cq32;   // per list: contracted quartets above / below thr
-    int* d_nk64 = nullptr;
+    int* d_ck64 = nullptr;               // FP64 kets per contracted bra pair (ctx->d_cprefix's offsets)
+    int* d_range64 = nullptr;            // FP64 part of each J range (ctx->d_range's layout)
   } split;
 };
 
@@ -164,15 +195,46 @@ struct qx_ctx {
 #define QX_SLOT_JK(c, k, f32) (QX_SLOT_JK0 + ((f32) * QX_NUM_CLASSES_MAX + (c)) * QX_JKPARTS_CAP + (k))
 #define QX_PROFILE_SLOTS (QX_SLOT_JK0 + 2 * QX_NUM_CLASSES_MAX * QX_JKPARTS_CAP)
 
+// J/K pass set-up and finish (qx_jk.hip)
+extern "C" {
+const double* qxk_rys_host(void);
+int qxk_jk_begin(const QxArgs* a, const QxJList* jl, long long nherm, double* J, double* K, long long n2,
+                 hipStream_t s);
+int qxk_j_finish(const QxArgs* a, const QxJList* jl, double* J, hipStream_t s);
+int qxk_jk_finish(const QxShellsDev* sh, const double* Jc, const double* Kp, double* J, double* K, hipStream_t s);
+}
+
+// An AO function as its Cartesian terms (one for s, p and Cartesian d; up to
+// three for a spherical d function).
+struct QxAoTerms {
+  int n, f[3];
+  double c[3];
+};
+
 // helper kernels (qx_kernels.hip)
 extern "C" {
 int qxk_fill(double* p, long long n, double v, hipStream_t s);
-int qxk_sym_half(const double* in, double* out, int n, hipStream_t s);    // out = (in + in^T)/2
 int qxk_add_copies(const double* copies, int ncopy, int n, double* out, hipStream_t s);  // out += sum of copies
 int qxk_cart_to_ao_mat(const QxShellsDev* sh, const double* in, double* out, hipStream_t s);   // T X T^T
 int qxk_ao_to_cart_mat(const QxShellsDev* sh, const double* in, double* out, hipStream_t s);   // T^T X T
-int qxk_cart_to_ao_axis(const QxShellsDev* sh, const double* in, double* out, long long outer, int axis_len_in,
-                        int axis_len_out, long long inner, hipStream_t s);
+// the same for up to three matrices in one launch; the Cartesian ones lie `stride` doubles apart
+int qxk_cart_to_ao_mats(const QxShellsDev* sh, const double* in, size_t stride, double* const* out, int count,
+                        hipStream_t s);
+int qxk_ao_to_cart_mats(const QxShellsDev* sh, const double* const* in, double* out, size_t stride, int count,
+                        hipStream_t s);
+// Pair matrix M (nslice matrices of ld x ld, `slice` doubles apart) -> tensor.
+// index: Cartesian function pair -> row (ncart^2 ints, -1 = screened out), fn:
+// row -> p * ncart + q, ao: per AO function up to three Cartesian terms
+// (qxk_pairm_tables fills them).
+int qxk_pairm_tables(const QxShellsDev* sh, const QxPairsDev* pr, int npairs, const QxPairIndex* ix, int* index,
+                     int* fn, QxAoTerms* ao, hipStream_t s);
+// every permutation of the elements of a panel of rows into a zeroed
+// Cartesian tensor: panel row k * cnt + i is component k of the class's pair
+// i0 + i (class X, ncomp components)
+int qxk_pairm_scatter(int ncart, const double* M, long long ld, long long slice, int nslice, const QxPairIndex* ix,
+                      const int* fn, int X, int ncomp, int i0, int cnt, double* out, hipStream_t s);
+int qxk_pairm_sym(double* M, long long ld, long long slice, int nslice, const QxPairIndex* ix, hipStream_t s);
+int qxk_pairm_expand(const QxShellsDev* sh, const double* M, long long ld, long long slice, int nslice,
+                     const int* index, const QxAoTerms* ao, double* out, hipStream_t s);
 int qxk_oei_deriv(const QxShellsDev* sh, double* dS, double* dT, double* dV, hipStream_t s);
-// grad += Pd . d/dtv d(T+V)/dR + Wd . d/dtv dS/dR (Cartesian Pd, Wd)
 }

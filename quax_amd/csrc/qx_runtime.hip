@@ -18,8 +18,9 @@
 #include <vector>
 
 #include "quax_amd.h"
-#include "qx_runtime.h"
 #include "qx_oei.h"
+#include "qx_runtime.h"
+#include "qx_rys.h"
 #include "qx_classes.inc"  // generated; in the build's generated-source directory
 
 static_assert(QX_GEN_LMAX == QX_LMAX_SUPPORTED, "generated kernels and runtime disagree on lmax");
@@ -67,6 +68,7 @@ T* dupload(qx_ctx* c, const std::vector<T>& v) {
 // scoped temporary device buffer
 struct DevBuf {
   void* p = nullptr;
+  explicit DevBuf(void* owned) : p(owned) {}
   explicit DevBuf(size_t bytes) { QX_HIP(hipMalloc(&p, std::max<size_t>(bytes, 8))); }
   ~DevBuf() { if (p) (void)hipFree(p); }
   double* d() const { return static_cast<double*>(p); }
@@ -211,12 +213,14 @@ int timed_launch(qx_ctx* c, int slot, long long pq, hipStream_t s, F&& launch) {
 }
 
 int launch_eri(qx_ctx* c, const QxWorkDev& w, int cls, const QxEpiDev& e, int fp32, hipStream_t s,
-               const QxPairsDev& pr, const QxPrimPairsDev& pp) {
+               const QxPairsDev& pr, const QxPrimPairsDev& pp, const QxPairM* pm = nullptr,
+               const QxKList* kl = nullptr) {
   QxArgs a;
   a.pr = pr; a.pp = pp; a.w = w; a.e = e; a.boys = c->d_boys;
-  QxLaunch L{fp32, s};
+  QxLaunch L{fp32, s, 0, pm, kl};
   const QxClassEntry& ent = qx_class_table[cls];
-  return timed_launch(c, QX_SLOT_ERI(cls, fp32 ? 1 : 0), w.nquart, s, [&] { return ent.eri(&a, &L); });
+  auto fn = kl && ent.rys_eri ? ent.rys_eri : ent.eri;
+  return timed_launch(c, QX_SLOT_ERI(cls, fp32 ? 1 : 0), w.nquart, s, [&] { return fn(&a, &L); });
 }
 
 // One kernel launch of a pass, with its estimated cost (flops).
@@ -248,15 +252,12 @@ void check_launch(int rc, const char* what);
 // With profiling on, each kernel's HIP events sit on the stream it runs on:
 // concurrent kernels are timed in place (one stream times each alone).
 //
-// side = false keeps the pass on the caller's stream.  The passes whose
-// kernels need more than ~6 KB of scratch per lane (derivative and
-// second-derivative tensors, the tangent kernels: up to 8.3 KB) run there:
-// each hardware queue grows its own scratch to the largest per-lane size it
-// has run, and growing a side stream's queue past ~8 KB per lane after the
-// process already holds scratch on its other queues has been refused by the
-// HSA runtime (HSA_STATUS_ERROR_OUT_OF_RESOURCES).  The caller's queue has
-// already run the largest kernels, the array-form ones of context set-up.
-// The streaming J/K and adjoint-gradient kernels stay under 6 KB per lane.
+// side = false keeps the pass on the caller's stream (callers that may not use
+// events or other streams).  Scratch: each hardware queue grows its own to the
+// largest per-lane size it has run, and growing a side stream's queue past
+// ~8 KB per lane once the process holds scratch on its other queues has been
+// refused by the HSA runtime (HSA_STATUS_ERROR_OUT_OF_RESOURCES); the build
+// keeps every kernel that runs here under 6 KB.
 void run_launches(qx_ctx* c, std::vector<Launch>& v, hipStream_t s, const char* what, bool side) {
   const int ns = side ? std::max(1, std::min<int>(c->nstreams, (int)v.size())) : 1;
   if (ns == 1) {
@@ -310,8 +311,9 @@ void frag_segment(const qx_ctx* c, int ko, int kn, int f, int& ss, int& se) {
 
 // Admissible kets of bra pair i (position in class X) in class Y: positions
 // [ss, ss + kc) of Y's list, i.e. the bra's fragment, Q_i Q_j >= bound (a
-// prefix of the descending segment) and canonical j <= i when X == Y.
-void ket_window(const qx_ctx* c, int X, int Y, int i, double bound, int& ss, int& kc) {
+// prefix of the descending segment) and, if asked for, canonical j <= i when
+// X == Y.
+void ket_window(const qx_ctx* c, int X, int Y, int i, double bound, int& ss, int& kc, bool canonical = true) {
   const int bo = c->class_pair_off[X], ko = c->class_pair_off[Y], kn = c->class_pair_cnt[Y];
   int se;
   frag_segment(c, ko, kn, c->h_pair_frag[bo + i], ss, se);
@@ -322,7 +324,51 @@ void ket_window(const qx_ctx* c, int X, int Y, int i, double bound, int& ss, int
     if (Qi * c->h_pair_Q[ko + mid] >= bound) lo = mid + 1; else hi = mid;
   }
   kc = lo - ss;
-  if (X == Y) kc = std::max(0, std::min(kc, i - ss + 1));
+  if (X == Y && canonical) kc = std::max(0, std::min(kc, i - ss + 1));
+}
+
+// Pseudo kets of class Y that bra pair P (any order of the two classes) meets
+// with Q_P Q_ket >= bound: the J kernels' ranges.
+QxRange pseudo_range(const qx_ctx* c, int P, int Y, double bound) {
+  const int X = c->h_pair_class[P], ko = c->class_pair_off[Y];
+  if (c->class_pair_cnt[Y] == 0) return {0, 0};
+  int ss, kc;
+  ket_window(c, X, Y, P - c->class_pair_off[X], bound, ss, kc, false);
+  if (kc <= 0) return {0, 0};
+  const int last = ko + ss + kc - 1;
+  return {c->h_pp_first[ko + ss], c->h_pp_first[last] + c->h_pp_n[last] - c->h_pp_first[ko + ss]};
+}
+
+// Hermite layout, J ranges and Rys tables.
+void setup_jk(qx_ctx* c) {
+  static const int order[6] = {0, 1, 2, 2, 3, 4};
+  QxJList& jl = c->jlist;
+  jl.npairs = c->npairs;
+  long long at = 0;
+  int u = 0;
+  for (int X = 0; X < 6; ++X) {
+    const int cnt = c->class_pair_cnt[X], off = c->class_pair_off[X];
+    const int nu = cnt ? c->h_pp_first[off + cnt - 1] + c->h_pp_n[off + cnt - 1] - c->h_pp_first[off] : 0;
+    jl.uoff[X] = u;
+    jl.hoff[X] = (int)at;
+    u += nu;
+    at += (long long)nu * qx_nherm(order[X]);
+  }
+  jl.uoff[6] = u;
+  QX_REQUIRE(at <= 0x7fffffff, QX_EUNSUPPORTED, "too many primitive pairs");
+  c->nherm = at;
+  std::vector<QxRange> r((size_t)6 * c->npairs);
+  for (int Y = 0; Y < 6; ++Y)
+    for (int P = 0; P < c->npairs; ++P) r[(size_t)Y * c->npairs + P] = pseudo_range(c, P, Y, c->tol * c->tol);
+  c->d_range = dupload(c, r);
+  c->d_herm = dalloc<double>(c, (size_t)4 * at);
+  c->d_rys = dalloc<double>(c, QX_RYS_DOUBLES);
+  QX_HIP(hipMemcpy(c->d_rys, qxk_rys_host(), QX_RYS_DOUBLES * sizeof(double), hipMemcpyHostToDevice));
+  jl.range = c->d_range;
+  jl.H = c->d_herm;
+  jl.P = c->d_herm + at;
+  jl.Hd = c->d_herm + 2 * at;
+  jl.Pd = c->d_herm + 3 * at;
 }
 
 void schwarz_and_lists(qx_ctx* c) {
@@ -445,6 +491,8 @@ void schwarz_and_lists(qx_ctx* c) {
     }
   std::vector<long long> allpre;
   std::vector<int> allkst;  // per bra pseudo pair: first ket (fragmented contexts)
+  std::vector<long long> allcpre;  // the same over contracted pairs
+  std::vector<int> allckst;
   std::vector<long long> kst_off;
   c->nquart_total = 0; c->npq_total = 0; c->store_total = 0;
   for (int X = 0; X < nclass; ++X) {
@@ -459,6 +507,8 @@ void schwarz_and_lists(qx_ctx* c) {
       wh.cls = class_index(X, Y);
       wh.bra_class = X; wh.ket_class = Y;
       wh.prefix_off = (long long)allpre.size();
+      wh.cprefix_off = (long long)allcpre.size();
+      allcpre.push_back(0);
       const int u0 = c->h_pp_first[bo];
       const int u1 = c->h_pp_first[bo + bn - 1] + c->h_pp_n[bo + bn - 1];
       allpre.push_back(0);
@@ -470,6 +520,9 @@ void schwarz_and_lists(qx_ctx* c) {
         int ss, kc;
         ket_window(c, X, Y, i, tol2, ss, kc);
         ncq += kc;
+        wh.maxket = std::max(wh.maxket, kc);
+        allcpre.push_back(ncq);
+        allckst.push_back(ss);
         {
           const int P = bo + i;
           const int A = c->atom[c->h_pair_sa[P]];
@@ -492,6 +545,8 @@ void schwarz_and_lists(qx_ctx* c) {
       wh.w.nket = (int)kcum[kn];
       wh.w.nquart = run;
       wh.w.diag = 0;
+      wh.ncq = ncq;
+      allckst.push_back(0);  // one entry per prefix entry
       wh.w.store_base = c->store_total;
       const int N = ncart(c->l[c->h_pair_sa[bo]]) * ncart(c->l[c->h_pair_sb[bo]]) *
                     ncart(c->l[c->h_pair_sa[ko]]) * ncart(c->l[c->h_pair_sb[ko]]);
@@ -503,14 +558,18 @@ void schwarz_and_lists(qx_ctx* c) {
         c->work.push_back(wh);
       } else {
         allpre.resize(wh.prefix_off);
+        allcpre.resize(wh.cprefix_off);
+        allckst.resize(wh.cprefix_off);
         allkst.resize(kst_off.back());
         kst_off.pop_back();
       }
     }
   }
   c->d_prefix = dupload(c, allpre);
+  c->d_cprefix = dupload(c, allcpre);
   if (c->fragmented) {
     c->d_kstart = dupload(c, allkst);
+    c->d_ckstart = dupload(c, allckst);
     c->d_pair_frag = dupload(c, c->h_pair_frag);
     // Cartesian function range of each fragment id (all kets of a bra pair
     // lie in its fragment, so a block's K' rows span at most this range)
@@ -528,8 +587,18 @@ void schwarz_and_lists(qx_ctx* c) {
       else c->kcols = std::max(c->kcols, hi[f] - lo[f]);
     }
     c->d_frag_col0 = dupload(c, lo);
+    // atom window of each fragment id: lowest atom, atoms up to the highest
+    std::vector<int> win(2 * (fmax + 1), 0);
+    for (int f = 0; f <= fmax; ++f) {
+      int a0 = c->natom, a1 = -1;
+      for (int at = 0; at < c->natom; ++at)
+        if (c->frag[at] == f) { a0 = std::min(a0, at); a1 = at; }
+      if (a1 >= 0) { win[2 * f] = a0; win[2 * f + 1] = a1 - a0 + 1; }
+    }
+    c->d_frag_atoms = dupload(c, win);
   }
   c->h_prefix = allpre;
+  c->h_cprefix = allcpre;
   c->h_kstart = allkst;
   c->h_kstart_off = kst_off;
   c->h_ppair.assign(c->npseudo, 0);
@@ -587,26 +656,24 @@ void end_ws(qx_ctx* c, hipStream_t s) {
 }
 
 // Mixed precision: for every quartet list, the number of FP64 kets of each
-// bra row at a Schwarz-bound threshold.  Kets of each bra pair are sorted by
+// bra pair at a Schwarz-bound threshold.  Kets of each bra pair are sorted by
 // descending Q, so for bra i the FP64 kets (Q_i Q_j >= thr^2) are a prefix of
-// its admissible kets; a masked launch (w.sel) then runs either part of the
-// unchanged list, keeping its block -> bra-row layout.
+// its admissible kets; a launch then takes either part of every row (kl.sel).
 void build_split(qx_ctx* c, double thr) {
   auto& S = c->split;
   if (S.thr == thr) return;
   QX_HIP(hipDeviceSynchronize());  // no kernel may still read the old counts
-  if (S.d_nk64) (void)hipFree(S.d_nk64);
+  for (int* p : {S.d_ck64, S.d_range64})
+    if (p) (void)hipFree(p);
   S = qx_ctx::Split{};
   const double tol2 = c->tol * c->tol, thr2 = thr * thr;
-  std::vector<int> nk;                 // per list, per bra row
-  std::vector<size_t> off;
+  std::vector<int> ck(c->h_cprefix.size(), 0);  // per list, per bra pair
   for (const auto& wh : c->work) {
     const int X = wh.bra_class, Y = wh.ket_class;
     const int bo = c->class_pair_off[X], bn = c->class_pair_cnt[X];
     const int ko = c->class_pair_off[Y], kn = c->class_pair_cnt[Y];
     std::vector<long long> kcum(kn + 1, 0);
     for (int j = 0; j < kn; ++j) kcum[j + 1] = kcum[j] + c->h_pp_n[ko + j];
-    off.push_back(nk.size());
     long long p64 = 0, p32 = 0, q64 = 0, q32 = 0;
     for (int i = 0; i < bn; ++i) {
       int ss, kc, ss2, k64;
@@ -615,23 +682,25 @@ void build_split(qx_ctx* c, double thr) {
       k64 = std::min(kc, k64);
       q64 += k64;
       q32 += kc - k64;
+      ck[wh.cprefix_off + i] = k64;
       const long long r64 = kcum[ss + k64] - kcum[ss], rall = kcum[ss + kc] - kcum[ss];
       for (int k = 0; k < c->h_pp_n[bo + i]; ++k) {
-        nk.push_back((int)r64);
         p64 += r64;
         p32 += rall - r64;
       }
     }
-    if ((long long)(nk.size() - off.back()) != wh.w.nbra)
-      throw QxError{QX_EHIP, "mixed-precision rows do not match the quartet list"};
     if (p64 + p32 != wh.w.nquart) throw QxError{QX_EHIP, "mixed-precision split lost quartets"};
     S.pq64.push_back(p64); S.pq32.push_back(p32);
     S.cq64.push_back(q64); S.cq32.push_back(q32);
   }
-  QX_HIP(hipMalloc(&S.d_nk64, std::max<size_t>(nk.size(), 1) * sizeof(int)));
-  if (!nk.empty()) QX_HIP(hipMemcpy(S.d_nk64, nk.data(), nk.size() * sizeof(int), hipMemcpyHostToDevice));
-  S.wm = c->work;
-  for (size_t i = 0; i < S.wm.size(); ++i) S.wm[i].w.nk64 = S.d_nk64 + off[i];
+  std::vector<int> r64((size_t)6 * c->npairs);
+  for (int Y = 0; Y < 6; ++Y)
+    for (int P = 0; P < c->npairs; ++P)
+      r64[(size_t)Y * c->npairs + P] = std::min(pseudo_range(c, P, Y, thr2).count, pseudo_range(c, P, Y, tol2).count);
+  QX_HIP(hipMalloc(&S.d_ck64, std::max<size_t>(ck.size(), 1) * sizeof(int)));
+  if (!ck.empty()) QX_HIP(hipMemcpy(S.d_ck64, ck.data(), ck.size() * sizeof(int), hipMemcpyHostToDevice));
+  QX_HIP(hipMalloc(&S.d_range64, std::max<size_t>(r64.size(), 1) * sizeof(int)));
+  if (!r64.empty()) QX_HIP(hipMemcpy(S.d_range64, r64.data(), r64.size() * sizeof(int), hipMemcpyHostToDevice));
   S.thr = thr;
 }
 
@@ -833,6 +902,7 @@ static void init_body(qx_ctx* c, int natom, const double* xyz_bohr, const double
     c->d_boys = dupload(c, boys_table());
     setup_shell_tables(c);
     schwarz_and_lists(c);
+    setup_jk(c);
     QX_HIP(hipDeviceSynchronize());
   }
 }
@@ -866,7 +936,9 @@ int qx_finalize(qx_ctx* c) {
   for (auto t : c->side) (void)hipStreamDestroy(t);
   for (auto e : c->fork_ev) (void)hipEventDestroy(e);
   if (c->ws_ev) (void)hipEventDestroy(c->ws_ev);
-  if (c->split.d_nk64) (void)hipFree(c->split.d_nk64);
+  for (int* p : {c->split.d_ck64, c->split.d_range64})
+    if (p) (void)hipFree(p);
+  if (c->pairm) (void)hipFree(c->pairm);
   for (void* p : c->allocs) (void)hipFree(p);
   delete c;
   return QX_OK;
@@ -927,93 +999,287 @@ long long qx_generate_multi_index_lookup(int nparams, int order, int* out, long 
   return count;
 }
 
-static void ao_tensor4_from_cart(qx_ctx* c, const double* cart, double* out, long long outer_slices, hipStream_t s) {
-  // four successive index transforms, Cartesian -> AO, per slice
-  const long long nc = c->ncart, nb = c->nbf;
-  DevBuf t1((size_t)outer_slices * nb * nc * nc * nc * sizeof(double));
-  DevBuf t2((size_t)outer_slices * nb * nb * nc * nc * sizeof(double));
-  check_launch(qxk_cart_to_ao_axis(&c->shells, cart, t1.d(), outer_slices, (int)nc, (int)nb, nc * nc * nc, s), "sph");
-  check_launch(qxk_cart_to_ao_axis(&c->shells, t1.d(), t2.d(), outer_slices * nb, (int)nc, (int)nb, nc * nc, s), "sph");
-  check_launch(qxk_cart_to_ao_axis(&c->shells, t2.d(), t1.d(), outer_slices * nb * nb, (int)nc, (int)nb, nc, s), "sph");
-  check_launch(qxk_cart_to_ao_axis(&c->shells, t1.d(), out, outer_slices * nb * nb * nb, (int)nc, (int)nb, 1, s), "sph");
-  QX_HIP(hipStreamSynchronize(s));
+// Workspace of one tensor pass: nslice pair matrices (or panels of one), the
+// index tables and the AO terms.  Up to QX_PAIRM_KEEP bytes stay with the
+// context, larger ones are allocated for the call.
+#define QX_PAIRM_KEEP ((size_t)1 << 30)
+#define QX_PAIRM_PANEL ((size_t)64 << 20)
+static const int kPairComps[6] = {1, 3, 9, 6, 18, 36};  // ss, ps, pp, ds, dp, dd
+
+struct PairMatrix {
+  QxPairIndex ix{};
+  long long ld = 0, slice = 0;
+  int nslice = 0;            // slices per pass; 0: M is one panel of `panel` rows
+  long long panel = 0;
+  double* M = nullptr;
+  int* index = nullptr;
+  int* fn = nullptr;
+  QxAoTerms* ao = nullptr;
+  std::unique_ptr<DevBuf> own;
+};
+
+// `bytes` of workspace, or null when the device has no room.
+static void* pairm_room(qx_ctx* c, PairMatrix& m, size_t bytes) {
+  void* p = nullptr;
+  if (bytes <= c->pairm_bytes) return c->pairm;
+  if (hipMalloc(&p, bytes) != hipSuccess) {
+    (void)hipGetLastError();
+    return nullptr;
+  }
+  if (bytes <= QX_PAIRM_KEEP) {
+    if (c->pairm) QX_HIP(hipFree(c->pairm));  // waits for passes that still read it
+    c->pairm = static_cast<double*>(p);
+    c->pairm_bytes = bytes;
+  } else {
+    m.own.reset(new DevBuf(p));
+  }
+  return p;
+}
+
+// Sets m up on stream s for up to `want` slices at a time: all of them where
+// the device (or pairm_limit) has room, else fewer, else row panels.
+static void begin_pairm(qx_ctx* c, PairMatrix& m, int want, hipStream_t s) {
+  int at = 0;
+  for (int X = 0; X < 6; ++X) {
+    m.ix.base[X] = at;
+    m.ix.cnt[X] = c->class_pair_cnt[X];
+    at += kPairComps[X] * c->class_pair_cnt[X];
+  }
+  m.ix.base[6] = at;
+  m.ld = std::max((at + 7) & ~7, 8);  // rows start on a 64-byte line
+  m.slice = m.ld * m.ld;
+  auto pad = [](size_t b) { return (b + 63) / 64 * 64; };
+  const size_t bi = pad((size_t)c->ncart * c->ncart * sizeof(int)), bf = pad((size_t)m.ld * sizeof(int));
+  const size_t tables = bi + bf + (size_t)c->nbf * sizeof(QxAoTerms);
+  void* p = nullptr;
+  size_t data = 0;
+  for (m.nslice = want; m.nslice >= 1 && !p; m.nslice = m.nslice > 1 ? (m.nslice + 1) / 2 : 0) {
+    data = (size_t)m.nslice * m.slice * sizeof(double);
+    if (c->pairm_limit && data > c->pairm_limit) continue;
+    if ((p = pairm_room(c, m, data + tables))) break;
+  }
+  if (!p) {
+    // panels scatter every element to its eight places, which needs no
+    // transform; a spherical tensor has always needed more room than this
+    if (c->pure) throw QxError{QX_ENOMEM, "no device memory for the pair matrix of a spherical tensor"};
+    m.nslice = 0;
+    m.panel = std::max<long long>(36, (long long)(QX_PAIRM_PANEL / (want * m.ld * sizeof(double))));
+    m.slice = m.panel * m.ld;
+    data = (size_t)want * m.slice * sizeof(double);
+    if (!(p = pairm_room(c, m, data + tables))) throw QxError{QX_ENOMEM, "no device memory for a tensor panel"};
+  }
+  m.M = static_cast<double*>(p);
+  char* q = static_cast<char*>(p) + data;
+  m.index = reinterpret_cast<int*>(q);
+  m.fn = reinterpret_cast<int*>(q + bi);
+  m.ao = reinterpret_cast<QxAoTerms*>(q + bi + bf);
+  (void)begin_ws(c, s);  // orders this pass after the previous user of the context's workspaces
+  check_launch(qxk_pairm_tables(&c->shells, &c->pr, c->npairs, &m.ix, m.index, m.fn, m.ao, s), "pair tables");
+}
+
+// Kets of one bra pair that a workgroup takes: enough workgroups to fill the
+// device a few times over, at least a few passes of the workgroup's lanes
+// each, since every workgroup clears, fills and flushes its rows once.
+#define QX_K_BLOCKS 4096
+#define QX_SUB_LANES 65536  // lanes below which contracted quartets are shared between lanes
+
+// The contracted list wh for a kernel of one lane per quartet in blocks of
+// `block` threads, or (block = 0) of the quadrature kernels.
+static QxKList k_list(const qx_ctx* c, const QxWorkHost& wh, int sel, int block) {
+  QxKList kl{};
+  kl.bra0 = c->class_pair_off[wh.bra_class]; kl.ket0 = c->class_pair_off[wh.ket_class];
+  kl.prefix = c->d_cprefix + wh.cprefix_off;
+  kl.kstart = c->fragmented ? c->d_ckstart + wh.cprefix_off : nullptr;
+  kl.n64 = c->split.d_ck64 ? c->split.d_ck64 + wh.cprefix_off : nullptr;
+  kl.sel = sel;
+  kl.nbra = c->class_pair_cnt[wh.bra_class];
+  kl.maxket = wh.maxket;
+  kl.nquart = wh.ncq;
+  kl.rys = c->d_rys;
+  kl.frag_atoms = c->d_frag_atoms;
+  // few contracted quartets: their primitive quartets are shared between up
+  // to 64 lanes, so that a small molecule still spreads over the device
+  const long long prims = (wh.w.nquart + wh.ncq - 1) / std::max(wh.ncq, 1LL);
+  kl.sub = (int)std::max<long long>(1, std::min<long long>({prims, 64, QX_SUB_LANES / std::max(wh.ncq, 1LL)}));
+  const long long per = std::max<long long>((wh.ncq + QX_K_BLOCKS - 1) / QX_K_BLOCKS, 1);
+  const int unit = block ? std::max(1, block / kl.sub) : 32;
+  kl.chunk = (int)std::min<long long>((per + unit - 1) / unit * unit, 1 << 20);
+  return kl;
+}
+
+// The contracted list wh with its place in M.
+static QxPairM pairm_list(const qx_ctx* c, const PairMatrix& m, const QxWorkHost& wh) {
+  QxPairM pm{};
+  const int X = wh.bra_class, Y = wh.ket_class;
+  pm.M = m.M; pm.ld = m.ld; pm.slice = m.slice;
+  pm.row0 = m.ix.base[X]; pm.rown = m.ix.cnt[X]; pm.rowp = c->class_pair_off[X];
+  pm.col0 = m.ix.base[Y]; pm.coln = m.ix.cnt[Y]; pm.colp = c->class_pair_off[Y];
+  pm.prefix = c->d_cprefix + wh.cprefix_off;
+  pm.kstart = c->fragmented ? c->d_ckstart + wh.cprefix_off : nullptr;
+  pm.nbra = c->class_pair_cnt[X];
+  pm.nquart = wh.ncq;
+  return pm;
+}
+
+// The same panel of a list for the quadrature kernels.
+static QxKList pairm_kets(const qx_ctx* c, const QxWorkHost& wh, const QxPairM& pm) {
+  QxKList kl = k_list(c, wh, 0, 0);
+  kl.bra0 = pm.rowp;
+  kl.prefix = pm.prefix;
+  kl.kstart = pm.kstart;
+  kl.nbra = pm.nbra;
+  kl.nquart = pm.nquart;
+  return kl;
+}
+
+// Evaluates the lists into nslice tensors at out: `launch(list, pm)` is one
+// list's kernel.  Whole matrices are mirrored and expanded; panels are
+// scattered.
+static void run_pairm(qx_ctx* c, PairMatrix& m, int nslice, double* out, hipStream_t s,
+                      const std::function<Launch(const QxWorkHost&, const QxPairM&)>& launch) {
+  std::vector<Launch> v;
+  if (m.nslice > 0) {
+    check_launch(qxk_fill(m.M, nslice * m.slice, 0.0, s), "fill");
+    for (const auto& wh : c->work) v.push_back(launch(wh, pairm_list(c, m, wh)));
+    run_launches(c, v, s, "pair matrix", true);
+    check_launch(qxk_pairm_sym(m.M, m.ld, m.slice, nslice, &m.ix, s), "pair mirror");
+    check_launch(qxk_pairm_expand(&c->shells, m.M, m.ld, m.slice, nslice, m.index, m.ao, out, s), "pair expand");
+    return;
+  }
+  const size_t nc = c->ncart, n4 = nc * nc * nc * nc;
+  check_launch(qxk_fill(out, (long long)(nslice * n4), 0.0, s), "fill");
+  for (int X = 0; X < 6; ++X) {
+    const int comps = kPairComps[X], step = (int)std::max<long long>(1, m.panel / comps);
+    for (int i0 = 0; i0 < m.ix.cnt[X]; i0 += step) {
+      const int cnt = std::min(step, m.ix.cnt[X] - i0);
+      check_launch(qxk_fill(m.M, nslice * m.slice, 0.0, s), "fill");
+      for (const auto& wh : c->work) {
+        if (wh.bra_class != X) continue;
+        QxPairM pm = pairm_list(c, m, wh);
+        const long long* pre = c->h_cprefix.data() + wh.cprefix_off;
+        pm.row0 = 0; pm.rown = cnt; pm.rowp += i0;
+        pm.prefix += i0;
+        if (pm.kstart) pm.kstart += i0;
+        pm.nbra = cnt;
+        pm.t0 = pre[i0];
+        pm.nquart = pre[i0 + cnt] - pre[i0];
+        v.push_back(launch(wh, pm));
+      }
+      run_launches(c, v, s, "pair matrix", false);
+      v.clear();
+      check_launch(qxk_pairm_scatter((int)nc, m.M, m.ld, m.slice, nslice, &m.ix, m.fn, X, comps, i0, cnt, out, s),
+                   "pair scatter");
+    }
+  }
+}
+
+static void end_pairm(qx_ctx* c, PairMatrix& m, hipStream_t s) {
+  end_ws(c, s);
+  if (m.own) QX_HIP(hipStreamSynchronize(s));  // freed on return
+}
+
+// The integral tensor (skip_single: single-atom quartets left out).
+static void eri_tensor(qx_ctx* c, int skip_single, double* out, hipStream_t s) {
+  PairMatrix m;
+  begin_pairm(c, m, 1, s);
+  QxEpiDev e{};
+  e.epi = QX_EPI_PAIRM; e.nbf = c->ncart; e.natom = c->natom; e.coord = -1; e.skip_single = skip_single;
+  run_pairm(c, m, 1, out, s, [&](const QxWorkHost& wh, const QxPairM& pm) {
+    const QxKList kl = pairm_kets(c, wh, pm);
+    return Launch{(double)pm.nquart * qx_class_table[wh.cls].eri_flops, [=](hipStream_t st) {
+                    return launch_eri(c, wh.w, wh.cls, e, 0, st, c->pr, c->pp, &pm, &kl);
+                  }};
+  });
+  end_pairm(c, m, s);
 }
 
 int qx_compute_2e_int(qx_ctx* c, double* out, void* stream) {
   if (!c || !out) return QX_EINVAL;
   return guarded(c, [&]() -> int {
     QX_HIP(hipSetDevice(c->device));
-    hipStream_t s = (hipStream_t)stream;
-    const size_t nc = c->ncart;
-    const size_t n4 = nc * nc * nc * nc;
-    DevBuf* tmp = c->pure ? new DevBuf(n4 * sizeof(double)) : nullptr;
-    std::unique_ptr<DevBuf> guard(tmp);
-    double* dst = c->pure ? tmp->d() : out;
-    check_launch(qxk_fill(dst, (long long)n4, 0.0, s), "fill");
-    QxEpiDev e{};
-    e.epi = QX_EPI_FULL; e.atomic = c->k1 ? 0 : 1; e.nbf = (int)nc; e.natom = c->natom; e.coord = -1; e.out = dst;
-    for (auto& wh : c->work) check_launch(launch_eri(c, wh.w, wh.cls, e, 0, s, c->pr, c->pp), "compute_2e_int");
-    if (c->pure) ao_tensor4_from_cart(c, dst, out, 1, s);
+    eri_tensor(c, 0, out, (hipStream_t)stream);
     return QX_OK;
   });
 }
 
-// Derivative kernels (every part) of one quartet list; sel / nq: the masked
-// part of the list the launch evaluates and its pseudo-pair quartet count.
-static void add_deriv_list(qx_ctx* c, const QxWorkHost& wh, const QxEpiDev& e, int fp32, int sel, long long nq,
-                           std::vector<Launch>& out) {
-  if (wh.w.nquart <= 0 || nq <= 0) return;
+// Adjoint-gradient kernels (every group of parts) of one quartet list; sel /
+// nq: the part of the list the launch evaluates and its pseudo-pair quartet
+// count.  dir: along tv instead.
+static void add_grad_list(qx_ctx* c, const QxWorkHost& wh, const QxEpiDev& e, int fp32, int sel, long long nq, bool dir,
+                          std::vector<Launch>& out) {
+  if (wh.ncq <= 0 || nq <= 0) return;
   const QxClassEntry& ent = qx_class_table[wh.cls];
-  // adjoint gradient: one launch per group of parts; tensor: one per part
-  const bool grad = e.epi == QX_EPI_GRAD;
-  const int nl = grad ? ent.ngroups : ent.nparts;
+  const int block = c->tile[1][wh.cls];
+  const QxKList kl = k_list(c, wh, sel, dir || qx_rys_g[wh.cls] ? 0 : block);
+  const int nl = dir ? 1 : ent.ngroups;
   for (int k = 0; k < nl; ++k) {
     QxArgs a;
     a.pr = c->pr; a.pp = c->pp; a.w = wh.w; a.e = e; a.boys = c->d_boys;
-    a.w.sel = sel;
-    if (grad) {
-      a.e.grad_wred = c->gwred[wh.cls];
-      a.e.grad_copies = std::min(std::max(c->gcopy[wh.cls], 1), a.e.grad_copies);
-    }
+    a.e.grad_wred = c->gwred[wh.cls];
+    a.e.grad_copies = std::min(std::max(c->gcopy[wh.cls], 1), a.e.grad_copies);
     const int slot = QX_SLOT_DERIV(wh.cls, k, fp32 ? 1 : 0);
-    auto fn = grad ? ent.grad[k] : ent.deri[k];
-    const double fl = grad ? ent.group_flops[k] : ent.part_flops[k];
-    const int block = grad ? c->tile[1][wh.cls] : 0;
-    out.push_back({(double)nq * fl, [c, a, fn, fp32, slot, nq, block](hipStream_t st) {
-                     QxLaunch L{fp32, st, block};
+    auto fn = dir ? ent.hess : ent.grad[k];
+    const double fl = dir ? 3.0 * ent.part_flops[0] * ent.nparts : ent.group_flops[k];
+    out.push_back({(double)nq * fl, [c, a, fn, fp32, slot, nq, block, kl, dir](hipStream_t st) {
+                     QxLaunch L{fp32, st, block, nullptr, &kl};
+                     if (dir) return fn(&a, &L);
                      return timed_launch(c, slot, nq, st, [&] { return fn(&a, &L); });
                    }});
   }
 }
 
-// J/K kernels (every part) of one quartet list, as add_deriv_list.
-static void add_jk_list(qx_ctx* c, const QxWorkHost& wh, const QxEpiDev& e, int fp32, int sel, long long nq,
-                        std::vector<Launch>& out) {
-  if (wh.w.nquart <= 0 || nq <= 0) return;
+// K kernel of one quartet list, as add_grad_list.
+static void add_k_list(qx_ctx* c, const QxWorkHost& wh, const QxEpiDev& e, int fp32, int sel, long long nq, bool dir,
+                       std::vector<Launch>& out) {
+  if (wh.ncq <= 0 || nq <= 0) return;
   const QxClassEntry& ent = qx_class_table[wh.cls];
-  for (int k = 0; k < ent.njk; ++k) {
+  const int block = c->tile[0][wh.cls];
+  const QxKList kl = k_list(c, wh, sel, dir || qx_rys_k[wh.cls] ? 0 : block);
+  const int nl = dir ? 1 : ent.njk;
+  for (int k = 0; k < nl; ++k) {
     QxArgs a;
     a.pr = c->pr; a.pp = c->pp; a.w = wh.w; a.e = e; a.boys = c->d_boys;
-    a.w.sel = sel;
     a.e.krows = e.krows && c->jkrows[wh.cls];
     const int slot = QX_SLOT_JK(wh.cls, k, fp32 ? 1 : 0);
-    auto fn = ent.jk[k];
-    const int block = c->tile[0][wh.cls];
-    out.push_back({(double)nq * ent.jk_flops[k], [c, a, fn, fp32, slot, nq, block](hipStream_t st) {
-                     QxLaunch L{fp32, st, block};
+    auto fn = dir ? ent.jkv : ent.jk[k];
+    out.push_back({(double)nq * ent.jk_flops[k], [c, a, fn, fp32, slot, nq, block, kl, dir](hipStream_t st) {
+                     QxLaunch L{fp32, st, block, nullptr, &kl};
+                     if (dir) return fn(&a, &L);
                      return timed_launch(c, slot, nq, st, [&] { return fn(&a, &L); });
                    }});
   }
 }
 
-static void add_deriv_launches(qx_ctx* c, const std::vector<QxWorkHost>& work, const QxEpiDev& e, int fp32,
-                               std::vector<Launch>& out) {
-  for (const auto& wh : work) add_deriv_list(c, wh, e, fp32, 0, wh.w.nquart, out);
-}
-
-static void add_jk_launches(qx_ctx* c, const std::vector<QxWorkHost>& work, const QxEpiDev& e, int fp32,
-                            std::vector<Launch>& out) {
-  for (const auto& wh : work) add_jk_list(c, wh, e, fp32, 0, wh.w.nquart, out);
+// J kernels of every bra class.  f32[X]: ket classes whose quartets beyond the
+// FP32 threshold run in FP32 (mixed precision).
+static void add_j_launches(qx_ctx* c, const QxEpiDev& e, const unsigned (&f32)[6], std::vector<Launch>& out) {
+  static const int order[6] = {0, 1, 2, 2, 3, 4};
+  const int nu_all = c->jlist.uoff[6];
+  // a workgroup walks every ket of its bra pseudo pair; with few bras the
+  // walk is shared out
+  const int split = std::min(8, std::max(1, 2048 / std::max(nu_all, 1)));
+  const int block = nu_all / split >= 512 ? 256 : 64;
+  for (int X = 5; X >= 0; --X) {
+    const long long nu = c->jlist.uoff[X + 1] - c->jlist.uoff[X];
+    if (nu <= 0) continue;
+    for (int pass = 0; pass < 2; ++pass) {
+      if (pass == 1 && f32[X] == 0) continue;
+      const int type = e.tv ? 2 : pass;
+      QxArgs a;
+      a.pr = c->pr; a.pp = c->pp; a.w = QxWorkDev{}; a.e = e; a.boys = c->d_boys;
+      QxJList jl = c->jlist;
+      jl.X = X;
+      jl.f32_classes = f32[X];
+      jl.n64 = c->split.d_range64;
+      auto fn = qx_j_table[order[X]];
+      const int slot = QX_SLOT_JK(class_index(X, X), 1, pass);
+      const double flops = 100.0 + 25.0 * (order[X] + 1) * (order[X] + 2);
+      out.push_back({(double)nu * nu_all * flops, [c, a, jl, fn, type, block, split, slot, nu, nu_all](hipStream_t st) {
+                       if (type == 2) return fn(&a, &jl, type, block, split, st);
+                       return timed_launch(c, slot, nu * nu_all, st, [&] { return fn(&a, &jl, type, block, split, st); });
+                     }});
+    }
+  }
 }
 
 // Mixed precision, per quartet list i of the split (pass 0 J/K, 1
@@ -1026,61 +1292,67 @@ static void add_jk_launches(qx_ctx* c, const std::vector<QxWorkHost>& work, cons
 static int mixed_mode(const qx_ctx* c, size_t i, int pass) {
   const auto& S = c->split;
   const long long p64 = S.pq64[i], p32 = S.pq32[i];
-  if (!c->fp32_ok[pass][S.wm[i].cls] || p32 < QX_MIXED_MIN_FRAC * (double)(p64 + p32)) return 0;
+  if (!c->fp32_ok[pass][c->work[i].cls] || p32 < QX_MIXED_MIN_FRAC * (double)(p64 + p32)) return 0;
   return p64 == 0 ? 1 : 2;
 }
 
 static void add_mixed_launches(qx_ctx* c, double thr, int pass, const QxEpiDev& e, std::vector<Launch>& out) {
   build_split(c, thr);
   const auto& S = c->split;
-  auto add = pass == 0 ? add_jk_list : add_deriv_list;
-  for (size_t i = 0; i < S.wm.size(); ++i) {
-    const QxWorkHost& wh = S.wm[i];
+  auto add = [&](const QxWorkHost& wh, int f32, int sel, long long nq) {
+    if (pass == 0) add_k_list(c, wh, e, f32, sel, nq, false, out);
+    else add_grad_list(c, wh, e, f32, sel, nq, false, out);
+  };
+  for (size_t i = 0; i < c->work.size(); ++i) {
+    const QxWorkHost& wh = c->work[i];
     switch (mixed_mode(c, i, pass)) {
-      case 0: add(c, wh, e, 0, 0, wh.w.nquart, out); break;
-      case 1: add(c, wh, e, 1, 0, wh.w.nquart, out); break;
+      case 0: add(wh, 0, 0, wh.w.nquart); break;
+      case 1: add(wh, 1, 0, wh.w.nquart); break;
       default:
-        add(c, wh, e, 0, 1, S.pq64[i], out);
-        add(c, wh, e, 1, 2, S.pq32[i], out);
+        add(wh, 0, 1, S.pq64[i]);
+        add(wh, 1, 2, S.pq32[i]);
     }
   }
 }
 
-static void launch_deriv_all(qx_ctx* c, const QxEpiDev& e, int fp32, hipStream_t s) {
-  std::vector<Launch> v;
-  add_deriv_launches(c, c->work, e, fp32, v);
-  run_launches(c, v, s, "eri derivative", false);
+// One list's derivative kernel (fp32 = 2: along e.tv) into the pair matrix.
+static Launch deri_launch(qx_ctx* c, const QxWorkHost& wh, const QxPairM& pm, const QxEpiDev& e, int type) {
+  const QxKList kl = pairm_kets(c, wh, pm);
+  QxArgs a;
+  a.pr = c->pr; a.pp = c->pp; a.w = wh.w; a.e = e; a.boys = c->d_boys;
+  const QxClassEntry& ent = qx_class_table[wh.cls];
+  return Launch{(double)pm.nquart * ent.part_flops[0] * ent.nparts, [=](hipStream_t st) {
+                  QxLaunch L{type, st, 0, &pm, &kl};
+                  return qx_class_table[wh.cls].deri(&a, &L);
+                }};
 }
 
+// First-derivative tensor slices: all 3N (coord < 0) or one, as many at a
+// time as begin_pairm found room for.
 static void deriv_tensor(qx_ctx* c, int coord, double* out, hipStream_t s) {
-  const size_t nc = c->ncart;
-  const size_t n4 = nc * nc * nc * nc;
-  const long long nslices = coord >= 0 ? 1 : 3LL * c->natom;
-  std::unique_ptr<DevBuf> tmp(c->pure ? new DevBuf(nslices * n4 * sizeof(double)) : nullptr);
-  double* dst = c->pure ? tmp->d() : out;
-  check_launch(qxk_fill(dst, (long long)(nslices * n4), 0.0, s), "fill");
-  QxEpiDev e{};
-  e.epi = QX_EPI_DFULL; e.atomic = 1; e.nbf = (int)nc; e.natom = c->natom; e.coord = coord; e.out = dst;
-  launch_deriv_all(c, e, 0, s);
-  if (c->pure) ao_tensor4_from_cart(c, dst, out, nslices, s);
-}
-
-// Tangent (second-derivative) kernels, every part of every class.
-static void add_dert_launches(qx_ctx* c, const QxEpiDev& e, std::vector<Launch>& out) {
-  for (const auto& wh : c->work) {
-    if (wh.w.nquart <= 0) continue;
-    const QxClassEntry& ent = qx_class_table[wh.cls];
-    for (int k = 0; k < ent.ntparts; ++k) {
-      QxArgs a;
-      a.pr = c->pr; a.pp = c->pp; a.w = wh.w; a.e = e; a.boys = c->d_boys;
-      auto fn = ent.dert[k];
-      const long long nq = wh.w.nquart;
-      out.push_back({(double)nq / ent.ntparts, [a, fn](hipStream_t st) {
-                       QxLaunch L{0, st};
-                       return fn(&a, &L);
-                     }});
+  const int nslices = coord >= 0 ? 1 : 3 * c->natom;
+  const size_t nb = c->nbf, nb4 = nb * nb * nb * nb;
+  PairMatrix m;
+  begin_pairm(c, m, nslices, s);
+  const int group = m.nslice > 0 ? m.nslice : nslices;
+  std::vector<int> map(3 * c->natom);
+  for (int y0 = 0; y0 < nslices; y0 += group) {
+    const int ny = std::min(group, nslices - y0);
+    QxEpiDev e{};
+    e.epi = QX_EPI_PAIRM; e.nbf = c->ncart; e.natom = c->natom; e.coord = coord;
+    std::unique_ptr<DevBuf> dmap;
+    if (ny < nslices) {
+      for (int y = 0; y < 3 * c->natom; ++y) map[y] = y >= y0 && y < y0 + ny ? y - y0 : -1;
+      dmap.reset(new DevBuf(map.size() * sizeof(int)));
+      QX_HIP(hipMemcpy(dmap->p, map.data(), map.size() * sizeof(int), hipMemcpyHostToDevice));
+      e.slot_map = static_cast<const int*>(dmap->p);
     }
+    run_pairm(c, m, ny, out + (size_t)y0 * nb4, s, [&](const QxWorkHost& wh, const QxPairM& pm) {
+      return deri_launch(c, wh, pm, e, 0);
+    });
+    if (dmap) QX_HIP(hipStreamSynchronize(s));
   }
+  end_pairm(c, m, s);
 }
 
 // Index of the coordinate pair (x <= y) among the m(m+1)/2 pairs in
@@ -1089,46 +1361,52 @@ static long long pair_index(int x, int y, int m) {
   return (long long)x * m - (long long)x * (x - 1) / 2 + (y - x);
 }
 
-// Second-derivative tensor: for each nuclear coordinate x the tangent
-// kernels along e_x give d2(ab|cd)/dx dy for every y; slices y >= x go to
-// pair (x, y) (all pairs when want < 0, else only pair `want` into slice 0).
-// Quartets on one atom are skipped, like the first-derivative tensor.
+// Second-derivative tensor: for each nuclear coordinate x the derivative
+// kernels in dual numbers along e_x give d2(ab|cd)/dx dy for every y; slices
+// y >= x are the consecutive pairs (x, y) (all pairs when want < 0, else only
+// pair `want` into slice 0), as many at a time as there is room for.  Quartets
+// on one atom are skipped, like the first-derivative tensor.
 static void deriv2_tensor(qx_ctx* c, long long want, double* out, hipStream_t s) {
-  const size_t nc = c->ncart;
-  const size_t n4 = nc * nc * nc * nc;
+  const size_t nb = c->nbf, nb4 = nb * nb * nb * nb;
   const int m = 3 * c->natom;
-  const long long npair = (long long)m * (m + 1) / 2;
-  const long long nslices = want >= 0 ? 1 : npair;
-  std::unique_ptr<DevBuf> tmp(c->pure ? new DevBuf(nslices * n4 * sizeof(double)) : nullptr);
-  double* dst = c->pure ? tmp->d() : out;
-  check_launch(qxk_fill(dst, (long long)(nslices * n4), 0.0, s), "fill");
-  std::vector<double> tv((size_t)m * m, 0.0);
-  std::vector<int> map((size_t)m * m, -1);
-  std::vector<int> xs;
-  for (int x = 0; x < m; ++x) {
-    tv[(size_t)x * m + x] = 1.0;
-    bool any = false;
-    for (int y = x; y < m; ++y) {
-      const long long q = pair_index(x, y, m);
-      if (want < 0) map[(size_t)x * m + y] = (int)q;
-      else if (q == want) map[(size_t)x * m + y] = 0;
-      any = any || map[(size_t)x * m + y] >= 0;
+  PairMatrix pmx;
+  begin_pairm(c, pmx, want >= 0 ? 1 : m, s);
+  const int room = pmx.nslice > 0 ? pmx.nslice : want >= 0 ? 1 : m;
+  struct Pass {
+    int x, y0, ny;
+  };
+  std::vector<Pass> passes;
+  for (int x = 0; x < m; ++x)
+    for (int y = x; y < m;) {
+      if (want >= 0) {
+        if (pair_index(x, y, m) == want) passes.push_back({x, y, 1});
+        ++y;
+        continue;
+      }
+      const int ny = std::min(room, m - y);
+      passes.push_back({x, y, ny});
+      y += ny;
     }
-    if (any) xs.push_back(x);
-  }
+  std::vector<double> tv((size_t)m * m, 0.0);
+  for (int x = 0; x < m; ++x) tv[(size_t)x * m + x] = 1.0;
+  std::vector<int> map(passes.size() * m, -1);
+  for (size_t k = 0; k < passes.size(); ++k)
+    for (int y = 0; y < passes[k].ny; ++y) map[k * m + passes[k].y0 + y] = y;
   DevBuf dtv(tv.size() * sizeof(double)), dmap(map.size() * sizeof(int));
   QX_HIP(hipMemcpy(dtv.d(), tv.data(), tv.size() * sizeof(double), hipMemcpyHostToDevice));
   QX_HIP(hipMemcpy(dmap.p, map.data(), map.size() * sizeof(int), hipMemcpyHostToDevice));
-  for (int x : xs) {
+  for (size_t k = 0; k < passes.size(); ++k) {
+    const Pass& ps = passes[k];
     QxEpiDev e{};
-    e.epi = QX_EPI_DFULL; e.atomic = 1; e.nbf = (int)nc; e.natom = c->natom; e.coord = -1; e.out = dst;
-    e.tv = dtv.d() + (size_t)x * m;
-    e.slot_map = static_cast<const int*>(dmap.p) + (size_t)x * m;
-    std::vector<Launch> v;
-    add_dert_launches(c, e, v);
-    run_launches(c, v, s, "eri second derivative", false);
+    e.epi = QX_EPI_PAIRM; e.nbf = c->ncart; e.natom = c->natom; e.coord = -1;
+    e.tv = dtv.d() + (size_t)ps.x * m;
+    e.slot_map = static_cast<const int*>(dmap.p) + k * m;
+    double* dst = out + (want >= 0 ? 0 : (size_t)pair_index(ps.x, ps.y0, m) * nb4);
+    run_pairm(c, pmx, ps.ny, dst, s, [&](const QxWorkHost& wh, const QxPairM& pm) {
+      return deri_launch(c, wh, pm, e, 2);
+    });
   }
-  if (c->pure) ao_tensor4_from_cart(c, dst, out, nslices, s);
+  end_pairm(c, pmx, s);
   QX_HIP(hipStreamSynchronize(s));  // dtv / dmap are freed on return
 }
 
@@ -1166,22 +1444,56 @@ int qx_compute_2e_deriv(qx_ctx* c, const int* dv, int len, double* out, void* st
     if (order == 0) {
       // the reference's order-0 call returns buffer 0 of a deriv-0 engine, i.e.
       // the integrals, with single-atom quartets skipped (libint_interface.cc:1180-1185)
-      const size_t nc = c->ncart;
-      const size_t n4 = nc * nc * nc * nc;
-      std::unique_ptr<DevBuf> tmp(c->pure ? new DevBuf(n4 * sizeof(double)) : nullptr);
-      double* dst = c->pure ? tmp->d() : out;
-      check_launch(qxk_fill(dst, (long long)n4, 0.0, s), "fill");
-      QxEpiDev e{};
-      e.epi = QX_EPI_FULL; e.atomic = c->k1 ? 0 : 1; e.nbf = (int)nc; e.natom = c->natom; e.coord = -1;
-      e.out = dst; e.skip_single = 1;
-      for (auto& wh : c->work) check_launch(launch_eri(c, wh.w, wh.cls, e, 0, s, c->pr, c->pp), "compute_2e_deriv");
-      if (c->pure) ao_tensor4_from_cart(c, dst, out, 1, s);
+      eri_tensor(c, 1, out, s);
       return QX_OK;
     }
     if (order == 1) deriv_tensor(c, coord, out, s);
     else deriv2_tensor(c, pair_index(c2[0], c2[1], len), out, s);
     return QX_OK;
   });
+}
+
+// J and K of D with work matrices w (2 n_cart^2 doubles, 3 for a spherical
+// basis), or (tv) of the integrals' derivative along tv; side: spread over the
+// side streams.
+static void jk_pass(qx_ctx* c, double* w, const double* D, double* J, double* K, int precision, double thr,
+                    const int* frag_skip, const double* tv, hipStream_t s, bool side) {
+  const size_t nc = c->ncart, n2 = nc * nc;
+  double *Jc = w, *Kp = w + n2;
+  QxArgs a;
+  a.pr = c->pr; a.pp = c->pp; a.w = QxWorkDev{}; a.boys = c->d_boys;
+  QxEpiDev& e = a.e;
+  e = QxEpiDev{};
+  e.epi = QX_EPI_JK; e.nbf = (int)nc; e.natom = c->natom; e.coord = -1; e.D = D; e.J = Jc; e.K = Kp;
+  if (c->pure) {
+    check_launch(qxk_ao_to_cart_mat(&c->shells, D, w + 2 * n2, s), "ao_to_cart");
+    e.D = w + 2 * n2;
+  }
+  set_krows(c, e);
+  if (frag_skip) {
+    e.frag_skip = frag_skip;
+    e.pair_frag = c->d_pair_frag;
+  }
+  e.tv = tv;
+  QxJList jl = c->jlist;
+  check_launch(qxk_jk_begin(&a, &jl, c->nherm, Jc, Kp, (long long)n2, s), "jk_begin");
+  std::vector<Launch> v;
+  unsigned f32[6] = {};
+  if (precision == QX_PREC_MIXED) {
+    add_mixed_launches(c, thr, 0, e, v);
+    for (size_t i = 0; i < c->work.size(); ++i)
+      if (mixed_mode(c, i, 0) != 0) {
+        const QxWorkHost& wh = c->work[i];
+        f32[wh.bra_class] |= 1u << wh.ket_class;
+        f32[wh.ket_class] |= 1u << wh.bra_class;
+      }
+  } else {
+    for (const auto& wh : c->work) add_k_list(c, wh, e, 0, 0, wh.w.nquart, tv != nullptr, v);
+  }
+  add_j_launches(c, e, f32, v);
+  run_launches(c, v, s, "jk_build", side);
+  check_launch(qxk_j_finish(&a, &jl, Jc, s), "j_finish");
+  check_launch(qxk_jk_finish(&c->shells, Jc, Kp, J, K, s), "jk_finish");
 }
 
 int qx_jk_build(qx_ctx* c, const double* D, double* J, double* K, int precision, double thr, void* stream) {
@@ -1197,39 +1509,8 @@ int qx_jk_build_masked(qx_ctx* c, const double* D, double* J, double* K, int pre
   return guarded(c, [&]() -> int {
     QX_HIP(hipSetDevice(c->device));
     hipStream_t s = (hipStream_t)stream;
-    const size_t nc = c->ncart, n2 = nc * nc;
     double* w = begin_ws(c, s);
-    double *Jp = w, *Kp = w + n2, *Dc = w + 2 * n2, *Js = w + 3 * n2, *Ks = w + 4 * n2;
-    const double* Dcart = D;
-    if (c->pure) {
-      check_launch(qxk_ao_to_cart_mat(&c->shells, D, Dc, s), "ao_to_cart");
-      Dcart = Dc;
-    }
-    check_launch(qxk_fill(Jp, (long long)n2, 0.0, s), "fill");
-    check_launch(qxk_fill(Kp, (long long)n2, 0.0, s), "fill");
-    QxEpiDev e{};
-    e.epi = QX_EPI_JK; e.nbf = (int)nc; e.natom = c->natom; e.coord = -1; e.D = Dcart; e.J = Jp; e.K = Kp;
-    set_krows(c, e);
-    if (frag_skip) {
-      e.frag_skip = frag_skip;
-      e.pair_frag = c->d_pair_frag;
-    }
-    std::vector<Launch> v;
-    if (precision == QX_PREC_MIXED) {
-      add_mixed_launches(c, thr, 0, e, v);
-    } else {
-      add_jk_launches(c, c->work, e, 0, v);
-    }
-    run_launches(c, v, s, "jk_build", true);
-    if (c->pure) {
-      check_launch(qxk_sym_half(Jp, Js, (int)nc, s), "sym");
-      check_launch(qxk_sym_half(Kp, Ks, (int)nc, s), "sym");
-      check_launch(qxk_cart_to_ao_mat(&c->shells, Js, J, s), "cart_to_ao");
-      check_launch(qxk_cart_to_ao_mat(&c->shells, Ks, K, s), "cart_to_ao");
-    } else {
-      check_launch(qxk_sym_half(Jp, J, (int)nc, s), "sym");
-      check_launch(qxk_sym_half(Kp, K, (int)nc, s), "sym");
-    }
+    jk_pass(c, w, D, J, K, precision, thr, frag_skip, nullptr, s, true);
     end_ws(c, s);
     return QX_OK;
   });
@@ -1252,38 +1533,7 @@ int qx_jk_build_noalloc(qx_ctx* c, const double* D, double* J, double* K, void* 
                                    std::to_string(nc) + " Cartesian functions) exceed the " +
                                    std::to_string(QX_NOALLOC_DOUBLES) + "-double scratch array"};
     QX_REQUIRE(c->scratch != nullptr, QX_EHIP, "jk_build_noalloc: scratch array not set up");
-    double* w = c->scratch;
-    double *Jp = w, *Kp = w + n2;
-    const double* Dcart = D;
-    if (c->pure) {
-      check_launch(qxk_ao_to_cart_mat(&c->shells, D, w + 2 * n2, s), "ao_to_cart");
-      Dcart = w + 2 * n2;
-    }
-    check_launch(qxk_fill(Jp, (long long)n2, 0.0, s), "fill");
-    check_launch(qxk_fill(Kp, (long long)n2, 0.0, s), "fill");
-    QxEpiDev e{};
-    e.epi = QX_EPI_JK; e.nbf = (int)nc; e.natom = c->natom; e.coord = -1; e.D = Dcart; e.J = Jp; e.K = Kp;
-    set_krows(c, e);
-    for (const auto& wh : c->work) {
-      if (wh.w.nquart <= 0) continue;
-      const QxClassEntry& ent = qx_class_table[wh.cls];
-      for (int k = 0; k < ent.njk; ++k) {
-        QxArgs a;
-        a.pr = c->pr; a.pp = c->pp; a.w = wh.w; a.e = e; a.boys = c->d_boys;
-        QxLaunch L{0, s};
-        check_launch(ent.jk[k](&a, &L), "jk_build_noalloc");
-      }
-    }
-    if (c->pure) {
-      double *Js = w + 3 * n2, *Ks = w + 4 * n2;
-      check_launch(qxk_sym_half(Jp, Js, (int)nc, s), "sym");
-      check_launch(qxk_sym_half(Kp, Ks, (int)nc, s), "sym");
-      check_launch(qxk_cart_to_ao_mat(&c->shells, Js, J, s), "cart_to_ao");
-      check_launch(qxk_cart_to_ao_mat(&c->shells, Ks, K, s), "cart_to_ao");
-    } else {
-      check_launch(qxk_sym_half(Jp, J, (int)nc, s), "sym");
-      check_launch(qxk_sym_half(Kp, K, (int)nc, s), "sym");
-    }
+    jk_pass(c, c->scratch, D, J, K, QX_PREC_FP64, 0.0, nullptr, nullptr, s, false);
     return QX_OK;
   });
 }
@@ -1309,11 +1559,12 @@ int qx_eri_grad(qx_ctx* c, const double* D, double* grad, int precision, double 
     e.grad = begin_grad_copies(c, s);
     e.grad_copies = QX_GRAD_COPIES;
     e.grad_win = c->grad_win;
+    e.pair_frag = c->d_pair_frag;
     std::vector<Launch> v;
     if (precision == QX_PREC_MIXED) {
       add_mixed_launches(c, thr, 1, e, v);
     } else {
-      add_deriv_launches(c, c->work, e, 0, v);
+      for (const auto& wh : c->work) add_grad_list(c, wh, e, 0, 0, wh.w.nquart, false, v);
     }
     run_launches(c, v, s, "eri_grad", true);
     check_launch(qxk_add_copies(c->gcopies, QX_GRAD_COPIES, 3 * c->natom, grad, s), "gradient copies");
@@ -1325,7 +1576,7 @@ int qx_eri_grad(qx_ctx* c, const double* D, double* grad, int precision, double 
 // Forward-over-reverse piece of the Hessian-vector product: the adjoint
 // contraction of the second-derivative integrals along v,
 // out[y] += sum_pqrs Gamma(D)_pqrs d/dv d(pq|rs)/dR_y, Gamma = 2 D_pq D_rs -
-// D_pr D_qs (tangent kernels, integrals recomputed, nothing stored).
+// D_pr D_qs (the gradient kernels in dual numbers, nothing stored).
 int qx_eri_hess_dir(qx_ctx* c, const double* D, const double* v, double* out, void* stream) {
   if (!c || !D || !v || !out) return QX_EINVAL;
   return guarded(c, [&]() -> int {
@@ -1343,9 +1594,10 @@ int qx_eri_hess_dir(qx_ctx* c, const double* D, const double* v, double* out, vo
     e.grad = begin_grad_copies(c, s);
     e.grad_copies = QX_GRAD_COPIES;
     e.grad_win = c->grad_win;
+    e.pair_frag = c->d_pair_frag;
     std::vector<Launch> L;
-    add_dert_launches(c, e, L);
-    run_launches(c, L, s, "eri_hess_dir", false);
+    for (const auto& wh : c->work) add_grad_list(c, wh, e, 0, 0, wh.w.nquart, true, L);
+    run_launches(c, L, s, "eri_hess_dir", true);
     check_launch(qxk_add_copies(c->gcopies, QX_GRAD_COPIES, 3 * c->natom, out, s), "gradient copies");
     end_ws(c, s);
     return QX_OK;
@@ -1360,31 +1612,8 @@ int qx_jk_deriv_dir(qx_ctx* c, const double* D, const double* v, double* J, doub
   return guarded(c, [&]() -> int {
     QX_HIP(hipSetDevice(c->device));
     hipStream_t s = (hipStream_t)stream;
-    const size_t nc = c->ncart, n2 = nc * nc;
     double* w = begin_ws(c, s);
-    double *Jp = w, *Kp = w + n2, *Dc = w + 2 * n2, *Js = w + 3 * n2, *Ks = w + 4 * n2;
-    const double* Dcart = D;
-    if (c->pure) {
-      check_launch(qxk_ao_to_cart_mat(&c->shells, D, Dc, s), "ao_to_cart");
-      Dcart = Dc;
-    }
-    check_launch(qxk_fill(Jp, (long long)n2, 0.0, s), "fill");
-    check_launch(qxk_fill(Kp, (long long)n2, 0.0, s), "fill");
-    QxEpiDev e{};
-    e.epi = QX_EPI_JKD; e.nbf = (int)nc; e.natom = c->natom; e.coord = -1; e.D = Dcart; e.J = Jp; e.K = Kp;
-    e.tv = v;
-    std::vector<Launch> L;
-    add_deriv_launches(c, c->work, e, 0, L);
-    run_launches(c, L, s, "jk_deriv_dir", false);
-    if (c->pure) {
-      check_launch(qxk_sym_half(Jp, Js, (int)nc, s), "sym");
-      check_launch(qxk_sym_half(Kp, Ks, (int)nc, s), "sym");
-      check_launch(qxk_cart_to_ao_mat(&c->shells, Js, J, s), "cart_to_ao");
-      check_launch(qxk_cart_to_ao_mat(&c->shells, Ks, K, s), "cart_to_ao");
-    } else {
-      check_launch(qxk_sym_half(Jp, J, (int)nc, s), "sym");
-      check_launch(qxk_sym_half(Kp, K, (int)nc, s), "sym");
-    }
+    jk_pass(c, w, D, J, K, QX_PREC_FP64, 0.0, nullptr, v, s, true);
     end_ws(c, s);
     return QX_OK;
   });
@@ -1416,13 +1645,12 @@ int qx_oei(qx_ctx* c, double* S, double* T, double* V, void* stream) {
     if (!c->pure) {
       run_oei(c, a, 0, s, "oei");
     } else {
-      DevBuf w(3 * n2 * 8);
-      a.S = w.d(); a.T = a.S + n2; a.V = a.T + n2;
+      double* w = begin_ws(c, s);
+      a.S = w; a.T = w + n2; a.V = w + 2 * n2;
       run_oei(c, a, 0, s, "oei");
-      check_launch(qxk_cart_to_ao_mat(&c->shells, a.S, S, s), "cart_to_ao");
-      check_launch(qxk_cart_to_ao_mat(&c->shells, a.T, T, s), "cart_to_ao");
-      check_launch(qxk_cart_to_ao_mat(&c->shells, a.V, V, s), "cart_to_ao");
-      QX_HIP(hipStreamSynchronize(s));
+      double* const out[3] = {S, T, V};
+      check_launch(qxk_cart_to_ao_mats(&c->shells, w, n2, out, 3, s), "cart_to_ao");
+      end_ws(c, s);
     }
     return QX_OK;
   });
@@ -1434,16 +1662,14 @@ static void oei_contract(qx_ctx* c, const double* Pd, const double* Wd, const do
   const size_t n2 = (size_t)c->ncart * c->ncart;
   QxOei a{};
   a.Pd = Pd; a.Wd = Wd; a.grad = grad; a.tv = v;
-  if (!c->pure) {
-    run_oei(c, a, v ? 2 : 1, s, what);
-  } else {
-    DevBuf w(2 * n2 * 8);
-    check_launch(qxk_ao_to_cart_mat(&c->shells, Pd, w.d(), s), "ao_to_cart");
-    check_launch(qxk_ao_to_cart_mat(&c->shells, Wd, w.d() + n2, s), "ao_to_cart");
-    a.Pd = w.d(); a.Wd = a.Pd + n2;
-    run_oei(c, a, v ? 2 : 1, s, what);
-    QX_HIP(hipStreamSynchronize(s));
+  if (c->pure) {
+    double* w = begin_ws(c, s);
+    const double* const in[2] = {Pd, Wd};
+    check_launch(qxk_ao_to_cart_mats(&c->shells, in, w, n2, 2, s), "ao_to_cart");
+    a.Pd = w; a.Wd = w + n2;
   }
+  run_oei(c, a, v ? 2 : 1, s, what);
+  if (c->pure) end_ws(c, s);
 }
 
 int qx_oei_grad(qx_ctx* c, const double* Pd, const double* Wd, double* grad, void* stream) {
@@ -1596,7 +1822,7 @@ int qx_mixed_pass_quartets(qx_ctx* c, double thr, int pass, long long* n64, long
     build_split(c, thr);
     const auto& S = c->split;
     long long a = 0, b = 0;
-    for (size_t i = 0; i < S.wm.size(); ++i) {
+    for (size_t i = 0; i < c->work.size(); ++i) {
       const bool f32 = pass < 0 || mixed_mode(c, i, pass) != 0;
       a += f32 ? S.cq64[i] : S.cq64[i] + S.cq32[i];
       b += f32 ? S.cq32[i] : 0;
@@ -1682,6 +1908,12 @@ int qx_set_fp32_classes(qx_ctx* c, int pass, const int* flags) {
 int qx_get_fp32_classes(const qx_ctx* c, int pass, int* flags) {
   if (!c || !flags || pass < 0 || pass > 1) return QX_EINVAL;
   for (int k = 0; k < QX_NUM_CLASSES; ++k) flags[k] = c->fp32_ok[pass][k];
+  return QX_OK;
+}
+
+int qx_set_tensor_limit(qx_ctx* c, long long bytes) {
+  if (!c || bytes < 0) return QX_EINVAL;
+  c->pairm_limit = (size_t)bytes;
   return QX_OK;
 }
 

@@ -231,6 +231,10 @@ class EriEngine:
     def set_streams(self, n: int):
         check(self.L.qx_set_streams(self.ctx, int(n)), self.ctx, "set_streams")
 
+    def set_tensor_limit(self, nbytes: int = 0):
+        """Most device memory of the tensor calls' pair matrices (0: what the device has)."""
+        check(self.L.qx_set_tensor_limit(self.ctx, int(nbytes)), self.ctx, "set_tensor_limit")
+
     def profile(self, on: bool):
         check(self.L.qx_profile_enable(self.ctx, 1 if on else 0), self.ctx)
 
