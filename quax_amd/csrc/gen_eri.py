@@ -821,7 +821,7 @@ def emit_class_files(cls, outdir, fp32):
         stats.append((cls, f"deriv{pi}", st))
     if nm in RYS_G:  # one kernel for the whole class
         groups = [list(range(len(parts)))]
-        write(f"cls_{nm}_g0.hip", [f"QX_DEFINE_RYS_G(d{nm}_g0, {la}, {lb}, {lc}, {ld}, {1 if fp32 else 0})"], "qx_rys.h")
+        write(f"cls_{nm}_g0.hip", [f"QX_DEFINE_RYS_G(d{nm}_g0, {la}, {lb}, {lc}, {ld})"], "qx_rys.h")
         return files, stats, len(parts), groups
     groups = part_groups(len(parts))
     for gi, members in enumerate(groups):

@@ -94,8 +94,8 @@ struct QxCoef<float> {
 };
 
 // Ix(i, j, k, l), i <= IA, k <= KC, l <= LD and one j <= JB, of one root and
-// direction into o[((i * (JB+1) + j) * (KC+1) + k) * (LD+1) + l].
-template <int IA, int JB, int KC, int LD, typename R>
+// direction into o[(i * (JB+1) + j) * NKS + k * (LD+1) + l].
+template <int IA, int JB, int KC, int LD, int NKS, typename R>
 __device__ __forceinline__ void qx_rys_1d(R start, R c0, R d0, R b10, R b01, R b00, R ab, R cd, int j, R* o) {
   using F = typename QxCoef<R>::T;
   constexpr int NM = IA + JB, MM = KC + LD;
@@ -117,7 +117,7 @@ __device__ __forceinline__ void qx_rys_1d(R start, R c0, R d0, R b10, R b01, R b
   const R t0 = j == 0 ? R(1) : j == 1 ? ab : ab * ab;
   const R t1 = j == 0 ? R(0) : j == 1 ? R(1) : F(2) * ab;
   const R t2 = j == 2 ? R(1) : R(0);
-  o += j * ((KC + 1) * (LD + 1));
+  o += j * NKS;
 #pragma unroll
   for (int i = 0; i <= IA; ++i) {
     R k[MM + 1];
@@ -134,7 +134,7 @@ __device__ __forceinline__ void qx_rys_1d(R start, R c0, R d0, R b10, R b01, R b
         for (int m = 0; m <= MM - l; ++m) k[m] = k[m + 1] + cd * k[m];
       }
 #pragma unroll
-      for (int kk = 0; kk <= KC; ++kk) o[(i * (JB + 1) * (KC + 1) + kk) * (LD + 1) + l] = k[kk];
+      for (int kk = 0; kk <= KC; ++kk) o[i * (JB + 1) * NKS + kk * (LD + 1) + l] = k[kk];
     }
   }
 }
@@ -209,7 +209,9 @@ struct QxRys {
   static constexpr int G = NA * NB;                       // lanes per quartet
   static constexpr int IA = LA + DER, KC = LC + DER;
   static constexpr int NKL = (KC + 1) * (LD + 1);
-  static constexpr int NG = (IA + 1) * (LB + 1) * NKL;    // 1D values per root and direction
+  static constexpr int NKS = NKL | 1;                     // stride of the (i, j) rows, odd against bank conflicts
+  static constexpr int NKU = (LC + 1) * (LD + 1);         // of an undifferentiated ket
+  static constexpr int NG = (IA + 1) * (LB + 1) * NKS;    // 1D values per root and direction
   static constexpr int STRIDE = (3 * N * NG) | 1;         // per quartet, odd against bank conflicts
   static constexpr int ONE = STRIDE + QX_RYS_PAR * N;     // LDS values of one quartet
   // quartets per wavefront: as many as its lanes hold and QX_RYS_LDS values allow
@@ -254,7 +256,7 @@ __device__ __forceinline__ void qx_rys_fill(const QxArgs& A_, const QxKList& kl,
     const int q = t / T, rdj = t - q * T, rd = rdj / (LB + 1), r = rd / 3, dim = rd - 3 * r;
     const R* o = par + (q * S::N + r) * QX_RYS_PAR;
     const R ab = dim == 0 ? a0 : dim == 1 ? a1 : a2;
-    qx_rys_1d<S::IA, LB, S::KC, LD, R>(dim == 0 ? o[9] : R(1), o[dim], o[3 + dim], o[6], o[7], o[8], ab, o[10 + dim],
+    qx_rys_1d<S::IA, LB, S::KC, LD, S::NKS, R>(dim == 0 ? o[9] : R(1), o[dim], o[3 + dim], o[6], o[7], o[8], ab, o[10 + dim],
                                        rdj - rd * (LB + 1), g + q * S::STRIDE + rd * S::NG);
   }
   qx_wave_sync();
@@ -280,7 +282,7 @@ struct QxRysLane {
       for (int j = 0; j < S::NB; ++j) e[d][1] = j == cb ? qx_comp(LB, j, d) : e[d][1];
     }
   }
-  __device__ __forceinline__ int off(int d) const { return (e[d][0] * (LB + 1) + e[d][1]) * S::NKL; }
+  __device__ __forceinline__ int off(int d) const { return (e[d][0] * (LB + 1) + e[d][1]) * S::NKS; }
 };
 
 // Most primitives of the kets in flight (wave-uniform).
@@ -441,10 +443,10 @@ struct QxRysRow {
 template <class S, int LB, int LD, typename R, typename F>
 __device__ __forceinline__ void qx_rys_row(const R* gd, int i, int j, int k, R ab, F wa, F wb, F wc,
                                            QxRysRow<S, LB, LD, R>& r) {
-  const R* o = gd + (i * (LB + 1) + j) * S::NKL + k * (LD + 1);
-  const R* up = o + (LB + 1) * S::NKL;
-  const R* dn = o - (i > 0 ? (LB + 1) * S::NKL : 0);
-  const R* bj = o - (j > 0 ? S::NKL : 0);
+  const R* o = gd + (i * (LB + 1) + j) * S::NKS + k * (LD + 1);
+  const R* up = o + (LB + 1) * S::NKS;
+  const R* dn = o - (i > 0 ? (LB + 1) * S::NKS : 0);
+  const R* bj = o - (j > 0 ? S::NKS : 0);
   const R* kd = o - (k > 0 ? LD + 1 : 0);
 #pragma unroll
   for (int l = 0; l <= LD; ++l) {
@@ -549,14 +551,16 @@ __global__ __launch_bounds__(QX_RYS_BLOCK) void qx_rd(QxArgs A_, QxKList kl, QxP
 // ---- adjoint gradient ------------------------------------------------------------
 // 8 f Gamma_abcd, Gamma = 2 D_ab D_cd - (D_ac D_bd + D_ad D_bc) / 2, for the
 // lane's (a, b) and every (c, d); summed against the derivative integrals.
-template <int LA, int LB, int LC, int LD, typename G, typename R>
-__global__ __launch_bounds__(QX_RYS_BLOCK) void qx_rg(QxArgs A_, QxKList kl) {
+// Per root the sum over (c, d) goes to the adjoint of each direction's 1D
+// values first (w: 5 multiply-adds per (c, d)), which then meets the raised
+// and lowered values: the nine derivative values per (c, d) are never formed.
+template <int LA, int LB, int LC, int LD, typename G>
+__global__ __launch_bounds__(QX_RYS_BLOCK, sizeof(G) == 8 ? 2 : 1) void qx_rg(QxArgs A_, QxKList kl) {
   using S = QxRys<LA, LB, LC, LD, 1>;
   constexpr int NC = S::NC, ND = S::ND;
-  using F = typename QxCoef<R>::T;
   HIP_DYNAMIC_SHARED(double, qx_sk)
   __shared__ double sg[QX_GRAD_LDS];
-  R* const g = reinterpret_cast<R*>(qx_sk) + (threadIdx.x >> 6) * S::LDS;
+  G* const g = reinterpret_cast<G*>(qx_sk) + (threadIdx.x >> 6) * S::LDS;
   QxKBlock b;
   if (!qx_k_block(A_, kl, b)) return;
   const QxGradTarget tgt = qx_grad_begin(A_, kl, b.P1, sg);
@@ -566,9 +570,12 @@ __global__ __launch_bounds__(QX_RYS_BLOCK) void qx_rg(QxArgs A_, QxKList kl) {
   const double dab = ln.in ? da[A_.pr.bfb[b.P1] + ln.cb] : 0.0;
   QxRysPair<G> bra;
   qx_rys_pair(A_, b.P1, u1, bra);
-  R ab[3];
+  double fi[3], fj[3];
 #pragma unroll
-  for (int d = 0; d < 3; ++d) qx_rys_cast(bra.AB[d], ab[d]);
+  for (int d = 0; d < 3; ++d) {
+    fi[d] = ln.e[d][0];
+    fj[d] = ln.e[d][1];
+  }
   double gb[6] = {};
   for (int j0 = b.j0 + (int)(threadIdx.x >> 6) * S::Q; j0 < b.j1; j0 += (int)(blockDim.x >> 6) * S::Q) {
     const int nq = min(S::Q, b.j1 - j0), pk0 = b.kst + j0;
@@ -576,7 +583,7 @@ __global__ __launch_bounds__(QX_RYS_BLOCK) void qx_rg(QxArgs A_, QxKList kl) {
     const bool in = ln.in && ln.slot < nq;
     const int P2 = pk0 + (in ? ln.slot : 0);
     const bool act = in && !qx_single_atom(A_, b.P1, P2);
-    R gam[NC * ND];
+    double gam[NC * ND];
     if (act) {
       const double f = 8.0 * qx_degeneracy(A_, b.P1, P2);
       const int ic = A_.pr.bfa[P2], id = A_.pr.bfb[P2];
@@ -591,7 +598,7 @@ __global__ __launch_bounds__(QX_RYS_BLOCK) void qx_rg(QxArgs A_, QxKList kl) {
         const double ac = da[ic + c], bc = db[ic + c];
         const double* dcd = A_.e.D + (size_t)(ic + c) * n + id;
 #pragma unroll
-        for (int d = 0; d < ND; ++d) gam[c * ND + d] = R(2.0 * f * dab * dcd[d] - (ac * bd[d] + bc * ad[d]));
+        for (int d = 0; d < ND; ++d) gam[c * ND + d] = 2.0 * f * dab * dcd[d] - (ac * bd[d] + bc * ad[d]);
       }
     }
     G v[9];
@@ -600,36 +607,55 @@ __global__ __launch_bounds__(QX_RYS_BLOCK) void qx_rg(QxArgs A_, QxKList kl) {
     for (int i1 = 0; i1 < n1; ++i1) {
       if (n1 > 1) qx_rys_pair(A_, b.P1, u1 + i1, bra);
       for (int i2 = 0; i2 < n2; ++i2) {
-        qx_rys_fill<S, LB, LD, G, R>(A_, kl, bra, pk0, nq, i2, g);
+        qx_rys_fill<S, LB, LD, G, G>(A_, kl, bra, pk0, nq, i2, g);
         if (!act || i2 >= A_.pr.pp_n[P2]) continue;
-        const F wa = (F)A_.pp.a2[u1 + i1], wb = (F)A_.pp.b2[u1 + i1], wc = (F)A_.pp.a2[A_.pr.pp_first[P2] + i2];
-        const R* gq = g + ln.slot * S::STRIDE;
+        const double wa = A_.pp.a2[u1 + i1], wb = A_.pp.b2[u1 + i1], wc = A_.pp.a2[A_.pr.pp_first[P2] + i2];
+        const G* gq = g + ln.slot * S::STRIDE;
 #pragma unroll 1
         for (int r = 0; r < S::N; ++r) {
-          QxRysRow<S, LB, LD, R> x[LC + 1], y[LC + 1], z[LC + 1];
+          const G* p[3];
+          G o[3][S::NKU], w[3][S::NKU];
 #pragma unroll
-          for (int k = 0; k <= LC; ++k) {
-            qx_rys_row<S, LB, LD, R, F>(gq + (3 * r + 0) * S::NG, ln.e[0][0], ln.e[0][1], k, ab[0], wa, wb, wc, x[k]);
-            qx_rys_row<S, LB, LD, R, F>(gq + (3 * r + 1) * S::NG, ln.e[1][0], ln.e[1][1], k, ab[1], wa, wb, wc, y[k]);
-            qx_rys_row<S, LB, LD, R, F>(gq + (3 * r + 2) * S::NG, ln.e[2][0], ln.e[2][1], k, ab[2], wa, wb, wc, z[k]);
+          for (int x = 0; x < 3; ++x) {
+            p[x] = gq + (3 * r + x) * S::NG + ln.off(x);
+#pragma unroll
+            for (int k = 0; k < S::NKU; ++k) {
+              o[x][k] = p[x][k];
+              w[x][k] = G(0.0);
+            }
           }
-          R s[9];
-#pragma unroll
-          for (int t = 0; t < 9; ++t) s[t] = R(0);
 #pragma unroll
           for (int c = 0; c < NC; ++c)
 #pragma unroll
             for (int d = 0; d < ND; ++d) {
-              const auto &xr = x[qx_comp(LC, c, 0)], &yr = y[qx_comp(LC, c, 1)], &zr = z[qx_comp(LC, c, 2)];
-              const int lx = qx_comp(LD, d, 0), ly = qx_comp(LD, d, 1), lz = qx_comp(LD, d, 2);
-              const R gx = gam[c * ND + d] * xr.o[lx], gy = gam[c * ND + d] * yr.o[ly];
-              const R xy = gx * yr.o[ly], xz = gx * zr.o[lz], yz = gy * zr.o[lz];
-              s[0] += xr.a[lx] * yz; s[1] += yr.a[ly] * xz; s[2] += zr.a[lz] * xy;
-              s[3] += xr.b[lx] * yz; s[4] += yr.b[ly] * xz; s[5] += zr.b[lz] * xy;
-              s[6] += xr.c[lx] * yz; s[7] += yr.c[ly] * xz; s[8] += zr.c[lz] * xy;
+              const int kx = qx_comp(LC, c, 0) * (LD + 1) + qx_comp(LD, d, 0);
+              const int ky = qx_comp(LC, c, 1) * (LD + 1) + qx_comp(LD, d, 1);
+              const int kz = qx_comp(LC, c, 2) * (LD + 1) + qx_comp(LD, d, 2);
+              const G gx = gam[c * ND + d] * o[0][kx], gz = gam[c * ND + d] * o[2][kz];
+              w[0][kx] += o[1][ky] * gz;
+              w[1][ky] += gx * o[2][kz];
+              w[2][kz] += gx * o[1][ky];
             }
 #pragma unroll
-          for (int t = 0; t < 9; ++t) v[t] += G(s[t]);
+          for (int x = 0; x < 3; ++x) {
+            __builtin_amdgcn_sched_barrier(0);  // one direction's operands at a time in registers
+            const G* up = p[x] + (LB + 1) * S::NKS;
+            const G* dn = p[x] - (ln.e[x][0] > 0 ? (LB + 1) * S::NKS : 0);
+            const G* bj = p[x] - (ln.e[x][1] > 0 ? S::NKS : 0);
+            G su(0.0), sd(0.0), so(0.0), sb(0.0), sc(0.0), sk(0.0);
+#pragma unroll
+            for (int k = 0; k < S::NKU; ++k) {
+              su += w[x][k] * up[k];
+              sd += w[x][k] * dn[k];
+              so += w[x][k] * o[x][k];
+              sb += w[x][k] * bj[k];
+              sc += w[x][k] * (k + LD + 1 < S::NKU ? o[x][k + LD + 1 < S::NKU ? k + LD + 1 : 0] : p[x][k + LD + 1]);
+              if (k > LD) sk += (double(k / (LD + 1)) * w[x][k]) * o[x][k > LD ? k - LD - 1 : 0];
+            }
+            v[x] += wa * su - fi[x] * sd;
+            v[3 + x] += wb * (su + bra.AB[x] * so) - fj[x] * sb;
+            v[6 + x] += wc * sc - sk;
+          }
         }
       }
     }
@@ -715,24 +741,21 @@ static inline dim3 qx_k_grid(const QxKList& kl) {
     return (int)hipGetLastError();                                                                \
   }
 
-// Adjoint gradient (FP64 or FP32), and its derivative along tv.
-template <int LA, int LB, int LC, int LD, typename G, typename R>
+// Adjoint gradient (in FP64 also where a mixed pass asks for FP32), and its
+// derivative along tv.
+template <int LA, int LB, int LC, int LD, typename G>
 static int qx_rg_go(const QxArgs* a, const QxLaunch* L) {
-  const size_t sh = 4 * (size_t)QxRys<LA, LB, LC, LD, 1>::LDS * sizeof(R);
-  hipLaunchKernelGGL((qx_rg<LA, LB, LC, LD, G, R>), qx_k_grid(*L->kl), dim3(QX_RYS_BLOCK), sh, L->stream, *a, *L->kl);
+  const size_t sh = 4 * (size_t)QxRys<LA, LB, LC, LD, 1>::LDS * sizeof(G);
+  hipLaunchKernelGGL((qx_rg<LA, LB, LC, LD, G>), qx_k_grid(*L->kl), dim3(QX_RYS_BLOCK), sh, L->stream, *a, *L->kl);
   return (int)hipGetLastError();
 }
-#define QX_DEFINE_RYS_G(NAME, LA, LB, LC, LD, WITH32)                                             \
+#define QX_DEFINE_RYS_G(NAME, LA, LB, LC, LD)                                                     \
   extern "C" int qx_launchg_##NAME(const QxArgs* a, const QxLaunch* L) {                          \
     if (!L->kl || L->kl->nquart <= 0 || L->kl->maxket <= 0) return 0;                             \
-    if (L->fp32) {                                                                                \
-      if constexpr (WITH32) return qx_rg_go<LA, LB, LC, LD, double, float>(a, L);                 \
-      return -1;                                                                                  \
-    }                                                                                             \
-    return qx_rg_go<LA, LB, LC, LD, double, double>(a, L);                                        \
+    return qx_rg_go<LA, LB, LC, LD, double>(a, L);                                                \
   }
 #define QX_DEFINE_RYS_H(NAME, LA, LB, LC, LD)                                                     \
   extern "C" int qx_launchh_##NAME(const QxArgs* a, const QxLaunch* L) {                          \
     if (!L->kl || L->kl->nquart <= 0 || L->kl->maxket <= 0) return 0;                             \
-    return a->e.tv ? qx_rg_go<LA, LB, LC, LD, qx_dual, qx_dual>(a, L) : -1;                       \
+    return a->e.tv ? qx_rg_go<LA, LB, LC, LD, qx_dual>(a, L) : -1;                       \
   }
