@@ -28,6 +28,7 @@ struct QxKList {
   int maxket;                 // most kets of one bra pair
   long long nquart;
   int chunk;                  // kets per workgroup
+  int ketprim;                // most primitives of a ket pair of the class
   int sub;                    // lanes that share one contracted quartet's primitives
   const double* rys;          // Rys root and weight tables
   const int* frag_atoms;      // gradient: first atom and atom count of each fragment (null: one fragment)

@@ -465,6 +465,8 @@ void schwarz_and_lists(qx_ctx* c) {
     return x.s2 < y.s2;
   });
   build_pair_arrays(c, scr, c->pr, c->pp, c->npseudo, &c->h_pp_first, &c->h_pp_n);
+  c->class_prims.assign(6, 1);
+  for (size_t i = 0; i < scr.size(); ++i) c->class_prims[scr[i].cls] = std::max(c->class_prims[scr[i].cls], c->h_pp_n[i]);
   c->npairs = (int)scr.size();
   c->h_pair_sa.resize(c->npairs); c->h_pair_sb.resize(c->npairs);
   c->h_pair_class.resize(c->npairs); c->h_pair_Q.resize(c->npairs); c->h_pair_frag.resize(c->npairs);
@@ -1095,6 +1097,7 @@ static QxKList k_list(const qx_ctx* c, const QxWorkHost& wh, int sel, int block)
   kl.nbra = c->class_pair_cnt[wh.bra_class];
   kl.maxket = wh.maxket;
   kl.nquart = wh.ncq;
+  kl.ketprim = c->class_prims[wh.ket_class];
   kl.rys = c->d_rys;
   kl.frag_atoms = c->d_frag_atoms;
   // few contracted quartets: their primitive quartets are shared between up

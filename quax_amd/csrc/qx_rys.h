@@ -83,6 +83,8 @@ __device__ __forceinline__ void qx_rys(const double* __restrict__ tab, qx_dual T
   }
 }
 
+#define QX_INLINE __attribute__((always_inline))
+
 // ---- 1D integrals -----------------------------------------------------------
 template <typename R>
 struct QxCoef {  // the type of a small integer factor
@@ -93,9 +95,9 @@ struct QxCoef<float> {
   using T = float;
 };
 
-// Ix(i, j, k, l), i <= IA, k <= KC, l <= LD and one j <= JB, of one root and
-// direction into o[(i * (JB+1) + j) * NKS + k * (LD+1) + l].
-template <int IA, int JB, int KC, int LD, int NKS, typename R>
+// Ix(i, j, k, l), i <= IA, k <= KC, l <= LD, of one root and direction into
+// o[(i * (JB+1) + j) * NKS + k * (LD+1) + l], for one j <= JB or (ALL) every j.
+template <int IA, int JB, int KC, int LD, int NKS, bool ALL, typename R>
 __device__ __forceinline__ void qx_rys_1d(R start, R c0, R d0, R b10, R b01, R b00, R ab, R cd, int j, R* o) {
   using F = typename QxCoef<R>::T;
   constexpr int NM = IA + JB, MM = KC + LD;
@@ -113,28 +115,33 @@ __device__ __forceinline__ void qx_rys_1d(R start, R c0, R d0, R b10, R b01, R b
       g[n][m] = v;
     }
   }
-  // (i, j) = sum_k binomial(j, k) ab^(j-k) (i + k), the same code for every j
-  const R t0 = j == 0 ? R(1) : j == 1 ? ab : ab * ab;
-  const R t1 = j == 0 ? R(0) : j == 1 ? R(1) : F(2) * ab;
-  const R t2 = j == 2 ? R(1) : R(0);
-  o += j * NKS;
+  // (i, j) = sum_k binomial(j, k) ab^(j-k) (i + k)
 #pragma unroll
-  for (int i = 0; i <= IA; ++i) {
-    R k[MM + 1];
+  for (int jj = 0; jj <= (ALL ? JB : 0); ++jj) {
+    if (ALL) j = jj;
+    const R t0 = j == 0 ? R(1) : j == 1 ? ab : ab * ab;
+    const R t1 = j == 0 ? R(0) : j == 1 ? R(1) : F(2) * ab;
+    const R t2 = j == 2 ? R(1) : R(0);
+    R* const oj = o + j * NKS;
 #pragma unroll
-    for (int m = 0; m <= MM; ++m) {
-      if (JB == 0) k[m] = g[i][m];
-      else if (JB == 1) k[m] = t0 * g[i][m] + t1 * g[i + 1 <= NM ? i + 1 : 0][m];
-      else k[m] = t0 * g[i][m] + t1 * g[i + 1 <= NM ? i + 1 : 0][m] + t2 * g[i + 2 <= NM ? i + 2 : 0][m];
-    }
+    for (int i = 0; i <= IA; ++i) {
+      R k[MM + 1];
 #pragma unroll
-    for (int l = 0; l <= LD; ++l) {
-      if (l > 0) {
-#pragma unroll
-        for (int m = 0; m <= MM - l; ++m) k[m] = k[m + 1] + cd * k[m];
+      for (int m = 0; m <= MM; ++m) {
+        if (JB == 0 || (ALL && jj == 0)) k[m] = g[i][m];
+        else if (ALL && jj == 1) k[m] = ab * g[i][m] + g[i + 1 <= NM ? i + 1 : 0][m];
+        else if (JB == 1) k[m] = t0 * g[i][m] + t1 * g[i + 1 <= NM ? i + 1 : 0][m];
+        else k[m] = t0 * g[i][m] + t1 * g[i + 1 <= NM ? i + 1 : 0][m] + t2 * g[i + 2 <= NM ? i + 2 : 0][m];
       }
 #pragma unroll
-      for (int kk = 0; kk <= KC; ++kk) o[i * (JB + 1) * NKS + kk * (LD + 1) + l] = k[kk];
+      for (int l = 0; l <= LD; ++l) {
+        if (l > 0) {
+#pragma unroll
+          for (int m = 0; m <= MM - l; ++m) k[m] = k[m + 1] + cd * k[m];
+        }
+#pragma unroll
+        for (int kk = 0; kk <= KC; ++kk) oj[i * (JB + 1) * NKS + kk * (LD + 1) + l] = k[kk];
+      }
     }
   }
 }
@@ -171,9 +178,10 @@ __device__ __forceinline__ void qx_rys_cast(qx_dual x, qx_dual& o) { o = x; }
 // b01, b00, the weight with all prefactors, and C - D.
 #define QX_RYS_PAR 13
 template <int N, typename G, typename R>
-__device__ __forceinline__ void qx_rys_params(const QxArgs& A_, const double* tab, const QxRysPair<G>& b, int P2, int u2,
-                                              int root, R* o) {
-  QxRysPair<G> k;
+__device__ __forceinline__ void qx_rys_params(const QxArgs& A_, const double* tab, int P1, int u1, int P2, int u2, int root,
+                                              R (&o)[QX_RYS_PAR]) {
+  QxRysPair<G> b, k;
+  qx_rys_pair(A_, P1, u1, b);
   qx_rys_pair(A_, P2, u2, k);
   const double p = b.p, q = k.p;
   const double pq = p + q, rs = 1.0 / sqrt(pq), opq = rs * rs, oo = 0.5 / (p * q);  // 1/2p = q oo, 1/2q = p oo
@@ -217,7 +225,14 @@ struct QxRys {
   // quartets per wavefront: as many as its lanes hold and QX_RYS_LDS values allow
   static constexpr int FIT = QX_RYS_LDS / ONE < 1 ? 1 : QX_RYS_LDS / ONE;
   static constexpr int Q = 64 / G < FIT ? 64 / G : FIT;
-  static constexpr int LDS = Q * ONE;                     // values per wavefront
+  static constexpr int LDS = (Q * ONE + 1) & ~1;          // values per wavefront
+  static constexpr int SUM = (Q * G) | 1;                 // row stride of the sums over a quartet's lanes
+  // 1D tasks: one per power of b, or all of them where that fits one pass of the wavefront better
+  static constexpr bool ALLJ = LB > 0 && 3 * Q * N * (LB + 1) > 64 && 3 * Q * N <= 64;
+  static constexpr int TASKS = 3 * N * (ALLJ ? 1 : LB + 1);  // per quartet
+  static constexpr int SETS = Q * N;                      // parameter sets of one step
+  static constexpr int STEPS = 64 / SETS;                 // steps whose sets one wavefront holds
+  static_assert(STEPS >= 1, "parameter sets of a step");
   // four wavefronts in dual numbers (16 bytes) and the gradient's accumulators fit a workgroup's 160 KB
   static_assert(4 * 16 * LDS + 8 * QX_GRAD_LDS <= 160 * 1024, "LDS of a quadrature workgroup");
 };
@@ -230,36 +245,76 @@ __device__ __forceinline__ void qx_wave_sync() {
   __builtin_amdgcn_wave_barrier();
 }
 
-// Fills the 1D integrals of up to Q quartets for primitive (i1, i2) of each;
-// every lane of the wavefront calls it.  One lane per (quartet, root) reads
-// the ket and the root table and leaves the recurrence parameters in LDS: read
-// by every 1D task itself, those loads (a table row and the pair data, each
-// lane at its own address) kept the CU's address unit busy four times longer
-// than the arithmetic took.
-template <class S, int LB, int LD, typename G, typename R>
-__device__ __forceinline__ void qx_rys_fill(const QxArgs& A_, const QxKList& kl, const QxRysPair<G>& bra, int pk0, int nq,
-                                            int i2, R* g) {
-  constexpr int T = 3 * S::N * (LB + 1);
-  R a0, a1, a2;
-  qx_rys_cast(bra.AB[0], a0);
-  qx_rys_cast(bra.AB[1], a1);
-  qx_rys_cast(bra.AB[2], a2);
+// Most primitives of the kets in flight (wave-uniform).
+__device__ __forceinline__ int qx_rys_prims(const QxArgs& A_, int pk0, int nq) {
+  int n = 1;
+  for (int q = 0; q < nq; ++q) n = max(n, A_.pr.pp_n[pk0 + q]);
+  return n;
+}
+
+// Runs the wavefront's share of a block's kets, Q at a time: begin(first ket,
+// how many), per primitive quartet step(i1, i2) with the 1D integrals at g,
+// end().  Every lane of the wavefront calls all three.
+//
+// Roots, weights and recurrence parameters of STEPS steps ahead (of several
+// ket groups, or for contracted pairs of several primitive quartets) are
+// worked out at once, one lane per (step, quartet, root), and kept in that
+// lane's registers: their chain of loads (pair, primitive, table row) and the
+// root polynomials would otherwise be waited for in every step, with a
+// handful of lanes busy.  A step's lanes then hand them to the 1D tasks
+// through LDS.  (Read by every 1D task itself, those loads kept the CU's
+// address unit busy four times longer than the arithmetic took.)
+template <class S, int LB, int LD, typename G, typename R, class Begin, class Step, class End>
+__device__ __forceinline__ void qx_rys_walk(const QxArgs& A_, const QxKList& kl, const QxKBlock& b, R* g, Begin begin, Step step,
+                                            End end) {
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), waves = blockDim.x >> 6;
+  const int u1 = A_.pr.pp_first[b.P1], n1 = A_.pr.pp_n[b.P1];
+  QxRysPair<G> bra;
+  qx_rys_pair(A_, b.P1, u1, bra);
+  R ab[3];
+#pragma unroll
+  for (int d = 0; d < 3; ++d) qx_rys_cast(bra.AB[d], ab[d]);
   R* const par = g + S::Q * S::STRIDE;
-  qx_wave_sync();  // the previous values have been read
-  for (int t = threadIdx.x & 63; t < nq * S::N; t += 64) {
-    const int q = t / S::N, pk = pk0 + q;
-    if (i2 < A_.pr.pp_n[pk])
-      qx_rys_params<S::N, G, R>(A_, kl.rys, bra, pk, A_.pr.pp_first[pk] + i2, t - q * S::N, par + t * QX_RYS_PAR);
+  const bool single = n1 == 1 && kl.ketprim == 1;
+  const int share = ((b.j1 - b.j0 + S::Q - 1) / S::Q + waves - 1) / waves * S::Q;
+  const int k0 = b.j0 + wave * share, k1 = min(b.j1, k0 + share);
+  const int ps = lane / S::SETS, pe = lane - ps * S::SETS, pq = pe / S::N, pr = pe - pq * S::N;  // the lane's set
+  R pv[QX_RYS_PAR];
+#pragma unroll
+  for (int i = 0; i < QX_RYS_PAR; ++i) pv[i] = R(0.0);
+  int held = 0;  // the step whose sets are next, single primitives
+  for (int k = k0; k < k1; k += S::Q) {
+    const int nq = min(S::Q, k1 - k), pk0 = b.kst + k;
+    const int n2 = kl.ketprim > 1 ? qx_rys_prims(A_, pk0, nq) : 1, nc = n1 * n2;
+    begin(pk0, nq);
+    for (int m = 0; m < nc; ++m) {
+      const int now = single ? held : m % S::STEPS;
+      if (now == 0) {
+        const int m1 = m + ps, i1 = single ? 0 : m1 / n2, i2 = single ? 0 : m1 - i1 * n2;
+        const int P2 = pk0 + (single ? ps * S::Q : 0) + pq;
+        if (ps < S::STEPS && (single ? P2 < b.kst + k1 : pq < nq && m1 < nc) && i2 < A_.pr.pp_n[min(P2, b.kst + k1 - 1)])
+          qx_rys_params<S::N, G, R>(A_, kl.rys, b.P1, u1 + i1, P2, A_.pr.pp_first[P2] + i2, pr, pv);
+      }
+      held = now + 1 < S::STEPS ? now + 1 : 0;
+      qx_wave_sync();  // the previous step's values have been read
+      if (ps == now) {
+#pragma unroll
+        for (int i = 0; i < QX_RYS_PAR; ++i) par[pe * QX_RYS_PAR + i] = pv[i];
+      }
+      qx_wave_sync();
+      for (int t = lane; t < nq * S::TASKS; t += 64) {
+        constexpr int J = S::ALLJ ? 1 : LB + 1;
+        const int q = t / S::TASKS, rdj = t - q * S::TASKS, rd = rdj / J, r = rd / 3, dim = rd - 3 * r;
+        const R* o = par + (q * S::N + r) * QX_RYS_PAR;
+        qx_rys_1d<S::IA, LB, S::KC, LD, S::NKS, S::ALLJ, R>(
+            dim == 0 ? o[9] : R(1), o[dim], o[3 + dim], o[6], o[7], o[8], dim == 0 ? ab[0] : dim == 1 ? ab[1] : ab[2],
+            o[10 + dim], rdj - rd * J, g + q * S::STRIDE + rd * S::NG);
+      }
+      qx_wave_sync();
+      step(m / n2, m - m / n2 * n2);
+    }
+    end();
   }
-  qx_wave_sync();
-  for (int t = threadIdx.x & 63; t < nq * T; t += 64) {
-    const int q = t / T, rdj = t - q * T, rd = rdj / (LB + 1), r = rd / 3, dim = rd - 3 * r;
-    const R* o = par + (q * S::N + r) * QX_RYS_PAR;
-    const R ab = dim == 0 ? a0 : dim == 1 ? a1 : a2;
-    qx_rys_1d<S::IA, LB, S::KC, LD, S::NKS, R>(dim == 0 ? o[9] : R(1), o[dim], o[3 + dim], o[6], o[7], o[8], ab, o[10 + dim],
-                                       rdj - rd * (LB + 1), g + q * S::STRIDE + rd * S::NG);
-  }
-  qx_wave_sync();
 }
 
 // The lane's bra function pair and quartet slot; exponents of (a, b) per direction.
@@ -284,13 +339,6 @@ struct QxRysLane {
   }
   __device__ __forceinline__ int off(int d) const { return (e[d][0] * (LB + 1) + e[d][1]) * S::NKS; }
 };
-
-// Most primitives of the kets in flight (wave-uniform).
-__device__ __forceinline__ int qx_rys_prims(const QxArgs& A_, int pk0, int nq) {
-  int n = 1;
-  for (int q = 0; q < nq; ++q) n = max(n, A_.pr.pp_n[pk0 + q]);
-  return n;
-}
 
 // I[c][d] += the lane's integrals of one primitive quartet.
 template <class S, int LC, int LD, typename R, typename T>
@@ -326,77 +374,69 @@ __global__ __launch_bounds__(QX_RYS_BLOCK_MAX) void qx_rk(QxArgs A_, QxKList kl)
   if (ROWS) qx_k_rows_begin<NA, NB, STAGE>(A_, b, qx_sk);
   const QxRysLane<S, LA, LB> ln;
   const int n = A_.e.nbf, ca = ln.ca, cb = ln.cb;
-  const int ia = A_.pr.bfa[b.P1], ib = A_.pr.bfb[b.P1], u1 = A_.pr.pp_first[b.P1], n1 = A_.pr.pp_n[b.P1];
-  QxRysPair<G> bra;
-  qx_rys_pair(A_, b.P1, u1, bra);
-  for (int j0 = b.j0 + (int)(threadIdx.x >> 6) * S::Q; j0 < b.j1; j0 += (int)(blockDim.x >> 6) * S::Q) {
-    const int nq = min(S::Q, b.j1 - j0), pk0 = b.kst + j0;
-    const int n2 = qx_rys_prims(A_, pk0, nq);
-    const bool act = ln.in && ln.slot < nq;
-    const int P2 = pk0 + (act ? ln.slot : 0);
-    G I[NC * ND];
+  const int ia = A_.pr.bfa[b.P1], ib = A_.pr.bfb[b.P1];
+  bool act = false;
+  int P2 = 0, pk = 0, nk = 0;
+  G I[NC * ND];
+  qx_rys_walk<S, LB, LD, G, R>(
+      A_, kl, b, g,
+      [&](int pk0, int nq) QX_INLINE {
+        pk = pk0;
+        nk = nq;
+        act = ln.in && ln.slot < nq;
+        P2 = pk0 + (act ? ln.slot : 0);
 #pragma unroll
-    for (int k = 0; k < NC * ND; ++k) I[k] = G(0.0);
-    for (int i1 = 0; i1 < n1; ++i1) {
-      if (n1 > 1) qx_rys_pair(A_, b.P1, u1 + i1, bra);
-      for (int i2 = 0; i2 < n2; ++i2) {
-        qx_rys_fill<S, LB, LD, G, R>(A_, kl, bra, pk0, nq, i2, g);
+        for (int k = 0; k < NC * ND; ++k) I[k] = G(0.0);
+      },
+      [&](int, int i2) QX_INLINE {
         if (act && i2 < A_.pr.pp_n[P2])
           qx_rys_sum<S, LC, LD>(g + ln.slot * S::STRIDE, ln.off(0), ln.off(1), ln.off(2), I);
-      }
-    }
-    if (act) {
-      const double fk = 2.0 * qx_degeneracy(A_, b.P1, P2);
-      const int ic = A_.pr.bfa[P2], id = A_.pr.bfb[P2];
-      const double *da, *db;
-      if (STAGE) {
-        da = qx_sk + (NA + NB + ca) * b.W - b.col0;
-        db = qx_sk + (NA + NB + NA + cb) * b.W - b.col0;
-      } else {
-        da = A_.e.D + (size_t)(ia + ca) * n;
-        db = A_.e.D + (size_t)(ib + cb) * n;
-      }
-      double *ra, *rb;
-      if (ROWS) {
-        ra = qx_sk + ca * b.W - b.col0;
-        rb = qx_sk + (NA + cb) * b.W - b.col0;
-      } else {
-        ra = A_.e.K + (size_t)(ia + ca) * n;
-        rb = A_.e.K + (size_t)(ib + cb) * n;
-      }
-      auto add = [&](double* p, double v) {
-        if (ROWS) atomicAdd(p, v);
-        else qx_atomic_add(p, v);
-      };
-      double bd[ND], ad[ND];
+      },
+      [&]() QX_INLINE {
+        static_assert((NC + ND) * S::SUM * sizeof(double) <= S::LDS * sizeof(R), "LDS of the lane sums");
+        double* const sum = reinterpret_cast<double*>(g);
+        const double fk = act ? 2.0 * qx_degeneracy(A_, b.P1, P2) : 0.0;
+        const int ic = A_.pr.bfa[P2], id = A_.pr.bfb[P2], lane = threadIdx.x & 63;
 #pragma unroll
-      for (int d = 0; d < ND; ++d) {
-        bd[d] = fk * db[id + d];
-        ad[d] = fk * da[id + d];
-      }
-      double kd[ND] = {}, ld[ND] = {};
+        for (int side = 0; side < 2; ++side) {  // K'_a from D_b, then K'_b from D_a
+          double v[NC + ND] = {};
+          if (act) {
+            const double* dx;
+            if (STAGE) dx = qx_sk + (side == 0 ? NA + NB + NA + cb : NA + NB + ca) * b.W - b.col0;
+            else dx = A_.e.D + (size_t)(side == 0 ? ib + cb : ia + ca) * n;
+            double xd[ND];
 #pragma unroll
-      for (int c = 0; c < NC; ++c) {
-        const double bc = fk * db[ic + c], ac = fk * da[ic + c];
-        double kc = 0.0, lc = 0.0;
+            for (int d = 0; d < ND; ++d) xd[d] = fk * dx[id + d];
 #pragma unroll
-        for (int d = 0; d < ND; ++d) {
-          const double v = qx_value(I[c * ND + d]);
-          kc += v * bd[d];
-          lc += v * ad[d];
-          kd[d] += v * bc;
-          ld[d] += v * ac;
+            for (int c = 0; c < NC; ++c) {
+              const double xc = fk * dx[ic + c];
+#pragma unroll
+              for (int d = 0; d < ND; ++d) {
+                const double t = qx_value(I[c * ND + d]);
+                v[c] += t * xd[d];
+                v[NC + d] += t * xc;
+              }
+            }
+          }
+          qx_wave_sync();
+          if (act) {
+#pragma unroll
+            for (int x = 0; x < NC + ND; ++x) sum[x * S::SUM + ln.slot * S::G + ln.ab] = v[x];
+          }
+          qx_wave_sync();
+          const int own = side == 0 ? NA : NB, len = side == 0 ? NB : NA;
+          for (int t = lane; t < nk * own * (NC + ND); t += 64) {
+            const int q = t / (own * (NC + ND)), cx = t - q * own * (NC + ND), o = cx / (NC + ND), x = cx - o * (NC + ND);
+            const double* w = sum + x * S::SUM + q * S::G + o * (side == 0 ? NB : 1);
+            double r = 0.0;
+#pragma unroll
+            for (int k = 0; k < len; ++k) r += w[k * (side == 0 ? 1 : NB)];
+            const int col = x < NC ? A_.pr.bfa[pk + q] + x : A_.pr.bfb[pk + q] + x - NC;
+            if (ROWS) atomicAdd(qx_sk + (side == 0 ? o : NA + o) * b.W + col - b.col0, r);
+            else qx_atomic_add(A_.e.K + (size_t)((side == 0 ? ia : ib) + o) * n + col, r);
+          }
         }
-        add(&ra[ic + c], kc);
-        add(&rb[ic + c], lc);
-      }
-#pragma unroll
-      for (int d = 0; d < ND; ++d) {
-        add(&ra[id + d], kd[d]);
-        add(&rb[id + d], ld[d]);
-      }
-    }
-  }
+      });
   if (ROWS) qx_k_rows_end<NA, NB>(A_, b, qx_sk);
 }
 
@@ -409,29 +449,28 @@ __global__ __launch_bounds__(QX_RYS_BLOCK) void qx_re(QxArgs A_, QxKList kl, QxP
   if (!qx_k_block(A_, kl, b)) return;
   double* const g = qx_sk + (threadIdx.x >> 6) * S::LDS;
   const QxRysLane<S, LA, LB> ln;
-  const int u1 = A_.pr.pp_first[b.P1], n1 = A_.pr.pp_n[b.P1];
-  QxRysPair<double> bra;
-  qx_rys_pair(A_, b.P1, u1, bra);
-  for (int j0 = b.j0 + (int)(threadIdx.x >> 6) * S::Q; j0 < b.j1; j0 += (int)(blockDim.x >> 6) * S::Q) {
-    const int nq = min(S::Q, b.j1 - j0), pk0 = b.kst + j0;
-    const int n2 = qx_rys_prims(A_, pk0, nq);
-    const bool act = ln.in && ln.slot < nq;
-    const int P2 = pk0 + (act ? ln.slot : 0);
-    double I[S::NC * S::ND] = {};
-    for (int i1 = 0; i1 < n1; ++i1) {
-      if (n1 > 1) qx_rys_pair(A_, b.P1, u1 + i1, bra);
-      for (int i2 = 0; i2 < n2; ++i2) {
-        qx_rys_fill<S, LB, LD, double, double>(A_, kl, bra, pk0, nq, i2, g);
+  bool act = false;
+  int P2 = 0;
+  double I[S::NC * S::ND];
+  qx_rys_walk<S, LB, LD, double, double>(
+      A_, kl, b, g,
+      [&](int pk0, int nq) QX_INLINE {
+        act = ln.in && ln.slot < nq;
+        P2 = pk0 + (act ? ln.slot : 0);
+#pragma unroll
+        for (int k = 0; k < S::NC * S::ND; ++k) I[k] = 0.0;
+      },
+      [&](int, int i2) QX_INLINE {
         if (act && i2 < A_.pr.pp_n[P2])
           qx_rys_sum<S, LC, LD>(g + ln.slot * S::STRIDE, ln.off(0), ln.off(1), ln.off(2), I);
-      }
-    }
-    if (act && !(A_.e.skip_single && qx_single_atom(A_, b.P1, P2))) {
-      double* m = pm.M + (pm.row0 + b.P1 - pm.rowp + (long long)ln.ab * pm.rown) * pm.ld + pm.col0 + (P2 - pm.colp);
+      },
+      [&]() QX_INLINE {
+        if (act && !(A_.e.skip_single && qx_single_atom(A_, b.P1, P2))) {
+          double* m = pm.M + (pm.row0 + b.P1 - pm.rowp + (long long)ln.ab * pm.rown) * pm.ld + pm.col0 + (P2 - pm.colp);
 #pragma unroll
-      for (int k = 0; k < S::NC * S::ND; ++k) m[(long long)k * pm.coln] = I[k];
-    }
-  }
+          for (int k = 0; k < S::NC * S::ND; ++k) m[(long long)k * pm.coln] = I[k];
+        }
+      });
 }
 
 // Values of one direction for the lane's (a, b), ket index k and all l: the
@@ -471,22 +510,27 @@ __global__ __launch_bounds__(QX_RYS_BLOCK) void qx_rd(QxArgs A_, QxKList kl, QxP
   QxKBlock b;
   if (!qx_k_block(A_, kl, b)) return;
   const QxRysLane<S, LA, LB> ln;
-  const int u1 = A_.pr.pp_first[b.P1], n1 = A_.pr.pp_n[b.P1];
-  QxRysPair<G> bra;
-  qx_rys_pair(A_, b.P1, u1, bra);
-  for (int j0 = b.j0 + (int)(threadIdx.x >> 6) * S::Q; j0 < b.j1; j0 += (int)(blockDim.x >> 6) * S::Q) {
-    const int nq = min(S::Q, b.j1 - j0), pk0 = b.kst + j0;
-    const int n2 = qx_rys_prims(A_, pk0, nq);
-    const bool in = ln.in && ln.slot < nq;
-    const int P2 = pk0 + (in ? ln.slot : 0);
-    const bool act = in && !qx_single_atom(A_, b.P1, P2);
-    const int at[4] = {A_.pr.atom_a[b.P1], A_.pr.atom_b[b.P1], A_.pr.atom_a[P2], A_.pr.atom_b[P2]};
-    double* m = pm.M + (pm.row0 + b.P1 - pm.rowp + (long long)ln.ab * pm.rown) * pm.ld + pm.col0 + (P2 - pm.colp);
-    for (int i1 = 0; i1 < n1; ++i1) {
-      if (n1 > 1) qx_rys_pair(A_, b.P1, u1 + i1, bra);
-      for (int i2 = 0; i2 < n2; ++i2) {
-        qx_rys_fill<S, LB, LD, G, G>(A_, kl, bra, pk0, nq, i2, g);
-        if (!act || i2 >= A_.pr.pp_n[P2]) continue;
+  const int u1 = A_.pr.pp_first[b.P1];
+  G ab[3];
+  {
+    QxRysPair<G> bra;
+    qx_rys_pair(A_, b.P1, u1, bra);
+#pragma unroll
+    for (int d = 0; d < 3; ++d) ab[d] = bra.AB[d];
+  }
+  bool act = false;
+  int P2 = 0, at[4];
+  qx_rys_walk<S, LB, LD, G, G>(
+      A_, kl, b, g,
+      [&](int pk0, int nq) QX_INLINE {
+        const bool in = ln.in && ln.slot < nq;
+        P2 = pk0 + (in ? ln.slot : 0);
+        act = in && !qx_single_atom(A_, b.P1, P2);
+        at[0] = A_.pr.atom_a[b.P1]; at[1] = A_.pr.atom_b[b.P1]; at[2] = A_.pr.atom_a[P2]; at[3] = A_.pr.atom_b[P2];
+      },
+      [&](int i1, int i2) QX_INLINE {
+        if (!act || i2 >= A_.pr.pp_n[P2]) return;
+        double* const m = pm.M + (pm.row0 + b.P1 - pm.rowp + (long long)ln.ab * pm.rown) * pm.ld + pm.col0 + (P2 - pm.colp);
         const double wa = A_.pp.a2[u1 + i1], wb = A_.pp.b2[u1 + i1], wc = A_.pp.a2[A_.pr.pp_first[P2] + i2];
         const G* gq = g + ln.slot * S::STRIDE;
 #pragma unroll 1
@@ -506,9 +550,9 @@ __global__ __launch_bounds__(QX_RYS_BLOCK) void qx_rd(QxArgs A_, QxKList kl, QxP
 #pragma unroll 1
           for (int r = 0; r < S::N; ++r) {
             QxRysRow<S, LB, LD, G> x, y, z;
-            qx_rys_row<S, LB, LD, G, double>(gq + (3 * r + 0) * S::NG, ln.e[0][0], ln.e[0][1], kx, bra.AB[0], wa, wb, wc, x);
-            qx_rys_row<S, LB, LD, G, double>(gq + (3 * r + 1) * S::NG, ln.e[1][0], ln.e[1][1], ky, bra.AB[1], wa, wb, wc, y);
-            qx_rys_row<S, LB, LD, G, double>(gq + (3 * r + 2) * S::NG, ln.e[2][0], ln.e[2][1], kz, bra.AB[2], wa, wb, wc, z);
+            qx_rys_row<S, LB, LD, G, double>(gq + (3 * r + 0) * S::NG, ln.e[0][0], ln.e[0][1], kx, ab[0], wa, wb, wc, x);
+            qx_rys_row<S, LB, LD, G, double>(gq + (3 * r + 1) * S::NG, ln.e[1][0], ln.e[1][1], ky, ab[1], wa, wb, wc, y);
+            qx_rys_row<S, LB, LD, G, double>(gq + (3 * r + 2) * S::NG, ln.e[2][0], ln.e[2][1], kz, ab[2], wa, wb, wc, z);
 #pragma unroll
             for (int d = 0; d < ND; ++d) {
               const int lx = qx_comp(LD, d, 0), ly = qx_comp(LD, d, 1), lz = qx_comp(LD, d, 2);
@@ -543,9 +587,8 @@ __global__ __launch_bounds__(QX_RYS_BLOCK) void qx_rd(QxArgs A_, QxKList kl, QxP
             }
           }
         }
-      }
-    }
-  }
+      },
+      [&]() QX_INLINE {});
 }
 
 // ---- adjoint gradient ------------------------------------------------------------
@@ -555,7 +598,7 @@ __global__ __launch_bounds__(QX_RYS_BLOCK) void qx_rd(QxArgs A_, QxKList kl, QxP
 // values first (w: 5 multiply-adds per (c, d)), which then meets the raised
 // and lowered values: the nine derivative values per (c, d) are never formed.
 template <int LA, int LB, int LC, int LD, typename G>
-__global__ __launch_bounds__(QX_RYS_BLOCK, sizeof(G) == 8 ? 2 : 1) void qx_rg(QxArgs A_, QxKList kl) {
+__global__ __launch_bounds__(QX_RYS_BLOCK, sizeof(G) == 8 && qx_ncart(LC) * qx_ncart(LD) < 36 ? 2 : 1) void qx_rg(QxArgs A_, QxKList kl) {
   using S = QxRys<LA, LB, LC, LD, 1>;
   constexpr int NC = S::NC, ND = S::ND;
   HIP_DYNAMIC_SHARED(double, qx_sk)
@@ -565,50 +608,56 @@ __global__ __launch_bounds__(QX_RYS_BLOCK, sizeof(G) == 8 ? 2 : 1) void qx_rg(Qx
   if (!qx_k_block(A_, kl, b)) return;
   const QxGradTarget tgt = qx_grad_begin(A_, kl, b.P1, sg);
   const QxRysLane<S, LA, LB> ln;
-  const int n = A_.e.nbf, u1 = A_.pr.pp_first[b.P1], n1 = A_.pr.pp_n[b.P1];
+  const int n = A_.e.nbf, u1 = A_.pr.pp_first[b.P1];
   const double *da = A_.e.D + (size_t)(A_.pr.bfa[b.P1] + ln.ca) * n, *db = A_.e.D + (size_t)(A_.pr.bfb[b.P1] + ln.cb) * n;
   const double dab = ln.in ? da[A_.pr.bfb[b.P1] + ln.cb] : 0.0;
-  QxRysPair<G> bra;
-  qx_rys_pair(A_, b.P1, u1, bra);
+  G ab[3];
+  {
+    QxRysPair<G> bra;
+    qx_rys_pair(A_, b.P1, u1, bra);
+#pragma unroll
+    for (int d = 0; d < 3; ++d) ab[d] = bra.AB[d];
+  }
   double fi[3], fj[3];
 #pragma unroll
   for (int d = 0; d < 3; ++d) {
     fi[d] = ln.e[d][0];
     fj[d] = ln.e[d][1];
   }
-  double gb[6] = {};
-  for (int j0 = b.j0 + (int)(threadIdx.x >> 6) * S::Q; j0 < b.j1; j0 += (int)(blockDim.x >> 6) * S::Q) {
-    const int nq = min(S::Q, b.j1 - j0), pk0 = b.kst + j0;
-    const int n2 = qx_rys_prims(A_, pk0, nq);
-    const bool in = ln.in && ln.slot < nq;
-    const int P2 = pk0 + (in ? ln.slot : 0);
-    const bool act = in && !qx_single_atom(A_, b.P1, P2);
-    double gam[NC * ND];
-    if (act) {
-      const double f = 8.0 * qx_degeneracy(A_, b.P1, P2);
-      const int ic = A_.pr.bfa[P2], id = A_.pr.bfb[P2];
-      double ad[ND], bd[ND];
+  double gb[6] = {}, gam[NC * ND];
+  G v[9];
+  bool act = false;
+  int P2 = 0, pk = 0, nk = 0;
+  qx_rys_walk<S, LB, LD, G, G>(
+      A_, kl, b, g,
+      [&](int pk0, int nq) QX_INLINE {
+        pk = pk0;
+        nk = nq;
+        const bool in = ln.in && ln.slot < nq;
+        P2 = pk0 + (in ? ln.slot : 0);
+        act = in && !qx_single_atom(A_, b.P1, P2);
+        if (act) {
+          const double f = 8.0 * qx_degeneracy(A_, b.P1, P2);
+          const int ic = A_.pr.bfa[P2], id = A_.pr.bfb[P2];
+          double ad[ND], bd[ND];
 #pragma unroll
-      for (int d = 0; d < ND; ++d) {
-        ad[d] = 0.5 * f * da[id + d];
-        bd[d] = 0.5 * f * db[id + d];
-      }
+          for (int d = 0; d < ND; ++d) {
+            ad[d] = 0.5 * f * da[id + d];
+            bd[d] = 0.5 * f * db[id + d];
+          }
 #pragma unroll
-      for (int c = 0; c < NC; ++c) {
-        const double ac = da[ic + c], bc = db[ic + c];
-        const double* dcd = A_.e.D + (size_t)(ic + c) * n + id;
+          for (int c = 0; c < NC; ++c) {
+            const double ac = da[ic + c], bc = db[ic + c];
+            const double* dcd = A_.e.D + (size_t)(ic + c) * n + id;
 #pragma unroll
-        for (int d = 0; d < ND; ++d) gam[c * ND + d] = 2.0 * f * dab * dcd[d] - (ac * bd[d] + bc * ad[d]);
-      }
-    }
-    G v[9];
+            for (int d = 0; d < ND; ++d) gam[c * ND + d] = 2.0 * f * dab * dcd[d] - (ac * bd[d] + bc * ad[d]);
+          }
+        }
 #pragma unroll
-    for (int t = 0; t < 9; ++t) v[t] = G(0.0);
-    for (int i1 = 0; i1 < n1; ++i1) {
-      if (n1 > 1) qx_rys_pair(A_, b.P1, u1 + i1, bra);
-      for (int i2 = 0; i2 < n2; ++i2) {
-        qx_rys_fill<S, LB, LD, G, G>(A_, kl, bra, pk0, nq, i2, g);
-        if (!act || i2 >= A_.pr.pp_n[P2]) continue;
+        for (int t = 0; t < 9; ++t) v[t] = G(0.0);
+      },
+      [&](int i1, int i2) QX_INLINE {
+        if (!act || i2 >= A_.pr.pp_n[P2]) return;
         const double wa = A_.pp.a2[u1 + i1], wb = A_.pp.b2[u1 + i1], wc = A_.pp.a2[A_.pr.pp_first[P2] + i2];
         const G* gq = g + ln.slot * S::STRIDE;
 #pragma unroll 1
@@ -653,24 +702,39 @@ __global__ __launch_bounds__(QX_RYS_BLOCK, sizeof(G) == 8 ? 2 : 1) void qx_rg(Qx
               if (k > LD) sk += (double(k / (LD + 1)) * w[x][k]) * o[x][k > LD ? k - LD - 1 : 0];
             }
             v[x] += wa * su - fi[x] * sd;
-            v[3 + x] += wb * (su + bra.AB[x] * so) - fj[x] * sb;
+            v[3 + x] += wb * (su + ab[x] * so) - fj[x] * sb;
             v[6 + x] += wc * sc - sk;
           }
         }
-      }
-    }
-    if (act) {
-      const int atc = 3 * A_.pr.atom_a[P2], atd = 3 * A_.pr.atom_b[P2];
+      },
+      [&]() QX_INLINE {
+        // the ket centres' terms, summed over the quartet's lanes in LDS: one
+        // LDS atomic per lane and direction would meet G-fold on each address
+        static_assert(6 * S::SUM * sizeof(double) <= S::LDS * sizeof(G), "LDS of the lane sums");
+        double* const sum = reinterpret_cast<double*>(g);
+        qx_wave_sync();
+        if (ln.in) {
 #pragma unroll
-      for (int x = 0; x < 3; ++x) {
-        const double a = qx_value(v[x]), bb = qx_value(v[3 + x]), c = qx_value(v[6 + x]);
-        gb[x] += a;
-        gb[3 + x] += bb;
-        tgt.add(atc + x, c);
-        tgt.add(atd + x, -(a + bb + c));
-      }
-    }
-  }
+          for (int x = 0; x < 3; ++x) {
+            const double a = act ? qx_value(v[x]) : 0.0, bb = act ? qx_value(v[3 + x]) : 0.0;
+            const double c = act ? qx_value(v[6 + x]) : 0.0;
+            gb[x] += a;
+            gb[3 + x] += bb;
+            sum[x * S::SUM + ln.slot * S::G + ln.ab] = c;
+            sum[(3 + x) * S::SUM + ln.slot * S::G + ln.ab] = -(a + bb + c);
+          }
+        }
+        qx_wave_sync();
+        constexpr int PARTS = S::G % 3 == 0 ? 3 : 1, LEN = S::G / PARTS;
+        for (int t = threadIdx.x & 63; t < nk * 6 * PARTS; t += 64) {
+          const int q = t / (6 * PARTS), e = t - q * 6 * PARTS, x = e / PARTS, part = e - x * PARTS;
+          const double* w = sum + x * S::SUM + q * S::G + part * LEN;
+          double r = 0.0;
+#pragma unroll
+          for (int k = 0; k < LEN; ++k) r += w[k];
+          tgt.add(3 * (x < 3 ? A_.pr.atom_a[pk + q] : A_.pr.atom_b[pk + q]) + (x < 3 ? x : x - 3), r);
+        }
+      });
   qx_grad_bra(A_, tgt, b.P1, gb);
   qx_grad_end(tgt);
 }
