@@ -1080,14 +1080,19 @@ static void begin_pairm(qx_ctx* c, PairMatrix& m, int want, hipStream_t s) {
 }
 
 // Kets of one bra pair that a workgroup takes: enough workgroups to fill the
-// device a few times over, at least a few passes of the workgroup's lanes
-// each, since every workgroup clears, fills and flushes its rows once.
+// device a few times over.  A K workgroup clears its K' rows, reads its density
+// rows and flushes with one global atomic per element of the rows, so it takes
+// QX_K_CHUNK primitive quartets or more where that leaves a quarter of
+// QX_K_BLOCKS workgroups (280 functions, all K kernels of a pass: 3.35 ms with
+// QX_K_BLOCKS, 2.83 ms with a quarter; of 672 functions' quartets a quarter
+// would already leave CUs idle at the end: (dd|dp) 8.1 ms at half, 8.9 ms).
 #define QX_K_BLOCKS 4096
+#define QX_K_CHUNK 2048LL
 #define QX_SUB_LANES 65536  // lanes below which contracted quartets are shared between lanes
 
 // The contracted list wh for a kernel of one lane per quartet in blocks of
-// `block` threads, or (block = 0) of the quadrature kernels.
-static QxKList k_list(const qx_ctx* c, const QxWorkHost& wh, int sel, int block) {
+// `block` threads, or (block = 0) of the quadrature kernels; rows: a K kernel.
+static QxKList k_list(const qx_ctx* c, const QxWorkHost& wh, int sel, int block, bool rows) {
   QxKList kl{};
   kl.bra0 = c->class_pair_off[wh.bra_class]; kl.ket0 = c->class_pair_off[wh.ket_class];
   kl.prefix = c->d_cprefix + wh.cprefix_off;
@@ -1102,9 +1107,10 @@ static QxKList k_list(const qx_ctx* c, const QxWorkHost& wh, int sel, int block)
   kl.frag_atoms = c->d_frag_atoms;
   // few contracted quartets: their primitive quartets are shared between up
   // to 64 lanes, so that a small molecule still spreads over the device
-  const long long prims = (wh.w.nquart + wh.ncq - 1) / std::max(wh.ncq, 1LL);
+  const long long prims = std::max((wh.w.nquart + wh.ncq - 1) / std::max(wh.ncq, 1LL), 1LL);
   kl.sub = (int)std::max<long long>(1, std::min<long long>({prims, 64, QX_SUB_LANES / std::max(wh.ncq, 1LL)}));
-  const long long per = std::max<long long>((wh.ncq + QX_K_BLOCKS - 1) / QX_K_BLOCKS, 1);
+  const long long most = (wh.ncq + QX_K_BLOCKS - 1) / QX_K_BLOCKS;
+  const long long per = std::max<long long>(rows ? std::max(most, std::min(4 * most, QX_K_CHUNK / prims)) : most, 1);
   const int unit = block ? std::max(1, block / kl.sub) : 32;
   kl.chunk = (int)std::min<long long>((per + unit - 1) / unit * unit, 1 << 20);
   return kl;
@@ -1126,7 +1132,7 @@ static QxPairM pairm_list(const qx_ctx* c, const PairMatrix& m, const QxWorkHost
 
 // The same panel of a list for the quadrature kernels.
 static QxKList pairm_kets(const qx_ctx* c, const QxWorkHost& wh, const QxPairM& pm) {
-  QxKList kl = k_list(c, wh, 0, 0);
+  QxKList kl = k_list(c, wh, 0, 0, false);
   kl.bra0 = pm.rowp;
   kl.prefix = pm.prefix;
   kl.kstart = pm.kstart;
@@ -1213,7 +1219,7 @@ static void add_grad_list(qx_ctx* c, const QxWorkHost& wh, const QxEpiDev& e, in
   if (wh.ncq <= 0 || nq <= 0) return;
   const QxClassEntry& ent = qx_class_table[wh.cls];
   const int block = c->tile[1][wh.cls];
-  const QxKList kl = k_list(c, wh, sel, dir || qx_rys_g[wh.cls] ? 0 : block);
+  const QxKList kl = k_list(c, wh, sel, dir || qx_rys_g[wh.cls] ? 0 : block, false);
   const int nl = dir ? 1 : ent.ngroups;
   for (int k = 0; k < nl; ++k) {
     QxArgs a;
@@ -1237,7 +1243,7 @@ static void add_k_list(qx_ctx* c, const QxWorkHost& wh, const QxEpiDev& e, int f
   if (wh.ncq <= 0 || nq <= 0) return;
   const QxClassEntry& ent = qx_class_table[wh.cls];
   const int block = c->tile[0][wh.cls];
-  const QxKList kl = k_list(c, wh, sel, dir || qx_rys_k[wh.cls] ? 0 : block);
+  const QxKList kl = k_list(c, wh, sel, dir || qx_rys_k[wh.cls] ? 0 : block, true);
   const int nl = dir ? 1 : ent.njk;
   for (int k = 0; k < nl; ++k) {
     QxArgs a;

@@ -225,8 +225,9 @@ struct QxRys {
   // quartets per wavefront: as many as its lanes hold and QX_RYS_LDS values allow
   static constexpr int FIT = QX_RYS_LDS / ONE < 1 ? 1 : QX_RYS_LDS / ONE;
   static constexpr int Q = 64 / G < FIT ? 64 / G : FIT;
-  static constexpr int LDS = (Q * ONE + 1) & ~1;          // values per wavefront
   static constexpr int SUM = (Q * G) | 1;                 // row stride of the sums over a quartet's lanes
+  static constexpr int SUMS = 2 * (DER ? 6 : NC + ND) * SUM;  // their LDS values (FP32: two per sum)
+  static constexpr int LDS = Q * ONE > SUMS ? (Q * ONE + 1) & ~1 : SUMS;  // values per wavefront
   // 1D tasks: one per power of b, or all of them where that fits one pass of the wavefront better
   static constexpr bool ALLJ = LB > 0 && 3 * Q * N * (LB + 1) > 64 && 3 * Q * N <= 64;
   static constexpr int TASKS = 3 * N * (ALLJ ? 1 : LB + 1);  // per quartet
