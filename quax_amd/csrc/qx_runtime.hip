@@ -309,37 +309,46 @@ void frag_segment(const qx_ctx* c, int ko, int kn, int f, int& ss, int& se) {
   se = (int)(std::upper_bound(fr, fr + kn, f) - fr);
 }
 
-// Admissible kets of bra pair i (position in class X) in class Y: positions
-// [ss, ss + kc) of Y's list, i.e. the bra's fragment, Q_i Q_j >= bound (a
-// prefix of the descending segment) and, if asked for, canonical j <= i when
-// X == Y.
-void ket_window(const qx_ctx* c, int X, int Y, int i, double bound, int& ss, int& kc, bool canonical = true) {
-  const int bo = c->class_pair_off[X], ko = c->class_pair_off[Y], kn = c->class_pair_cnt[Y];
-  int se;
-  frag_segment(c, ko, kn, c->h_pair_frag[bo + i], ss, se);
-  const double Qi = c->h_pair_Q[bo + i];
-  int lo = ss, hi = se;
-  while (lo < hi) {
-    const int mid = (lo + hi) / 2;
-    if (Qi * c->h_pair_Q[ko + mid] >= bound) lo = mid + 1; else hi = mid;
+// Admissible kets of every bra pair of class X in class Y: positions
+// [first, first + count) of Y's list, i.e. the bra's fragment and
+// Q_bra Q_ket >= bound, a prefix of the segment, which is sorted by descending
+// Q.  The bras of a fragment are too, so the prefix only shrinks from one to
+// the next.  (`canonical`: j <= i when X == Y.)
+std::vector<QxRange> ket_windows(const qx_ctx* c, int X, int Y, double bound, bool canonical = true) {
+  const int bo = c->class_pair_off[X], bn = c->class_pair_cnt[X];
+  const int ko = c->class_pair_off[Y], kn = c->class_pair_cnt[Y];
+  std::vector<QxRange> w(bn);
+  int ss = 0, end = 0;
+  for (int i = 0; i < bn; ++i) {
+    if (i == 0 || c->h_pair_frag[bo + i] != c->h_pair_frag[bo + i - 1])
+      frag_segment(c, ko, kn, c->h_pair_frag[bo + i], ss, end);
+    while (end > ss && !(c->h_pair_Q[bo + i] * c->h_pair_Q[ko + end - 1] >= bound)) --end;
+    int kc = end - ss;
+    if (X == Y && canonical) kc = std::max(0, std::min(kc, i - ss + 1));
+    w[i] = {ss, kc};
   }
-  kc = lo - ss;
-  if (X == Y && canonical) kc = std::max(0, std::min(kc, i - ss + 1));
+  return w;
 }
 
-// Pseudo kets of class Y that bra pair P (any order of the two classes) meets
-// with Q_P Q_ket >= bound: the J kernels' ranges.
-QxRange pseudo_range(const qx_ctx* c, int P, int Y, double bound) {
-  const int X = c->h_pair_class[P], ko = c->class_pair_off[Y];
-  if (c->class_pair_cnt[Y] == 0) return {0, 0};
-  int ss, kc;
-  ket_window(c, X, Y, P - c->class_pair_off[X], bound, ss, kc, false);
-  if (kc <= 0) return {0, 0};
-  const int last = ko + ss + kc - 1;
-  return {c->h_pp_first[ko + ss], c->h_pp_first[last] + c->h_pp_n[last] - c->h_pp_first[ko + ss]};
+// Pseudo kets of each class that every pair (any order of the two classes)
+// meets with Q_P Q_ket >= bound: the J kernels' ranges, [Y * npairs + pair].
+std::vector<QxRange> pseudo_ranges(const qx_ctx* c, double bound) {
+  std::vector<QxRange> r((size_t)6 * c->npairs, QxRange{0, 0});
+  for (int X = 0; X < 6; ++X)
+    for (int Y = 0; Y < 6; ++Y) {
+      const int ko = c->class_pair_off[Y];
+      const auto w = ket_windows(c, X, Y, bound, false);
+      for (size_t i = 0; i < w.size(); ++i) {
+        if (w[i].count <= 0) continue;
+        const int first = ko + w[i].first, last = first + w[i].count - 1;
+        r[(size_t)Y * c->npairs + c->class_pair_off[X] + i] = {c->h_pp_first[first],
+                                                               c->h_pp_first[last] + c->h_pp_n[last] - c->h_pp_first[first]};
+      }
+    }
+  return r;
 }
 
-// Hermite layout, J ranges and Rys tables.
+// Hermite layout and J ranges.
 void setup_jk(qx_ctx* c) {
   static const int order[6] = {0, 1, 2, 2, 3, 4};
   QxJList& jl = c->jlist;
@@ -357,13 +366,8 @@ void setup_jk(qx_ctx* c) {
   jl.uoff[6] = u;
   QX_REQUIRE(at <= 0x7fffffff, QX_EUNSUPPORTED, "too many primitive pairs");
   c->nherm = at;
-  std::vector<QxRange> r((size_t)6 * c->npairs);
-  for (int Y = 0; Y < 6; ++Y)
-    for (int P = 0; P < c->npairs; ++P) r[(size_t)Y * c->npairs + P] = pseudo_range(c, P, Y, c->tol * c->tol);
-  c->d_range = dupload(c, r);
+  c->d_range = dupload(c, pseudo_ranges(c, c->tol * c->tol));
   c->d_herm = dalloc<double>(c, (size_t)4 * at);
-  c->d_rys = dalloc<double>(c, QX_RYS_DOUBLES);
-  QX_HIP(hipMemcpy(c->d_rys, qxk_rys_host(), QX_RYS_DOUBLES * sizeof(double), hipMemcpyHostToDevice));
   jl.range = c->d_range;
   jl.H = c->d_herm;
   jl.P = c->d_herm + at;
@@ -373,6 +377,8 @@ void setup_jk(qx_ctx* c) {
 
 void schwarz_and_lists(qx_ctx* c) {
   const int ns = c->nshell;
+  c->d_rys = dalloc<double>(c, QX_RYS_DOUBLES);
+  QX_HIP(hipMemcpy(c->d_rys, qxk_rys_host(), QX_RYS_DOUBLES * sizeof(double), hipMemcpyHostToDevice));
   // ---- every shell pair, class-sorted, for the Schwarz pass
   std::vector<PairRec> all;
   for (int s1 = 0; s1 < ns; ++s1)
@@ -420,7 +426,10 @@ void schwarz_and_lists(qx_ctx* c) {
     w.nquart = p.back(); w.store_base = 0; w.diag = 1;
     QxEpiDev e{};
     e.epi = QX_EPI_SCHWARZ; e.out = diag.d(); e.nbf = c->ncart; e.natom = c->natom; e.coord = -1;
-    int rc = launch_eri(c, w, class_index(X, X), e, 0, 0, pr_all, pp_all);
+    QxKList kl{};
+    kl.bra0 = lo; kl.nbra = hi - lo; kl.rys = c->d_rys;
+    for (int i = lo; i < hi; ++i) kl.ketprim = std::max(kl.ketprim, cnt[i]);
+    int rc = launch_eri(c, w, class_index(X, X), e, 0, 0, pr_all, pp_all, nullptr, &kl);
     if (rc != 0) {
       for (auto* q : bufs) delete q;
       check_launch(rc, "schwarz");
@@ -516,11 +525,9 @@ void schwarz_and_lists(qx_ctx* c) {
       allpre.push_back(0);
       kst_off.push_back((long long)allkst.size());
       long long run = 0, ncq = 0;
+      const auto window = ket_windows(c, X, Y, tol2);
       for (int i = 0; i < bn; ++i) {
-        // kets with Q_i Q_j >= tol^2 form a prefix of the descending list
-        // (of the bra's fragment segment)
-        int ss, kc;
-        ket_window(c, X, Y, i, tol2, ss, kc);
+        const int ss = window[i].first, kc = window[i].count;
         ncq += kc;
         wh.maxket = std::max(wh.maxket, kc);
         allcpre.push_back(ncq);
@@ -677,11 +684,9 @@ void build_split(qx_ctx* c, double thr) {
     std::vector<long long> kcum(kn + 1, 0);
     for (int j = 0; j < kn; ++j) kcum[j + 1] = kcum[j] + c->h_pp_n[ko + j];
     long long p64 = 0, p32 = 0, q64 = 0, q32 = 0;
+    const auto all = ket_windows(c, X, Y, tol2), fp64 = ket_windows(c, X, Y, thr2);
     for (int i = 0; i < bn; ++i) {
-      int ss, kc, ss2, k64;
-      ket_window(c, X, Y, i, tol2, ss, kc);
-      ket_window(c, X, Y, i, thr2, ss2, k64);
-      k64 = std::min(kc, k64);
+      const int ss = all[i].first, kc = all[i].count, k64 = std::min(kc, fp64[i].count);
       q64 += k64;
       q32 += kc - k64;
       ck[wh.cprefix_off + i] = k64;
@@ -695,10 +700,9 @@ void build_split(qx_ctx* c, double thr) {
     S.pq64.push_back(p64); S.pq32.push_back(p32);
     S.cq64.push_back(q64); S.cq32.push_back(q32);
   }
-  std::vector<int> r64((size_t)6 * c->npairs);
-  for (int Y = 0; Y < 6; ++Y)
-    for (int P = 0; P < c->npairs; ++P)
-      r64[(size_t)Y * c->npairs + P] = std::min(pseudo_range(c, P, Y, thr2).count, pseudo_range(c, P, Y, tol2).count);
+  const auto rall = pseudo_ranges(c, tol2), rthr = pseudo_ranges(c, thr2);
+  std::vector<int> r64(rall.size());
+  for (size_t i = 0; i < r64.size(); ++i) r64[i] = std::min(rall[i].count, rthr[i].count);
   QX_HIP(hipMalloc(&S.d_ck64, std::max<size_t>(ck.size(), 1) * sizeof(int)));
   if (!ck.empty()) QX_HIP(hipMemcpy(S.d_ck64, ck.data(), ck.size() * sizeof(int), hipMemcpyHostToDevice));
   QX_HIP(hipMalloc(&S.d_range64, std::max<size_t>(r64.size(), 1) * sizeof(int)));

@@ -474,6 +474,30 @@ __global__ __launch_bounds__(QX_RYS_BLOCK) void qx_re(QxArgs A_, QxKList kl, QxP
       });
 }
 
+// The Schwarz pass: (ab|ab) of every pair, one wavefront each, by pair and
+// function pair.
+template <int LA, int LB>
+__global__ __launch_bounds__(64) void qx_rs(QxArgs A_, QxKList kl) {
+  using S = QxRys<LA, LB, LA, LB, 0>;
+  HIP_DYNAMIC_SHARED(double, qx_sk)
+  const int P = kl.bra0 + (int)blockIdx.x;
+  const QxKBlock b{P, 0, 1, P, 0, 0};
+  const QxRysLane<S, LA, LB> ln;
+  double I[S::NC * S::ND] = {};
+  qx_rys_walk<S, LB, LB, double, double>(
+      A_, kl, b, qx_sk, [&](int, int) QX_INLINE {},
+      [&](int, int) QX_INLINE {
+        if (ln.slot == 0) qx_rys_sum<S, LA, LB>(qx_sk, ln.off(0), ln.off(1), ln.off(2), I);
+      },
+      [&]() QX_INLINE {
+        if (ln.slot != 0) return;
+        double v = 0.0;
+#pragma unroll
+        for (int k = 0; k < S::NC * S::ND; ++k) v = k == ln.ab ? I[k] : v;
+        A_.e.out[(long long)P * QX_PAIR_STRIDE + ln.ab] = v;
+      });
+}
+
 // Values of one direction for the lane's (a, b), ket index k and all l: the
 // integral (o), d/dA (a), d/dB (b) and d/dC (c) factors.
 template <class S, int LB, int LD, typename R>
@@ -787,7 +811,16 @@ static inline dim3 qx_k_grid(const QxKList& kl) {
 // L->fp32 = 2 their derivatives along tv) into the pair matrix.
 #define QX_DEFINE_RYS_E(NAME, LA, LB, LC, LD)                                                     \
   extern "C" int qx_launchr_##NAME(const QxArgs* a, const QxLaunch* L) {                          \
-    if (!L->kl || !L->pm || L->kl->nquart <= 0 || L->kl->maxket <= 0) return 0;                   \
+    if (!L->kl) return -1;                                                                        \
+    if constexpr (LA == LC && LB == LD) {                                                         \
+      if (a->e.epi == QX_EPI_SCHWARZ) {                                                           \
+        if (L->kl->nbra <= 0) return 0;                                                           \
+        const size_t one = sizeof(double) * QxRys<LA, LB, LA, LB, 0>::LDS;                        \
+        hipLaunchKernelGGL((qx_rs<LA, LB>), dim3((unsigned)L->kl->nbra), dim3(64), one, L->stream, *a, *L->kl); \
+        return (int)hipGetLastError();                                                            \
+      }                                                                                           \
+    }                                                                                             \
+    if (!L->pm || L->kl->nquart <= 0 || L->kl->maxket <= 0) return 0;                   \
     const size_t sh = 4 * sizeof(double) * QxRys<LA, LB, LC, LD, 0>::LDS;                         \
     hipLaunchKernelGGL((qx_re<LA, LB, LC, LD>), qx_k_grid(*L->kl), dim3(QX_RYS_BLOCK), sh, L->stream, *a, *L->kl, *L->pm); \
     return (int)hipGetLastError();                                                                \
