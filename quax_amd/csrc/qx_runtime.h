@@ -205,13 +205,6 @@ int qxk_j_finish(const QxArgs* a, const QxJList* jl, double* J, hipStream_t s);
 int qxk_jk_finish(const QxShellsDev* sh, const double* Jc, const double* Kp, double* J, double* K, hipStream_t s);
 }
 
-// An AO function as its Cartesian terms (one for s, p and Cartesian d; up to
-// three for a spherical d function).
-struct QxAoTerms {
-  int n, f[3];
-  double c[3];
-};
-
 // helper kernels (qx_kernels.hip)
 extern "C" {
 int qxk_fill(double* p, long long n, double v, hipStream_t s);
@@ -227,15 +220,17 @@ int qxk_ao_to_cart_mats(const QxShellsDev* sh, const double* const* in, double* 
 // index: Cartesian function pair -> row (ncart^2 ints, -1 = screened out), fn:
 // row -> p * ncart + q, ao: per AO function up to three Cartesian terms
 // (qxk_pairm_tables fills them).
-int qxk_pairm_tables(const QxShellsDev* sh, const QxPairsDev* pr, int npairs, const QxPairIndex* ix, int* index,
-                     int* fn, QxAoTerms* ao, hipStream_t s);
+int qxk_pairm_tables(const QxShellsDev* sh, const QxPairsDev* pr, int npairs, const QxPairIndex* ix, long long ld, int* index,
+                     int* fn, hipStream_t s);
 // every permutation of the elements of a panel of rows into a zeroed
 // Cartesian tensor: panel row k * cnt + i is component k of the class's pair
 // i0 + i (class X, ncomp components)
 int qxk_pairm_scatter(int ncart, const double* M, long long ld, long long slice, int nslice, const QxPairIndex* ix,
                       const int* fn, int X, int ncomp, int i0, int cnt, double* out, hipStream_t s);
 int qxk_pairm_sym(double* M, long long ld, long long slice, int nslice, const QxPairIndex* ix, hipStream_t s);
-int qxk_pairm_expand(const QxShellsDev* sh, const double* M, long long ld, long long slice, int nslice,
-                     const int* index, const QxAoTerms* ao, double* out, hipStream_t s);
+int qxk_pairm_expand(int n, const double* M, long long ld, long long slice, int nslice, const int* index, const int* fn,
+                     double* out, hipStream_t s);
+int qxk_pairm_ao(const QxShellsDev* sh, const QxPairIndex* ix, const int* fn, double* M, long long ld, long long slice,
+                 int nslice, hipStream_t s);
 int qxk_oei_deriv(const QxShellsDev* sh, double* dS, double* dT, double* dV, hipStream_t s);
 }

@@ -1005,8 +1005,8 @@ long long qx_generate_multi_index_lookup(int nparams, int order, int* out, long 
   return count;
 }
 
-// Workspace of one tensor pass: nslice pair matrices (or panels of one), the
-// index tables and the AO terms.  Up to QX_PAIRM_KEEP bytes stay with the
+// Workspace of one tensor pass: nslice pair matrices (or panels of one), and
+// the index tables.  Up to QX_PAIRM_KEEP bytes stay with the
 // context, larger ones are allocated for the call.
 #define QX_PAIRM_KEEP ((size_t)1 << 30)
 #define QX_PAIRM_PANEL ((size_t)64 << 20)
@@ -1020,7 +1020,6 @@ struct PairMatrix {
   double* M = nullptr;
   int* index = nullptr;
   int* fn = nullptr;
-  QxAoTerms* ao = nullptr;
   std::unique_ptr<DevBuf> own;
 };
 
@@ -1055,8 +1054,8 @@ static void begin_pairm(qx_ctx* c, PairMatrix& m, int want, hipStream_t s) {
   m.ld = std::max((at + 7) & ~7, 8);  // rows start on a 64-byte line
   m.slice = m.ld * m.ld;
   auto pad = [](size_t b) { return (b + 63) / 64 * 64; };
-  const size_t bi = pad((size_t)c->ncart * c->ncart * sizeof(int)), bf = pad((size_t)m.ld * sizeof(int));
-  const size_t tables = bi + bf + (size_t)c->nbf * sizeof(QxAoTerms);
+  const size_t bi = pad((size_t)c->nbf * c->nbf * sizeof(int)), bf = pad((size_t)m.ld * sizeof(int));
+  const size_t tables = bi + bf;
   void* p = nullptr;
   size_t data = 0;
   for (m.nslice = want; m.nslice >= 1 && !p; m.nslice = m.nslice > 1 ? (m.nslice + 1) / 2 : 0) {
@@ -1078,9 +1077,8 @@ static void begin_pairm(qx_ctx* c, PairMatrix& m, int want, hipStream_t s) {
   char* q = static_cast<char*>(p) + data;
   m.index = reinterpret_cast<int*>(q);
   m.fn = reinterpret_cast<int*>(q + bi);
-  m.ao = reinterpret_cast<QxAoTerms*>(q + bi + bf);
   (void)begin_ws(c, s);  // orders this pass after the previous user of the context's workspaces
-  check_launch(qxk_pairm_tables(&c->shells, &c->pr, c->npairs, &m.ix, m.index, m.fn, m.ao, s), "pair tables");
+  check_launch(qxk_pairm_tables(&c->shells, &c->pr, c->npairs, &m.ix, m.ld, m.index, m.fn, s), "pair tables");
 }
 
 // Kets of one bra pair that a workgroup takes: enough workgroups to fill the
@@ -1155,8 +1153,9 @@ static void run_pairm(qx_ctx* c, PairMatrix& m, int nslice, double* out, hipStre
     check_launch(qxk_fill(m.M, nslice * m.slice, 0.0, s), "fill");
     for (const auto& wh : c->work) v.push_back(launch(wh, pairm_list(c, m, wh)));
     run_launches(c, v, s, "pair matrix", true);
+    check_launch(qxk_pairm_ao(&c->shells, &m.ix, m.fn, m.M, m.ld, m.slice, nslice, s), "pair transform");
     check_launch(qxk_pairm_sym(m.M, m.ld, m.slice, nslice, &m.ix, s), "pair mirror");
-    check_launch(qxk_pairm_expand(&c->shells, m.M, m.ld, m.slice, nslice, m.index, m.ao, out, s), "pair expand");
+    check_launch(qxk_pairm_expand(c->nbf, m.M, m.ld, m.slice, nslice, m.index, m.fn, out, s), "pair expand");
     return;
   }
   const size_t nc = c->ncart, n4 = nc * nc * nc * nc;
