@@ -544,13 +544,12 @@ def herm(L):
     return [(t, u, v) for t in range(L + 1) for u in range(L + 1 - t) for v in range(L + 1 - t - u)]
 
 
-def emit_j(L1, outdir, lmax, fp32):
-    """jeng_<L1>.hip: the J kernel of bra pairs of total angular momentum L1:
-    per ket order L2 a body that runs the Hermite Coulomb recursion
+def j_cores(L1, L2s):
+    """Per ket order L2 a body that runs the Hermite Coulomb recursion
     R^n_{t+1} = t R^{n+1}_{t-1} + X R^{n+1}_t and contracts it with the ket's
     Hermite density."""
     out = []
-    for L2 in range(2 * lmax + 1):
+    for L2 in L2s:
         L = L1 + L2
         H1, H2 = herm(L1), herm(L2)
         S = [f"template <typename G, typename R>\n__device__ __forceinline__ void qx_jc_{L1}{L2}(R X, R Y, R Z, "
@@ -582,9 +581,34 @@ def emit_j(L1, outdir, lmax, fp32):
                 S.append(f"  j[{m}] += h[{k}] * G({v});")
         S.append("}")
         out += S + [""]
+    return out
+
+
+def emit_j(L1, outdir, lmax, fp32):
+    """jeng_<L1>.hip, jengv_<L1>.hip: the J kernels of bra pairs of total
+    angular momentum L1 (FP64 and FP32; dual numbers)."""
     cases = " ".join(f"QX_J_CASE({L1}, {L2})" for L2 in range(2 * lmax + 1))
-    out.append(f"QX_DEFINE_J_KERNEL({L1}, {1 if fp32 else 0}, {cases})")
-    path = os.path.join(outdir, f"jeng_{L1}.hip")
+    paths = []
+    for name, last in (("jeng", f"QX_DEFINE_J_KERNEL({L1}, {1 if fp32 else 0}, {cases})"),
+                       ("jengv", f"QX_DEFINE_JV_KERNEL({L1}, {cases})")):
+        paths.append(os.path.join(outdir, f"{name}_{L1}.hip"))
+        with open(paths[-1], "w") as fh:
+            fh.write("\n".join(['#include "../qx_jk.h"', ""] + j_cores(L1, range(2 * lmax + 1)) + [last, ""]))
+    return paths
+
+
+def emit_small(outdir):
+    """jk_small.hip: every K and J body of s and p shells in one kernel."""
+    out = []
+    for l in canonical_classes(1)[1]:
+        nm = "".join(map(str, l))
+        na, nb, nc, nd = map(ncart, l)
+        out += emit_eri_core(l)[1] + [f"QX_DEFINE_K_BODY(e{nm}_0, {na}, {nb}, {nc}, {nd})", ""]
+    for L1 in range(3):
+        cases = " ".join(f"QX_J_CASE({L1}, {L2})" for L2 in range(3))
+        out += j_cores(L1, range(3)) + [f"QX_DEFINE_J_BODY({L1}, {cases})", ""]
+    out.append("QX_DEFINE_SMALL()")
+    path = os.path.join(outdir, "jk_small.hip")
     with open(path, "w") as fh:
         fh.write("\n".join(['#include "../qx_jk.h"', ""] + out + [""]))
     return path
@@ -855,7 +879,9 @@ def main():
         flops[cls] = (s[0][2]["flops"], [st["flops"] for _, _, st in s[1:]], [st["ncomb"] for _, _, st in s[1:]])
     pairs = [(a, b) for a in range(lmax + 1) for b in range(a + 1)]
     files += [emit_oei(a, b, outdir) for a, b in pairs]
-    files += [emit_j(L, outdir, lmax, fp32) for L in range(2 * lmax + 1)]
+    for L in range(2 * lmax + 1):
+        files += emit_j(L, outdir, lmax, fp32)
+    files.append(emit_small(outdir))
     with open(os.path.join(outdir, "qx_rys.inc"), "w") as fh:
         fh.write(rys_tables())
     D = ["// generated: kernel launch tables indexed by canonical class id", "#pragma once",
@@ -918,6 +944,7 @@ def main():
         D.append(f"static const unsigned char qx_rys_{name}[QX_NUM_CLASSES] = {{")
         D.append("  " + ", ".join(str(int("".join(map(str, cls)) in table)) for cls in classes))
         D.append("};")
+    D.append('extern "C" int qx_launch_small(const QxArgs*, const QxSmall*, unsigned, hipStream_t);')
     D.append("// one-electron kernels per shell-pair class")
     D += [f'extern "C" int qx_launch_oei_{a}{b}(const QxOei*, int, hipStream_t);' for a, b in pairs]
     D.append(f"static int (*const qx_oei_table[{len(pairs)}])(const QxOei*, int, hipStream_t) = {{"

@@ -293,10 +293,11 @@ __device__ __forceinline__ void qx_j_kets(const QxArgs& A_, const QxJList& jl, i
                             [](R x, R y, R z, const R (&b)[L1 + L2 + 1], const G (&h)[qx_nherm(L2)], \
                                G (&jj)[qx_nherm(L1)]) { qx_jc_##L1##L2<G, R>(x, y, z, b, h, jj); }); \
     break;
-#define QX_DEFINE_J_KERNEL(L1, WITH32, CASES)                                                     \
-  template <typename G, typename R>                                                               \
-  __global__ __launch_bounds__(QX_BLOCK_MAX) void qx_jeng_##L1(QxArgs A_, QxJList jl) {           \
-    const int u = jl.uoff[jl.X] + (int)blockIdx.x;                                                \
+// (The kernels take the body as a macro: through a device function, the
+// compiler keeps a copy of the list argument in scratch, and the dual-number
+// kernel of dd bras, 3.5 KB of scratch, then returned wrong potentials.)
+#define QX_J_BODY(L1, bx, by, ny, ...)\
+    const int u = jl.uoff[jl.X] + (int)(bx);                                                             \
     const int P = A_.pp.pair[u];                                                                  \
     if (A_.e.frag_skip && A_.e.frag_skip[A_.e.pair_frag[P]]) return;                              \
     constexpr int N1 = qx_nherm(L1);                                                              \
@@ -317,28 +318,50 @@ __device__ __forceinline__ void qx_j_kets(const QxArgs& A_, const QxJList& jl, i
       }                                                                                           \
       const int len = hi - lo;                                                                    \
       if (len <= 0) continue;                                                                     \
-      const int v0 = r.first + lo + (int)((long long)len * blockIdx.y / gridDim.y);               \
-      const int v1 = r.first + lo + (int)((long long)len * (blockIdx.y + 1) / gridDim.y);         \
+      const int v0 = r.first + lo + (int)((long long)len * (by) / (ny));                              \
+      const int v1 = r.first + lo + (int)((long long)len * ((by) + 1) / (ny));                        \
       switch (Y == 0 ? 0 : Y == 1 ? 1 : Y <= 3 ? 2 : Y - 1) {                                     \
-        CASES                                                                                     \
+        __VA_ARGS__                                                                               \
       }                                                                                           \
     }                                                                                             \
     const long long m = jl.uoff[jl.X + 1] - jl.uoff[jl.X];                                        \
     _Pragma("unroll") for (int t = 0; t < N1; ++t) {                                              \
       const G s = qx_wave_total(j[t]);                                                            \
-      if (__lane_id() == 0) qx_potential_add(s, jl.P, jl.Pd, jl.hoff[jl.X] + t * m + blockIdx.x); \
-    }                                                                                             \
+      if (__lane_id() == 0) qx_potential_add(s, jl.P, jl.Pd, jl.hoff[jl.X] + t * m + (bx));         \
+    }
+#define QX_DEFINE_J_BODY(L1, ...)                                                                 \
+  template <typename G, typename R>                                                               \
+  __device__ __forceinline__ void qx_jb_##L1(const QxArgs& A_, const QxJList& jl, int x, int y, int n) { \
+    QX_J_BODY(L1, x, y, n, __VA_ARGS__)                                                           \
+  }
+#define QX_DEFINE_J_KERNEL(L1, WITH32, ...)                                                       \
+  template <typename G, typename R>                                                               \
+  __global__ __launch_bounds__(QX_BLOCK_MAX) void qx_jeng_##L1(QxArgs A_, QxJList jl) {           \
+    QX_J_BODY(L1, blockIdx.x, blockIdx.y, gridDim.y, __VA_ARGS__)                                 \
   }                                                                                               \
+  extern "C" int qx_launch_jengv_##L1(const QxArgs*, const QxJList*, int, int, hipStream_t);      \
   /* type: 0 FP64, 1 FP32 recursion, 2 derivative along tv */                                       \
   extern "C" int qx_launch_jeng_##L1(const QxArgs* a, const QxJList* jl, int type, int block, int split, hipStream_t s) { \
     const int nu = jl->uoff[jl->X + 1] - jl->uoff[jl->X];                                         \
     if (nu <= 0) return 0;                                                                        \
+    if (type == 2) return qx_launch_jengv_##L1(a, jl, block, split, s);                           \
     const dim3 grid((unsigned)nu, (unsigned)split);                                               \
     if (type == 0) hipLaunchKernelGGL((qx_jeng_##L1<double, double>), grid, dim3(block), 0, s, *a, *jl); \
-    else if (type == 1) {                                                                         \
+    else {                                                                                        \
       if constexpr (WITH32) hipLaunchKernelGGL((qx_jeng_##L1<double, float>), grid, dim3(block), 0, s, *a, *jl); \
       else return -1;                                                                             \
-    } else hipLaunchKernelGGL((qx_jeng_##L1<qx_dual, qx_dual>), grid, dim3(block), 0, s, *a, *jl); \
+    }                                                                                             \
+    return (int)hipGetLastError();                                                                \
+  }
+#define QX_DEFINE_JV_KERNEL(L1, ...)                                                              \
+  __global__ __launch_bounds__(QX_BLOCK_MAX) void qx_jengv_##L1(QxArgs A_, QxJList jl) {          \
+    using G = qx_dual;                                                                            \
+    using R = qx_dual;                                                                            \
+    QX_J_BODY(L1, blockIdx.x, blockIdx.y, gridDim.y, __VA_ARGS__)                                 \
+  }                                                                                               \
+  extern "C" int qx_launch_jengv_##L1(const QxArgs* a, const QxJList* jl, int block, int split, hipStream_t s) { \
+    const dim3 grid((unsigned)(jl->uoff[jl->X + 1] - jl->uoff[jl->X]), (unsigned)split);          \
+    hipLaunchKernelGGL(qx_jengv_##L1, grid, dim3(block), 0, s, *a, *jl);                          \
     return (int)hipGetLastError();                                                                \
   }
 
@@ -356,13 +379,12 @@ __device__ __forceinline__ void qx_load_block(const double* d, int stride, doubl
 struct QxKBlock {
   int P1, j0, j1, kst, W, col0;
 };
-__device__ __forceinline__ bool qx_k_block(const QxArgs& A_, const QxKList& kl, QxKBlock& b) {
-  const int i = blockIdx.x;
+__device__ __forceinline__ bool qx_k_block(const QxArgs& A_, const QxKList& kl, int i, int part, QxKBlock& b) {
   b.P1 = kl.bra0 + i;
   int lo = 0, hi = (int)(kl.prefix[i + 1] - kl.prefix[i]);
   if (kl.sel == 1) hi = min(hi, kl.n64[i]);
   if (kl.sel == 2) lo = min(hi, kl.n64[i]);
-  b.j0 = lo + (int)blockIdx.y * kl.chunk;
+  b.j0 = lo + part * kl.chunk;
   b.j1 = min(hi, b.j0 + kl.chunk);
   if (b.j0 >= hi) return false;
   if (A_.e.frag_skip && A_.e.frag_skip[A_.e.pair_frag[b.P1]]) return false;
@@ -370,6 +392,10 @@ __device__ __forceinline__ bool qx_k_block(const QxArgs& A_, const QxKList& kl, 
   b.W = A_.e.kcols > 0 ? A_.e.kcols : A_.e.nbf;
   b.col0 = A_.e.frag_col0 ? A_.e.frag_col0[A_.e.pair_frag[b.P1]] : 0;
   return true;
+}
+
+__device__ __forceinline__ bool qx_k_block(const QxArgs& A_, const QxKList& kl, QxKBlock& b) {
+  return qx_k_block(A_, kl, blockIdx.x, blockIdx.y, b);
 }
 
 // Zeroes the K' rows (and fills the density rows behind them).
@@ -429,12 +455,9 @@ __device__ __forceinline__ void qx_k_add(const QxArgs& A_, const QxKBlock& b, in
 }
 
 // K kernel of a light class: one lane per contracted quartet.
-#define QX_DEFINE_K_KERNEL(NAME, NA, NB, NC, ND, WITH32)                                          \
+#define QX_DEFINE_K_BODY(NAME, NA, NB, NC, ND)                                                    \
   template <typename R, bool ROWS, bool STAGE>                                                    \
-  __global__ __launch_bounds__(QX_BLOCK_MAX) void qx_kk_##NAME(QxArgs A_, QxKList kl) {           \
-    HIP_DYNAMIC_SHARED(double, qx_sk)                                                             \
-    QxKBlock b;                                                                                   \
-    if (!qx_k_block(A_, kl, b)) return;                                                           \
+  __device__ __forceinline__ void qx_kd_##NAME(const QxArgs& A_, const QxKList& kl, const QxKBlock& b, double* qx_sk) { \
     if (ROWS) qx_k_rows_begin<NA, NB, STAGE>(A_, b, qx_sk);                                       \
     const int n_ = A_.e.nbf;                                                                      \
     for (int t = (int)threadIdx.x; t < (b.j1 - b.j0) * kl.sub; t += (int)blockDim.x) {            \
@@ -460,6 +483,14 @@ __device__ __forceinline__ void qx_k_add(const QxArgs& A_, const QxKBlock& b, in
       qx_k_add<NA, NB, NC, ND, ROWS>(A_, b, P2, qx_sk, kac, kad, kbc, kbd);                       \
     }                                                                                             \
     if (ROWS) qx_k_rows_end<NA, NB>(A_, b, qx_sk);                                                \
+  }
+#define QX_DEFINE_K_KERNEL(NAME, NA, NB, NC, ND, WITH32)                                          \
+  QX_DEFINE_K_BODY(NAME, NA, NB, NC, ND)                                                          \
+  template <typename R, bool ROWS, bool STAGE>                                                    \
+  __global__ __launch_bounds__(QX_BLOCK_MAX) void qx_kk_##NAME(QxArgs A_, QxKList kl) {           \
+    HIP_DYNAMIC_SHARED(double, qx_sk)                                                             \
+    QxKBlock b;                                                                                   \
+    if (qx_k_block(A_, kl, b)) qx_kd_##NAME<R, ROWS, STAGE>(A_, kl, b, qx_sk);                    \
   }                                                                                               \
   QX_DEFINE_K_LAUNCHER(NAME, NA, NB, qx_kk_##NAME, WITH32, L->block > 0 ? L->block : QX_BLOCK, 0)
 
@@ -487,4 +518,49 @@ __device__ __forceinline__ void qx_k_add(const QxArgs& A_, const QxKBlock& b, in
       return -1;                                                                                  \
     }                                                                                             \
     return qx_k_go_##NAME<double>(a, L);                                                          \
+  }
+
+// ---- small s, p molecules ------------------------------------------------------
+// Every K and J list of a context without d shells in one launch: the lists'
+// workgroups one after the other, each of QX_SMALL_BLOCK threads.  A molecule
+// of a few atoms leaves most of the device idle in any one of the nine
+// kernels, whose times (7-16 us each, a chain of loads and one primitive loop)
+// and launches then add up.
+#define QX_SMALL_BLOCK 128
+struct QxSmall {
+  QxKList k[6];   // 0000, 1000, 1010, 1100, 1110, 1111
+  QxJList j[3];   // bra ss, ps, pp
+  int end[9];     // workgroups of the lists up to each one
+  int split;      // workgroups that share a J bra's kets
+};
+#define QX_DEFINE_SMALL()                                                                         \
+  __global__ __launch_bounds__(QX_SMALL_BLOCK) void qx_small(QxArgs A_, QxSmall sm) {             \
+    HIP_DYNAMIC_SHARED(double, qx_sk)                                                             \
+    const int w = blockIdx.x;                                                                     \
+    int i = 0;                                                                                    \
+    while (i < 8 && w >= sm.end[i]) ++i;                                                          \
+    const int at = w - (i ? sm.end[i - 1] : 0);                                                   \
+    if (i >= 6) {                                                                                 \
+      const int by = at % sm.split, bx = at / sm.split;                                           \
+      if (i == 6) qx_jb_0<double, double>(A_, sm.j[0], bx, by, sm.split);                         \
+      else if (i == 7) qx_jb_1<double, double>(A_, sm.j[1], bx, by, sm.split);                    \
+      else qx_jb_2<double, double>(A_, sm.j[2], bx, by, sm.split);                                \
+      return;                                                                                     \
+    }                                                                                             \
+    const QxKList& kl = sm.k[i];                                                                  \
+    QxKBlock b;                                                                                   \
+    if (!qx_k_block(A_, kl, at % kl.nbra, at / kl.nbra, b)) return;                               \
+    switch (i) {                                                                                  \
+      case 0: qx_kd_e0000_0<double, true, true>(A_, kl, b, qx_sk); break;                         \
+      case 1: qx_kd_e1000_0<double, true, true>(A_, kl, b, qx_sk); break;                         \
+      case 2: qx_kd_e1010_0<double, true, true>(A_, kl, b, qx_sk); break;                         \
+      case 3: qx_kd_e1100_0<double, true, true>(A_, kl, b, qx_sk); break;                         \
+      case 4: qx_kd_e1110_0<double, true, true>(A_, kl, b, qx_sk); break;                         \
+      default: qx_kd_e1111_0<double, true, true>(A_, kl, b, qx_sk); break;                        \
+    }                                                                                             \
+  }                                                                                               \
+  extern "C" int qx_launch_small(const QxArgs* a, const QxSmall* sm, unsigned lds, hipStream_t s) { \
+    if (sm->end[8] <= 0) return 0;                                                                \
+    hipLaunchKernelGGL(qx_small, dim3((unsigned)sm->end[8]), dim3(QX_SMALL_BLOCK), lds, s, *a, *sm); \
+    return (int)hipGetLastError();                                                                \
   }

@@ -274,7 +274,7 @@ __global__ void k_pairm_scatter(int nc, const double* M, long long ld, long long
 #define PM_LDS_TRI (150 * 1024)  // a triangle takes one panel up to here (n <= 195)
 #define PM_LDS_ROWS (72 * 1024)  // rows of a panel beyond: two workgroups per CU
 // An output row pair goes out without a stay in the caches: nothing reads it here.
-typedef double pm_dv2 __attribute__((ext_vector_type(2)));
+typedef double pm_dv2 __attribute__((vector_size(16)));
 template <bool TRI>
 __global__ __launch_bounds__(1024) void k_pairm_expand(int n, const double* M, long long ld, long long slice,
                                                       const int* index, const int* fn, int rows, double* out) {
