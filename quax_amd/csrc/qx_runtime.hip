@@ -1113,7 +1113,13 @@ static QxKList k_list(const qx_ctx* c, const QxWorkHost& wh, int sel, int block,
   kl.sub = (int)std::max<long long>(1, std::min<long long>({prims, 64, QX_SUB_LANES / std::max(wh.ncq, 1LL)}));
   const long long most = (wh.ncq + QX_K_BLOCKS - 1) / QX_K_BLOCKS;
   const long long per = std::max<long long>(rows ? std::max(most, std::min(4 * most, QX_K_CHUNK / prims)) : most, 1);
-  const int unit = block ? std::max(1, block / kl.sub) : 32;
+  // quadrature: in short lists as little as one step of each of a block's four
+  // wavefronts (60 functions: a derivative tensor's kernels 1.27 ms in shares
+  // of 32 kets, 0.70 ms so; of the long lists of 280 functions' gradient shares
+  // of 40 cost 2 % more than of 64)
+  static const int kPairFns[6] = {1, 3, 9, 6, 18, 36};
+  const int step = 4 * (64 / kPairFns[wh.bra_class]);
+  const int unit = block ? std::max(1, block / kl.sub) : per <= 16 ? std::min(step, 32) : 32;
   kl.chunk = (int)std::min<long long>((per + unit - 1) / unit * unit, 1 << 20);
   return kl;
 }
@@ -1268,7 +1274,9 @@ static void add_j_launches(qx_ctx* c, const QxEpiDev& e, const unsigned (&f32)[6
   static const int order[6] = {0, 1, 2, 2, 3, 4};
   const int nu_all = c->jlist.uoff[6];
   // a workgroup walks every ket of its bra pseudo pair; with few bras the
-  // walk is shared out
+  // walk is shared out.  (Not further by class: every workgroup passes through
+  // the code of all ket classes, and the 210 dd bras of 280 functions took
+  // 587 us in 9 shares each, 160 us whole.)
   const int split = std::min(8, std::max(1, 2048 / std::max(nu_all, 1)));
   const int block = nu_all / split >= 512 ? 256 : 64;
   for (int X = 5; X >= 0; --X) {
