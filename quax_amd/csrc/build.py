@@ -147,13 +147,19 @@ def kernel_scratch(obj: str, tmp: str) -> list:
 
 
 def check_streaming_scratch(objs, verbose=True):
-    """Fails the build when a streaming J/K (cls_*_j*) or adjoint-gradient
-    (cls_*_g*) kernel needs more than STREAMING_SCRATCH_MAX bytes of scratch
-    per lane."""
+    """Fails the build when a kernel that runs on side streams needs more than
+    STREAMING_SCRATCH_MAX bytes of scratch per lane: K (cls_*_j*), J (jeng*),
+    gradient (cls_*_g*), tensor (cls_*_r*, cls_*_d*) and second-derivative
+    (cls_*_v*) kernels, and the array form (cls_*_e) of the classes without a
+    quadrature one."""
     if not os.path.exists(os.path.join(LLVM_BIN, "clang-offload-bundler")):
         print("scratch check skipped: no clang-offload-bundler", flush=True)
         return
-    streaming = [o for o in objs if re.match(r"cls_\d{4}_[jg]\d+\.hip\.", os.path.basename(o))]
+    names = [os.path.basename(o) for o in objs]
+    quad = {n[4:8] for n in names if re.match(r"cls_\d{4}_r0\.hip\.", n)}
+    streaming = [o for o, n in zip(objs, names)
+                 if re.match(r"(cls_\d{4}_[jgrdv]\d+|jengv?_\d)\.hip\.", n)
+                 or (re.match(r"cls_\d{4}_e\.hip\.", n) and n[4:8] not in quad)]
     worst = ("", 0)
     with tempfile.TemporaryDirectory() as tmp:
         for o in streaming:

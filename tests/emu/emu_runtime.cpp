@@ -28,7 +28,7 @@ void lane_main(int lane) {
     P.bar->arrive_and_wait();  // start of a block (or shutdown)
     if (P.quit.load()) return;
     blockIdx.x = P.cur_block % P.grid.x;
-    blockIdx.y = P.cur_block / P.grid.x;
+    blockIdx.y = (P.cur_block / P.grid.x) % P.grid.y; blockIdx.z = P.cur_block / (P.grid.x * P.grid.y);
     blockDim = P.block;
     gridDim = P.grid;
     if ((unsigned)lane < P.block.x) P.body();
@@ -50,9 +50,11 @@ static unsigned wave_size(unsigned l) {
   return std::min<unsigned>(64, g_sync_n - w0);
 }
 
+void wave_sync() { wave_bar().arrive_and_wait(); }
+
 void run_grid(dim3 grid, dim3 block, const std::function<void()>& body) {
-  const int lanes = 256;
-  if (block.x > 256) {
+  const int lanes = 512;
+  if (block.x > 512) {
     std::fprintf(stderr, "emu: block size %u > 256 not supported\n", block.x);
     std::abort();
   }

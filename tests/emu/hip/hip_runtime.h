@@ -59,6 +59,11 @@ inline hipError_t hipMalloc(void** p, size_t n) {
   *p = std::malloc(n);
   return *p ? hipSuccess : hipErrorOutOfMemory;
 }
+template <class T>
+inline hipError_t hipMalloc(T** p, size_t n) { return hipMalloc(reinterpret_cast<void**>(p), n); }
+#define __align__(n) __attribute__((aligned(n)))
+#define HIP_SYMBOL(x) ((const void*)(x))
+inline hipError_t hipGetSymbolAddress(void** p, const void* sym) { *p = const_cast<void*>(sym); return hipSuccess; }
 inline hipError_t hipFree(void* p) {
   std::free(p);
   return hipSuccess;
@@ -104,9 +109,12 @@ int shfl_xor(int v, int off);
 unsigned long long ballot(bool p);
 void syncthreads();
 int syncthreads_or(int p);
+void wave_sync();
 }  // namespace emu
 
 #define __syncthreads() emu::syncthreads()
+#define __builtin_amdgcn_fence(a, b) ((void)0)
+#define __builtin_amdgcn_wave_barrier() emu::wave_sync()
 inline int __syncthreads_or(int p) { return emu::syncthreads_or(p); }
 inline double __shfl_xor(double v, int off, int = 64) { return emu::shfl_xor(v, off); }
 inline int __shfl_xor(int v, int off, int = 64) { return emu::shfl_xor(v, off); }
@@ -160,3 +168,8 @@ inline void emu_launch(K kernel, dim3 grid, dim3 block, size_t shmem, A... args)
 
 using std::max;
 using std::min;
+inline int __builtin_amdgcn_readfirstlane(int x) { return x; }
+inline void __builtin_amdgcn_sched_barrier(int) {}
+template <class T> inline void __builtin_nontemporal_store(T v, T* p) { *p = v; }
+struct alignas(16) double2 { double x, y; };
+inline double2 make_double2(double x, double y) { return {x, y}; }
