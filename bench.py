@@ -44,6 +44,7 @@ def kernel_table(eng):
     """Per profile slot: kernel name and algorithmic flops per primitive
     quartet (including the epilogue contraction)."""
     import ctypes
+    from quax_amd.csrc import gen_eri  # which classes run by quadrature
     L = eng.L
     ncart = lambda l: (l + 1) * (l + 2) // 2
     classes = {}
@@ -77,9 +78,15 @@ def kernel_table(eng):
         if kind.value == 0:
             info[slot] = (f"qx_k_e{nm}<{tp}>", ef, nm, key)
         elif kind.value == 2:
-            info[slot] = (f"qx_kj_e{nm}_{part.value}<{tp}>", jf[part.value] if part.value < njk else 0.0, nm, key)
+            # part 0: K of the class; part 1: J of the bra pairs (la, lb), booked under (la lb|la lb)
+            args = ", ".join(map(str, l4))
+            name = f"qx_rk<{args}, {tp}>" if nm in gen_eri.RYS_K else f"qx_kk_e{nm}_{part.value}<{tp}>"
+            if part.value:
+                name = f"qx_jeng_{l4[0] + l4[1]}<{tp}>"
+            info[slot] = (name, jf[part.value] if part.value < njk else 0.0, nm, key)
         elif part.value < npart:
-            info[slot] = (f"qx_kg_d{nm}_g{part.value}<{tp}>", pf[part.value], nm, key)
+            name = f"qx_rg<{', '.join(map(str, l4))}>" if nm in gen_eri.RYS_G else f"qx_kg_d{nm}_g{part.value}<{tp}>"
+            info[slot] = (name, pf[part.value], nm, key)
         else:
             info[slot] = (f"unused slot {slot}", 0.0, nm, key)
     return info

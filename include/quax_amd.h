@@ -266,19 +266,18 @@ int qx_scf_matrix(qx_scf* scf, int which, double* out, void* stream);
 void qx_scf_destroy(qx_scf* scf);
 const char* qx_scf_last_error(const qx_scf* scf);
 
-/* Quartet tiles (no reference counterpart): threads per workgroup -- the
- * primitive quartets one workgroup evaluates, and the quartets that share
- * its LDS K' rows -- of the streaming kernels of each class, per pass
+/* Quartet tiles (no reference counterpart): threads per workgroup, and so the
+ * quartets that share its LDS K' rows, of the K and gradient kernels with one
+ * lane per quartet (the quadrature classes ignore it), per pass
  * (0 = J/K, 1 = adjoint gradient); block[qx_num_classes()], multiples of
  * 64 up to 256, or NULL for the built-in table (picked by the autotuner,
  * quax_amd/csrc/tune.py --tiles, from GPU timings). */
 int qx_set_class_tiles(qx_ctx* ctx, int pass, const int* block);
 int qx_get_class_tiles(const qx_ctx* ctx, int pass, int* block);
 /* Per class (flags[qx_num_classes()], NULL = built-in table): whether the
- * adjoint-gradient kernels sum the terms of centres that are the same atom
- * on every lane of a wavefront across the wavefront before their LDS
- * accumulators (cheaper LDS atomics, ~200 cross-lane operations per wave);
- * the autotuner picks it per class. */
+ * adjoint-gradient kernels sum the bra centres' terms across the wavefront
+ * before they add them to the LDS accumulators at the end of a workgroup; the
+ * autotuner picks it per class. */
 int qx_set_grad_wave_reduce(qx_ctx* ctx, const int* flags);
 int qx_get_grad_wave_reduce(const qx_ctx* ctx, int* flags);
 /* Per class (copies[qx_num_classes()], 1..64, NULL = built-in table): how
@@ -357,9 +356,9 @@ int qx_max_parts(void);
  * arrays of qx_max_parts() entries.  Derivative profile slots of the gradient
  * pass are indexed by group. */
 int qx_class_groups(int cls, int* ngroups, double* flops, int* nparts);
-/* The J/K pass launches one kernel per range of a components of a class:
- * number of parts and FP operations per primitive quartet of each (J/K
- * epilogue included); flops holds up to 8 entries. */
+/* Parts of a class's K kernel (one) and its FP operations per primitive
+ * quartet (contraction included); flops holds up to 8 entries.  The J kernels
+ * are booked as part 1 of the classes (X|X). */
 int qx_class_jk(int cls, int* nparts, double* flops);
 int qx_profile_enable(qx_ctx* ctx, int on);
 int qx_profile_read(qx_ctx* ctx, double* ms, long long* launches, long long* pquartets);

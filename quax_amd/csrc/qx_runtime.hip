@@ -1312,6 +1312,7 @@ static void add_j_launches(qx_ctx* c, const QxEpiDev& e, const unsigned (&f32)[6
 static int mixed_mode(const qx_ctx* c, size_t i, int pass) {
   const auto& S = c->split;
   const long long p64 = S.pq64[i], p32 = S.pq32[i];
+  if (pass == 1 && qx_rys_g[c->work[i].cls]) return 0;  // the quadrature gradient has no FP32 form
   if (!c->fp32_ok[pass][c->work[i].cls] || p32 < QX_MIXED_MIN_FRAC * (double)(p64 + p32)) return 0;
   return p64 == 0 ? 1 : 2;
 }
