@@ -614,6 +614,35 @@ def emit_small(outdir):
     return path
 
 
+def emit_small_grad(outdir):
+    """grad_small.hip: every gradient body of s and p shells in one kernel;
+    also the class of each of its lists."""
+    out, cases, lists = [], [], []
+    for ci, cls in enumerate(canonical_classes(1)[1]):
+        nm = "".join(map(str, cls))
+        for pi, part in enumerate(deriv_parts(cls)):
+            out += [emit_deriv_core(cls, pi, part)[0], ""]
+            cases += [f"    case {len(lists)}:",
+                      "      qx_grad_block(A_, kl, b, sg, [&](int P1, int P2, int u1, int u2, double (&g)[QX_GRAD_NCOMB]) {",
+                      f"        qx_gr_d{nm}_{pi}<double>(A_, P1, P2, u1, u2, g);", "      });", "      break;"]
+            lists.append(ci)
+    n = len(lists)
+    out += [f"__constant__ int qx_small_class[{n}] = {{{', '.join(map(str, lists))}}};",
+            "__global__ __launch_bounds__(QX_SMALL_BLOCK) void qx_small_grad(QxArgs A_, QxSmallGrad sm) {",
+            "  __shared__ double sg[QX_GRAD_LDS];", "  const int w = blockIdx.x;", "  int i = 0;",
+            f"  while (i < {n - 1} && w >= sm.end[i]) ++i;", "  const int at = w - (i ? sm.end[i - 1] : 0);",
+            "  const QxKList& kl = sm.k[qx_small_class[i]];", "  QxKBlock b;",
+            "  if (!qx_k_block(A_, kl, at % kl.nbra, at / kl.nbra, b)) return;", "  switch (i) {"] + cases + ["  }", "}",
+            'extern "C" int qx_launch_small_grad(const QxArgs* a, const QxSmallGrad* sm, hipStream_t s) {',
+            f"  if (sm->end[{n - 1}] <= 0) return 0;",
+            f"  hipLaunchKernelGGL(qx_small_grad, dim3((unsigned)sm->end[{n - 1}]), dim3(QX_SMALL_BLOCK), 0, s, *a, *sm);",
+            "  return (int)hipGetLastError();", "}"]
+    path = os.path.join(outdir, "grad_small.hip")
+    with open(path, "w") as fh:
+        fh.write("\n".join(['#include "../qx_grad.h"', ""] + out + [""]))
+    return path, lists
+
+
 def emit_oei(la, lb, outdir):
     """oei_<la><lb>.hip: the attraction recurrences of one shell-pair class
     (the ERI bra recurrence with W - P = C - P and the (ss|ss) integrals
@@ -855,7 +884,9 @@ def emit_class_files(cls, outdir, fp32):
         kern = ["template <typename R>",
                 f"__global__ __launch_bounds__(QX_BLOCK_MAX){attr} void qx_kg_d{nm}_g{gi}(QxArgs A_, QxKList kl) {{",
                 "  __shared__ double sg[QX_GRAD_LDS];",
-                "  qx_grad_block(A_, kl, sg, [&](int P1, int P2, int u1, int u2, double (&g)[QX_GRAD_NCOMB]) {",
+                "  QxKBlock b;",
+                "  if (!qx_k_block(A_, kl, b)) return;",
+                "  qx_grad_block(A_, kl, b, sg, [&](int P1, int P2, int u1, int u2, double (&g)[QX_GRAD_NCOMB]) {",
                 f"    qx_gr_d{nm}_{pi}<R>(A_, P1, P2, u1, u2, g);", "  });", "}",
                 f"QX_DEFINE_GRAD_LAUNCHER(d{nm}_g{gi}, {1 if fp32 else 0})"]
         write(f"cls_{nm}_g{gi}.hip", [gsrc[pi] for pi in members] + [""] + kern, "qx_grad.h")
@@ -882,6 +913,8 @@ def main():
     for L in range(2 * lmax + 1):
         files += emit_j(L, outdir, lmax, fp32)
     files.append(emit_small(outdir))
+    path, small = emit_small_grad(outdir)
+    files.append(path)
     with open(os.path.join(outdir, "qx_rys.inc"), "w") as fh:
         fh.write(rys_tables())
     D = ["// generated: kernel launch tables indexed by canonical class id", "#pragma once",
@@ -944,6 +977,9 @@ def main():
         D.append(f"static const unsigned char qx_rys_{name}[QX_NUM_CLASSES] = {{")
         D.append("  " + ", ".join(str(int("".join(map(str, cls)) in table)) for cls in classes))
         D.append("};")
+    D.append('extern "C" int qx_launch_small_grad(const QxArgs*, const QxSmallGrad*, hipStream_t);')
+    D.append(f"static const int qx_small_grad_class[{len(small)}] = {{{', '.join(map(str, small))}}};")
+    D.append(f"#define QX_SMALL_GRADS {len(small)}")
     D.append('extern "C" int qx_launch_small(const QxArgs*, const QxSmall*, unsigned, hipStream_t);')
     D.append("// one-electron kernels per shell-pair class")
     D += [f'extern "C" int qx_launch_oei_{a}{b}(const QxOei*, int, hipStream_t);' for a, b in pairs]

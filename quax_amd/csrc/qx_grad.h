@@ -61,9 +61,7 @@ __device__ __forceinline__ void qx_grad_bra(const QxArgs& A_, const QxGradTarget
 // d/dA, d/dB, d/dC sums.
 #define QX_GRAD_NCOMB 9
 template <class Part>
-__device__ __forceinline__ void qx_grad_block(const QxArgs& A_, const QxKList& kl, double* sg, Part part) {
-  QxKBlock b;
-  if (!qx_k_block(A_, kl, b)) return;
+__device__ __forceinline__ void qx_grad_block(const QxArgs& A_, const QxKList& kl, const QxKBlock& b, double* sg, Part part) {
   const QxGradTarget tgt = qx_grad_begin(A_, kl, b.P1, sg);
   const int u1 = A_.pr.pp_first[b.P1], n1 = A_.pr.pp_n[b.P1];
   double gb[6] = {};
@@ -104,3 +102,10 @@ __device__ __forceinline__ void qx_grad_block(const QxArgs& A_, const QxKList& k
     }                                                                                             \
     return (int)hipGetLastError();                                                                \
   }
+
+// Every gradient kernel of a context without d shells in one launch (as
+// qx_small of the J/K pass): QX_SMALL_GRADS of them, each a class's list.
+struct QxSmallGrad {
+  QxKList k[6];  // per class: 0000, 1000, 1010, 1100, 1110, 1111
+  int end[16];   // workgroups of the kernels up to each one
+};

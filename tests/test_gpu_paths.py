@@ -52,9 +52,9 @@ def test_one_launch_pass_equals_separate_kernels(gpu, symbols):
     bs = BasisSet.build(mol, "sto-3g", pure=False)
     D = _density(bs.nbf(), 1)
     with _engine(mol, bs, ints_tol=1e-12) as eng:
-        one = eng.jk(D)
+        one = (*eng.jk(D), eng.eri_grad(D))
         eng.profile(True)
-        for a, b in zip(one, eng.jk(D)):
+        for a, b in zip(one, (*eng.jk(D), eng.eri_grad(D))):
             _close(a, b)
 
 
