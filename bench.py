@@ -544,7 +544,7 @@ def main():
     eng.set_streams(args.streams)
 
     table = kernel_table(eng)
-    eri_slots = [k for k in range(len(ms)) if table[k][0].startswith("qx_kj")]
+    eri_slots = [k for k in range(len(ms)) if table[k][3].startswith("jk")]
     eri_ms = float(ms[eri_slots].sum()) / args.steps
     deri_ms = float(ms.sum()) / args.steps - eri_ms
     slot = int(np.argmax(ms))
