@@ -309,7 +309,12 @@ def _classes(var, default):
 
 
 # classes whose K, adjoint gradient and (stored) integrals come from the
-# Rys-quadrature kernels (qx_rys.h) instead of the one-lane-per-quartet bodies
+# Rys-quadrature kernels (qx_rys.h) instead of the one-lane-per-quartet bodies.
+# 280 functions, one lane / quadrature in us: K 2110 183/797, 2111 283/308, 2120
+# 299/412, 2210 119/373, 2220 350/289 (but 7.4/12.4 ms in FP32 at 672 functions),
+# 2121 829/288, 2211 530/228; gradient 1111 216/318, 2020 201/290, 2011 205/472,
+# 2110 370/1608, and the split one-lane bodies of the listed classes 1.3 to 3
+# times the quadrature's
 RYS_K = _classes("QX_RYS_K", "2121 2211 2221 2222")
 RYS_G = _classes("QX_RYS_G", "2111 2120 2121 2210 2211 2220 2221 2222")
 RYS_E = _classes("QX_RYS_E", "2111 2120 2121 2211 2220 2221 2222")

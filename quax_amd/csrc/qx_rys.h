@@ -264,7 +264,8 @@ __device__ __forceinline__ int qx_rys_prims(const QxArgs& A_, int pk0, int nq) {
 // root polynomials would otherwise be waited for in every step, with a
 // handful of lanes busy.  A step's lanes then hand them to the 1D tasks
 // through LDS.  (Read by every 1D task itself, those loads kept the CU's
-// address unit busy four times longer than the arithmetic took.)
+// address unit busy four times longer than the arithmetic took; one step at a
+// time, (dd|ps) of a 280-function gradient took 1.22 ms against 1.08 so.)
 template <class S, int LB, int LD, typename G, typename R, class Begin, class Step, class End>
 __device__ __forceinline__ void qx_rys_walk(const QxArgs& A_, const QxKList& kl, const QxKBlock& b, R* g, Begin begin, Step step,
                                             End end) {
@@ -364,6 +365,11 @@ __device__ __forceinline__ void qx_rys_sum(const R* gq, int ox, int oy, int oz, 
 }
 
 // ---- K ------------------------------------------------------------------------
+// Bound by latency at two or three wavefronts per SIMD (a quarter of the FP64
+// issue rate) and LDS.  K'_a then K'_b: a lane's sums over (c, d) are added
+// over its quartet's lanes in LDS, one atomic per row element instead of one
+// per lane ((dd|dp) of 280 functions 457 -> 357 us, (dp|dp) 403 -> 336, with
+// larger shares of kets per workgroup 322 and 291).
 template <int LA, int LB, int LC, int LD, typename G, typename R, bool ROWS, bool STAGE>
 __global__ __launch_bounds__(QX_RYS_BLOCK_MAX) void qx_rk(QxArgs A_, QxKList kl) {
   using S = QxRys<LA, LB, LC, LD, 0>;
@@ -621,7 +627,10 @@ __global__ __launch_bounds__(QX_RYS_BLOCK) void qx_rd(QxArgs A_, QxKList kl, QxP
 // lane's (a, b) and every (c, d); summed against the derivative integrals.
 // Per root the sum over (c, d) goes to the adjoint of each direction's 1D
 // values first (w: 5 multiply-adds per (c, d)), which then meets the raised
-// and lowered values: the nine derivative values per (c, d) are never formed.
+// and lowered values: the nine derivative values per (c, d) are never formed
+// ((dd|dp) of 280 functions: 1.77 ms at one wavefront per SIMD -> 0.98 at two).
+// Bound by LDS reads and FP64 issue in about equal parts at two wavefronts per
+// SIMD; three (168 registers) spill and take 2.2 ms.
 template <int LA, int LB, int LC, int LD, typename G>
 __global__ __launch_bounds__(QX_RYS_BLOCK, sizeof(G) == 8 && qx_ncart(LC) * qx_ncart(LD) < 36 ? 2 : 1) void qx_rg(QxArgs A_, QxKList kl) {
   using S = QxRys<LA, LB, LC, LD, 1>;
@@ -735,6 +744,7 @@ __global__ __launch_bounds__(QX_RYS_BLOCK, sizeof(G) == 8 && qx_ncart(LC) * qx_n
       [&]() QX_INLINE {
         // the ket centres' terms, summed over the quartet's lanes in LDS: one
         // LDS atomic per lane and direction would meet G-fold on each address
+        // ((dd|ps) of 280 functions: 1.08 -> 0.79 ms)
         static_assert(6 * S::SUM * sizeof(double) <= S::LDS * sizeof(G), "LDS of the lane sums");
         double* const sum = reinterpret_cast<double*>(g);
         qx_wave_sync();
