@@ -128,8 +128,12 @@ int qx_jk_build(qx_ctx* ctx, const double* D, double* J, double* K, int precisio
  * qx_jk_noalloc_capacity() doubles (24 MiB, held by every GPU the library
  * runs on until the process ends): 2 n_cart^2 doubles for Cartesian bases,
  * 5 n_cart^2 for spherical ones; larger contexts return QX_EINVAL with a
- * message.  All kernels run in turn on `stream`.  Calls that overlap on one
- * GPU share the array and race; the array is cleared on every call. */
+ * message.  Its other work memory belongs to the context, was allocated by
+ * qx_initialize and is used by this call alone.  All kernels run in turn on
+ * `stream`, without events (qx_profile_* does not see them).  A call may
+ * overlap the context's other passes on another stream; two of these calls
+ * that overlap on one GPU share the array and race.  What a call accumulates
+ * into is cleared on every call. */
 int qx_jk_build_noalloc(qx_ctx* ctx, const double* D, double* J, double* K, void* stream);
 long long qx_jk_noalloc_capacity(void);
 

@@ -98,6 +98,7 @@ struct qx_ctx {
   QxRange* d_range = nullptr;
   QxJList jlist{};
   double* d_herm = nullptr;
+  double* d_herm_own = nullptr;          // value parts (H, P) of qx_jk_build_noalloc
   long long nherm = 0;
   double* d_rys = nullptr;
   // pair-matrix workspace of the tensor entry points, kept up to

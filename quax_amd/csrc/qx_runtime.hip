@@ -198,10 +198,10 @@ hipEvent_t take_event(qx_ctx* c) {
 }
 
 // Runs one kernel launch, bracketed by HIP events on its stream when
-// profiling is on.
+// profiling is on (and the pass may use events: `timed`).
 template <class F>
-int timed_launch(qx_ctx* c, int slot, long long pq, hipStream_t s, F&& launch) {
-  if (!c->profiling || pq <= 0) return launch();
+int timed_launch(qx_ctx* c, int slot, long long pq, hipStream_t s, F&& launch, bool timed = true) {
+  if (!timed || !c->profiling || pq <= 0) return launch();
   hipEvent_t a = take_event(c), b = take_event(c);
   QX_HIP(hipEventRecord(a, s));
   const int rc = launch();
@@ -348,6 +348,12 @@ std::vector<QxRange> pseudo_ranges(const qx_ctx* c, double bound) {
   return r;
 }
 
+// Work matrices of qx_jk_build_noalloc in the file-scope array `scratch`.
+#define QX_NOALLOC_DOUBLES (3ull << 20)
+// Doubles of it that a context is charged with (the documented limit; a
+// spherical pass uses three of its five matrices).
+size_t noalloc_doubles(const qx_ctx* c) { return (size_t)(c->pure ? 5 : 2) * c->ncart * c->ncart; }
+
 // Hermite layout and J ranges.
 void setup_jk(qx_ctx* c) {
   static const int order[6] = {0, 1, 2, 2, 3, 4};
@@ -373,6 +379,8 @@ void setup_jk(qx_ctx* c) {
   jl.P = c->d_herm + at;
   jl.Hd = c->d_herm + 2 * at;
   jl.Pd = c->d_herm + 3 * at;
+  // the allocation-free pass has its own, as it may run beside another pass
+  if (noalloc_doubles(c) <= QX_NOALLOC_DOUBLES) c->d_herm_own = dalloc<double>(c, (size_t)2 * at);
 }
 
 void schwarz_and_lists(qx_ctx* c) {
@@ -761,7 +769,6 @@ void setup_shell_tables(qx_ctx* c) {
 // bases) or 2 n_cart^2 up to n_cart = 1254 (Cartesian).  Host code never
 // uses the array's name as an address: qx_initialize looks up its device
 // address once per device and keeps it in g_scratch_ptr.
-#define QX_NOALLOC_DOUBLES (3ull << 20)
 static __device__ __align__(256) double scratch[QX_NOALLOC_DOUBLES];
 
 #define QX_MAX_DEVICES 64
@@ -1248,7 +1255,7 @@ static void add_grad_list(qx_ctx* c, const QxWorkHost& wh, const QxEpiDev& e, in
 
 // K kernel of one quartet list, as add_grad_list.
 static void add_k_list(qx_ctx* c, const QxWorkHost& wh, const QxEpiDev& e, int fp32, int sel, long long nq, bool dir,
-                       std::vector<Launch>& out) {
+                       std::vector<Launch>& out, bool timed = true) {
   if (wh.ncq <= 0 || nq <= 0) return;
   const QxClassEntry& ent = qx_class_table[wh.cls];
   const int block = c->tile[0][wh.cls];
@@ -1260,19 +1267,19 @@ static void add_k_list(qx_ctx* c, const QxWorkHost& wh, const QxEpiDev& e, int f
     a.e.krows = e.krows && c->jkrows[wh.cls];
     const int slot = QX_SLOT_JK(wh.cls, k, fp32 ? 1 : 0);
     auto fn = dir ? ent.jkv : ent.jk[k];
-    out.push_back({(double)nq * ent.jk_flops[k], [c, a, fn, fp32, slot, nq, block, kl, dir](hipStream_t st) {
+    out.push_back({(double)nq * ent.jk_flops[k], [c, a, fn, fp32, slot, nq, block, kl, dir, timed](hipStream_t st) {
                      QxLaunch L{fp32, st, block, nullptr, &kl};
-                     if (dir) return fn(&a, &L);
-                     return timed_launch(c, slot, nq, st, [&] { return fn(&a, &L); });
+                     return timed_launch(c, slot, nq, st, [&] { return fn(&a, &L); }, timed && !dir);
                    }});
   }
 }
 
 // J kernels of every bra class.  f32[X]: ket classes whose quartets beyond the
 // FP32 threshold run in FP32 (mixed precision).
-static void add_j_launches(qx_ctx* c, const QxEpiDev& e, const unsigned (&f32)[6], std::vector<Launch>& out) {
+static void add_j_launches(qx_ctx* c, const QxEpiDev& e, const QxJList& lists, const unsigned (&f32)[6],
+                           std::vector<Launch>& out, bool timed) {
   static const int order[6] = {0, 1, 2, 2, 3, 4};
-  const int nu_all = c->jlist.uoff[6];
+  const int nu_all = lists.uoff[6];
   // a workgroup walks every ket of its bra pseudo pair; with few bras the
   // walk is shared out.  (Not further by class: every workgroup passes through
   // the code of all ket classes, and the 210 dd bras of 280 functions took
@@ -1280,23 +1287,23 @@ static void add_j_launches(qx_ctx* c, const QxEpiDev& e, const unsigned (&f32)[6
   const int split = std::min(8, std::max(1, 2048 / std::max(nu_all, 1)));
   const int block = nu_all / split >= 512 ? 256 : 64;
   for (int X = 5; X >= 0; --X) {
-    const long long nu = c->jlist.uoff[X + 1] - c->jlist.uoff[X];
+    const long long nu = lists.uoff[X + 1] - lists.uoff[X];
     if (nu <= 0) continue;
     for (int pass = 0; pass < 2; ++pass) {
       if (pass == 1 && f32[X] == 0) continue;
       const int type = e.tv ? 2 : pass;
       QxArgs a;
       a.pr = c->pr; a.pp = c->pp; a.w = QxWorkDev{}; a.e = e; a.boys = c->d_boys;
-      QxJList jl = c->jlist;
+      QxJList jl = lists;
       jl.X = X;
       jl.f32_classes = f32[X];
       jl.n64 = c->split.d_range64;
       auto fn = qx_j_table[order[X]];
       const int slot = QX_SLOT_JK(class_index(X, X), 1, pass);
       const double flops = 100.0 + 25.0 * (order[X] + 1) * (order[X] + 2);
-      out.push_back({(double)nu * nu_all * flops, [c, a, jl, fn, type, block, split, slot, nu, nu_all](hipStream_t st) {
-                       if (type == 2) return fn(&a, &jl, type, block, split, st);
-                       return timed_launch(c, slot, nu * nu_all, st, [&] { return fn(&a, &jl, type, block, split, st); });
+      out.push_back({(double)nu * nu_all * flops, [c, a, jl, fn, type, block, split, slot, nu, nu_all, timed](hipStream_t st) {
+                       return timed_launch(c, slot, nu * nu_all, st, [&] { return fn(&a, &jl, type, block, split, st); },
+                                           timed && type != 2);
                      }});
     }
   }
@@ -1481,8 +1488,8 @@ int qx_compute_2e_deriv(qx_ctx* c, const int* dv, int len, double* out, void* st
 // registers of the largest class and one block size for all cost more than the
 // launches.
 #define QX_SMALL_QUARTETS 2000000
-static bool small_pass(qx_ctx* c, const QxEpiDev& e, QxSmall& sm, size_t& lds) {
-  if (c->profiling || !e.krows || c->class_pair_cnt[3] + c->class_pair_cnt[4] + c->class_pair_cnt[5] > 0) return false;
+static bool small_pass(qx_ctx* c, const QxEpiDev& e, const QxJList& jl, bool timed, QxSmall& sm, size_t& lds) {
+  if ((timed && c->profiling) || !e.krows || c->class_pair_cnt[3] + c->class_pair_cnt[4] + c->class_pair_cnt[5] > 0) return false;
   if (c->npq_total > QX_SMALL_QUARTETS) return false;
   sm = QxSmall{};
   long long blocks[9] = {};
@@ -1496,11 +1503,11 @@ static bool small_pass(qx_ctx* c, const QxEpiDev& e, QxSmall& sm, size_t& lds) {
     lds = std::max(lds, 2 * (ncart(at < 1 ? 0 : 1) + ncart(at < 3 ? 0 : 1)) * W * sizeof(double));
   }
   if (lds > QX_K_STAGE_MAX) return false;
-  sm.split = std::min(8, std::max(1, 2048 / std::max(c->jlist.uoff[6], 1)));
+  sm.split = std::min(8, std::max(1, 2048 / std::max(jl.uoff[6], 1)));
   for (int X = 0; X < 3; ++X) {
-    sm.j[X] = c->jlist;
+    sm.j[X] = jl;
     sm.j[X].X = X;
-    blocks[6 + X] = (long long)(c->jlist.uoff[X + 1] - c->jlist.uoff[X]) * sm.split;
+    blocks[6 + X] = (long long)(jl.uoff[X + 1] - jl.uoff[X]) * sm.split;
   }
   long long end = 0;
   for (int i = 0; i < 9; ++i) {
@@ -1535,10 +1542,12 @@ static bool small_grad(const qx_ctx* c, QxSmallGrad& sm) {
 }
 
 // J and K of D with work matrices w (2 n_cart^2 doubles, 3 for a spherical
-// basis), or (tv) of the integrals' derivative along tv; side: spread over the
-// side streams.
+// basis), or (tv) of the integrals' derivative along tv.  herm: Hermite
+// densities and potentials (2 nherm doubles) of a pass that may run beside the
+// context's other passes: it touches no memory of theirs, keeps to stream s and
+// uses no events.  Null: the context's, spread over the side streams.
 static void jk_pass(qx_ctx* c, double* w, const double* D, double* J, double* K, int precision, double thr,
-                    const int* frag_skip, const double* tv, hipStream_t s, bool side) {
+                    const int* frag_skip, const double* tv, hipStream_t s, double* herm = nullptr) {
   const size_t nc = c->ncart, n2 = nc * nc;
   double *Jc = w, *Kp = w + n2;
   QxArgs a;
@@ -1557,12 +1566,18 @@ static void jk_pass(qx_ctx* c, double* w, const double* D, double* J, double* K,
   }
   e.tv = tv;
   QxJList jl = c->jlist;
+  const bool alone = herm != nullptr;
+  if (alone) {
+    jl.H = herm;
+    jl.P = herm + c->nherm;
+    jl.Hd = jl.Pd = nullptr;
+  }
   check_launch(qxk_jk_begin(&a, &jl, c->nherm, Jc, Kp, (long long)n2, s), "jk_begin");
   std::vector<Launch> v;
   unsigned f32[6] = {};
   QxSmall sm;
   size_t lds = 0;
-  if (precision == QX_PREC_FP64 && !tv && small_pass(c, e, sm, lds)) {
+  if (precision == QX_PREC_FP64 && !tv && small_pass(c, e, jl, !alone, sm, lds)) {
     check_launch(qx_launch_small(&a, &sm, (unsigned)lds, s), "jk_build");
     check_launch(qxk_j_finish(&a, &jl, Jc, s), "j_finish");
     check_launch(qxk_jk_finish(&c->shells, Jc, Kp, J, K, s), "jk_finish");
@@ -1577,10 +1592,10 @@ static void jk_pass(qx_ctx* c, double* w, const double* D, double* J, double* K,
         f32[wh.ket_class] |= 1u << wh.bra_class;
       }
   } else {
-    for (const auto& wh : c->work) add_k_list(c, wh, e, 0, 0, wh.w.nquart, tv != nullptr, v);
+    for (const auto& wh : c->work) add_k_list(c, wh, e, 0, 0, wh.w.nquart, tv != nullptr, v, !alone);
   }
-  add_j_launches(c, e, f32, v);
-  run_launches(c, v, s, "jk_build", side);
+  add_j_launches(c, e, jl, f32, v, !alone);
+  run_launches(c, v, s, "jk_build", !alone);
   check_launch(qxk_j_finish(&a, &jl, Jc, s), "j_finish");
   check_launch(qxk_jk_finish(&c->shells, Jc, Kp, J, K, s), "jk_finish");
 }
@@ -1599,30 +1614,31 @@ int qx_jk_build_masked(qx_ctx* c, const double* D, double* J, double* K, int pre
     QX_HIP(hipSetDevice(c->device));
     hipStream_t s = (hipStream_t)stream;
     double* w = begin_ws(c, s);
-    jk_pass(c, w, D, J, K, precision, thr, frag_skip, nullptr, s, true);
+    jk_pass(c, w, D, J, K, precision, thr, frag_skip, nullptr, s);
     end_ws(c, s);
     return QX_OK;
   });
 }
 
 // qx_jk_build (FP64) without any device allocation: the J'/K' work
-// matrices live in the scratch array, every class kernel runs in turn on the
-// caller's stream (no side streams, events or timing), and the work matrices
-// are cleared by a fill kernel on every call.  Calls that overlap on one GPU
-// share the array and race.
+// matrices live in the scratch array, the Hermite densities and potentials in
+// memory of the context that only this call writes, every kernel runs in turn
+// on the caller's stream (no side streams, events or timing), and the pass's
+// first kernel clears what it accumulates into.  So it may overlap the
+// context's other passes; two of these calls that overlap on one GPU share the
+// array and race.
 int qx_jk_build_noalloc(qx_ctx* c, const double* D, double* J, double* K, void* stream) {
   if (!c || !D || !J || !K) return QX_EINVAL;
   return guarded(c, [&]() -> int {
     QX_HIP(hipSetDevice(c->device));
     hipStream_t s = (hipStream_t)stream;
-    const size_t nc = c->ncart, n2 = nc * nc;
-    const size_t need = (c->pure ? 5 : 2) * n2;
+    const size_t need = noalloc_doubles(c);
     if (need > QX_NOALLOC_DOUBLES)
       throw QxError{QX_EINVAL, "jk_build_noalloc: " + std::to_string(need) + " doubles of work matrices (" +
-                                   std::to_string(nc) + " Cartesian functions) exceed the " +
+                                   std::to_string(c->ncart) + " Cartesian functions) exceed the " +
                                    std::to_string(QX_NOALLOC_DOUBLES) + "-double scratch array"};
     QX_REQUIRE(c->scratch != nullptr, QX_EHIP, "jk_build_noalloc: scratch array not set up");
-    jk_pass(c, c->scratch, D, J, K, QX_PREC_FP64, 0.0, nullptr, nullptr, s, false);
+    jk_pass(c, c->scratch, D, J, K, QX_PREC_FP64, 0.0, nullptr, nullptr, s, c->d_herm_own);
     return QX_OK;
   });
 }
@@ -1712,7 +1728,7 @@ int qx_jk_deriv_dir(qx_ctx* c, const double* D, const double* v, double* J, doub
     QX_HIP(hipSetDevice(c->device));
     hipStream_t s = (hipStream_t)stream;
     double* w = begin_ws(c, s);
-    jk_pass(c, w, D, J, K, QX_PREC_FP64, 0.0, nullptr, v, s, true);
+    jk_pass(c, w, D, J, K, QX_PREC_FP64, 0.0, nullptr, v, s);
     end_ws(c, s);
     return QX_OK;
   });

@@ -1,0 +1,83 @@
+"""Passes that share a context, a stream or a capture with others.
+
+Results are compared with the same entry point called alone: FP64 sums of the
+same terms, whose order differs by atomics only, so 1e-12 of the largest
+element."""
+import ctypes
+
+import numpy as np
+import pytest
+
+from quax_amd.basis import BasisSet
+from quax_amd.molecule import synthetic_cluster
+
+pytestmark = pytest.mark.gpu
+
+
+def _density(n, seed):
+    X = np.random.default_rng(seed).standard_normal((n, n)) * 0.3
+    return X @ X.T / n
+
+
+def _same(a, b):
+    assert bool(a.isfinite().all())
+    assert (a - b).abs().max().item() <= 1e-12 * max(1.0, b.abs().max().item())
+
+
+def _noalloc(eng, D, J, K):
+    from quax_amd import _lib
+    _lib.check(eng.L.qx_jk_build_noalloc(eng.ctx, _lib.ptr(D), _lib.ptr(J), _lib.ptr(K), eng._stream()), eng.ctx)
+
+
+def _context(basis, pure):
+    from quax_amd.engine import EriEngine
+    mol = synthetic_cluster(2, 1, 11, n_o=1) if basis == "sto-3g" else synthetic_cluster(3, 1, 11)
+    return EriEngine(mol, BasisSet.build(mol, basis, pure=pure), ints_tol=1e-12)
+
+
+@pytest.mark.parametrize("basis,pure", [("sto-3g", False), ("even-tempered", True)])
+def test_noalloc_pass_beside_another_pass(gpu, basis, pure):
+    """Both passes in flight on two streams of one context, with densities of
+    different size, and a captured allocation-free pass replayed beside the other."""
+    torch = gpu
+    with _context(basis, pure) as eng:
+        n = eng.nbf
+        D1, D2 = (torch.as_tensor(_density(n, k) * s, device="cuda") for k, s in ((1, 1.0), (2, 50.0)))
+        ref1, ref2 = [x.clone() for x in eng.jk(D1)], [x.clone() for x in eng.jk(D2)]
+        new = lambda: torch.full((n, n), float("nan"), dtype=torch.float64, device="cuda")
+        J, K, Jg, Kg = new(), new(), new(), new()
+        s1, s2 = torch.cuda.Stream(), torch.cuda.Stream()
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            _noalloc(eng, D1, Jg, Kg)
+        for rep in range(12):
+            out = (new(), new())
+            torch.cuda.synchronize()
+            with torch.cuda.stream(s1):
+                if rep % 2:
+                    graph.replay()
+                else:
+                    _noalloc(eng, D1, J, K)
+            with torch.cuda.stream(s2):
+                eng.jk(D2, out=out)
+            torch.cuda.synchronize()
+            for got, want in zip((Jg, Kg) if rep % 2 else (J, K), ref1):
+                _same(got, want)
+            for got, want in zip(out, ref2):
+                _same(got, want)
+
+
+@pytest.mark.parametrize("basis,pure", [("sto-3g", False), ("even-tempered", True)])
+def test_noalloc_pass_uses_no_events(gpu, basis, pure):
+    torch = gpu
+    with _context(basis, pure) as eng:
+        n = eng.nbf
+        D = torch.as_tensor(_density(n, 3), device="cuda")
+        J, K = (torch.empty((n, n), dtype=torch.float64, device="cuda") for _ in range(2))
+        eng.profile(True)
+        _noalloc(eng, D, J, K)
+        assert eng.profile_read()[1].sum() == 0
+        for got, want in zip((J, K), eng.jk(D)):
+            _same(got, want)
+        assert eng.profile_read()[1].sum() > 0
