@@ -439,13 +439,16 @@ def emit_eri_core(l):
     stats = dict(vrr=len(v.lines), vrr_flops=v.nflop, hrr=len(h.lines), hrr_flops=h.nflop, L=Lt, N=N,
                  flops=core_flops(Lt, v.nflop, h.nflop))
     # K form: the integrals of all primitives are summed as [e0|f0], then
-    # transferred and contracted with the density blocks one by one
+    # transferred and contracted with the density blocks one by one, all in
+    # FP64 also where the recursion is FP32 (summed in FP32, K of 49 x 49
+    # primitives was off by 2.7e-7 of its norm; rounded after the sum, 2.4e-8;
+    # rounded per primitive quartet only, 1.5e-9)
     K = [f"template <typename R>\n__device__ __forceinline__ void qx_kb_e{nm}_0(const QxArgs& A_, int P1, int P2, int s_, int ns_, "
          f"const double (&Dac)[{NA * NC}], const double (&Dad)[{NA * ND}], const double (&Dbc)[{NB * NC}], "
          f"const double (&Dbd)[{NB * ND}], double (&kac)[{NA * NC}], double (&kad)[{NA * ND}], "
          f"double (&kbc)[{NB * NC}], double (&kbd)[{NB * ND}]) {{"]
     names = {ac: f"s_{ac[0][0]}{ac[0][1]}{ac[0][2]}_{ac[1][0]}{ac[1][1]}{ac[1][2]}" for ac in sorted(vn)}
-    K += [f"  R {x}(0);" for x in names.values()]
+    K += [f"  double {x} = 0.0;" for x in names.values()]
     K.append("  const int v1_ = A_.pr.pp_first[P1], v2_ = A_.pr.pp_first[P2], n2_ = A_.pr.pp_n[P2];")
     K.append("  for (int k_ = s_; k_ < A_.pr.pp_n[P1] * n2_; k_ += ns_) {")
     K.append("  const int u1 = v1_ + k_ / n2_, u2 = v2_ + k_ % n2_;")
@@ -455,8 +458,9 @@ def emit_eri_core(l):
     body = [x for x in body if x not in transfer]
     emit_vrr_consts(body, v.lines)
     body += ["  " + x for x in v.lines]
-    body += [f"  {names[ac]} += {vn[ac]};" for ac in sorted(vn)]
-    K += ["  " + x for x in body] + ["  }"] + transfer
+    body += [f"  {names[ac]} += (double){vn[ac]};" for ac in sorted(vn)]
+    fp64 = lambda x: x.replace("const R ", "const double ").replace("(R)", "")
+    K += ["  " + x for x in body] + ["  }"] + [fp64(x) for x in transfer]
     groups = []
     for k in range(N):
         i, rem = divmod(k, NB * NC * ND)
@@ -467,7 +471,7 @@ def emit_eri_core(l):
             f"  {{ const double v_ = qx_value({outs[k]});",
             f"    kac[{ik}] += v_ * Dbd[{jl}]; kad[{il}] += v_ * Dbc[{jk}];",
             f"    kbc[{jk}] += v_ * Dad[{il}]; kbd[{jl}] += v_ * Dac[{ik}]; }}"]))
-    K += ["  " + x if not x.startswith("  ") else x for x in interleave(h.lines, groups)]
+    K += ["  " + x if not x.startswith("  ") else x for x in interleave([fp64(x) for x in h.lines], groups)]
     K.append("}")
     # K epilogue: 4 fused multiply-adds per integral
     return "\n".join(L), ["\n".join(K)], dict(stats, jk_flops=[core_flops(Lt, v.nflop, h.nflop) + 8 * N])

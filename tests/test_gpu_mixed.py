@@ -16,7 +16,7 @@ import pytest
 
 import oracle
 from quax_amd import workloads
-from quax_amd.basis import BasisSet
+from quax_amd.basis import BasisSet, Shell
 from quax_amd.molecule import Molecule
 from test_gpu_eri import contracted_d_cluster, small_d_cluster
 
@@ -185,3 +185,25 @@ def test_mixed_threshold_is_validated(gpu):
                 eng.eri_grad(D, precision=MIXED, fp32_threshold=bad)
         with pytest.raises(QuaxNativeError):
             eng.set_streams(0)
+
+
+def test_fp32_pass_sums_primitives_in_fp64(gpu):
+    """Contracted s shells of seven primitives, all in FP32: a primitive
+    quartet's integral is rounded to FP32 once and everything after it is FP64,
+    so J and K of a density with one element (one positive quartet per element,
+    2401 primitive ones) are within 2^-24 of the FP64 result, element by
+    element.  Enough quartets that one lane sums all primitives of one."""
+    n = 30
+    mol = Molecule(["H"] * n, np.random.default_rng(0).uniform(0, 9, (n, 3)))
+    exps, coefs = list(np.geomspace(60.0, 0.2, 7)), [0.1, 0.2, 0.3, 0.4, 0.3, 0.2, 0.1]
+    bs = BasisSet("s7", [Shell(0, a, exps, coefs) for a in range(n)])
+    D = np.zeros((n, n))
+    D[4, 4] = 1.0
+    with _engine(mol, bs) as eng:
+        _all_fp32(eng)
+        assert eng.mixed_quartets(1e300, 0) == (0, eng.num_quartets())
+        for x32, x64 in zip(eng.jk(D, precision=MIXED, fp32_threshold=1e300), eng.jk(D)):
+            err = (x32 - x64).abs().cpu().numpy()
+            x64 = x64.cpu().numpy()
+            assert x64.min() >= 0.0 and err.max() > 0.0
+            assert (err <= 2.0 ** -24 * x64 + 1e-14 * x64.max()).all()
