@@ -121,12 +121,12 @@ def build_h5(verbose=True):
     return H5_LIB
 
 
-# Scratch per lane allowed to the streaming J/K and adjoint-gradient kernels,
-# which run on up to four streams: a side stream's hardware queue that has to
+# Scratch per lane allowed to the generated kernels, which run on up to four
+# streams: a side stream's hardware queue that has to
 # grow its scratch past ~8 KB per lane, once the process holds scratch on its
 # other queues, has been refused by the HSA runtime (the queue aborts with
-# HSA_STATUS_ERROR_OUT_OF_RESOURCES).  Larger kernels run on the caller's
-# stream only.
+# HSA_STATUS_ERROR_OUT_OF_RESOURCES).  The caller's stream is no safer: nothing
+# a context runs before grows its scratch.
 STREAMING_SCRATCH_MAX = 6144
 LLVM_BIN = os.path.join(ROCM, "llvm", "bin")
 
@@ -147,19 +147,12 @@ def kernel_scratch(obj: str, tmp: str) -> list:
 
 
 def check_streaming_scratch(objs, verbose=True):
-    """Fails the build when a kernel that runs on side streams needs more than
-    STREAMING_SCRATCH_MAX bytes of scratch per lane: K (cls_*_j*), J (jeng*),
-    gradient (cls_*_g*), tensor (cls_*_r*, cls_*_d*) and second-derivative
-    (cls_*_v*) kernels, and the array form (cls_*_e) of the classes without a
-    quadrature one."""
+    """Fails the build when a generated kernel needs more than
+    STREAMING_SCRATCH_MAX bytes of scratch per lane."""
     if not os.path.exists(os.path.join(LLVM_BIN, "clang-offload-bundler")):
         print("scratch check skipped: no clang-offload-bundler", flush=True)
         return
-    names = [os.path.basename(o) for o in objs]
-    quad = {n[4:8] for n in names if re.match(r"cls_\d{4}_r0\.hip\.", n)}
-    streaming = [o for o, n in zip(objs, names)
-                 if re.match(r"(cls_\d{4}_[jgrdv]\d+|jengv?_\d)\.hip\.", n)
-                 or (re.match(r"cls_\d{4}_e\.hip\.", n) and n[4:8] not in quad)]
+    streaming = [o for o in objs if not os.path.basename(o).startswith("qx_")]
     worst = ("", 0)
     with tempfile.TemporaryDirectory() as tmp:
         for o in streaming:

@@ -845,9 +845,9 @@ def part_groups(nparts):
 
 
 def emit_class_files(cls, outdir, fp32):
-    """Writes, per class: cls_<l>_e.hip (array-form ERI kernel), cls_<l>_j0.hip
-    (K), cls_<l>_r0.hip (integrals into the pair matrix by quadrature, heavy
-    classes), cls_<l>_d0.hip (derivative slices), cls_<l>_v0.hip (directional
+    """Writes, per class: cls_<l>_e.hip (integrals: array-form kernel, or by
+    quadrature for the heavy classes, whose array form would need 1 to 18 KB of
+    scratch per lane), cls_<l>_j0.hip (K), cls_<l>_d0.hip (derivative slices), cls_<l>_v0.hip (directional
     derivatives of K and of the adjoint gradient) and cls_<l>_g<k>.hip (adjoint
     gradient: one kernel by quadrature, or one per derivative part)."""
     la, lb, lc, ld = cls
@@ -863,14 +863,15 @@ def emit_class_files(cls, outdir, fp32):
         files.append(path)
 
     src_e, jks, st = emit_eri_core(cls)
-    write(f"cls_{nm}_e.hip", [src_e, "", f"QX_DEFINE_ERI_KERNEL(e{nm}, {N}, {dims})"], "qx_pairm.h")
+    if nm in RYS_E:
+        write(f"cls_{nm}_e.hip", [f"QX_DEFINE_RYS_E(e{nm}, {la}, {lb}, {lc}, {ld})"], "qx_rys.h")
+    else:
+        write(f"cls_{nm}_e.hip", [src_e, "", f"QX_DEFINE_ERI_KERNEL(e{nm}, {N}, {dims})"], "qx_pairm.h")
     if nm in RYS_K:
         write(f"cls_{nm}_j0.hip", [f"QX_DEFINE_RYS_K(e{nm}_0, {la}, {lb}, {lc}, {ld}, {1 if fp32 else 0})"], "qx_rys.h")
     else:
         write(f"cls_{nm}_j0.hip", [jks[0], "", f"QX_DEFINE_K_KERNEL(e{nm}_0, {dims}, {1 if fp32 else 0})"], "qx_jk.h")
     stats.append((cls, "eri", st))
-    if nm in RYS_E:
-        write(f"cls_{nm}_r0.hip", [f"QX_DEFINE_RYS_E(e{nm}, {la}, {lb}, {lc}, {ld})"], "qx_rys.h")
     write(f"cls_{nm}_d0.hip", [f"QX_DEFINE_RYS_D(d{nm}, {la}, {lb}, {lc}, {ld})"], "qx_rys.h")
     write(f"cls_{nm}_v0.hip", [f"QX_DEFINE_RYS_KV(e{nm}, {la}, {lb}, {lc}, {ld})",
                                f"QX_DEFINE_RYS_H(d{nm}, {la}, {lb}, {lc}, {ld})"], "qx_rys.h")
@@ -937,7 +938,7 @@ def main():
         D.append(f'extern "C" int qx_launch_e{nm}(const QxArgs*, const QxLaunch*);')
         for pi in range(len(jkf[cls])):
             D.append(f'extern "C" int qx_launchj_e{nm}_{pi}(const QxArgs*, const QxLaunch*);')
-        names = [f"qx_launch_d{nm}", f"qx_launchv_e{nm}", f"qx_launchh_d{nm}"] + ([f"qx_launchr_e{nm}"] if nm in RYS_E else [])
+        names = [f"qx_launch_d{nm}", f"qx_launchv_e{nm}", f"qx_launchh_d{nm}"]
         D += [f'extern "C" int {x}(const QxArgs*, const QxLaunch*);' for x in names]
         for gi in range(len(groups[cls])):
             D.append(f'extern "C" int qx_launchg_d{nm}_g{gi}(const QxArgs*, const QxLaunch*);')
@@ -953,8 +954,7 @@ def main():
         gps = ", ".join(str(len(g)) for g in groups[cls])
         jl = ", ".join(f"qx_launchj_e{nm}_{pi}" for pi in range(len(jkf[cls])))
         jfs = ", ".join(f"{x:.1f}" for x in jkf[cls])
-        re = f"qx_launchr_e{nm}" if nm in RYS_E else "nullptr"
-        D.append(f"  {{{cls[0]}, {cls[1]}, {cls[2]}, {cls[3]}, qx_launch_e{nm}, {re}, qx_launch_d{nm}, qx_launchv_e{nm}, "
+        D.append(f"  {{{cls[0]}, {cls[1]}, {cls[2]}, {cls[3]}, qx_launch_e{nm}, qx_launch_d{nm}, qx_launchv_e{nm}, "
                  f"qx_launchh_d{nm}, {len(jkf[cls])}, {{{jl}}}, {{{jfs}}}, {nparts[cls]}, {len(groups[cls])}, {{{gl}}}, "
                  f"{ef:.1f}, {{{pfs}}}, {{{pcs}}}, {{{gfs}}}, {{{gps}}}}},")
     D.append("};")

@@ -292,8 +292,7 @@ __device__ __forceinline__ long long qx_dfull_slice(const QxEpiDev& e, int y) {
 
 struct QxClassEntry {
   int la, lb, lc, ld;
-  int (*eri)(const QxArgs*, const QxLaunch*);      // array form (store, Schwarz, pair matrix)
-  int (*rys_eri)(const QxArgs*, const QxLaunch*);  // pair matrix by quadrature (null: array form)
+  int (*eri)(const QxArgs*, const QxLaunch*);      // integrals (store, Schwarz, pair matrix): array form or quadrature
   int (*deri)(const QxArgs*, const QxLaunch*);     // derivative (fp32 = 2: tangent) slices of the pair matrix
   int (*jkv)(const QxArgs*, const QxLaunch*);      // K of the directional derivative
   int (*hess)(const QxArgs*, const QxLaunch*);     // adjoint gradient's directional derivative

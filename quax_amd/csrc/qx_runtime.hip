@@ -213,14 +213,12 @@ int timed_launch(qx_ctx* c, int slot, long long pq, hipStream_t s, F&& launch, b
 }
 
 int launch_eri(qx_ctx* c, const QxWorkDev& w, int cls, const QxEpiDev& e, int fp32, hipStream_t s,
-               const QxPairsDev& pr, const QxPrimPairsDev& pp, const QxPairM* pm = nullptr,
-               const QxKList* kl = nullptr) {
+               const QxPairsDev& pr, const QxPrimPairsDev& pp, const QxPairM* pm, const QxKList* kl) {
   QxArgs a;
   a.pr = pr; a.pp = pp; a.w = w; a.e = e; a.boys = c->d_boys;
   QxLaunch L{fp32, s, 0, pm, kl};
   const QxClassEntry& ent = qx_class_table[cls];
-  auto fn = kl && ent.rys_eri ? ent.rys_eri : ent.eri;
-  return timed_launch(c, QX_SLOT_ERI(cls, fp32 ? 1 : 0), w.nquart, s, [&] { return fn(&a, &L); });
+  return timed_launch(c, QX_SLOT_ERI(cls, fp32 ? 1 : 0), w.nquart, s, [&] { return ent.eri(&a, &L); });
 }
 
 // One kernel launch of a pass, with its estimated cost (flops).
@@ -1853,7 +1851,10 @@ int qx_eri_store(qx_ctx* c, double* out, void* stream) {
     hipStream_t s = (hipStream_t)stream;
     QxEpiDev e{};
     e.epi = QX_EPI_STORE; e.nbf = c->ncart; e.natom = c->natom; e.coord = -1; e.out = out;
-    for (auto& wh : c->work) check_launch(launch_eri(c, wh.w, wh.cls, e, 0, s, c->pr, c->pp), "eri_store");
+    for (auto& wh : c->work) {
+      const QxKList kl = k_list(c, wh, 0, 0, false);
+      check_launch(launch_eri(c, wh.w, wh.cls, e, 0, s, c->pr, c->pp, nullptr, &kl), "eri_store");
+    }
     return QX_OK;
   });
 }

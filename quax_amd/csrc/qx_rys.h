@@ -448,6 +448,7 @@ __global__ __launch_bounds__(QX_RYS_BLOCK_MAX) void qx_rk(QxArgs A_, QxKList kl)
 }
 
 // ---- integrals and derivative integrals into the pair matrix --------------------
+// (or, QX_EPI_STORE, into the class-blocked array of a single-primitive basis)
 template <int LA, int LB, int LC, int LD>
 __global__ __launch_bounds__(QX_RYS_BLOCK) void qx_re(QxArgs A_, QxKList kl, QxPairM pm) {
   using S = QxRys<LA, LB, LC, LD, 0>;
@@ -473,9 +474,13 @@ __global__ __launch_bounds__(QX_RYS_BLOCK) void qx_re(QxArgs A_, QxKList kl, QxP
       },
       [&]() QX_INLINE {
         if (act && !(A_.e.skip_single && qx_single_atom(A_, b.P1, P2))) {
-          double* m = pm.M + (pm.row0 + b.P1 - pm.rowp + (long long)ln.ab * pm.rown) * pm.ld + pm.col0 + (P2 - pm.colp);
+          const bool store = A_.e.epi == QX_EPI_STORE;
+          double* m = store ? A_.e.out + A_.w.store_base + (long long)ln.ab * (S::NC * S::ND) * kl.nquart +
+                                  kl.prefix[blockIdx.x] + (P2 - b.kst)
+                            : pm.M + (pm.row0 + b.P1 - pm.rowp + (long long)ln.ab * pm.rown) * pm.ld + pm.col0 + (P2 - pm.colp);
+          const long long step = store ? kl.nquart : pm.coln;
 #pragma unroll
-          for (int k = 0; k < S::NC * S::ND; ++k) m[(long long)k * pm.coln] = I[k];
+          for (int k = 0; k < S::NC * S::ND; ++k) m[k * step] = I[k];
         }
       });
 }
@@ -817,11 +822,11 @@ static inline dim3 qx_k_grid(const QxKList& kl) {
     return a->e.tv ? qx_rk_go_v##NAME<qx_dual, qx_dual>(a, L) : -1;                               \
   }
 
-// Integrals (QX_DEFINE_RYS_E) and derivative integrals (QX_DEFINE_RYS_D, with
+// Integrals (QX_DEFINE_RYS_E: pair matrix, store, Schwarz) and derivative integrals (QX_DEFINE_RYS_D, with
 // L->fp32 = 2 their derivatives along tv) into the pair matrix.
 #define QX_DEFINE_RYS_E(NAME, LA, LB, LC, LD)                                                     \
-  extern "C" int qx_launchr_##NAME(const QxArgs* a, const QxLaunch* L) {                          \
-    if (!L->kl) return -1;                                                                        \
+  extern "C" int qx_launch_##NAME(const QxArgs* a, const QxLaunch* L) {                           \
+    if (!L->kl || L->fp32 || a->e.epi == QX_EPI_JK) return -1;                                    \
     if constexpr (LA == LC && LB == LD) {                                                         \
       if (a->e.epi == QX_EPI_SCHWARZ) {                                                           \
         if (L->kl->nbra <= 0) return 0;                                                           \
@@ -830,9 +835,12 @@ static inline dim3 qx_k_grid(const QxKList& kl) {
         return (int)hipGetLastError();                                                            \
       }                                                                                           \
     }                                                                                             \
-    if (!L->pm || L->kl->nquart <= 0 || L->kl->maxket <= 0) return 0;                   \
+    if (L->kl->nquart <= 0 || L->kl->maxket <= 0) return 0;                                       \
+    const bool store = a->e.epi == QX_EPI_STORE;                                                  \
+    if (store ? L->kl->ketprim != 1 : !L->pm) return -1;                                          \
     const size_t sh = 4 * sizeof(double) * QxRys<LA, LB, LC, LD, 0>::LDS;                         \
-    hipLaunchKernelGGL((qx_re<LA, LB, LC, LD>), qx_k_grid(*L->kl), dim3(QX_RYS_BLOCK), sh, L->stream, *a, *L->kl, *L->pm); \
+    hipLaunchKernelGGL((qx_re<LA, LB, LC, LD>), qx_k_grid(*L->kl), dim3(QX_RYS_BLOCK), sh, L->stream, *a, *L->kl, \
+                       store ? QxPairM{} : *L->pm);                                               \
     return (int)hipGetLastError();                                                                \
   }
 #define QX_DEFINE_RYS_D(NAME, LA, LB, LC, LD)                                                     \

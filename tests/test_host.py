@@ -298,3 +298,21 @@ def test_streaming_kernels_fit_side_stream_scratch():
         sizes = build.kernel_scratch(objs["cls_2221_j0"], tmp)
     assert sizes and all(name.startswith("_Z") and size >= 0 for name, size in sizes)
     build.check_streaming_scratch(list(objs.values()), verbose=False)
+
+
+def test_no_generated_kernel_outgrows_the_scratch_budget():
+    """Every kernel generated by the last build, on whichever stream it runs, needs
+    at most 6 KB of scratch per lane: set-up runs none of the largest ones, so
+    neither a side stream's queue nor the caller's has grown before."""
+    import glob
+    import tempfile
+    from quax_amd.csrc import build
+    objs = []
+    for src in glob.glob(os.path.join(build.GEN, "*.hip")):
+        built = glob.glob(os.path.join(build.OBJ, os.path.basename(src) + ".*.o"))
+        objs += [max(built, key=os.path.getmtime)] if built else []
+    if not objs or not os.path.exists(os.path.join(build.LLVM_BIN, "clang-offload-bundler")):
+        pytest.skip("no built objects or no offload bundler")
+    with tempfile.TemporaryDirectory() as tmp:
+        big = [k for o in objs for k in build.kernel_scratch(o, tmp) if k[1] > build.STREAMING_SCRATCH_MAX]
+    assert not big
