@@ -615,7 +615,7 @@ def emit_small(outdir):
         out += emit_eri_core(l)[1] + [f"QX_DEFINE_K_BODY(e{nm}_0, {na}, {nb}, {nc}, {nd})", ""]
     for L1 in range(3):
         cases = " ".join(f"QX_J_CASE({L1}, {L2})" for L2 in range(3))
-        out += j_cores(L1, range(3)) + [f"QX_DEFINE_J_BODY({L1}, {cases})", ""]
+        out += j_cores(L1, range(3)) + [f"#define QX_SMALL_CASES_{L1} {cases}", ""]
     out.append("QX_DEFINE_SMALL()")
     path = os.path.join(outdir, "jk_small.hip")
     with open(path, "w") as fh:

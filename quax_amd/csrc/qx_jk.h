@@ -300,8 +300,9 @@ __device__ __forceinline__ void qx_j_kets(const QxArgs& A_, const QxJList& jl, i
                                G (&jj)[qx_nherm(L1)]) { qx_jc_##L1##L2<G, R>(x, y, z, b, h, jj); }); \
     break;
 // (The kernels take the body as a macro: through a device function, the
-// compiler keeps a copy of the list argument in scratch, and the dual-number
-// kernel of dd bras, 3.5 KB of scratch, then returned wrong potentials.)
+// compiler kept a copy of the list argument in scratch, and the dual-number
+// kernel of dd bras, 3.5 KB of scratch, then returned wrong potentials.  The
+// build compares the kernels' scratch with what they need without a copy.)
 #define QX_J_BODY(L1, bx, by, ny, ...)\
     const int u = jl.uoff[jl.X] + (int)(bx);                                                             \
     const int P = A_.pp.pair[u];                                                                  \
@@ -335,11 +336,6 @@ __device__ __forceinline__ void qx_j_kets(const QxArgs& A_, const QxJList& jl, i
       const G s = qx_wave_total(j[t]);                                                            \
       if (__lane_id() == 0) qx_potential_add(s, jl.P, jl.Pd, jl.hoff[jl.X] + t * m + (bx));         \
     }
-#define QX_DEFINE_J_BODY(L1, ...)                                                                 \
-  template <typename G, typename R>                                                               \
-  __device__ __forceinline__ void qx_jb_##L1(const QxArgs& A_, const QxJList& jl, int x, int y, int n) { \
-    QX_J_BODY(L1, x, y, n, __VA_ARGS__)                                                           \
-  }
 #define QX_DEFINE_J_KERNEL(L1, WITH32, ...)                                                       \
   template <typename G, typename R>                                                               \
   __global__ __launch_bounds__(QX_BLOCK_MAX) void qx_jeng_##L1(QxArgs A_, QxJList jl) {           \
@@ -539,6 +535,15 @@ struct QxSmall {
   int end[9];     // workgroups of the lists up to each one
   int split;      // workgroups that share a J bra's kets
 };
+#define QX_SMALL_J(L1, ...)                                                                       \
+  if (i == 6 + L1) {                                                                              \
+    using G = double;                                                                             \
+    using R = double;                                                                             \
+    const QxJList& jl = sm.j[L1];                                                                 \
+    const int by = at % sm.split, bx = at / sm.split;                                             \
+    QX_J_BODY(L1, bx, by, sm.split, __VA_ARGS__)                                                  \
+    return;                                                                                       \
+  }
 #define QX_DEFINE_SMALL()                                                                         \
   __global__ __launch_bounds__(QX_SMALL_BLOCK) void qx_small(QxArgs A_, QxSmall sm) {             \
     HIP_DYNAMIC_SHARED(double, qx_sk)                                                             \
@@ -546,13 +551,9 @@ struct QxSmall {
     int i = 0;                                                                                    \
     while (i < 8 && w >= sm.end[i]) ++i;                                                          \
     const int at = w - (i ? sm.end[i - 1] : 0);                                                   \
-    if (i >= 6) {                                                                                 \
-      const int by = at % sm.split, bx = at / sm.split;                                           \
-      if (i == 6) qx_jb_0<double, double>(A_, sm.j[0], bx, by, sm.split);                         \
-      else if (i == 7) qx_jb_1<double, double>(A_, sm.j[1], bx, by, sm.split);                    \
-      else qx_jb_2<double, double>(A_, sm.j[2], bx, by, sm.split);                                \
-      return;                                                                                     \
-    }                                                                                             \
+    QX_SMALL_J(0, QX_SMALL_CASES_0)                                                               \
+    QX_SMALL_J(1, QX_SMALL_CASES_1)                                                               \
+    QX_SMALL_J(2, QX_SMALL_CASES_2)                                                               \
     const QxKList& kl = sm.k[i];                                                                  \
     QxKBlock b;                                                                                   \
     if (!qx_k_block(A_, kl, at % kl.nbra, at / kl.nbra, b)) return;                               \

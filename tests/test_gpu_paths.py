@@ -182,3 +182,23 @@ def test_transformation_tile_edges(gpu, n, m):
     for c in C:
         ref = np.tensordot(ref, c, axes=[(0,), (0,)])
     _close(partial_tei_transformation(G, *C), ref)
+
+
+@pytest.mark.parametrize("prims", [1, 3])
+@pytest.mark.parametrize("pure", [False, True])
+def test_directional_jk_against_the_derivative_tensor(gpu, pure, prims):
+    """The dual-number J and K kernels of every class against the first-derivative
+    tensor contracted with the direction and the density."""
+    import torch
+    mol = Molecule(["C", "O", "C"], np.array([[0.0, 0.1, -0.3], [1.3, 2.0, 0.4], [-1.1, 0.9, 2.2]]))
+    geo = lambda x: list(x * 2.5 ** np.arange(prims))
+    bs = BasisSet("spd", _shells(3, [(0, geo(0.5)), (1, geo(0.4)), (2, geo(0.6))]), pure=pure)
+    D = _density(bs.nbf(), 10)
+    v = np.random.default_rng(11).standard_normal(9)
+    with _engine(mol, bs, ints_tol=1e-14) as eng:
+        n = eng.nbf
+        G = torch.tensordot(torch.as_tensor(v, device="cuda"), eng.eri_deriv_core(1), dims=1)
+        J, K = eng.jk_deriv_dir(D, v)
+        Dt = torch.as_tensor(D, device="cuda").reshape(-1)
+        _close(J, (G.reshape(n * n, n * n) @ Dt).reshape(n, n))
+        _close(K, (G.permute(0, 2, 1, 3).reshape(n * n, n * n) @ Dt).reshape(n, n))

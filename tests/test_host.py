@@ -316,3 +316,19 @@ def test_no_generated_kernel_outgrows_the_scratch_budget():
     with tempfile.TemporaryDirectory() as tmp:
         big = [k for o in objs for k in build.kernel_scratch(o, tmp) if k[1] > build.STREAMING_SCRATCH_MAX]
     assert not big
+
+
+def test_build_refuses_a_scratch_copy_of_kernel_arguments(monkeypatch):
+    """Kernels that hold their lists as one argument may not need more scratch than
+    they do without a copy of it; the others only have the common budget."""
+    from quax_amd.csrc import build
+    if not os.path.exists(os.path.join(build.LLVM_BIN, "clang-offload-bundler")):
+        pytest.skip("no offload bundler")
+    size = {}
+    monkeypatch.setattr(build, "kernel_scratch", lambda o, tmp: [("kernel", size["now"])])
+    for name, most in [*build.ARGUMENT_SCRATCH.items(), ("cls_2222_j0", build.STREAMING_SCRATCH_MAX)]:
+        size["now"] = most
+        build.check_streaming_scratch([f"{name}.hip.0.o"], verbose=False)
+        size["now"] = most + 304
+        with pytest.raises(RuntimeError):
+            build.check_streaming_scratch([f"{name}.hip.0.o"], verbose=False)
