@@ -321,10 +321,14 @@ int qx_jk_build_masked(qx_ctx* ctx, const double* D, double* J, double* K, int p
 int qx_set_streams(qx_ctx* ctx, int nstreams);
 
 /* Most device memory (bytes; 0 = what the device has) that the tensor entry
- * points (compute_2e_int, eri_deriv_core(1), compute_2e_deriv of order 0 and
- * 1) take for their function-pair matrices; a tighter limit makes them work
- * through fewer derivative slices at a time and then through row panels, with
- * the same result. */
+ * points (compute_2e_int, eri_deriv_core, compute_2e_deriv) take for their
+ * function-pair matrices, beside index tables of 4 bytes per function pair.  A
+ * tighter limit makes them work through fewer derivative slices at a time and
+ * then, in a Cartesian basis, through row panels, with the same result; 36 rows
+ * of one slice are taken at least.  A spherical basis needs room for one slice
+ * (QX_ENOMEM below that).  Up to 1 GiB of the matrices stays with the context
+ * until qx_finalize or a limit below it; larger ones are allocated and freed by
+ * each call, which then waits for the device. */
 int qx_set_tensor_limit(qx_ctx* ctx, long long bytes);
 
 /* Measurement support (no reference counterpart).

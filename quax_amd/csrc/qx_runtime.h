@@ -102,7 +102,8 @@ struct qx_ctx {
   long long nherm = 0;
   double* d_rys = nullptr;
   // pair-matrix workspace of the tensor entry points, kept up to
-  // QX_PAIRM_KEEP bytes; passes that use it are ordered like those on ws
+  // QX_PAIRM_KEEP bytes (and pairm_limit); passes that use it are ordered like
+  // those on ws
   double* pairm = nullptr;
   size_t pairm_bytes = 0;
   size_t pairm_limit = 0;                // most bytes of pair matrices per pass (0: what the device has)

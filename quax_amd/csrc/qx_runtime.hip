@@ -1020,24 +1020,32 @@ static const int kPairComps[6] = {1, 3, 9, 6, 18, 36};  // ss, ps, pp, ds, dp, d
 struct PairMatrix {
   QxPairIndex ix{};
   long long ld = 0, slice = 0;
-  int nslice = 0;            // slices per pass; 0: M is one panel of `panel` rows
-  long long panel = 0;
+  int nslice = 0;            // slices per pass
+  long long panel = 0;       // M is one panel of this many rows of each slice (0: whole slices)
   double* M = nullptr;
   int* index = nullptr;
   int* fn = nullptr;
   std::unique_ptr<DevBuf> own;
 };
 
+// Gives the kept workspace back; hipFree waits for passes that still read it.
+static void drop_pairm(qx_ctx* c) {
+  void* p = c->pairm;
+  c->pairm = nullptr;
+  c->pairm_bytes = 0;
+  if (p) QX_HIP(hipFree(p));
+}
+
 // `bytes` of workspace, or null when the device has no room.
 static void* pairm_room(qx_ctx* c, PairMatrix& m, size_t bytes) {
   void* p = nullptr;
   if (bytes <= c->pairm_bytes) return c->pairm;
+  drop_pairm(c);  // before the larger one, which may need its room
   if (hipMalloc(&p, bytes) != hipSuccess) {
     (void)hipGetLastError();
     return nullptr;
   }
   if (bytes <= QX_PAIRM_KEEP) {
-    if (c->pairm) QX_HIP(hipFree(c->pairm));  // waits for passes that still read it
     c->pairm = static_cast<double*>(p);
     c->pairm_bytes = bytes;
   } else {
@@ -1047,7 +1055,8 @@ static void* pairm_room(qx_ctx* c, PairMatrix& m, size_t bytes) {
 }
 
 // Sets m up on stream s for up to `want` slices at a time: all of them where
-// the device (or pairm_limit) has room, else fewer, else row panels.
+// the device (or pairm_limit) has room, else fewer, else row panels of as many
+// slices as take 36 rows each, the components of one dd pair.
 static void begin_pairm(qx_ctx* c, PairMatrix& m, int want, hipStream_t s) {
   int at = 0;
   for (int X = 0; X < 6; ++X) {
@@ -1068,15 +1077,19 @@ static void begin_pairm(qx_ctx* c, PairMatrix& m, int want, hipStream_t s) {
     if (c->pairm_limit && data > c->pairm_limit) continue;
     if ((p = pairm_room(c, m, data + tables))) break;
   }
+  const size_t row = m.ld * sizeof(double);
   if (!p) {
     // panels scatter every element to its eight places, which needs no
     // transform; a spherical tensor has always needed more room than this
     if (c->pure) throw QxError{QX_ENOMEM, "no device memory for the pair matrix of a spherical tensor"};
-    m.nslice = 0;
-    m.panel = std::max<long long>(36, (long long)(QX_PAIRM_PANEL / (want * m.ld * sizeof(double))));
-    m.slice = m.panel * m.ld;
-    data = (size_t)want * m.slice * sizeof(double);
-    if (!(p = pairm_room(c, m, data + tables))) throw QxError{QX_ENOMEM, "no device memory for a tensor panel"};
+    for (size_t room = c->pairm_limit ? std::min(c->pairm_limit, QX_PAIRM_PANEL) : QX_PAIRM_PANEL; !p; room /= 2) {
+      m.nslice = (int)std::min<size_t>(want, std::max<size_t>(1, room / (36 * row)));
+      m.panel = (long long)std::max<size_t>(36, room / (m.nslice * row));
+      m.slice = m.panel * m.ld;
+      data = (size_t)m.nslice * m.slice * sizeof(double);
+      p = pairm_room(c, m, data + tables);
+      if (!p && data <= 36 * row) throw QxError{QX_ENOMEM, "no device memory for a tensor panel"};
+    }
   }
   m.M = static_cast<double*>(p);
   char* q = static_cast<char*>(p) + data;
@@ -1160,7 +1173,7 @@ static QxKList pairm_kets(const qx_ctx* c, const QxWorkHost& wh, const QxPairM& 
 static void run_pairm(qx_ctx* c, PairMatrix& m, int nslice, double* out, hipStream_t s,
                       const std::function<Launch(const QxWorkHost&, const QxPairM&)>& launch) {
   std::vector<Launch> v;
-  if (m.nslice > 0) {
+  if (m.panel == 0) {
     check_launch(qxk_fill(m.M, nslice * m.slice, 0.0, s), "fill");
     for (const auto& wh : c->work) v.push_back(launch(wh, pairm_list(c, m, wh)));
     run_launches(c, v, s, "pair matrix", true);
@@ -1360,7 +1373,7 @@ static void deriv_tensor(qx_ctx* c, int coord, double* out, hipStream_t s) {
   const size_t nb = c->nbf, nb4 = nb * nb * nb * nb;
   PairMatrix m;
   begin_pairm(c, m, nslices, s);
-  const int group = m.nslice > 0 ? m.nslice : nslices;
+  const int group = m.nslice;
   std::vector<int> map(3 * c->natom);
   for (int y0 = 0; y0 < nslices; y0 += group) {
     const int ny = std::min(group, nslices - y0);
@@ -1397,7 +1410,7 @@ static void deriv2_tensor(qx_ctx* c, long long want, double* out, hipStream_t s)
   const int m = 3 * c->natom;
   PairMatrix pmx;
   begin_pairm(c, pmx, want >= 0 ? 1 : m, s);
-  const int room = pmx.nslice > 0 ? pmx.nslice : want >= 0 ? 1 : m;
+  const int room = pmx.nslice;
   struct Pass {
     int x, y0, ny;
   };
@@ -2029,8 +2042,12 @@ int qx_get_fp32_classes(const qx_ctx* c, int pass, int* flags) {
 
 int qx_set_tensor_limit(qx_ctx* c, long long bytes) {
   if (!c || bytes < 0) return QX_EINVAL;
-  c->pairm_limit = (size_t)bytes;
-  return QX_OK;
+  return guarded(c, [&]() -> int {
+    QX_HIP(hipSetDevice(c->device));
+    c->pairm_limit = (size_t)bytes;
+    if (bytes > 0 && c->pairm_bytes > c->pairm_limit) drop_pairm(c);
+    return QX_OK;
+  });
 }
 
 int qx_set_streams(qx_ctx* c, int n) {

@@ -232,7 +232,8 @@ class EriEngine:
         check(self.L.qx_set_streams(self.ctx, int(n)), self.ctx, "set_streams")
 
     def set_tensor_limit(self, nbytes: int = 0):
-        """Most device memory of the tensor calls' pair matrices (0: what the device has)."""
+        """Most device memory of the tensor calls' pair matrices (0: what the
+        device has); gives back what the engine keeps beyond it."""
         check(self.L.qx_set_tensor_limit(self.ctx, int(nbytes)), self.ctx, "set_tensor_limit")
 
     def profile(self, on: bool):

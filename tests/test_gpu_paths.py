@@ -117,6 +117,61 @@ def test_tensors_in_row_panels_equal_whole(gpu):
             _close(eng.eri_deriv_core(1), deriv)
 
 
+def _three_atoms(kind, pure):
+    from quax_amd.engine import EriEngine
+    mol = _line(3, 2.1)
+    more = [2.5, 0.8] if kind == "contracted" else []
+    bs = BasisSet("spd", _shells(3, [(0, [0.9] + more), (1, [1.1] + more), (2, [0.7])]), pure=pure)
+    return EriEngine(mol, bs, ints_tol=1e-14, fragments=[0, 1, 0] if kind == "fragments" else None)
+
+
+@pytest.mark.parametrize("kind", ["single", "contracted", "fragments"])
+def test_tensors_in_many_row_panels(gpu, kind):
+    """36 rows at a time: every dd pair is a panel of its own, in one slice per
+    pass, so panels and slices start inside their lists."""
+    import ctypes
+    with _three_atoms(kind, False) as eng:
+        whole = eng.compute_2e_int(), eng.eri_deriv_core(1), eng.eri_deriv_core(2)
+        eng.set_tensor_limit(4096)
+        eng.profile(True)
+        panels = eng.compute_2e_int()
+        launches = eng.profile_read()[1]
+        eng.profile(False)
+        l4, most = (ctypes.c_int * 4)(), {}
+        for slot in np.flatnonzero(launches):
+            k, c, p, f = (ctypes.c_int() for _ in range(4))
+            eng.L.qx_profile_slot(int(slot), *(ctypes.byref(x) for x in (k, c, p, f)))
+            eng.L.qx_class_info(c.value, l4, None)
+            most[tuple(l4)] = launches[slot]
+        assert most[2, 2, 2, 2] == (4 if kind == "fragments" else 6) and most[2, 1, 0, 0] > 1
+        _close(panels, whole[0])
+        _close(eng.eri_deriv_core(1), whole[1])
+        _close(eng.eri_deriv_core(2), whole[2])
+
+
+@pytest.mark.parametrize("pure", [False, True])
+def test_second_derivative_tensor_in_slices(gpu, pure):
+    with _three_atoms("contracted", pure) as eng:
+        whole = eng.eri_deriv_core(2)
+        eng.set_tensor_limit(4 * 520 * 520 * 8)  # four of nine slices
+        _close(eng.eri_deriv_core(2), whole)
+        _close(eng.compute_2e_deriv([1, 0, 0, 0, 0, 0, 0, 0, 1]), whole[8])
+
+
+def test_kept_tensor_workspace_is_given_back(gpu):
+    torch = gpu
+    mol = _line(2, 2.1)
+    bs = BasisSet("spd", _shells(2, [(0, [0.9]), (1, [1.1]), (2, [0.7]), (2, [1.9]), (2, [0.3])]), pure=True)
+    with _engine(mol, bs, ints_tol=1e-14) as eng:
+        eng.set_tensor_limit(0)
+        free = lambda: torch.cuda.mem_get_info()[0]
+        out = eng.eri_deriv_core(1)
+        held = free()
+        eng.set_tensor_limit(10 * 1024 * 1024)  # one slice
+        assert free() > held
+        _close(eng.eri_deriv_core(1), out)
+
+
 @pytest.mark.parametrize("n_c,pure", [(1, True), (2, False), (7, True)])
 def test_expansion_of_a_tensor(gpu, n_c, pure):
     """28 functions of one carbon (one workgroup's triangle, even rows), 60
