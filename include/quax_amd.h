@@ -328,7 +328,9 @@ int qx_set_streams(qx_ctx* ctx, int nstreams);
  * of one slice are taken at least.  A spherical basis needs room for one slice
  * (QX_ENOMEM below that).  Up to 1 GiB of the matrices stays with the context
  * until qx_finalize or a limit below it; larger ones are allocated and freed by
- * each call, which then waits for the device. */
+ * each call, which then waits for the device.  A call of order 0 or 1 on a stream
+ * under HIP graph capture gets matrices of its own, which stay until qx_finalize
+ * for the graph's replays. */
 int qx_set_tensor_limit(qx_ctx* ctx, long long bytes);
 
 /* Measurement support (no reference counterpart).

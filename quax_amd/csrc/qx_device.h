@@ -72,7 +72,8 @@ struct QxWorkDev {         // one (bra class, ket class) quartet list
 struct QxEpiDev {
   int epi;
   int nbf, natom;
-  int coord;                 // PAIRM derivatives: -1 = all 3N slices, else one coordinate
+  int coord;                 // PAIRM derivatives: -1 = every coordinate's slice, else one coordinate
+  int slice0, nslice;        // PAIRM derivatives: the slices are coordinates [slice0, slice0 + nslice) (nslice 0: coord rule)
   double* out;
   const double* D;           // density, Cartesian nbf x nbf (JK, GRAD)
   double* J; double* K;      // unsymmetrised J', K' (JK)
@@ -84,7 +85,6 @@ struct QxEpiDev {
   int grad_wred;             // GRAD: sum the bra centres' terms across the wavefront before LDS
   int grad_win;              // GRAD: widest LDS atom window in doubles (0 or >= QX_GRAD_LDS: QX_GRAD_LDS)
   const double* tv;          // 3N geometry direction: seed of the directional-derivative kernels
-  const int* slot_map;       // PAIRM derivatives: output slice of coordinate y (-1: none); null = coord rule
   int skip_single;           // PAIRM integrals: leave out quartets with all four centres on one atom
   const int* frag_skip;      // JK: per fragment, nonzero = leave its quartets out (null: none)
   const int* pair_frag;      // fragment of each sorted shell pair (fragmented contexts)
@@ -273,11 +273,11 @@ __device__ __forceinline__ bool qx_single_atom(const QxArgs& A_, int P1, int P2)
   return a == A_.pr.atom_b[P1] && a == A_.pr.atom_a[P2] && a == A_.pr.atom_b[P2];
 }
 
-// Output slice of nuclear coordinate y in a derivative-tensor scatter:
-// slot_map[y] when given (-1 = not wanted), else every slice (coord < 0) or
-// only coordinate `coord` into slice 0.
+// Output slice of nuclear coordinate y in a derivative-tensor pass (-1: not
+// wanted): its place in the pass's range, or every slice (coord < 0), or only
+// coordinate `coord` into slice 0.
 __device__ __forceinline__ long long qx_dfull_slice(const QxEpiDev& e, int y) {
-  if (e.slot_map) return e.slot_map[y];
+  if (e.nslice) return y >= e.slice0 && y < e.slice0 + e.nslice ? y - e.slice0 : -1;
   if (e.coord >= 0) return y == e.coord ? 0 : -1;
   return y;
 }

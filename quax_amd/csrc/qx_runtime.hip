@@ -654,13 +654,17 @@ static double* begin_grad_copies(qx_ctx* c, hipStream_t s) {
   return c->gcopies;
 }
 
+// Orders a pass on stream s after the previous user of the context's
+// workspaces.
+void order_ws(qx_ctx* c, hipStream_t s) {
+  if (!c->ws_ev) QX_HIP(hipEventCreateWithFlags(&c->ws_ev, hipEventDisableTiming));
+  if (c->ws_used && !c->capturing) QX_HIP(hipStreamWaitEvent(s, c->ws_ev, 0));
+}
+
 // Work matrices of a J/K or gradient pass on stream s (see qx_ctx::ws).
 double* begin_ws(qx_ctx* c, hipStream_t s) {
-  if (!c->ws) {
-    c->ws = dalloc<double>(c, (size_t)5 * c->ncart * c->ncart);
-    QX_HIP(hipEventCreateWithFlags(&c->ws_ev, hipEventDisableTiming));
-  }
-  if (c->ws_used && !c->capturing) QX_HIP(hipStreamWaitEvent(s, c->ws_ev, 0));
+  if (!c->ws) c->ws = dalloc<double>(c, (size_t)5 * c->ncart * c->ncart);
+  order_ws(c, s);
   return c->ws;
 }
 
@@ -1025,27 +1029,51 @@ struct PairMatrix {
   double* M = nullptr;
   int* index = nullptr;
   int* fn = nullptr;
+  bool captured = false;     // the pass is being captured
   std::unique_ptr<DevBuf> own;
 };
 
+// Device memory calls that a capture in progress, here or in another thread,
+// does not refuse.
+struct RelaxedCapture {
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+  ~RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+};
+
+static bool is_capturing(hipStream_t s) {
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(s, &st) != hipSuccess) {
+    (void)hipGetLastError();  // the default stream while another one is captured
+    return false;
+  }
+  return st != hipStreamCaptureStatusNone;
+}
+
 // Gives the kept workspace back; hipFree waits for passes that still read it.
 static void drop_pairm(qx_ctx* c) {
+  const RelaxedCapture relaxed;
   void* p = c->pairm;
   c->pairm = nullptr;
   c->pairm_bytes = 0;
   if (p) QX_HIP(hipFree(p));
 }
 
-// `bytes` of workspace, or null when the device has no room.
+// `bytes` of workspace, or null when the device has no room.  A captured pass
+// gets its own, which stays until the context goes: replays use it whatever the
+// context has done since.
 static void* pairm_room(qx_ctx* c, PairMatrix& m, size_t bytes) {
+  const RelaxedCapture relaxed;
   void* p = nullptr;
-  if (bytes <= c->pairm_bytes) return c->pairm;
-  drop_pairm(c);  // before the larger one, which may need its room
+  if (bytes <= c->pairm_bytes && !m.captured) return c->pairm;
+  if (!m.captured) drop_pairm(c);  // before the larger one, which may need its room
   if (hipMalloc(&p, bytes) != hipSuccess) {
     (void)hipGetLastError();
     return nullptr;
   }
-  if (bytes <= QX_PAIRM_KEEP) {
+  if (m.captured) {
+    c->allocs.push_back(p);
+  } else if (bytes <= QX_PAIRM_KEEP) {
     c->pairm = static_cast<double*>(p);
     c->pairm_bytes = bytes;
   } else {
@@ -1058,6 +1086,7 @@ static void* pairm_room(qx_ctx* c, PairMatrix& m, size_t bytes) {
 // the device (or pairm_limit) has room, else fewer, else row panels of as many
 // slices as take 36 rows each, the components of one dd pair.
 static void begin_pairm(qx_ctx* c, PairMatrix& m, int want, hipStream_t s) {
+  m.captured = is_capturing(s);
   int at = 0;
   for (int X = 0; X < 6; ++X) {
     m.ix.base[X] = at;
@@ -1095,7 +1124,7 @@ static void begin_pairm(qx_ctx* c, PairMatrix& m, int want, hipStream_t s) {
   char* q = static_cast<char*>(p) + data;
   m.index = reinterpret_cast<int*>(q);
   m.fn = reinterpret_cast<int*>(q + bi);
-  (void)begin_ws(c, s);  // orders this pass after the previous user of the context's workspaces
+  if (!m.captured) order_ws(c, s);
   check_launch(qxk_pairm_tables(&c->shells, &c->pr, c->npairs, &m.ix, m.ld, m.index, m.fn, s), "pair tables");
 }
 
@@ -1176,7 +1205,7 @@ static void run_pairm(qx_ctx* c, PairMatrix& m, int nslice, double* out, hipStre
   if (m.panel == 0) {
     check_launch(qxk_fill(m.M, nslice * m.slice, 0.0, s), "fill");
     for (const auto& wh : c->work) v.push_back(launch(wh, pairm_list(c, m, wh)));
-    run_launches(c, v, s, "pair matrix", true);
+    run_launches(c, v, s, "pair matrix", !m.captured);
     check_launch(qxk_pairm_ao(&c->shells, &m.ix, m.fn, m.M, m.ld, m.slice, nslice, s), "pair transform");
     check_launch(qxk_pairm_sym(m.M, m.ld, m.slice, nslice, &m.ix, s), "pair mirror");
     check_launch(qxk_pairm_expand(c->nbf, m.M, m.ld, m.slice, nslice, m.index, m.fn, out, s), "pair expand");
@@ -1210,6 +1239,7 @@ static void run_pairm(qx_ctx* c, PairMatrix& m, int nslice, double* out, hipStre
 }
 
 static void end_pairm(qx_ctx* c, PairMatrix& m, hipStream_t s) {
+  if (m.captured) return;
   end_ws(c, s);
   if (m.own) QX_HIP(hipStreamSynchronize(s));  // freed on return
 }
@@ -1374,22 +1404,17 @@ static void deriv_tensor(qx_ctx* c, int coord, double* out, hipStream_t s) {
   PairMatrix m;
   begin_pairm(c, m, nslices, s);
   const int group = m.nslice;
-  std::vector<int> map(3 * c->natom);
   for (int y0 = 0; y0 < nslices; y0 += group) {
     const int ny = std::min(group, nslices - y0);
     QxEpiDev e{};
     e.epi = QX_EPI_PAIRM; e.nbf = c->ncart; e.natom = c->natom; e.coord = coord;
-    std::unique_ptr<DevBuf> dmap;
     if (ny < nslices) {
-      for (int y = 0; y < 3 * c->natom; ++y) map[y] = y >= y0 && y < y0 + ny ? y - y0 : -1;
-      dmap.reset(new DevBuf(map.size() * sizeof(int)));
-      QX_HIP(hipMemcpy(dmap->p, map.data(), map.size() * sizeof(int), hipMemcpyHostToDevice));
-      e.slot_map = static_cast<const int*>(dmap->p);
+      e.slice0 = y0;
+      e.nslice = ny;
     }
     run_pairm(c, m, ny, out + (size_t)y0 * nb4, s, [&](const QxWorkHost& wh, const QxPairM& pm) {
       return deri_launch(c, wh, pm, e, 0);
     });
-    if (dmap) QX_HIP(hipStreamSynchronize(s));
   }
   end_pairm(c, m, s);
 }
@@ -1428,25 +1453,21 @@ static void deriv2_tensor(qx_ctx* c, long long want, double* out, hipStream_t s)
     }
   std::vector<double> tv((size_t)m * m, 0.0);
   for (int x = 0; x < m; ++x) tv[(size_t)x * m + x] = 1.0;
-  std::vector<int> map(passes.size() * m, -1);
-  for (size_t k = 0; k < passes.size(); ++k)
-    for (int y = 0; y < passes[k].ny; ++y) map[k * m + passes[k].y0 + y] = y;
-  DevBuf dtv(tv.size() * sizeof(double)), dmap(map.size() * sizeof(int));
+  DevBuf dtv(tv.size() * sizeof(double));
   QX_HIP(hipMemcpy(dtv.d(), tv.data(), tv.size() * sizeof(double), hipMemcpyHostToDevice));
-  QX_HIP(hipMemcpy(dmap.p, map.data(), map.size() * sizeof(int), hipMemcpyHostToDevice));
-  for (size_t k = 0; k < passes.size(); ++k) {
-    const Pass& ps = passes[k];
+  for (const Pass& ps : passes) {
     QxEpiDev e{};
     e.epi = QX_EPI_PAIRM; e.nbf = c->ncart; e.natom = c->natom; e.coord = -1;
     e.tv = dtv.d() + (size_t)ps.x * m;
-    e.slot_map = static_cast<const int*>(dmap.p) + k * m;
+    e.slice0 = ps.y0;
+    e.nslice = ps.ny;
     double* dst = out + (want >= 0 ? 0 : (size_t)pair_index(ps.x, ps.y0, m) * nb4);
     run_pairm(c, pmx, ps.ny, dst, s, [&](const QxWorkHost& wh, const QxPairM& pm) {
       return deri_launch(c, wh, pm, e, 2);
     });
   }
   end_pairm(c, pmx, s);
-  QX_HIP(hipStreamSynchronize(s));  // dtv / dmap are freed on return
+  QX_HIP(hipStreamSynchronize(s));  // dtv is freed on return
 }
 
 int qx_eri_deriv_core(qx_ctx* c, int order, double* out, void* stream) {

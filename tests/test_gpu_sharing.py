@@ -81,3 +81,59 @@ def test_noalloc_pass_uses_no_events(gpu, basis, pure):
         for got, want in zip((J, K), eng.jk(D)):
             _same(got, want)
         assert eng.profile_read()[1].sum() > 0
+
+
+@pytest.mark.parametrize("warm", [False, True])
+@pytest.mark.parametrize("basis,pure", [("sto-3g", False), ("even-tempered", False), ("even-tempered", True)])
+def test_captured_tensor_passes(gpu, basis, pure, warm):
+    """Integral and first-derivative tensors under capture, in a fresh context and
+    in one whose workspace other passes have used, replayed between eager passes
+    that use and give back that workspace."""
+    torch = gpu
+    from quax_amd.engine import EriEngine
+    mol = synthetic_cluster(1, 1, 5)
+    calls = [lambda e: e.compute_2e_int(), lambda e: e.eri_deriv_core(1),
+             lambda e: e.compute_2e_deriv([0] * 6), lambda e: e.compute_2e_deriv([0, 0, 0, 0, 1, 0])]
+    with EriEngine(mol, BasisSet.build(mol, basis, pure=pure), ints_tol=1e-12) as ref_eng:
+        ref = [f(ref_eng).clone() for f in calls]
+    for f, want in zip(calls, ref):
+        with EriEngine(mol, BasisSet.build(mol, basis, pure=pure), ints_tol=1e-12) as eng:
+            D = torch.as_tensor(_density(eng.nbf, 4), device="cuda")
+            if warm:
+                calls[1](eng)
+                eng.jk(D)
+            torch.cuda.synchronize()
+            graph = torch.cuda.CUDAGraph()
+            with torch.cuda.graph(graph):
+                out = f(eng)
+            for rep in range(4):
+                out.fill_(float("nan"))
+                graph.replay()
+                torch.cuda.synchronize()
+                _same(out, want)
+                for other, w in zip(calls, ref):
+                    _same(other(eng), w)
+                eng.jk(D)
+                if rep == 1:
+                    eng.set_tensor_limit(1 << 30)
+                    eng.set_tensor_limit(0)
+
+
+def test_captured_tensor_pass_in_slices(gpu):
+    torch = gpu
+    from quax_amd.engine import EriEngine
+    mol = synthetic_cluster(1, 1, 5)
+    with EriEngine(mol, BasisSet.build(mol, "sto-3g", pure=False), ints_tol=1e-12) as eng:
+        want = eng.eri_deriv_core(1).clone()
+        for limit in (24 * 24 * 8 * 2, 4096):  # two of six slices; row panels
+            eng.set_tensor_limit(limit)
+            torch.cuda.synchronize()
+            graph = torch.cuda.CUDAGraph()
+            with torch.cuda.graph(graph):
+                out = eng.eri_deriv_core(1)
+            for _ in range(3):
+                out.fill_(float("nan"))
+                graph.replay()
+                torch.cuda.synchronize()
+                _same(out, want)
+                _same(eng.eri_deriv_core(1), want)
