@@ -270,7 +270,13 @@ int qx_scf_matrix(qx_scf* scf, int which, double* out, void* stream);
 void qx_scf_destroy(qx_scf* scf);
 const char* qx_scf_last_error(const qx_scf* scf);
 
-/* Quartet tiles (no reference counterpart): threads per workgroup, and so the
+/* Tuning per class.  A basis of s and p shells alone runs a J/K pass of up to
+ * 2e6 primitive quartets, or a gradient of up to 1e7, in one launch on the
+ * caller's stream, as long as the setters below are at their defaults for these
+ * classes and profiling is off; otherwise, and in every other basis, each class
+ * is a launch of its own.
+ *
+ * Quartet tiles (no reference counterpart): threads per workgroup, and so the
  * quartets that share its LDS K' rows, of the K and gradient kernels with one
  * lane per quartet (the quadrature classes ignore it), per pass
  * (0 = J/K, 1 = adjoint gradient); block[qx_num_classes()], multiples of
@@ -340,7 +346,8 @@ int qx_set_tensor_limit(qx_ctx* ctx, long long bytes);
  * number of derivative kernel parts of class cls.
  * qx_profile_enable(1) resets and starts recording a HIP event pair around
  * every kernel launch, on the stream the kernel runs on (with
- * qx_set_streams(ctx, 1) every kernel is timed alone); qx_profile_read
+ * qx_set_streams(ctx, 1) every kernel is timed alone) and launches every class
+ * by itself (see the tuning calls); qx_profile_read
  * synchronises and returns, per
  * slot, the summed kernel time in ms, the launch count and the primitive-pair
  * quartets processed.  Arrays hold qx_profile_slots() entries;

@@ -1513,6 +1513,17 @@ int qx_compute_2e_deriv(qx_ctx* c, const int* dv, int len, double* out, void* st
   });
 }
 
+// Whether the caller left the per-class tuning of the s and p classes' kernels
+// (pass 0 J/K, 1 gradient) as it is built in: one launch for all has none.
+static bool default_tuning(const qx_ctx* c, int pass) {
+  for (int k = 0; k < 6; ++k) {
+    if (c->tile[pass][k] != qx_tile_default[k][pass]) return false;
+    if (pass == 0 && !c->jkrows[k]) return false;
+    if (pass == 1 && (c->gwred[k] != qx_gwred_default[k] || c->gcopy[k] != qx_gcopy_default[k])) return false;
+  }
+  return true;
+}
+
 // The lists of a pass as one launch, where no shell is above p and the whole
 // pass has at most QX_SMALL_QUARTETS primitive quartets: minimal basis, 3 atoms
 // 49 us against 128 in separate launches, 8 atoms (0.7 million) 92 against 135,
@@ -1521,7 +1532,7 @@ int qx_compute_2e_deriv(qx_ctx* c, const int* dv, int len, double* out, void* st
 // launches.
 #define QX_SMALL_QUARTETS 2000000
 static bool small_pass(qx_ctx* c, const QxEpiDev& e, const QxJList& jl, bool timed, QxSmall& sm, size_t& lds) {
-  if ((timed && c->profiling) || !e.krows || c->class_pair_cnt[3] + c->class_pair_cnt[4] + c->class_pair_cnt[5] > 0) return false;
+  if ((timed && c->profiling) || !e.krows || !default_tuning(c, 0) || c->class_pair_cnt[3] + c->class_pair_cnt[4] + c->class_pair_cnt[5] > 0) return false;
   if (c->npq_total > QX_SMALL_QUARTETS) return false;
   sm = QxSmall{};
   long long blocks[9] = {};
@@ -1556,7 +1567,8 @@ static bool small_pass(qx_ctx* c, const QxEpiDev& e, const QxJList& jl, bool tim
 #define QX_SMALL_GRAD_QUARTETS 10000000
 static_assert(QX_SMALL_GRADS <= 16, "lists of the one-launch gradient");
 static bool small_grad(const qx_ctx* c, QxSmallGrad& sm) {
-  if (c->profiling || c->class_pair_cnt[3] + c->class_pair_cnt[4] + c->class_pair_cnt[5] > 0) return false;
+  if (c->profiling || !default_tuning(c, 1) || c->class_pair_cnt[3] + c->class_pair_cnt[4] + c->class_pair_cnt[5] > 0)
+    return false;
   if (c->npq_total > QX_SMALL_GRAD_QUARTETS) return false;
   sm = QxSmallGrad{};
   long long blocks[6] = {}, end = 0;

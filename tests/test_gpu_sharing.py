@@ -119,6 +119,49 @@ def test_captured_tensor_passes(gpu, basis, pure, warm):
                     eng.set_tensor_limit(0)
 
 
+def _kernels(torch, call):
+    """Kernel launches of a call, from the graph it is captured into."""
+    hip = ctypes.CDLL("libamdhip64.so")
+    graph = torch.cuda.CUDAGraph(keep_graph=True)
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph):
+        call()
+    raw, n = ctypes.c_void_p(graph.raw_cuda_graph()), ctypes.c_size_t()
+    assert hip.hipGraphGetNodes(raw, None, ctypes.byref(n)) == 0
+    nodes = (ctypes.c_void_p * n.value)()
+    assert hip.hipGraphGetNodes(raw, nodes, ctypes.byref(n)) == 0
+    kinds = [ctypes.c_int() for _ in nodes]
+    assert all(hip.hipGraphNodeGetType(ctypes.c_void_p(x), ctypes.byref(k)) == 0 for x, k in zip(nodes, kinds))
+    return sum(k.value == 0 for k in kinds)
+
+
+@pytest.mark.parametrize("setter,value,pass_", [("set_class_tiles", 192, 0), ("set_jk_rows", 0, 0),
+                                                ("set_class_tiles", 192, 1), ("set_grad_copies", 2, 1),
+                                                ("set_grad_wave_reduce", None, 1)])
+def test_tuning_calls_reach_small_molecules(gpu, setter, value, pass_):
+    """A small s, p molecule's one launch gives way to the class kernels that a
+    tuning call addresses, with the same results, and comes back with the defaults."""
+    torch = gpu
+    with _context("sto-3g", False) as eng:
+        D = torch.as_tensor(_density(eng.nbf, 5), device="cuda")
+        out = [torch.empty((eng.nbf, eng.nbf), dtype=torch.float64, device="cuda") for _ in range(2)]
+        run = (lambda: eng.jk(D, out=out)) if pass_ == 0 else (lambda: (eng.eri_grad(D),))
+        want = [x.clone() for x in run()]
+        one = _kernels(torch, run)
+        set_ = getattr(eng, setter)
+        args = (pass_,) if setter == "set_class_tiles" else ()
+        n = len(eng.jk_rows())
+        flags = [value] * n if value is not None else [not f for f in eng.grad_wave_reduce()]
+        set_(*args, flags)
+        for got, w in zip(run(), want):
+            _same(got, w)
+        assert _kernels(torch, run) >= one + 5  # six class lists at least
+        set_(*args, None)
+        assert _kernels(torch, run) == one
+        for got, w in zip(run(), want):
+            _same(got, w)
+
+
 def test_captured_tensor_pass_in_slices(gpu):
     torch = gpu
     from quax_amd.engine import EriEngine
