@@ -222,7 +222,9 @@ const char* qx_gemm_last_error(void);
  * qx_set_fp32_classes: per-class policy of a pass, flags[qx_num_classes()]
  * (nonzero = FP32 allowed), or the built-in default (from timings of FP32
  * against FP64 kernels per class) when flags is NULL; qx_get_fp32_classes
- * reads it. */
+ * reads it.  The classes whose gradient is by quadrature, (dp|pp), (dp|ds),
+ * (dp|dp) and (dd|ps) to (dd|dd), have no FP32 gradient: they run it in FP64
+ * whatever the policy allows. */
 int qx_mixed_quartets(qx_ctx* ctx, double fp32_threshold, long long* n_fp64, long long* n_fp32);
 int qx_mixed_pass_quartets(qx_ctx* ctx, double fp32_threshold, int pass, long long* n_fp64, long long* n_fp32);
 int qx_set_fp32_classes(qx_ctx* ctx, int pass, const int* flags);

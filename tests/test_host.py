@@ -280,6 +280,16 @@ def test_tuned_tables_reach_the_generated_class_table(tmp_path):
         assert f32 == (int(nm in tuning["fp32"]["jk"]), int(nm in tuning["fp32"]["grad"])), nm
 
 
+def test_built_in_policy_names_only_kernels_that_exist():
+    """The default FP32 policy and quartet tiles of the gradient leave out the
+    classes whose gradient is by quadrature: it has neither."""
+    from quax_amd.csrc import gen_eri
+    with open(os.path.join(ROOT, "quax_amd", "csrc", "deriv_budget.json")) as fh:
+        tuning = json.load(fh)
+    assert gen_eri.RYS_G and not gen_eri.RYS_G & (set(tuning["fp32"]["grad"]) | set(tuning["tiles"]["grad"]))
+    assert gen_eri.RYS_K and not gen_eri.RYS_K & set(tuning["tiles"]["jk"])
+
+
 def test_streaming_kernels_fit_side_stream_scratch():
     """Every streaming J/K and adjoint-gradient kernel of the last build needs
     at most 6 KB of scratch per lane (the side streams' budget; read from the
