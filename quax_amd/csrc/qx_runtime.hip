@@ -914,7 +914,8 @@ static void init_body(qx_ctx* c, int natom, const double* xyz_bohr, const double
     for (double v : c->exps) QX_REQUIRE(v > 0 && std::isfinite(v), QX_EINVAL, "exponents must be positive");
     for (int s = 0; s < nshell; ++s)
       normalize_shell(c->l[s], c->nprim[s], &c->exps[c->poff[s]], coefs + c->poff[s], &c->coefs[c->poff[s]]);
-    c->d_boys = dupload(c, boys_table());
+    static const std::vector<double> boys = boys_table();  // 0.5 ms of long double arithmetic, once per process
+    c->d_boys = dupload(c, boys);
     setup_shell_tables(c);
     schwarz_and_lists(c);
     setup_jk(c);
