@@ -20,7 +20,7 @@ struct QxGradTarget {
 __device__ __forceinline__ QxGradTarget qx_grad_begin(const QxArgs& A_, const QxKList& kl, int P1, double* lds) {
   QxGradTarget t;
   const int nc = A_.e.grad_copies > 1 ? A_.e.grad_copies : 1;
-  t.g = A_.e.grad + (size_t)((blockIdx.x + blockIdx.y * 7) % nc) * (size_t)(3 * A_.e.natom);
+  t.g = A_.e.grad + (size_t)((blockIdx.x + blockIdx.y * 7 + blockIdx.z * 13) % nc) * (size_t)(3 * A_.e.natom);
   const int cap = A_.e.grad_win > 0 && A_.e.grad_win < QX_GRAD_LDS ? A_.e.grad_win : QX_GRAD_LDS;
   t.lo = 0;
   t.w = 3 * A_.e.natom;

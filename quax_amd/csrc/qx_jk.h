@@ -35,7 +35,8 @@ struct QxKList {
   long long nquart;
   int chunk;                  // kets per workgroup
   int ketprim;                // most primitives of a ket pair of the class
-  int sub;                    // lanes that share one contracted quartet's primitives
+  int sub;                    // lanes that share one contracted quartet's primitives (one-lane kernels)
+  int psplit;                 // workgroups that share them (quadrature kernels; grid z)
   const double* rys;          // Rys root and weight tables
   const int* frag_atoms;      // gradient: first atom and atom count of each fragment (null: one fragment)
 };

@@ -96,13 +96,12 @@ __global__ void k_fill_int(int* p, long long n, int v) {
     p[i] = v;
 }
 
-// One thread per screened shell pair: the rows of its AO function pairs (index)
-// and the function pair of each row (fn: higher << 16 | lower, -1 for a
-// component no pair has).  A pair's AO components take the first of the rows
-// its Cartesian ones had.
-__global__ void k_pairm_index(QxShellsDev sh, QxPairsDev pr, int npairs, QxPairIndex ix, int* index, int* fn) {
-  const int P = blockIdx.x * blockDim.x + threadIdx.x;
-  if (P >= npairs) return;
+// Screened shell pair P: the rows of its AO function pairs (index) and the
+// function pair of each row (fn: higher << 16 | lower, -1 for a component no
+// pair has).  A pair's AO components take the first of the rows its Cartesian
+// ones had.
+__device__ __forceinline__ void pairm_index(const QxShellsDev& sh, const QxPairsDev& pr, int P, const QxPairIndex& ix,
+                                            int* index, int* fn) {
   const int la = sh.l[pr.sa[P]], lb = sh.l[pr.sb[P]], n = sh.nbf;
   const int na = sh.pure && la > 1 ? 2 * la + 1 : (la + 1) * (la + 2) / 2;
   const int nb = sh.pure && lb > 1 ? 2 * lb + 1 : (lb + 1) * (lb + 2) / 2;
@@ -118,6 +117,23 @@ __global__ void k_pairm_index(QxShellsDev sh, QxPairsDev pr, int npairs, QxPairI
       index[(size_t)g * n + f] = row;
       fn[row] = max(f, g) << 16 | min(f, g);
     }
+}
+__global__ void k_pairm_index(QxShellsDev sh, QxPairsDev pr, int npairs, QxPairIndex ix, int* index, int* fn) {
+  const int P = blockIdx.x * blockDim.x + threadIdx.x;
+  if (P < npairs) pairm_index(sh, pr, P, ix, index, fn);
+}
+
+// The tables of a small context and its cleared matrices in one workgroup:
+// launches are most of such a tensor's time (two functions 57 us in four
+// launches, ONEWG here).
+#define PM_SMALL 16384  // doubles of the matrices, ints of the tables
+__global__ __launch_bounds__(1024) void k_pairm_small(QxShellsDev sh, QxPairsDev pr, int npairs, QxPairIndex ix, int ld,
+                                                     int* index, int* fn, double* M, int nm) {
+  for (int i = threadIdx.x; i < sh.nbf * sh.nbf; i += blockDim.x) index[i] = -1;
+  for (int i = threadIdx.x; i < ld; i += blockDim.x) fn[i] = -1;
+  for (int i = threadIdx.x; i < nm; i += blockDim.x) M[i] = 0.0;
+  __syncthreads();
+  for (int P = threadIdx.x; P < npairs; P += blockDim.x) pairm_index(sh, pr, P, ix, index, fn);
 }
 
 // Class and pair position of row r.
@@ -270,13 +286,15 @@ __global__ void k_pairm_scatter(int nc, const double* M, long long ld, long long
 // tensor's HBM writes.  Transforming to AO functions here, with a gather
 // through an index table per (r, u), took 1196 us for the 112-function tensor
 // (1.26 GB), with one lane per ket shell pair 822 us; this takes 330 and the
-// two transforming passes 125.
+// two transforming passes 125.  HALF: M is not mirrored, an element of the other
+// half is read where it is stored (small matrices: a launch less).
+#define PM_HALF 512  // rows
 #define PM_LDS_TRI (150 * 1024)  // a triangle takes one panel up to here (n <= 195)
 #define PM_LDS_ROWS (72 * 1024)  // rows of a panel beyond: two workgroups per CU
 // An output row pair goes out without a stay in the caches: nothing reads it here.
 typedef double pm_dv2 __attribute__((vector_size(16)));
-template <bool TRI>
-__global__ __launch_bounds__(1024) void k_pairm_expand(int n, const double* M, long long ld, long long slice,
+template <bool TRI, bool HALF>
+__global__ __launch_bounds__(1024) void k_pairm_expand(int n, const double* M, long long ld, long long slice, QxPairIndex ix,
                                                       const int* index, const int* fn, int rows, double* out) {
   HIP_DYNAMIC_SHARED(double, row)
   const long long t = blockIdx.x;
@@ -291,11 +309,20 @@ __global__ __launch_bounds__(1024) void k_pairm_expand(int n, const double* M, l
   const int from = index[(size_t)p * n + q];
   if (from >= 0) {
     const double* m = M + (long long)blockIdx.y * slice + from * ld;
+    int X = 0, pos = 0;
+    if (HALF) pairm_row(ix, from, X, pos);
 #pragma unroll 4
     for (int c = threadIdx.x; c < ld; c += blockDim.x) {
       const int f = fn[c], r = f >> 16, u = f & 0xffff;
       if (f < 0) continue;
-      const double v = m[c];
+      double v;
+      if (HALF) {
+        int Y, j;
+        pairm_row(ix, c, Y, j);
+        v = X > Y || (X == Y && pos >= j) ? m[c] : M[(long long)blockIdx.y * slice + c * ld + from];
+      } else {
+        v = m[c];
+      }
       if (TRI) {
         row[r * (r + 1) / 2 + u] = v;
       } else {
@@ -598,8 +625,13 @@ int qxk_ao_to_cart_mat(const QxShellsDev* sh, const double* in, double* out, hip
 }
 
 int qxk_pairm_tables(const QxShellsDev* sh, const QxPairsDev* pr, int npairs, const QxPairIndex* ix, long long ld, int* index,
-                     int* fn, hipStream_t s) {
+                     int* fn, double* M, long long nm, int* cleared, hipStream_t s) {
   const long long n2 = (long long)sh->nbf * sh->nbf;
+  *cleared = n2 + ld <= PM_SMALL && nm <= PM_SMALL;
+  if (*cleared) {
+    hipLaunchKernelGGL(k_pairm_small, dim3(1), dim3(1024), 0, s, *sh, *pr, npairs, *ix, (int)ld, index, fn, M, (int)nm);
+    return (int)hipGetLastError();
+  }
   hipLaunchKernelGGL(k_fill_int, dim3(std::min(nblk(n2, 256), 4096u)), dim3(256), 0, s, index, n2, -1);
   hipLaunchKernelGGL(k_fill_int, dim3(std::min(nblk(ld, 256), 4096u)), dim3(256), 0, s, fn, ld, -1);
   if (npairs > 0)
@@ -619,9 +651,14 @@ int qxk_pairm_ao(const QxShellsDev* sh, const QxPairIndex* ix, const int* fn, do
   return (int)hipGetLastError();
 }
 
-int qxk_pairm_sym(double* M, long long ld, long long slice, int nslice, const QxPairIndex* ix, hipStream_t s) {
+// Whether the expansion reads the stored half (M is then not mirrored).
+static bool pairm_half(int n, long long ld) {
+  return ld <= PM_HALF && (size_t)n * (n + 1) / 2 * sizeof(double) <= PM_LDS_TRI;
+}
+
+int qxk_pairm_sym(int n, double* M, long long ld, long long slice, int nslice, const QxPairIndex* ix, hipStream_t s) {
   const long long T = (ld + PM_TILE - 1) / PM_TILE, tiles = T * (T + 1) / 2;
-  if (tiles <= 0 || nslice <= 0) return 0;
+  if (tiles <= 0 || nslice <= 0 || pairm_half(n, ld)) return 0;
   if (tiles > 0x7fffffffLL || nslice > 65535) return (int)hipErrorInvalidValue;
   hipLaunchKernelGGL(k_pairm_sym, dim3((unsigned)tiles, (unsigned)nslice), dim3(256), 0, s, M, ld, slice, *ix);
   return (int)hipGetLastError();
@@ -637,8 +674,8 @@ int qxk_pairm_scatter(int ncart, const double* M, long long ld, long long slice,
   return (int)hipGetLastError();
 }
 
-int qxk_pairm_expand(int n, const double* M, long long ld, long long slice, int nslice, const int* index, const int* fn,
-                     double* out, hipStream_t s) {
+int qxk_pairm_expand(int n, const double* M, long long ld, long long slice, int nslice, const QxPairIndex* ix,
+                     const int* index, const int* fn, double* out, hipStream_t s) {
   if (nslice <= 0) return 0;
   const size_t tri = (size_t)n * (n + 1) / 2 * sizeof(double);
   const bool one = tri <= PM_LDS_TRI;
@@ -647,8 +684,9 @@ int qxk_pairm_expand(int n, const double* M, long long ld, long long slice, int 
   const dim3 grid((unsigned)((long long)n * (n + 1) / 2), (unsigned)nslice, (unsigned)((n + rows - 1) / rows));
   if (nslice > 65535 || bytes > PM_LDS_TRI) return (int)hipErrorInvalidValue;
   const dim3 block(n < 96 ? 512 : 1024);  // 112 functions: 464 us with 256 threads, 371 with 512, 328 with 1024
-  if (one) hipLaunchKernelGGL(k_pairm_expand<true>, grid, block, bytes, s, n, M, ld, slice, index, fn, rows, out);
-  else hipLaunchKernelGGL(k_pairm_expand<false>, grid, block, bytes, s, n, M, ld, slice, index, fn, rows, out);
+  if (pairm_half(n, ld)) hipLaunchKernelGGL((k_pairm_expand<true, true>), grid, block, bytes, s, n, M, ld, slice, *ix, index, fn, rows, out);
+  else if (one) hipLaunchKernelGGL((k_pairm_expand<true, false>), grid, block, bytes, s, n, M, ld, slice, *ix, index, fn, rows, out);
+  else hipLaunchKernelGGL((k_pairm_expand<false, false>), grid, block, bytes, s, n, M, ld, slice, *ix, index, fn, rows, out);
   return (int)hipGetLastError();
 }
 

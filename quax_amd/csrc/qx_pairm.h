@@ -26,6 +26,8 @@ struct QxPairM {
   const int* kstart;         // per bra pair: first admissible ket pair (null = 0)
   int nbra;
   long long nquart;          // contracted quartets
+  int sub;                   // adjacent lanes that share one contracted quartet's primitives (array-form kernels): a
+                             // power of two up to 64
   long long t0;              // number of the first one (a panel of bra pairs starts inside the list)
 };
 
@@ -42,25 +44,33 @@ __device__ __forceinline__ void qx_locate_pairs(const QxPairM& pm, long long t, 
 }
 
 template <int NAB, int NCD, typename R>
-__device__ __forceinline__ void qx_pairm_eri(const QxPairM& pm, int P1, int P2, const R (&o)[NAB * NCD]) {
+__device__ __forceinline__ void qx_pairm_eri(const QxPairM& pm, int P1, int P2, bool lead, const R (&o)[NAB * NCD]) {
   double* m = pm.M + (long long)(pm.row0 + P1 - pm.rowp) * pm.ld + pm.col0 + (P2 - pm.colp);
 #pragma unroll
   for (int ij = 0; ij < NAB; ++ij)
 #pragma unroll
-    for (int kl = 0; kl < NCD; ++kl) m[(long long)ij * pm.rown * pm.ld + (long long)kl * pm.coln] = (double)o[ij * NCD + kl];
+    for (int kl = 0; kl < NCD; ++kl) {
+      double v = (double)o[ij * NCD + kl];
+      for (int off = pm.sub >> 1; off > 0; off >>= 1) v += __shfl_xor(v, off);  // launch-uniform
+      if (lead) m[(long long)ij * pm.rown * pm.ld + (long long)kl * pm.coln] = v;
+    }
 }
 
 // ---- array-form kernels ---------------------------------------------------
-// The integral cores add to their output array, so that a PAIRM launch (one
-// lane per contracted quartet) sums its primitive quartets in place; the
-// other epilogues run one lane per primitive quartet.
+// The integral cores add to their output array, so that a PAIRM launch sums its
+// primitive quartets in place: one lane per contracted quartet, or pm.sub of
+// them in a small molecule, each a share, and the shares meet in cross-lane sums
+// (by atomics, the tensor of 8 atoms in a minimal basis took 442 us against 138).
+// The other epilogues run one lane per primitive quartet.
 struct QxArrayQuartet {
-  int P1, P2, u1, u2, n1, n2;
+  int P1, P2, u1, u2, n1, n2, k0, ks;  // primitive quartets k0, k0 + ks, ...
 };
 __device__ __forceinline__ bool qx_array_quartet(const QxArgs& A_, const QxPairM& pm, long long t, QxArrayQuartet& q) {
   if (A_.e.epi == QX_EPI_PAIRM) {
-    if (t >= pm.nquart) return false;
-    qx_locate_pairs(pm, t, q.P1, q.P2);
+    if (t >= pm.nquart * pm.sub) return false;
+    q.ks = pm.sub;
+    q.k0 = (int)(t % pm.sub);
+    qx_locate_pairs(pm, t / pm.sub, q.P1, q.P2);
     q.u1 = A_.pr.pp_first[q.P1];
     q.u2 = A_.pr.pp_first[q.P2];
     q.n1 = A_.pr.pp_n[q.P1];
@@ -68,13 +78,14 @@ __device__ __forceinline__ bool qx_array_quartet(const QxArgs& A_, const QxPairM
   } else {
     if (t >= A_.w.nquart) return false;
     qx_locate(A_, t, q.u1, q.u2, q.P1, q.P2);
-    q.n1 = q.n2 = 1;
+    q.n1 = q.n2 = q.ks = 1;
+    q.k0 = 0;
   }
   return true;
 }
 
 static inline dim3 qx_array_grid(const QxArgs* a, const QxLaunch* L, long long& nq) {
-  nq = a->e.epi == QX_EPI_PAIRM ? (L->pm ? L->pm->nquart : 0) : a->w.nquart;
+  nq = a->e.epi == QX_EPI_PAIRM ? (L->pm ? L->pm->nquart * L->pm->sub : 0) : a->w.nquart;
   return dim3((unsigned)((nq + QX_BLOCK - 1) / QX_BLOCK));
 }
 
@@ -86,9 +97,9 @@ static inline dim3 qx_array_grid(const QxArgs* a, const QxLaunch* L, long long& 
     if (!qx_array_quartet(A_, pm, t, q)) return;                                                  \
     if (A_.e.skip_single && qx_single_atom(A_, q.P1, q.P2)) return;                               \
     double o[N] = {};                                                                             \
-    for (int i = 0; i < q.n1; ++i)                                                                \
-      for (int j = 0; j < q.n2; ++j) qx_core_##NAME<double>(A_, q.P1, q.P2, q.u1 + i, q.u2 + j, o); \
-    if (A_.e.epi == QX_EPI_PAIRM) qx_pairm_eri<NA * NB, NC * ND, double>(pm, q.P1, q.P2, o);      \
+    for (int k = q.k0; k < q.n1 * q.n2; k += q.ks)                                                \
+      qx_core_##NAME<double>(A_, q.P1, q.P2, q.u1 + k / q.n2, q.u2 + k % q.n2, o);                \
+    if (A_.e.epi == QX_EPI_PAIRM) qx_pairm_eri<NA * NB, NC * ND, double>(pm, q.P1, q.P2, q.k0 == 0, o);      \
     else qx_epi_eri<NA, NB, NC, ND, double>(A_, t, q.P1, q.P2, o, true);                          \
   }                                                                                               \
   extern "C" int qx_launch_##NAME(const QxArgs* a, const QxLaunch* L) {                           \

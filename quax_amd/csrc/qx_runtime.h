@@ -219,19 +219,19 @@ int qxk_cart_to_ao_mats(const QxShellsDev* sh, const double* in, size_t stride, 
 int qxk_ao_to_cart_mats(const QxShellsDev* sh, const double* const* in, double* out, size_t stride, int count,
                         hipStream_t s);
 // Pair matrix M (nslice matrices of ld x ld, `slice` doubles apart) -> tensor.
-// index: Cartesian function pair -> row (ncart^2 ints, -1 = screened out), fn:
-// row -> p * ncart + q, ao: per AO function up to three Cartesian terms
-// (qxk_pairm_tables fills them).
+// index: AO function pair -> row (nbf^2 ints, -1 = screened out), fn: row ->
+// higher << 16 | lower function, -1 for none (qxk_pairm_tables fills them, and
+// clears the nm doubles at M where the context is small: cleared).
 int qxk_pairm_tables(const QxShellsDev* sh, const QxPairsDev* pr, int npairs, const QxPairIndex* ix, long long ld, int* index,
-                     int* fn, hipStream_t s);
+                     int* fn, double* M, long long nm, int* cleared, hipStream_t s);
 // every permutation of the elements of a panel of rows into a zeroed
 // Cartesian tensor: panel row k * cnt + i is component k of the class's pair
 // i0 + i (class X, ncomp components)
 int qxk_pairm_scatter(int ncart, const double* M, long long ld, long long slice, int nslice, const QxPairIndex* ix,
                       const int* fn, int X, int ncomp, int i0, int cnt, double* out, hipStream_t s);
-int qxk_pairm_sym(double* M, long long ld, long long slice, int nslice, const QxPairIndex* ix, hipStream_t s);
-int qxk_pairm_expand(int n, const double* M, long long ld, long long slice, int nslice, const int* index, const int* fn,
-                     double* out, hipStream_t s);
+int qxk_pairm_sym(int n, double* M, long long ld, long long slice, int nslice, const QxPairIndex* ix, hipStream_t s);
+int qxk_pairm_expand(int n, const double* M, long long ld, long long slice, int nslice, const QxPairIndex* ix,
+                     const int* index, const int* fn, double* out, hipStream_t s);
 int qxk_pairm_ao(const QxShellsDev* sh, const QxPairIndex* ix, const int* fn, double* M, long long ld, long long slice,
                  int nslice, hipStream_t s);
 int qxk_oei_deriv(const QxShellsDev* sh, double* dS, double* dT, double* dV, hipStream_t s);

@@ -1030,6 +1030,7 @@ struct PairMatrix {
   double* M = nullptr;
   int* index = nullptr;
   int* fn = nullptr;
+  int cleared = 0;           // M is cleared for the first pass
   bool captured = false;     // the pass is being captured
   std::unique_ptr<DevBuf> own;
 };
@@ -1126,7 +1127,8 @@ static void begin_pairm(qx_ctx* c, PairMatrix& m, int want, hipStream_t s) {
   m.index = reinterpret_cast<int*>(q);
   m.fn = reinterpret_cast<int*>(q + bi);
   if (!m.captured) order_ws(c, s);
-  check_launch(qxk_pairm_tables(&c->shells, &c->pr, c->npairs, &m.ix, m.ld, m.index, m.fn, s), "pair tables");
+  check_launch(qxk_pairm_tables(&c->shells, &c->pr, c->npairs, &m.ix, m.ld, m.index, m.fn, m.M, m.nslice * m.slice, &m.cleared,
+                                s), "pair tables");
 }
 
 // Kets of one bra pair that a workgroup takes: enough workgroups to fill the
@@ -1138,7 +1140,17 @@ static void begin_pairm(qx_ctx* c, PairMatrix& m, int want, hipStream_t s) {
 // would already leave CUs idle at the end: (dd|dp) 8.1 ms at half, 8.9 ms).
 #define QX_K_BLOCKS 4096
 #define QX_K_CHUNK 2048LL
+#define QX_RYS_BLOCKS 1024LL  // quadrature workgroups below which they share primitive quartets
 #define QX_SUB_LANES 65536  // lanes below which contracted quartets are shared between lanes
+
+// Primitive quartets of a contracted quartet of the list (mean, rounded up).
+static long long list_prims(const QxWorkHost& wh) {
+  return std::max((wh.w.nquart + wh.ncq - 1) / std::max(wh.ncq, 1LL), 1LL);
+}
+// Lanes that share them: few contracted quartets still spread over the device.
+static int shared_lanes(const QxWorkHost& wh) {
+  return (int)std::max<long long>(1, std::min<long long>({list_prims(wh), 64, QX_SUB_LANES / std::max(wh.ncq, 1LL)}));
+}
 
 // The contracted list wh for a kernel of one lane per quartet in blocks of
 // `block` threads, or (block = 0) of the quadrature kernels; rows: a K kernel.
@@ -1155,10 +1167,8 @@ static QxKList k_list(const qx_ctx* c, const QxWorkHost& wh, int sel, int block,
   kl.ketprim = c->class_prims[wh.ket_class];
   kl.rys = c->d_rys;
   kl.frag_atoms = c->d_frag_atoms;
-  // few contracted quartets: their primitive quartets are shared between up
-  // to 64 lanes, so that a small molecule still spreads over the device
-  const long long prims = std::max((wh.w.nquart + wh.ncq - 1) / std::max(wh.ncq, 1LL), 1LL);
-  kl.sub = (int)std::max<long long>(1, std::min<long long>({prims, 64, QX_SUB_LANES / std::max(wh.ncq, 1LL)}));
+  const long long prims = list_prims(wh);
+  kl.sub = shared_lanes(wh);
   const long long most = (wh.ncq + QX_K_BLOCKS - 1) / QX_K_BLOCKS;
   const long long per = std::max<long long>(rows ? std::max(most, std::min(4 * most, QX_K_CHUNK / prims)) : most, 1);
   // quadrature: in short lists as little as one step of each of a block's four
@@ -1169,6 +1179,9 @@ static QxKList k_list(const qx_ctx* c, const QxWorkHost& wh, int sel, int block,
   const int step = 4 * (64 / kPairFns[wh.bra_class]);
   const int unit = block ? std::max(1, block / kl.sub) : per <= 16 ? std::min(step, 32) : 32;
   kl.chunk = (int)std::min<long long>((per + unit - 1) / unit * unit, 1 << 20);
+  // quadrature workgroups that share a bra's primitive quartets, four or more each
+  const long long blocks = (long long)kl.nbra * ((kl.maxket + kl.chunk - 1) / std::max(kl.chunk, 1));
+  kl.psplit = block ? 1 : (int)std::max<long long>(1, std::min(prims / 4, QX_RYS_BLOCKS / std::max(blocks, 1LL)));
   return kl;
 }
 
@@ -1183,6 +1196,7 @@ static QxPairM pairm_list(const qx_ctx* c, const PairMatrix& m, const QxWorkHost
   pm.kstart = c->fragmented ? c->d_ckstart + wh.cprefix_off : nullptr;
   pm.nbra = c->class_pair_cnt[X];
   pm.nquart = wh.ncq;
+  for (pm.sub = 1; 2 * pm.sub <= shared_lanes(wh);) pm.sub *= 2;
   return pm;
 }
 
@@ -1198,18 +1212,20 @@ static QxKList pairm_kets(const qx_ctx* c, const QxWorkHost& wh, const QxPairM& 
 }
 
 // Evaluates the lists into nslice tensors at out: `launch(list, pm)` is one
-// list's kernel.  Whole matrices are mirrored and expanded; panels are
-// scattered.
-static void run_pairm(qx_ctx* c, PairMatrix& m, int nslice, double* out, hipStream_t s,
+// list's kernel; others_only: it leaves out quartets on a single atom.  Whole
+// matrices are mirrored and expanded; panels are scattered.
+static void run_pairm(qx_ctx* c, PairMatrix& m, int nslice, bool others_only, double* out, hipStream_t s,
                       const std::function<Launch(const QxWorkHost&, const QxPairM&)>& launch) {
   std::vector<Launch> v;
   if (m.panel == 0) {
-    check_launch(qxk_fill(m.M, nslice * m.slice, 0.0, s), "fill");
-    for (const auto& wh : c->work) v.push_back(launch(wh, pairm_list(c, m, wh)));
+    if (!m.cleared) check_launch(qxk_fill(m.M, nslice * m.slice, 0.0, s), "fill");
+    m.cleared = 0;
+    for (const auto& wh : c->work)
+      if (!others_only || c->ndq_class[wh.cls] > 0) v.push_back(launch(wh, pairm_list(c, m, wh)));
     run_launches(c, v, s, "pair matrix", !m.captured);
     check_launch(qxk_pairm_ao(&c->shells, &m.ix, m.fn, m.M, m.ld, m.slice, nslice, s), "pair transform");
-    check_launch(qxk_pairm_sym(m.M, m.ld, m.slice, nslice, &m.ix, s), "pair mirror");
-    check_launch(qxk_pairm_expand(c->nbf, m.M, m.ld, m.slice, nslice, m.index, m.fn, out, s), "pair expand");
+    check_launch(qxk_pairm_sym(c->nbf, m.M, m.ld, m.slice, nslice, &m.ix, s), "pair mirror");
+    check_launch(qxk_pairm_expand(c->nbf, m.M, m.ld, m.slice, nslice, &m.ix, m.index, m.fn, out, s), "pair expand");
     return;
   }
   const size_t nc = c->ncart, n4 = nc * nc * nc * nc;
@@ -1251,7 +1267,7 @@ static void eri_tensor(qx_ctx* c, int skip_single, double* out, hipStream_t s) {
   begin_pairm(c, m, 1, s);
   QxEpiDev e{};
   e.epi = QX_EPI_PAIRM; e.nbf = c->ncart; e.natom = c->natom; e.coord = -1; e.skip_single = skip_single;
-  run_pairm(c, m, 1, out, s, [&](const QxWorkHost& wh, const QxPairM& pm) {
+  run_pairm(c, m, 1, skip_single != 0, out, s, [&](const QxWorkHost& wh, const QxPairM& pm) {
     const QxKList kl = pairm_kets(c, wh, pm);
     return Launch{(double)pm.nquart * qx_class_table[wh.cls].eri_flops, [=](hipStream_t st) {
                     return launch_eri(c, wh.w, wh.cls, e, 0, st, c->pr, c->pp, &pm, &kl);
@@ -1413,7 +1429,7 @@ static void deriv_tensor(qx_ctx* c, int coord, double* out, hipStream_t s) {
       e.slice0 = y0;
       e.nslice = ny;
     }
-    run_pairm(c, m, ny, out + (size_t)y0 * nb4, s, [&](const QxWorkHost& wh, const QxPairM& pm) {
+    run_pairm(c, m, ny, true, out + (size_t)y0 * nb4, s, [&](const QxWorkHost& wh, const QxPairM& pm) {
       return deri_launch(c, wh, pm, e, 0);
     });
   }
@@ -1463,7 +1479,7 @@ static void deriv2_tensor(qx_ctx* c, long long want, double* out, hipStream_t s)
     e.slice0 = ps.y0;
     e.nslice = ps.ny;
     double* dst = out + (want >= 0 ? 0 : (size_t)pair_index(ps.x, ps.y0, m) * nb4);
-    run_pairm(c, pmx, ps.ny, dst, s, [&](const QxWorkHost& wh, const QxPairM& pm) {
+    run_pairm(c, pmx, ps.ny, true, dst, s, [&](const QxWorkHost& wh, const QxPairM& pm) {
       return deri_launch(c, wh, pm, e, 2);
     });
   }

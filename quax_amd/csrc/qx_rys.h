@@ -255,7 +255,9 @@ __device__ __forceinline__ int qx_rys_prims(const QxArgs& A_, int pk0, int nq) {
 
 // Runs the wavefront's share of a block's kets, Q at a time: begin(first ket,
 // how many), per primitive quartet step(i1, i2) with the 1D integrals at g,
-// end().  Every lane of the wavefront calls all three.
+// end().  Every lane of the wavefront calls all three.  Workgroups of one grid
+// column share the primitive quartets: the few long sums of a small contracted
+// molecule would otherwise run one after the other in a handful of wavefronts.
 //
 // Roots, weights and recurrence parameters of STEPS steps ahead (of several
 // ket groups, or for contracted pairs of several primitive quartets) are
@@ -287,10 +289,13 @@ __device__ __forceinline__ void qx_rys_walk(const QxArgs& A_, const QxKList& kl,
   int held = 0;  // the step whose sets are next, single primitives
   for (int k = k0; k < k1; k += S::Q) {
     const int nq = min(S::Q, k1 - k), pk0 = b.kst + k;
-    const int n2 = kl.ketprim > 1 ? qx_rys_prims(A_, pk0, nq) : 1, nc = n1 * n2;
+    // the workgroup's share of the primitive quartets
+    const int n2 = kl.ketprim > 1 ? qx_rys_prims(A_, pk0, nq) : 1, all = n1 * n2;
+    const int mb = (int)((long long)all * blockIdx.z / gridDim.z), nc = (int)((long long)all * (blockIdx.z + 1) / gridDim.z);
+    if (mb >= nc) continue;
     begin(pk0, nq);
-    for (int m = 0; m < nc; ++m) {
-      const int now = single ? held : m % S::STEPS;
+    for (int m = mb; m < nc; ++m) {
+      const int now = single ? held : (m - mb) % S::STEPS;
       if (now == 0) {
         const int m1 = m + ps, i1 = single ? 0 : m1 / n2, i2 = single ? 0 : m1 - i1 * n2;
         const int P2 = pk0 + (single ? ps * S::Q : 0) + pq;
@@ -480,7 +485,10 @@ __global__ __launch_bounds__(QX_RYS_BLOCK) void qx_re(QxArgs A_, QxKList kl, QxP
                             : pm.M + (pm.row0 + b.P1 - pm.rowp + (long long)ln.ab * pm.rown) * pm.ld + pm.col0 + (P2 - pm.colp);
           const long long step = store ? kl.nquart : pm.coln;
 #pragma unroll
-          for (int k = 0; k < S::NC * S::ND; ++k) m[k * step] = I[k];
+          for (int k = 0; k < S::NC * S::ND; ++k) {
+            if (gridDim.z > 1) qx_atomic_add(&m[k * step], I[k]);
+            else m[k * step] = I[k];
+          }
         }
       });
 }
@@ -536,7 +544,7 @@ __device__ __forceinline__ void qx_rys_row(const R* gd, int i, int j, int k, R a
 // First-derivative integrals into the slices of the coordinates (G = qx_dual:
 // their derivatives along tv).  One ket c component at a time keeps the nine
 // derivative values of its d components in registers; contracted quartets add
-// up in place, which no other lane touches.
+// up in the matrix, by atomics that no step waits for.
 template <int LA, int LB, int LC, int LD, typename G>
 __global__ __launch_bounds__(QX_RYS_BLOCK) void qx_rd(QxArgs A_, QxKList kl, QxPairM pm) {
   using S = QxRys<LA, LB, LC, LD, 1>;
@@ -546,7 +554,7 @@ __global__ __launch_bounds__(QX_RYS_BLOCK) void qx_rd(QxArgs A_, QxKList kl, QxP
   QxKBlock b;
   if (!qx_k_block(A_, kl, b)) return;
   const QxRysLane<S, LA, LB> ln;
-  const int u1 = A_.pr.pp_first[b.P1];
+  const int u1 = A_.pr.pp_first[b.P1], prims = A_.pr.pp_n[b.P1] * kl.ketprim;
   G ab[3];
   {
     QxRysPair<G> bra;
@@ -598,7 +606,6 @@ __global__ __launch_bounds__(QX_RYS_BLOCK) void qx_rd(QxArgs A_, QxKList kl, QxP
               v[6][d] += x.c[lx] * yz; v[7][d] += y.c[ly] * xz; v[8][d] += z.c[lz] * xy;
             }
           }
-          const bool first = i1 == 0 && i2 == 0;
 #pragma unroll
           for (int ce = 0; ce < 4; ++ce) {
             bool lead = true;  // the first centre of its atom stores the atom's sum
@@ -618,7 +625,8 @@ __global__ __launch_bounds__(QX_RYS_BLOCK) void qx_rd(QxArgs A_, QxKList kl, QxP
 #pragma unroll
               for (int d = 0; d < ND; ++d) {
                 const double s = f0 * qx_value(v[x][d]) + f1 * qx_value(v[3 + x][d]) + f2 * qx_value(v[6 + x][d]);
-                o[(long long)d * pm.coln] = first ? s : o[(long long)d * pm.coln] + s;
+                if (prims > 1) qx_atomic_add(&o[(long long)d * pm.coln], s);
+                else o[(long long)d * pm.coln] = s;
               }
             }
           }
@@ -781,7 +789,7 @@ __global__ __launch_bounds__(QX_RYS_BLOCK, sizeof(G) == 8 && qx_ncart(LC) * qx_n
 
 // ---- launchers ----------------------------------------------------------------------
 static inline dim3 qx_k_grid(const QxKList& kl) {
-  return dim3((unsigned)kl.nbra, (unsigned)((kl.maxket + kl.chunk - 1) / kl.chunk));
+  return dim3((unsigned)kl.nbra, (unsigned)((kl.maxket + kl.chunk - 1) / kl.chunk), (unsigned)kl.psplit);
 }
 
 // K by quadrature (FP64 or FP32), and its directional derivative along tv.
