@@ -318,6 +318,11 @@ def _classes(var, default):
 RYS_K = _classes("QX_RYS_K", "2121 2211 2221 2222")
 RYS_G = _classes("QX_RYS_G", "2111 2120 2121 2210 2211 2220 2221 2222")
 RYS_E = _classes("QX_RYS_E", "2111 2120 2121 2211 2220 2221 2222")
+# classes whose adjoint gradient's directional derivative is by quadrature.  One
+# lane / quadrature in us, both in dual numbers: 196 functions 0000 42/493, 1010
+# 157/1294, 1111 511/1219, 2011 302/1012, 2020 134/892, 2110 489/580, 2200 80/205;
+# 12 atoms, minimal basis 0000 49/463, 1010 160/1143, 1110 117/1022, 1111 202/628
+RYS_H = _classes("QX_RYS_H", "2111 2120 2121 2210 2211 2220 2221 2222")
 
 
 def _ranges(n, k):
@@ -363,6 +368,29 @@ def deriv_parts(l, budget=None):
     return [part((a, a + 1), (b, b + 1), r) for a in range(NA) for b in range(NB) for r in _ranges(NC, kc)]
 
 
+def emit_setup_tangent(L, Lt):
+    """Set-up of a dual-number body: every geometric quantity is a qx_dual whose
+    derivative part follows the atoms along A_.e.tv (exponents are fixed)."""
+    L.append("  const double p = A_.pp.p[u1], q = A_.pp.p[u2];")
+    L.append("  const QxTanPair tb_ = qx_tan_pair(A_, P1, u1), tk_ = qx_tan_pair(A_, P2, u2);")
+    L.append("  const R Px = tb_.P[0], Py = tb_.P[1], Pz = tb_.P[2];")
+    L.append("  const R Qx = tk_.P[0], Qy = tk_.P[1], Qz = tk_.P[2];")
+    L.append("  const R Ax = tb_.A[0], Ay = tb_.A[1], Az = tb_.A[2];")
+    L.append("  const R Cx = tk_.A[0], Cy = tk_.A[1], Cz = tk_.A[2];")
+    L.append("  const R ABx = tb_.AB[0], ABy = tb_.AB[1], ABz = tb_.AB[2];")
+    L.append("  const R CDx = tk_.AB[0], CDy = tk_.AB[1], CDz = tk_.AB[2];")
+    L.append("  const double pq = p + q, opq = 1.0 / pq;")
+    L.append("  const R Wx = (p * Px + q * Qx) * opq, Wy = (p * Py + q * Qy) * opq, Wz = (p * Pz + q * Qz) * opq;")
+    L.append("  const R PQx = Px - Qx, PQy = Py - Qy, PQz = Pz - Qz;")
+    L.append("  const double rho = p * q * opq;")
+    L.append("  const R T = rho * (PQx * PQx + PQy * PQy + PQz * PQz);")
+    L.append(f"  R F[{Lt + 1}];")
+    L.append(f"  qx_boys_tan<{Lt}>(T, A_.boys, F);")
+    L.append("  const R pref = (QX_TWO_PI_5_2 / (p * q * sqrt(pq))) * (tb_.K * tk_.K);")
+    for m in range(Lt + 1):
+        L.append(f"  const R b{m} = pref * F[{m}];")
+
+
 def emit_setup(L, Lt, deriv_w):
     L.append("  const double p = A_.pp.p[u1], Kab = A_.pp.K[u1];")
     L.append("  const double Px = A_.pp.Px[u1], Py = A_.pp.Py[u1], Pz = A_.pp.Pz[u1];")
@@ -384,7 +412,8 @@ def emit_setup(L, Lt, deriv_w):
         L.append(f"  const R b{m} = (R)(pref * F[{m}]);")
 
 
-def emit_vrr_consts(L, vrr_lines):
+def emit_vrr_consts(L, vrr_lines, S="R"):
+    """S: type of the factors that depend on exponents alone."""
     used = "\n".join(vrr_lines)
     for ax in AX:
         if f"PA{ax}" in used:
@@ -396,23 +425,30 @@ def emit_vrr_consts(L, vrr_lines):
         if f"WQ{ax}" in used:
             L.append(f"  const R WQ{ax} = (R)(W{ax} - Q{ax});")
     if "oo2p " in used:
-        L.append("  const R oo2p = (R)(0.5 / p);")
+        L.append(f"  const {S} oo2p = ({S})(0.5 / p);")
     if "oo2q " in used:
-        L.append("  const R oo2q = (R)(0.5 / q);")
+        L.append(f"  const {S} oo2q = ({S})(0.5 / q);")
     if "oo2pq " in used:
-        L.append("  const R oo2pq = (R)(0.5 * opq);")
+        L.append(f"  const {S} oo2pq = ({S})(0.5 * opq);")
     if " rp " in used:
-        L.append("  const R rp = (R)(q * opq);")
+        L.append(f"  const {S} rp = ({S})(q * opq);")
     if " rq " in used:
-        L.append("  const R rq = (R)(p * opq);")
+        L.append(f"  const {S} rq = ({S})(p * opq);")
 
 
-def _head(L, fn, sig, Lt, v, vn, ret="void", inline="__forceinline__"):
-    L.append(f"template <typename R>\n__device__ {inline} {ret} {fn}(const QxArgs& A_, int P1, int P2, "
-             f"int u1, int u2{sig}) {{")
-    emit_setup(L, Lt, False)
-    emit_vrr_consts(L, v.lines)
-    L += ["  " + x for x in v.lines]
+def _head(L, fn, sig, Lt, v, vn, ret="void", inline="__forceinline__", tangent=False):
+    if tangent:
+        L.append(f"__device__ {inline} {ret} {fn}(const QxArgs& A_, int P1, int P2, int u1, int u2{sig}) {{")
+        L.append("  using R = qx_dual;")
+        emit_setup_tangent(L, Lt)
+        emit_vrr_consts(L, v.lines, "double")
+        L += ["  " + x.replace("R(", "double(") for x in v.lines]
+    else:
+        L.append(f"template <typename R>\n__device__ {inline} {ret} {fn}(const QxArgs& A_, int P1, int P2, "
+                 f"int u1, int u2{sig}) {{")
+        emit_setup(L, Lt, False)
+        emit_vrr_consts(L, v.lines)
+        L += ["  " + x for x in v.lines]
     for (a, c), name in sorted(vn.items()):
         L.append(f"  const R s_{a[0]}{a[1]}{a[2]}_{c[0]}{c[1]}{c[2]} = {name};")
 
@@ -477,10 +513,11 @@ def emit_eri_core(l):
     return "\n".join(L), ["\n".join(K)], dict(stats, jk_flops=[core_flops(Lt, v.nflop, h.nflop) + 8 * N])
 
 
-def emit_deriv_core(l, pi, part):
+def emit_deriv_core(l, pi, part, tangent=False):
     """One derivative part: qx_gr_d* contracts each derivative integral with
     the density pair product as soon as it is formed (the adjoint gradient),
-    so no derivative block is ever held whole."""
+    so no derivative block is ever held whole.  tangent: qx_gt_d*, the same of
+    the integrals' derivative along A_.e.tv."""
     la, lb, lc, ld = l
     nn = (ncart(la), ncart(lb), ncart(lc), ncart(ld))
     NA, NB, NC_, ND = nn
@@ -494,8 +531,9 @@ def emit_deriv_core(l, pi, part):
     Lt = sum(l) + 1
     nm = "".join(map(str, l))
     NC = len(combos)
-    wexpr = {"A": "(R)A_.pp.a2[u1]", "B": "(R)A_.pp.b2[u1]", "C": "(R)A_.pp.a2[u2]", "D": "(R)A_.pp.b2[u2]"}
-    wdecl = [f"  const R w{c} = {wexpr[c]};" for c in sorted(set(cc for cc, _ in combos))]
+    S = "double" if tangent else "R"  # factors without a derivative part
+    wexpr = {"A": "A_.pp.a2[u1]", "B": "A_.pp.b2[u1]", "C": "A_.pp.a2[u2]", "D": "A_.pp.b2[u2]"}
+    wdecl = [f"  const {S} w{c} = ({S}){wexpr[c]};" for c in sorted(set(cc for cc, _ in combos))]
     # per element: expressions of each combo and the position after which all exist
     elems = []
     ti = 0
@@ -519,11 +557,11 @@ def emit_deriv_core(l, pi, part):
                             dn = outs[ti]
                             last = max(last, pos[ti])
                             ti += 1
-                        exprs.append(f"w{cn} * {up}" + (f" - R({n}) * {dn}" if dn else ""))
+                        exprs.append(f"w{cn} * {up}" + (f" - {S}({n}) * {dn}" if dn else ""))
                     elems.append((e, le, last, exprs))
     # streaming adjoint form
     G = []
-    _head(G, f"qx_gr_d{nm}_{pi}", f", double (&g)[{NC}]", Lt, v, vn)
+    _head(G, f"qx_{'gt' if tangent else 'gr'}_d{nm}_{pi}", f", double (&g)[{NC}]", Lt, v, vn, tangent=tangent)
     G += wdecl
     emit_dblocks(G, nn)
     groups = []
@@ -534,7 +572,7 @@ def emit_deriv_core(l, pi, part):
         ij, kl, ik, il, jk, jl = i * NB + j, kk * ND + ll, i * NC_ + kk, i * ND + ll, j * NC_ + kk, j * ND + ll
         st = [f"  {{ const double G_ = 2.0 * Dab[{ij}] * Dcd[{kl}] - 0.5 * (Dac[{ik}] * Dbd[{jl}] + "
               f"Dad[{il}] * Dbc[{jk}]);"]
-        st += [f"    g[{ci}] += G_ * (double)({ex});" for ci, ex in enumerate(exprs)]
+        st += [f"    g[{ci}] += G_ * {'qx_value' if tangent else '(double)'}({ex});" for ci, ex in enumerate(exprs)]
         st.append("  }")
         groups.append((last, st))
     G += ["  " + x if not x.startswith("  ") else x for x in interleave(h.lines, groups)]
@@ -873,9 +911,20 @@ def emit_class_files(cls, outdir, fp32):
         write(f"cls_{nm}_j0.hip", [jks[0], "", f"QX_DEFINE_K_KERNEL(e{nm}_0, {dims}, {1 if fp32 else 0})"], "qx_jk.h")
     stats.append((cls, "eri", st))
     write(f"cls_{nm}_d0.hip", [f"QX_DEFINE_RYS_D(d{nm}, {la}, {lb}, {lc}, {ld})"], "qx_rys.h")
-    write(f"cls_{nm}_v0.hip", [f"QX_DEFINE_RYS_KV(e{nm}, {la}, {lb}, {lc}, {ld})",
-                               f"QX_DEFINE_RYS_H(d{nm}, {la}, {lb}, {lc}, {ld})"], "qx_rys.h")
     parts = deriv_parts(cls)
+    if nm in RYS_H:
+        hess = [f"QX_DEFINE_RYS_H(d{nm}, {la}, {lb}, {lc}, {ld})"]
+    else:
+        hess = []
+        for pi, part in enumerate(parts):
+            hess += [emit_deriv_core(cls, pi, part, tangent=True)[0], "",
+                     f"__global__ __launch_bounds__(QX_BLOCK_MAX) void qx_kgv_d{nm}_{pi}(QxArgs A_, QxKList kl) {{",
+                     "  __shared__ double sg[QX_GRAD_LDS];", "  QxKBlock b;", "  if (!qx_k_block(A_, kl, b)) return;",
+                     "  qx_grad_block(A_, kl, b, sg, [&](int P1, int P2, int u1, int u2, double (&g)[QX_GRAD_NCOMB]) {",
+                     f"    qx_gt_d{nm}_{pi}(A_, P1, P2, u1, u2, g);", "  });", "}"]
+        kernels = ", ".join(f"qx_kgv_d{nm}_{pi}" for pi in range(len(parts)))
+        hess.append(f"QX_DEFINE_GRADV_LAUNCHER(d{nm}, {kernels})")
+    write(f"cls_{nm}_v0.hip", [f"QX_DEFINE_RYS_KV(e{nm}, {la}, {lb}, {lc}, {ld})", ""] + hess, "qx_rys.h")
     gsrc = []
     for pi, part in enumerate(parts):
         src_g, st, (cmask, xmask, dinv, NC) = emit_deriv_core(cls, pi, part)
@@ -981,8 +1030,9 @@ def main():
           for L in range(2 * lmax + 1)]
     D.append(f"static int (*const qx_j_table[{2 * lmax + 1}])(const QxArgs*, const QxJList*, int, int, int, hipStream_t) = {{"
              + ", ".join(f"qx_launch_jeng_{L}" for L in range(2 * lmax + 1)) + "};")
-    for name, table in (("k", RYS_K), ("g", RYS_G)):
-        D.append(f"// per class: {'K' if name == 'k' else 'the adjoint gradient'} by Rys quadrature")
+    for name, table, what in (("k", RYS_K, "K"), ("g", RYS_G, "the adjoint gradient"),
+                              ("h", RYS_H, "the adjoint gradient's directional derivative")):
+        D.append(f"// per class: {what} by Rys quadrature")
         D.append(f"static const unsigned char qx_rys_{name}[QX_NUM_CLASSES] = {{")
         D.append("  " + ", ".join(str(int("".join(map(str, cls)) in table)) for cls in classes))
         D.append("};")

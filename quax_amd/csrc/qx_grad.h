@@ -103,6 +103,19 @@ __device__ __forceinline__ void qx_grad_block(const QxArgs& A_, const QxKList& k
     return (int)hipGetLastError();                                                                \
   }
 
+// Launcher of the generated kernels of a class's directional derivative.
+#define QX_DEFINE_GRADV_LAUNCHER(NAME, ...)                                                       \
+  extern "C" int qx_launchh_##NAME(const QxArgs* a, const QxLaunch* L) {                          \
+    if (!L->kl || L->kl->nquart <= 0 || L->kl->maxket <= 0) return 0;                             \
+    const int bs = qx_launch_block(L);                                                            \
+    if (bs % 64 || bs > QX_BLOCK_MAX) return (int)hipErrorInvalidValue;                           \
+    if (!a->e.tv) return -1;                                                                      \
+    const QxKList& kl = *L->kl;                                                                   \
+    const dim3 grid((unsigned)kl.nbra, (unsigned)((kl.maxket + kl.chunk - 1) / kl.chunk));        \
+    for (auto kernel : {__VA_ARGS__}) hipLaunchKernelGGL(kernel, grid, dim3(bs), 0, L->stream, *a, kl); \
+    return (int)hipGetLastError();                                                                \
+  }
+
 // Every gradient kernel of a context without d shells in one launch (as
 // qx_small of the J/K pass): QX_SMALL_GRADS of them, each a class's list.
 struct QxSmallGrad {

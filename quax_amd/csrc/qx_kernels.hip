@@ -124,8 +124,8 @@ __global__ void k_pairm_index(QxShellsDev sh, QxPairsDev pr, int npairs, QxPairI
 }
 
 // The tables of a small context and its cleared matrices in one workgroup:
-// launches are most of such a tensor's time (two functions 57 us in four
-// launches, ONEWG here).
+// launches are most of such a tensor's time (two functions: 57 us with
+// three launches more, 27 us).
 #define PM_SMALL 16384  // doubles of the matrices, ints of the tables
 __global__ __launch_bounds__(1024) void k_pairm_small(QxShellsDev sh, QxPairsDev pr, int npairs, QxPairIndex ix, int ld,
                                                      int* index, int* fn, double* M, int nm) {

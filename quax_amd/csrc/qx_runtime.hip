@@ -257,6 +257,11 @@ void check_launch(int rc, const char* what);
 // refused by the HSA runtime (HSA_STATUS_ERROR_OUT_OF_RESOURCES); the build
 // keeps every kernel that runs here under 6 KB.
 void run_launches(qx_ctx* c, std::vector<Launch>& v, hipStream_t s, const char* what, bool side) {
+  // two small launches cost less in turn than the events of a fork (H2's
+  // directional J/K 47 us against 71)
+  double cost = 0.0;
+  for (const auto& x : v) cost += x.cost;
+  if (v.size() <= 2 && cost < 1e8) side = false;
   const int ns = side ? std::max(1, std::min<int>(c->nstreams, (int)v.size())) : 1;
   if (ns == 1) {
     for (auto& x : v) check_launch(x.go(s), what);
@@ -1293,7 +1298,7 @@ static void add_grad_list(qx_ctx* c, const QxWorkHost& wh, const QxEpiDev& e, in
   if (wh.ncq <= 0 || nq <= 0) return;
   const QxClassEntry& ent = qx_class_table[wh.cls];
   const int block = c->tile[1][wh.cls];
-  const QxKList kl = k_list(c, wh, sel, dir || qx_rys_g[wh.cls] ? 0 : block, false);
+  const QxKList kl = k_list(c, wh, sel, (dir ? qx_rys_h : qx_rys_g)[wh.cls] ? 0 : block, false);
   const int nl = dir ? 1 : ent.ngroups;
   for (int k = 0; k < nl; ++k) {
     QxArgs a;
