@@ -257,3 +257,70 @@ def test_directional_jk_against_the_derivative_tensor(gpu, pure, prims):
         Dt = torch.as_tensor(D, device="cuda").reshape(-1)
         _close(J, (G.reshape(n * n, n * n) @ Dt).reshape(n, n))
         _close(K, (G.permute(0, 2, 1, 3).reshape(n * n, n * n) @ Dt).reshape(n, n))
+
+
+def _molecules_as_fragments():
+    """Uneven molecules of s and p shells side by side, and each by itself."""
+    mols = [synthetic_cluster(0, 2, 3, n_o=1), synthetic_cluster(2, 1, 4), Molecule(["H"], np.zeros((1, 3))),
+            synthetic_cluster(1, 4, 6)]
+    xyz = np.vstack([np.asarray(m.geometry()).reshape(-1, 3) + [0.0, 0.0, 25.0 * k] for k, m in enumerate(mols)])
+    sym = [m.symbol(i) for m in mols for i in range(m.natom())]
+    frag = [k for k, m in enumerate(mols) for _ in range(m.natom())]
+    return mols, Molecule(sym, xyz), frag
+
+
+def test_one_launch_passes_and_tensors_of_fragments(gpu):
+    """The one-launch J/K (whole and with fragments left out), the gradient and the
+    tensors of a batch of minimal-basis molecules against one context each."""
+    import torch
+    mols, comb, frag = _molecules_as_fragments()
+    nb = [BasisSet.build(m, "sto-3g").nbf() for m in mols]
+    off = np.concatenate([[0], np.cumsum(nb)])
+    D = np.zeros((off[-1],) * 2)
+    for k, n in enumerate(nb):
+        D[off[k]:off[k + 1], off[k]:off[k + 1]] = _density(n, 20 + k)
+    with _engine(comb, BasisSet.build(comb, "sto-3g"), ints_tol=1e-14, fragments=frag) as eng:
+        J, K = eng.jk(D)
+        skip = [0, 1, 0, 1]
+        Js, Ks = eng.jk(D, frag_skip=skip)
+        g = eng.eri_grad(D).reshape(-1, 3)
+        G, dG = eng.compute_2e_int(), eng.eri_deriv_core(1)
+    inside = torch.zeros_like(G, dtype=torch.bool)
+    at = 0
+    for k, m in enumerate(mols):
+        s = slice(off[k], off[k + 1])
+        a = slice(at, at + m.natom())
+        at += m.natom()
+        inside[s, s, s, s] = True
+        with _engine(m, BasisSet.build(m, "sto-3g"), ints_tol=1e-14) as one:
+            Jk, Kk = one.jk(D[s, s])
+            _close(J[s, s], Jk)
+            _close(K[s, s], Kk)
+            _close(Js[s, s], Jk * (1 - skip[k]))
+            _close(Ks[s, s], Kk * (1 - skip[k]))
+            _close(g[a], one.eri_grad(D[s, s]).reshape(-1, 3))
+            _close(G[s, s, s, s], one.compute_2e_int())
+            _close(dG[3 * a.start:3 * a.stop, s, s, s, s], one.eri_deriv_core(1))
+    assert (G[~inside] == 0).all() and (dG[:, ~inside] == 0).all()
+
+
+@pytest.mark.parametrize("n_c,extra,offset", [(1, 0, 1), (2, 1, 0), (2, 1, 1), (7, 1, 0), (7, 2, 1)])
+def test_expansion_odd_or_unaligned(gpu, n_c, extra, offset):
+    """An odd number of functions, and an output off its 16-byte line, on both
+    sides of the largest triangle: no wide stores."""
+    import torch
+    from quax_amd import _lib
+    mol = synthetic_cluster(n_c, 0, 9) if n_c > 1 else Molecule(["C"], np.zeros((1, 3)))
+    bs = BasisSet.build(mol, "even-tempered", pure=True)
+    bs = BasisSet("more", bs.shells + [Shell(0, 0, [0.05 * 3 ** k], [1.0]) for k in range(extra)], pure=True)
+    with _engine(mol, bs, ints_tol=1e-12) as eng:
+        n = eng.nbf
+        assert n % 2 == extra % 2 and (n > 195) == (n_c == 7)
+        buf = torch.full((n ** 4 + 2,), float("nan"), dtype=torch.float64, device="cuda")
+        out = buf[offset:offset + n ** 4]
+        assert out.data_ptr() % 16 == 8 * offset
+        _lib.check(eng.L.qx_compute_2e_int(eng.ctx, _lib.ptr(out), eng._stream()), eng.ctx)
+        assert torch.isnan(buf[:offset]).all() and torch.isnan(buf[offset + n ** 4:]).all()
+        D = _density(n, 21)
+        J = (out.view(n * n, n * n) @ torch.as_tensor(D, device="cuda").reshape(-1)).reshape(n, n)
+        _close(eng.jk(D)[0], J)
