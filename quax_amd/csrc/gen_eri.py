@@ -256,16 +256,13 @@ def interleave(hlines, groups):
     return out
 
 
-def emit_dblocks(L, nn, arrays=True):
+def emit_dblocks(L, nn):
     """Loads the six density blocks of the quartet (double) from A_.e.D into
-    local arrays; arrays=False only sets up the indices (the caller reads D
-    where each value is used)."""
+    local arrays."""
     NA, NB, NC, ND = nn
     L.append("  const int n_ = A_.e.nbf;")
     L.append("  const double* Dm_ = A_.e.D;")
     L.append("  const int ia_ = A_.pr.bfa[P1], ib_ = A_.pr.bfb[P1], ic_ = A_.pr.bfa[P2], id_ = A_.pr.bfb[P2];")
-    if not arrays:
-        return
     for nm, r0, nr, c0, nc in (("Dab", "ia_", NA, "ib_", NB), ("Dcd", "ic_", NC, "id_", ND),
                                ("Dac", "ia_", NA, "ic_", NC), ("Dad", "ia_", NA, "id_", ND),
                                ("Dbc", "ib_", NB, "ic_", NC), ("Dbd", "ib_", NB, "id_", ND)):
@@ -310,9 +307,10 @@ def _classes(var, default):
 
 # classes whose K, adjoint gradient and (stored) integrals come from the
 # Rys-quadrature kernels (qx_rys.h) instead of the one-lane-per-quartet bodies.
-# 280 functions, one lane / quadrature in us: K 2110 183/797, 2111 283/308, 2120
-# 299/412, 2210 119/373, 2220 350/289 (but 7.4/12.4 ms in FP32 at 672 functions),
-# 2121 829/288, 2211 530/228; gradient 1111 216/318, 2020 201/290, 2011 205/472,
+# 280 functions, one lane / quadrature in us, all FP64: K 2110 183/797, 2111 283/308,
+# 2120 299/412, 2210 119/373, 2220 350/289 (but 7.7/11.9 ms at 672 functions, where
+# K' and density rows fill a CU's LDS and the quadrature has four wavefronts on it:
+# the one-lane form stays, 0.06 ms slower at 280), 2121 829/288, 2211 530/228; gradient 1111 216/318, 2020 201/290, 2011 205/472,
 # 2110 370/1608, and the split one-lane bodies of the listed classes 1.3 to 3
 # times the quadrature's
 RYS_K = _classes("QX_RYS_K", "2121 2211 2221 2222")

@@ -1,16 +1,16 @@
-// Device-side definitions shared by the generated per-class ERI kernels:
-// argument structs, the Boys function, quartet lookup and the epilogues.
+// Device-side definitions shared by every kernel of the library: argument
+// structs, the Boys function, dual numbers and quartet lookup.
 //
 // Work decomposition.  Screened shell pairs are sorted by class and, within a
 // class, by descending Schwarz bound.  Each contracted pair expands into its
-// primitive pairs ("pseudo pairs", stored contiguously per pair).  One thread
-// evaluates one pseudo-pair quartet; a contracted quartet is the sum of its
-// pseudo-pair quartets, so every epilogue that is linear in the integrals
-// (J/K, gradient, tensor scatter with atomics) contracts by accumulation.
-// For a bra pseudo pair i the admissible ket pseudo pairs form a prefix of the
-// ket list (Schwarz-sorted, canonical j <= i within one class), so a work list
-// is a running-count array over bra pseudo pairs and thread t finds its bra by
-// binary search.
+// primitive pairs ("pseudo pairs", stored contiguously per pair); a contracted
+// quartet is the sum of its pseudo-pair quartets.  For a bra pair the
+// admissible kets of a class form a prefix of its list (Schwarz-sorted,
+// canonical j <= i within one class), so a work list is a running-count array
+// over the bra pairs.  The K, gradient and quadrature kernels give a workgroup
+// one bra pair and a run of its kets and sum a contracted quartet's primitives
+// in registers; the array-form kernels (qx_pairm.h) find a thread's quartet by
+// binary search.  The stored integrals use the same lists over pseudo pairs.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -169,8 +169,6 @@ __device__ __forceinline__ qx_dual operator/(qx_dual a, double b) { return {a.v 
 __device__ __forceinline__ qx_dual& operator+=(qx_dual& a, qx_dual b) { a = a + b; return a; }
 __device__ __forceinline__ qx_dual& operator-=(qx_dual& a, qx_dual b) { a = a - b; return a; }
 __device__ __forceinline__ qx_dual& operator*=(qx_dual& a, qx_dual b) { a = a * b; return a; }
-// the derivative part (what a tangent kernel writes out)
-__device__ __forceinline__ double qx_tan(qx_dual x) { return x.d; }
 
 // F_m(T) along the tangent: dF_m/dT = -F_{m+1}
 template <int M>
@@ -264,10 +262,7 @@ __device__ __forceinline__ void qx_epi_eri(const QxArgs& A_, long long t, int P1
   }
 }
 
-// ---- derivative epilogues --------------------------------------------
-// dv holds NCOMB blocks of N, ordered over centres in CMASK (A=1, B=2, C=4,
-// D=8) then Cartesian directions in XMASK.  With DINV the part covers A, B, C
-// in all directions and d/dD = -(d/dA + d/dB + d/dC).
+// ---- derivatives -------------------------------------------------------
 __device__ __forceinline__ bool qx_single_atom(const QxArgs& A_, int P1, int P2) {
   const int a = A_.pr.atom_a[P1];
   return a == A_.pr.atom_b[P1] && a == A_.pr.atom_a[P2] && a == A_.pr.atom_b[P2];
@@ -282,9 +277,7 @@ __device__ __forceinline__ long long qx_dfull_slice(const QxEpiDev& e, int y) {
   return y;
 }
 
-// ---- kernel definitions (instantiated once per generated file) --------
-#define QX_GRID(nq) dim3((unsigned)(((nq) + QX_BLOCK - 1) / QX_BLOCK))
-
+// ---- kernel tables --------------------------------------------------------
 #define QX_GRAD_LDS 768  // block-level gradient accumulators (3 x the atoms of a block's window)
 
 #define QX_DPARTS_CAP 128  // most derivative parts one class may be split into

@@ -1,9 +1,9 @@
-// Helper kernels of the ERI library: fills, symmetrisation, Cartesian <->
-// spherical transforms, and the one-electron integrals (overlap, kinetic,
-// nuclear attraction) with their first nuclear derivatives.
+// Helper kernels of the ERI library: fills, Cartesian <-> spherical transforms,
+// the pair matrix's way to a tensor, and the derivative matrices of the
+// one-electron integrals (their values and contracted derivatives: qx_oei.h).
 //
-// One-electron integrals are O(n^2 N) work next to the O(n^4) two-electron
-// path, so these kernels favour compact generic code: one thread per ordered
+// The derivative matrices are O(n^2 N) work next to the O(n^4) two-electron
+// path, so their kernel favours compact generic code: one thread per ordered
 // shell pair, 1D Obara-Saika tables for S and T, an Obara-Saika vertical
 // recurrence on the bra for V followed by the binomial transfer
 // (a|O|b) = sum_k C(b,k) AB^(b-k) (a+k|O|0) per Cartesian direction.
@@ -81,8 +81,7 @@ __device__ __forceinline__ void ao_to_cart_at(const QxShellsDev& sh, const doubl
   out[t] = acc;
 }
 
-// Up to three matrices at once (grid row y): the kernels' arithmetic is that of
-// the single forms above.
+// Up to three matrices at once (grid row y).
 struct MatPtrs {
   const double* in[3];
   double* out[3];
@@ -683,7 +682,9 @@ int qxk_pairm_expand(int n, const double* M, long long ld, long long slice, int 
   const size_t bytes = one ? tri : (size_t)rows * n * sizeof(double);
   const dim3 grid((unsigned)((long long)n * (n + 1) / 2), (unsigned)nslice, (unsigned)((n + rows - 1) / rows));
   if (nslice > 65535 || bytes > PM_LDS_TRI) return (int)hipErrorInvalidValue;
-  const dim3 block(n < 96 ? 512 : 1024);  // 112 functions: 464 us with 256 threads, 371 with 512, 328 with 1024
+  // 256 / 512 / 1024 threads in us: 28 functions 7 / 6 / 7 (three slices 8 / 9 / 12), 56 functions 19 / 17.5 / 19,
+  // 84 functions 103 / 96 / 94, 92 functions 137 / 132 / 126, 112 functions 441 / 359 / 310
+  const dim3 block(n < 64 ? 512 : 1024);
   if (pairm_half(n, ld)) hipLaunchKernelGGL((k_pairm_expand<true, true>), grid, block, bytes, s, n, M, ld, slice, *ix, index, fn, rows, out);
   else if (one) hipLaunchKernelGGL((k_pairm_expand<true, false>), grid, block, bytes, s, n, M, ld, slice, *ix, index, fn, rows, out);
   else hipLaunchKernelGGL((k_pairm_expand<false, false>), grid, block, bytes, s, n, M, ld, slice, *ix, index, fn, rows, out);

@@ -8,12 +8,12 @@
 // Cartesian function pairs, M[row of (a, b)][column of (c, d)], whose index is
 //   class base + component * (pairs of the class) + (pair position):
 // consecutive lanes (consecutive ket pairs) write consecutive doubles, each
-// element once and without atomics, also for contracted shells, because one
-// lane sums all primitive quartets of its contracted quartet.  A quarter of
-// the tensor's bytes is written this way; the runtime then mirrors M
+// element once, also for contracted shells, whose primitive quartets are summed
+// before the store (derivatives of contracted quartets add up in M by atomics).
+// A quarter of the tensor's bytes is written this way; the runtime then
+// brings M to AO functions in a spherical basis (qxk_pairm_ao), mirrors it
 // (qxk_pairm_sym) and expands it row by row into the tensor with coalesced
-// stores, applying the Cartesian -> spherical transform on the way
-// (qxk_pairm_expand).
+// stores (qxk_pairm_expand).
 #pragma once
 #include "qx_device.h"
 

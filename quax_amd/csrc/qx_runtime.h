@@ -84,7 +84,6 @@ struct qx_ctx {
   std::vector<double> h_pair_Q;
   std::vector<int> h_pair_frag;
   std::vector<int> class_pair_off, class_pair_cnt;   // per pair class, in sorted pairs
-  std::vector<int> class_pp_off, class_pp_cnt;       // per pair class, in pseudo pairs
   std::vector<int> class_prims;                      // per pair class: most primitives of a pair
   // quartet lists (one per canonical class)
   std::vector<QxWorkHost> work;

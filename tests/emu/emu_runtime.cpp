@@ -55,7 +55,7 @@ void wave_sync() { wave_bar().arrive_and_wait(); }
 void run_grid(dim3 grid, dim3 block, const std::function<void()>& body) {
   const int lanes = 512;
   if (block.x > 512) {
-    std::fprintf(stderr, "emu: block size %u > 256 not supported\n", block.x);
+    std::fprintf(stderr, "emu: block size %u > 512 not supported\n", block.x);
     std::abort();
   }
   if (!g_pool) {
