@@ -126,7 +126,7 @@ __global__ void k_pairm_index(QxShellsDev sh, QxPairsDev pr, int npairs, QxPairI
 // launches are most of such a tensor's time (two functions: 57 us with
 // three launches more, 27 us).
 #define PM_SMALL 16384  // doubles of the matrices, ints of the tables
-__global__ __launch_bounds__(1024) void k_pairm_small(QxShellsDev sh, QxPairsDev pr, int npairs, QxPairIndex ix, int ld,
+__global__ __launch_bounds__(512) void k_pairm_small(QxShellsDev sh, QxPairsDev pr, int npairs, QxPairIndex ix, int ld,
                                                      int* index, int* fn, double* M, int nm) {
   for (int i = threadIdx.x; i < sh.nbf * sh.nbf; i += blockDim.x) index[i] = -1;
   for (int i = threadIdx.x; i < ld; i += blockDim.x) fn[i] = -1;
@@ -628,7 +628,7 @@ int qxk_pairm_tables(const QxShellsDev* sh, const QxPairsDev* pr, int npairs, co
   const long long n2 = (long long)sh->nbf * sh->nbf;
   *cleared = n2 + ld <= PM_SMALL && nm <= PM_SMALL;
   if (*cleared) {
-    hipLaunchKernelGGL(k_pairm_small, dim3(1), dim3(1024), 0, s, *sh, *pr, npairs, *ix, (int)ld, index, fn, M, (int)nm);
+    hipLaunchKernelGGL(k_pairm_small, dim3(1), dim3(512), 0, s, *sh, *pr, npairs, *ix, (int)ld, index, fn, M, (int)nm);
     return (int)hipGetLastError();
   }
   hipLaunchKernelGGL(k_fill_int, dim3(std::min(nblk(n2, 256), 4096u)), dim3(256), 0, s, index, n2, -1);

@@ -93,14 +93,16 @@ static inline dim3 qx_array_grid(const QxArgs* a, const QxLaunch* L, long long& 
 #define QX_DEFINE_ERI_KERNEL(NAME, N, NA, NB, NC, ND)                                             \
   __global__ __launch_bounds__(QX_BLOCK) void qx_k_##NAME(QxArgs A_, QxPairM pm) {                \
     const long long t = (long long)blockIdx.x * QX_BLOCK + threadIdx.x;                          \
-    QxArrayQuartet q;                                                                             \
-    if (!qx_array_quartet(A_, pm, t, q)) return;                                                  \
-    if (A_.e.skip_single && qx_single_atom(A_, q.P1, q.P2)) return;                               \
+    QxArrayQuartet q{};                                                                           \
+    bool on = qx_array_quartet(A_, pm, t, q);                                                     \
+    if (on && A_.e.skip_single) on = !qx_single_atom(A_, q.P1, q.P2);                             \
     double o[N] = {};                                                                             \
-    for (int k = q.k0; k < q.n1 * q.n2; k += q.ks)                                                \
-      qx_core_##NAME<double>(A_, q.P1, q.P2, q.u1 + k / q.n2, q.u2 + k % q.n2, o);                \
-    if (A_.e.epi == QX_EPI_PAIRM) qx_pairm_eri<NA * NB, NC * ND, double>(pm, q.P1, q.P2, q.k0 == 0, o);      \
-    else qx_epi_eri<NA, NB, NC, ND, double>(A_, t, q.P1, q.P2, o, true);                          \
+    if (on)                                                                                       \
+      for (int k = q.k0; k < q.n1 * q.n2; k += q.ks)                                              \
+        qx_core_##NAME<double>(A_, q.P1, q.P2, q.u1 + k / q.n2, q.u2 + k % q.n2, o);              \
+    /* every lane: the sums over a quartet's lanes are cross-lane */                              \
+    if (A_.e.epi == QX_EPI_PAIRM) qx_pairm_eri<NA * NB, NC * ND, double>(pm, q.P1, q.P2, on && q.k0 == 0, o); \
+    else qx_epi_eri<NA, NB, NC, ND, double>(A_, t, q.P1, q.P2, o, on);                            \
   }                                                                                               \
   extern "C" int qx_launch_##NAME(const QxArgs* a, const QxLaunch* L) {                           \
     long long nq;                                                                                 \

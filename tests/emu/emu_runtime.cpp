@@ -76,7 +76,7 @@ void run_grid(dim3 grid, dim3 block, const std::function<void()>& body) {
   P.body = body;
   P.grid = grid;
   P.block = block;
-  for (unsigned b = 0; b < grid.x * grid.y; ++b) {
+  for (unsigned b = 0; b < grid.x * grid.y * grid.z; ++b) {
     P.cur_block = b;
     P.bar->arrive_and_wait();
     P.bar->arrive_and_wait();

@@ -26,6 +26,7 @@
 
 #define __global__
 #define __device__
+#define __constant__ static
 #define __host__
 #define __forceinline__ inline
 #define __launch_bounds__(...)
