@@ -44,16 +44,18 @@ __device__ __forceinline__ void qx_locate_pairs(const QxPairM& pm, long long t, 
 }
 
 template <int NAB, int NCD, typename R>
-__device__ __forceinline__ void qx_pairm_eri(const QxPairM& pm, int P1, int P2, bool lead, const R (&o)[NAB * NCD]) {
+__device__ __forceinline__ void qx_pairm_eri(const QxPairM& pm, int P1, int P2, bool lead, R (&o)[NAB * NCD]) {
+  if (pm.sub > 1) {  // launch-uniform
+#pragma unroll
+    for (int k = 0; k < NAB * NCD; ++k)
+      for (int off = pm.sub >> 1; off > 0; off >>= 1) o[k] += __shfl_xor(o[k], off);
+  }
+  if (!lead) return;
   double* m = pm.M + (long long)(pm.row0 + P1 - pm.rowp) * pm.ld + pm.col0 + (P2 - pm.colp);
 #pragma unroll
   for (int ij = 0; ij < NAB; ++ij)
 #pragma unroll
-    for (int kl = 0; kl < NCD; ++kl) {
-      double v = (double)o[ij * NCD + kl];
-      for (int off = pm.sub >> 1; off > 0; off >>= 1) v += __shfl_xor(v, off);  // launch-uniform
-      if (lead) m[(long long)ij * pm.rown * pm.ld + (long long)kl * pm.coln] = v;
-    }
+    for (int kl = 0; kl < NCD; ++kl) m[(long long)ij * pm.rown * pm.ld + (long long)kl * pm.coln] = (double)o[ij * NCD + kl];
 }
 
 // ---- array-form kernels ---------------------------------------------------

@@ -290,9 +290,14 @@ __device__ __forceinline__ void qx_rys_walk(const QxArgs& A_, const QxKList& kl,
   for (int k = k0; k < k1; k += S::Q) {
     const int nq = min(S::Q, k1 - k), pk0 = b.kst + k;
     // the workgroup's share of the primitive quartets
-    const int n2 = kl.ketprim > 1 ? qx_rys_prims(A_, pk0, nq) : 1, all = n1 * n2;
-    const int mb = (int)((long long)all * blockIdx.z / gridDim.z), nc = (int)((long long)all * (blockIdx.z + 1) / gridDim.z);
-    if (mb >= nc) continue;
+    const int n2 = kl.ketprim > 1 ? qx_rys_prims(A_, pk0, nq) : 1;
+    int mb = 0, nc = n1 * n2;
+    if (kl.psplit > 1) {
+      const long long all = nc;
+      mb = (int)(all * blockIdx.z / kl.psplit);
+      nc = (int)(all * (blockIdx.z + 1) / kl.psplit);
+      if (mb >= nc) continue;
+    }
     begin(pk0, nq);
     for (int m = mb; m < nc; ++m) {
       const int now = single ? held : (m - mb) % S::STEPS;
@@ -454,7 +459,7 @@ __global__ __launch_bounds__(QX_RYS_BLOCK_MAX) void qx_rk(QxArgs A_, QxKList kl)
 
 // ---- integrals and derivative integrals into the pair matrix --------------------
 // (or, QX_EPI_STORE, into the class-blocked array of a single-primitive basis)
-template <int LA, int LB, int LC, int LD>
+template <int LA, int LB, int LC, int LD, bool STORE>
 __global__ __launch_bounds__(QX_RYS_BLOCK) void qx_re(QxArgs A_, QxKList kl, QxPairM pm) {
   using S = QxRys<LA, LB, LC, LD, 0>;
   HIP_DYNAMIC_SHARED(double, qx_sk)
@@ -479,15 +484,20 @@ __global__ __launch_bounds__(QX_RYS_BLOCK) void qx_re(QxArgs A_, QxKList kl, QxP
       },
       [&]() QX_INLINE {
         if (act && !(A_.e.skip_single && qx_single_atom(A_, b.P1, P2))) {
-          const bool store = A_.e.epi == QX_EPI_STORE;
-          double* m = store ? A_.e.out + A_.w.store_base + (long long)ln.ab * (S::NC * S::ND) * kl.nquart +
-                                  kl.prefix[blockIdx.x] + (P2 - b.kst)
-                            : pm.M + (pm.row0 + b.P1 - pm.rowp + (long long)ln.ab * pm.rown) * pm.ld + pm.col0 + (P2 - pm.colp);
-          const long long step = store ? kl.nquart : pm.coln;
+          if (STORE) {
+            double* m = A_.e.out + A_.w.store_base + (long long)ln.ab * (S::NC * S::ND) * kl.nquart + kl.prefix[blockIdx.x] +
+                        (P2 - b.kst);
 #pragma unroll
-          for (int k = 0; k < S::NC * S::ND; ++k) {
-            if (gridDim.z > 1) qx_atomic_add(&m[k * step], I[k]);
-            else m[k * step] = I[k];
+            for (int k = 0; k < S::NC * S::ND; ++k) m[k * kl.nquart] = I[k];
+            return;
+          }
+          double* m = pm.M + (pm.row0 + b.P1 - pm.rowp + (long long)ln.ab * pm.rown) * pm.ld + pm.col0 + (P2 - pm.colp);
+          if (kl.psplit > 1) {
+#pragma unroll
+            for (int k = 0; k < S::NC * S::ND; ++k) qx_atomic_add(&m[(long long)k * pm.coln], I[k]);
+          } else {
+#pragma unroll
+            for (int k = 0; k < S::NC * S::ND; ++k) m[(long long)k * pm.coln] = I[k];
           }
         }
       });
@@ -847,8 +857,12 @@ static inline dim3 qx_k_grid(const QxKList& kl) {
     const bool store = a->e.epi == QX_EPI_STORE;                                                  \
     if (store ? L->kl->ketprim != 1 : !L->pm) return -1;                                          \
     const size_t sh = 4 * sizeof(double) * QxRys<LA, LB, LC, LD, 0>::LDS;                         \
-    hipLaunchKernelGGL((qx_re<LA, LB, LC, LD>), qx_k_grid(*L->kl), dim3(QX_RYS_BLOCK), sh, L->stream, *a, *L->kl, \
-                       store ? QxPairM{} : *L->pm);                                               \
+    if (store)                                                                                    \
+      hipLaunchKernelGGL((qx_re<LA, LB, LC, LD, true>), qx_k_grid(*L->kl), dim3(QX_RYS_BLOCK), sh, L->stream, *a, \
+                         *L->kl, QxPairM{});                                                      \
+    else                                                                                          \
+      hipLaunchKernelGGL((qx_re<LA, LB, LC, LD, false>), qx_k_grid(*L->kl), dim3(QX_RYS_BLOCK), sh, L->stream, *a, \
+                         *L->kl, *L->pm);                                                         \
     return (int)hipGetLastError();                                                                \
   }
 #define QX_DEFINE_RYS_D(NAME, LA, LB, LC, LD)                                                     \
