@@ -150,9 +150,9 @@ def measured_traffic(workload, kernel):
     if not os.path.exists(path):
         return None
     for line in open(path):
-        f = line.split()
-        if len(f) == 3 and not line.startswith("#") and f[0] == workload and f[1] == kernel:
-            return float(f[2])
+        f = line.split()  # workload, kernel (template arguments hold blanks), bytes
+        if len(f) >= 3 and not line.startswith("#") and f[0] == workload and " ".join(f[1:-1]) == kernel:
+            return float(f[-1])
     return None
 
 

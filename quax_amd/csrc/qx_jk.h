@@ -15,10 +15,12 @@
 // A quartet's integrals are contracted over its primitives before the
 // horizontal recurrence, so a contracted quartet updates K once.
 //
-// J is bound by FP64 issue (84 % of it for the ps|, pp| bras of 280 functions;
-// 0.69 ms of 3.05 ms in all).  K of the light classes is bound by LDS atomics
-// and the rows' flush, K of the d classes that stay here by their registers
-// (512, one wavefront per SIMD).  With J and K in one kernel, six streams of
+// J is bound by instruction issue and the latency of its chains together (VALU
+// issue 39-53 % of the cycles, FP64 24-32 %, for all bras below dd; 0.69 ms of
+// 3.05 ms in all).  K of the light classes is bound by LDS atomics and the rows'
+// flush (LDS busy 20-43 %), K of the d classes that stay here by their registers
+// and scratch ((dp|pp), (dp|ds), (dd|ds): 0.5-2.2 KB per lane, 0.5-1.2 GB of HBM
+// traffic per launch).  With J and K in one kernel, six streams of
 // atomics per integral, the same pass took 8.5 ms.
 #pragma once
 #include "qx_device.h"

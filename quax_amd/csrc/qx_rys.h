@@ -375,8 +375,8 @@ __device__ __forceinline__ void qx_rys_sum(const R* gq, int ox, int oy, int oz, 
 }
 
 // ---- K ------------------------------------------------------------------------
-// Bound by latency at two or three wavefronts per SIMD (a quarter of the FP64
-// issue rate) and LDS.  K'_a then K'_b: a lane's sums over (c, d) are added
+// Bound by LDS (busy 51-54 % of the cycles) and latency at two or three
+// wavefronts per SIMD (FP64 issue 17-26 %).  K'_a then K'_b: a lane's sums over (c, d) are added
 // over its quartet's lanes in LDS, one atomic per row element instead of one
 // per lane ((dd|dp) of 280 functions 457 -> 357 us, (dp|dp) 403 -> 336, with
 // larger shares of kets per workgroup 322 and 291).
@@ -652,7 +652,7 @@ __global__ __launch_bounds__(QX_RYS_BLOCK) void qx_rd(QxArgs A_, QxKList kl, QxP
 // values first (w: 5 multiply-adds per (c, d)), which then meets the raised
 // and lowered values: the nine derivative values per (c, d) are never formed
 // ((dd|dp) of 280 functions: 1.77 ms at one wavefront per SIMD -> 0.98 at two).
-// Bound by LDS reads and FP64 issue in about equal parts at two wavefronts per
+// Bound by LDS reads (busy 52-68 % of the cycles) and VALU issue (41-53 %) at two wavefronts per
 // SIMD; three (168 registers) spill and take 2.2 ms.
 template <int LA, int LB, int LC, int LD, typename G>
 __global__ __launch_bounds__(QX_RYS_BLOCK, sizeof(G) == 8 && qx_ncart(LC) * qx_ncart(LD) < 36 ? 2 : 1) void qx_rg(QxArgs A_, QxKList kl) {
