@@ -608,12 +608,11 @@ void schwarz_and_lists(qx_ctx* c) {
     }
     c->d_frag_col0 = dupload(c, lo);
     // atom window of each fragment id: lowest atom, atoms up to the highest
-    std::vector<int> win(2 * (fmax + 1), 0);
-    for (int f = 0; f <= fmax; ++f) {
-      int a0 = c->natom, a1 = -1;
-      for (int at = 0; at < c->natom; ++at)
-        if (c->frag[at] == f) { a0 = std::min(a0, at); a1 = at; }
-      if (a1 >= 0) { win[2 * f] = a0; win[2 * f + 1] = a1 - a0 + 1; }
+    std::vector<int> win(2 * (size_t)(fmax + 1), 0);
+    for (int at = 0; at < c->natom; ++at) {
+      int* w = &win[2 * (size_t)c->frag[at]];
+      if (w[1] == 0) w[0] = at;
+      w[1] = at - w[0] + 1;
     }
     c->d_frag_atoms = dupload(c, win);
   }
