@@ -316,10 +316,11 @@ def _classes(var, default):
 RYS_K = _classes("QX_RYS_K", "2121 2211 2221 2222")
 RYS_G = _classes("QX_RYS_G", "2111 2120 2121 2210 2211 2220 2221 2222")
 RYS_E = _classes("QX_RYS_E", "2111 2120 2121 2211 2220 2221 2222")
-# classes whose adjoint gradient's directional derivative is by quadrature.  One
-# lane / quadrature in us, both in dual numbers: 196 functions 0000 42/493, 1010
+# classes whose directional derivatives (K and adjoint gradient) are by quadrature.
+# Gradient, one lane / quadrature in us, both in dual numbers: 196 functions 0000 42/493, 1010
 # 157/1294, 1111 511/1219, 2011 302/1012, 2020 134/892, 2110 489/580, 2200 80/205;
-# 12 atoms, minimal basis 0000 49/463, 1010 160/1143, 1110 117/1022, 1111 202/628
+# 12 atoms, minimal basis 0000 49/463, 1010 160/1143, 1110 117/1022, 1111 202/628;
+# whole directional J/K pass 2.3/3.1 ms and 0.37/0.77 ms
 RYS_H = _classes("QX_RYS_H", "2111 2120 2121 2210 2211 2220 2221 2222")
 
 
@@ -451,6 +452,59 @@ def _head(L, fn, sig, Lt, v, vn, ret="void", inline="__forceinline__", tangent=F
         L.append(f"  const R s_{a[0]}{a[1]}{a[2]}_{c[0]}{c[1]}{c[2]} = {name};")
 
 
+def emit_k_body(l, h, v, vn, outs, pos, tangent=False):
+    """K body of a class (qx_kb_e*): the integrals of all primitives are summed
+    as [e0|f0], then transferred and contracted with the density blocks one by
+    one, all in FP64 also where the recursion is FP32 (summed in FP32, K of 49 x
+    49 primitives was off by 2.7e-7 of its norm; rounded after the sum, 2.4e-8;
+    rounded per primitive quartet only, 1.5e-9).  tangent: qx_kb_ve*, the same
+    of the integrals' derivative along A_.e.tv."""
+    NA, NB, NC, ND = (ncart(x) for x in l)
+    N = NA * NB * NC * ND
+    nm = "".join(map(str, l))
+    S = "R" if tangent else "double"  # type of the sums and the transfer
+    K = [f"template <typename R>\n__device__ __forceinline__ void qx_kb_{f've{nm}' if tangent else f'e{nm}_0'}(const QxArgs& A_, int P1, int P2, "
+         f"int s_, int ns_, const double (&Dac)[{NA * NC}], const double (&Dad)[{NA * ND}], const double (&Dbc)[{NB * NC}], "
+         f"const double (&Dbd)[{NB * ND}], double (&kac)[{NA * NC}], double (&kad)[{NA * ND}], "
+         f"double (&kbc)[{NB * NC}], double (&kbd)[{NB * ND}]) {{"]
+    names = {ac: f"s_{ac[0][0]}{ac[0][1]}{ac[0][2]}_{ac[1][0]}{ac[1][1]}{ac[1][2]}" for ac in sorted(vn)}
+    K += [f"  {S} {x}(0.0);" for x in names.values()]
+    K.append("  const int v1_ = A_.pr.pp_first[P1], v2_ = A_.pr.pp_first[P2], n2_ = A_.pr.pp_n[P2];")
+    K.append("  for (int k_ = s_; k_ < A_.pr.pp_n[P1] * n2_; k_ += ns_) {")
+    K.append("  const int u1 = v1_ + k_ / n2_, u2 = v2_ + k_ % n2_;")
+    body = []
+    if tangent:
+        emit_setup_tangent(body, sum(l))
+        emit_vrr_consts(body, v.lines, "double")
+        body += ["  " + x.replace("R(", "double(") for x in v.lines]
+    else:
+        emit_setup(body, sum(l), False)
+        emit_vrr_consts(body, v.lines)
+        body += ["  " + x for x in v.lines]
+    body = [x for x in body if not x.startswith(("  const R ABx", "  const R CDx"))]
+    body += [f"  {names[ac]} += ({S}){vn[ac]};" for ac in sorted(vn)]
+    K += ["  " + x for x in body] + ["  }"]
+    if tangent:
+        K.append("  const QxTanPair tb_ = qx_tan_pair(A_, P1, v1_), tk_ = qx_tan_pair(A_, P2, v2_);")
+    for cd, pair, tan in (("AB", "P1", "tb_"), ("CD", "P2", "tk_")):
+        K.append(f"  const {S} " + ", ".join(f"{cd}{ax} = {tan}.AB[{i}]" if tangent else f"{cd}{ax} = A_.pr.AB{ax}[{pair}]"
+                                             for i, ax in enumerate(AX)) + ";")
+    groups = []
+    for k in range(N):
+        i, rem = divmod(k, NB * NC * ND)
+        j, rem = divmod(rem, NC * ND)
+        kk, ll = divmod(rem, ND)
+        ik, il, jk, jl = i * NC + kk, i * ND + ll, j * NC + kk, j * ND + ll
+        groups.append((pos[k], [
+            f"  {{ const double v_ = qx_value({outs[k]});",
+            f"    kac[{ik}] += v_ * Dbd[{jl}]; kad[{il}] += v_ * Dbc[{jk}];",
+            f"    kbc[{jk}] += v_ * Dad[{il}]; kbd[{jl}] += v_ * Dac[{ik}]; }}"]))
+    hrr = [x.replace("const R ", f"const {S} ") for x in h.lines]
+    K += ["  " + x if not x.startswith("  ") else x for x in interleave(hrr, groups)]
+    K.append("}")
+    return "\n".join(K)
+
+
 def emit_eri_core(l):
     """Two bodies per class: qx_core_e* adds the integrals to an array (the
     pair-matrix / store / Schwarz epilogues), qx_kb_e* sums the primitive
@@ -472,43 +526,9 @@ def emit_eri_core(l):
     L.append("}")
     stats = dict(vrr=len(v.lines), vrr_flops=v.nflop, hrr=len(h.lines), hrr_flops=h.nflop, L=Lt, N=N,
                  flops=core_flops(Lt, v.nflop, h.nflop))
-    # K form: the integrals of all primitives are summed as [e0|f0], then
-    # transferred and contracted with the density blocks one by one, all in
-    # FP64 also where the recursion is FP32 (summed in FP32, K of 49 x 49
-    # primitives was off by 2.7e-7 of its norm; rounded after the sum, 2.4e-8;
-    # rounded per primitive quartet only, 1.5e-9)
-    K = [f"template <typename R>\n__device__ __forceinline__ void qx_kb_e{nm}_0(const QxArgs& A_, int P1, int P2, int s_, int ns_, "
-         f"const double (&Dac)[{NA * NC}], const double (&Dad)[{NA * ND}], const double (&Dbc)[{NB * NC}], "
-         f"const double (&Dbd)[{NB * ND}], double (&kac)[{NA * NC}], double (&kad)[{NA * ND}], "
-         f"double (&kbc)[{NB * NC}], double (&kbd)[{NB * ND}]) {{"]
-    names = {ac: f"s_{ac[0][0]}{ac[0][1]}{ac[0][2]}_{ac[1][0]}{ac[1][1]}{ac[1][2]}" for ac in sorted(vn)}
-    K += [f"  double {x} = 0.0;" for x in names.values()]
-    K.append("  const int v1_ = A_.pr.pp_first[P1], v2_ = A_.pr.pp_first[P2], n2_ = A_.pr.pp_n[P2];")
-    K.append("  for (int k_ = s_; k_ < A_.pr.pp_n[P1] * n2_; k_ += ns_) {")
-    K.append("  const int u1 = v1_ + k_ / n2_, u2 = v2_ + k_ % n2_;")
-    body = []
-    emit_setup(body, Lt, False)
-    transfer = [x for x in body if x.startswith("  const R ABx") or x.startswith("  const R CDx")]
-    body = [x for x in body if x not in transfer]
-    emit_vrr_consts(body, v.lines)
-    body += ["  " + x for x in v.lines]
-    body += [f"  {names[ac]} += (double){vn[ac]};" for ac in sorted(vn)]
-    fp64 = lambda x: x.replace("const R ", "const double ").replace("(R)", "")
-    K += ["  " + x for x in body] + ["  }"] + [fp64(x) for x in transfer]
-    groups = []
-    for k in range(N):
-        i, rem = divmod(k, NB * NC * ND)
-        j, rem = divmod(rem, NC * ND)
-        kk, ll = divmod(rem, ND)
-        ik, il, jk, jl = i * NC + kk, i * ND + ll, j * NC + kk, j * ND + ll
-        groups.append((pos[k], [
-            f"  {{ const double v_ = qx_value({outs[k]});",
-            f"    kac[{ik}] += v_ * Dbd[{jl}]; kad[{il}] += v_ * Dbc[{jk}];",
-            f"    kbc[{jk}] += v_ * Dad[{il}]; kbd[{jl}] += v_ * Dac[{ik}]; }}"]))
-    K += ["  " + x if not x.startswith("  ") else x for x in interleave([fp64(x) for x in h.lines], groups)]
-    K.append("}")
+    K = emit_k_body(l, h, v, vn, outs, pos)
     # K epilogue: 4 fused multiply-adds per integral
-    return "\n".join(L), ["\n".join(K)], dict(stats, jk_flops=[core_flops(Lt, v.nflop, h.nflop) + 8 * N])
+    return "\n".join(L), [K], dict(stats, jk_flops=[core_flops(Lt, v.nflop, h.nflop) + 8 * N])
 
 
 def emit_deriv_core(l, pi, part, tangent=False):
@@ -922,7 +942,12 @@ def emit_class_files(cls, outdir, fp32):
                      f"    qx_gt_d{nm}_{pi}(A_, P1, P2, u1, u2, g);", "  });", "}"]
         kernels = ", ".join(f"qx_kgv_d{nm}_{pi}" for pi in range(len(parts)))
         hess.append(f"QX_DEFINE_GRADV_LAUNCHER(d{nm}, {kernels})")
-    write(f"cls_{nm}_v0.hip", [f"QX_DEFINE_RYS_KV(e{nm}, {la}, {lb}, {lc}, {ld})", ""] + hess, "qx_rys.h")
+    if nm in RYS_H:
+        kv = [f"QX_DEFINE_RYS_KV(e{nm}, {la}, {lb}, {lc}, {ld})", ""]
+    else:
+        T = [(a, b, c, d) for a in comps(la) for b in comps(lb) for c in comps(lc) for d in comps(ld)]
+        kv = [emit_k_body(cls, *build_dag(T), tangent=True), "", f"QX_DEFINE_KV_KERNEL(e{nm}, {dims})", ""]
+    write(f"cls_{nm}_v0.hip", kv + hess, "qx_rys.h")
     gsrc = []
     for pi, part in enumerate(parts):
         src_g, st, (cmask, xmask, dinv, NC) = emit_deriv_core(cls, pi, part)
@@ -1029,7 +1054,7 @@ def main():
     D.append(f"static int (*const qx_j_table[{2 * lmax + 1}])(const QxArgs*, const QxJList*, int, int, int, hipStream_t) = {{"
              + ", ".join(f"qx_launch_jeng_{L}" for L in range(2 * lmax + 1)) + "};")
     for name, table, what in (("k", RYS_K, "K"), ("g", RYS_G, "the adjoint gradient"),
-                              ("h", RYS_H, "the adjoint gradient's directional derivative")):
+                              ("h", RYS_H, "the directional derivatives of K and of the adjoint gradient")):
         D.append(f"// per class: {what} by Rys quadrature")
         D.append(f"static const unsigned char qx_rys_{name}[QX_NUM_CLASSES] = {{")
         D.append("  " + ", ".join(str(int("".join(map(str, cls)) in table)) for cls in classes))

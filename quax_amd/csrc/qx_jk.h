@@ -489,7 +489,7 @@ __device__ __forceinline__ void qx_k_add(const QxArgs& A_, const QxKBlock& b, in
     }                                                                                             \
     if (ROWS) qx_k_rows_end<NA, NB>(A_, b, qx_sk);                                                \
   }
-#define QX_DEFINE_K_KERNEL(NAME, NA, NB, NC, ND, WITH32)                                          \
+#define QX_DEFINE_KK(NAME, NA, NB, NC, ND)                                                        \
   QX_DEFINE_K_BODY(NAME, NA, NB, NC, ND)                                                          \
   template <typename R, bool ROWS, bool STAGE>                                                    \
   __global__ __launch_bounds__(QX_BLOCK_MAX) void qx_kk_##NAME(QxArgs A_, QxKList kl) {           \
@@ -497,25 +497,27 @@ __device__ __forceinline__ void qx_k_add(const QxArgs& A_, const QxKBlock& b, in
     QxKBlock b;                                                                                   \
     if (qx_k_block(A_, kl, b)) qx_kd_##NAME<R, ROWS, STAGE>(A_, kl, b, qx_sk);                    \
   }                                                                                               \
-  QX_DEFINE_K_LAUNCHER(NAME, NA, NB, qx_kk_##NAME, WITH32, L->block > 0 ? L->block : QX_BLOCK, 0)
+  QX_DEFINE_K_GO(NAME, NA, NB)
 
 // Launcher of a K kernel template <R, ROWS, STAGE>: K' rows in LDS when they
-// fit, density rows too when both do.  EXTRA: further LDS bytes per R.
-#define QX_DEFINE_K_LAUNCHER(NAME, NA, NB, KERNEL, WITH32, BLOCK, EXTRA)                          \
+// fit, density rows too when both do.
+#define QX_DEFINE_K_GO(NAME, NA, NB)                                                              \
   template <typename R>                                                                           \
   static int qx_k_go_##NAME(const QxArgs* a, const QxLaunch* L) {                                 \
     const QxKList& kl = *L->kl;                                                                   \
-    const int bs = (BLOCK);                                                                       \
+    const int bs = qx_launch_block(L);                                                            \
     if (bs % 64 || bs > QX_BLOCK_MAX) return (int)hipErrorInvalidValue;                           \
     const size_t W = a->e.kcols > 0 ? a->e.kcols : a->e.nbf, rows = ((NA) + (NB)) * W * sizeof(double); \
-    const size_t extra = (EXTRA) * sizeof(R);                                                     \
-    const bool fit1 = a->e.krows && rows + extra <= QX_K_LDS_MAX, fit2 = fit1 && 2 * rows + extra <= QX_K_STAGE_MAX; \
+    const bool fit1 = a->e.krows && rows <= QX_K_LDS_MAX, fit2 = fit1 && 2 * rows <= QX_K_STAGE_MAX; \
     const dim3 grid((unsigned)kl.nbra, (unsigned)((kl.maxket + kl.chunk - 1) / kl.chunk));        \
-    if (fit2) hipLaunchKernelGGL((KERNEL<R, true, true>), grid, dim3(bs), 2 * rows + extra, L->stream, *a, kl); \
-    else if (fit1) hipLaunchKernelGGL((KERNEL<R, true, false>), grid, dim3(bs), rows + extra, L->stream, *a, kl); \
-    else hipLaunchKernelGGL((KERNEL<R, false, false>), grid, dim3(bs), extra, L->stream, *a, kl); \
+    if (fit2) hipLaunchKernelGGL((qx_kk_##NAME<R, true, true>), grid, dim3(bs), 2 * rows, L->stream, *a, kl); \
+    else if (fit1) hipLaunchKernelGGL((qx_kk_##NAME<R, true, false>), grid, dim3(bs), rows, L->stream, *a, kl); \
+    else hipLaunchKernelGGL((qx_kk_##NAME<R, false, false>), grid, dim3(bs), 0, L->stream, *a, kl); \
     return (int)hipGetLastError();                                                                \
-  }                                                                                               \
+  }
+// FP64 and FP32 K kernels of a class, and (KV) K of the directional derivative.
+#define QX_DEFINE_K_KERNEL(NAME, NA, NB, NC, ND, WITH32)                                          \
+  QX_DEFINE_KK(NAME, NA, NB, NC, ND)                                                              \
   extern "C" int qx_launchj_##NAME(const QxArgs* a, const QxLaunch* L) {                          \
     if (!L->kl || L->kl->nquart <= 0 || L->kl->maxket <= 0) return 0;                             \
     if (L->fp32) {                                                                                \
@@ -523,6 +525,12 @@ __device__ __forceinline__ void qx_k_add(const QxArgs& A_, const QxKBlock& b, in
       return -1;                                                                                  \
     }                                                                                             \
     return qx_k_go_##NAME<double>(a, L);                                                          \
+  }
+#define QX_DEFINE_KV_KERNEL(NAME, NA, NB, NC, ND)                                                 \
+  QX_DEFINE_KK(v##NAME, NA, NB, NC, ND)                                                           \
+  extern "C" int qx_launchv_##NAME(const QxArgs* a, const QxLaunch* L) {                          \
+    if (!L->kl || L->kl->nquart <= 0 || L->kl->maxket <= 0) return 0;                             \
+    return a->e.tv ? qx_k_go_v##NAME<qx_dual>(a, L) : -1;                                         \
   }
 
 // ---- small s, p molecules ------------------------------------------------------
