@@ -268,7 +268,7 @@ __device__ __forceinline__ int qx_rys_prims(const QxArgs& A_, int pk0, int nq) {
 // through LDS.  (Read by every 1D task itself, those loads kept the CU's
 // address unit busy four times longer than the arithmetic took; one step at a
 // time, (dd|ps) of a 280-function gradient took 1.22 ms against 1.08 so.)
-template <class S, int LB, int LD, typename G, typename R, class Begin, class Step, class End>
+template <class S, int LB, int LD, typename G, typename R, bool SHARE = true, class Begin, class Step, class End>
 __device__ __forceinline__ void qx_rys_walk(const QxArgs& A_, const QxKList& kl, const QxKBlock& b, R* g, Begin begin, Step step,
                                             End end) {
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), waves = blockDim.x >> 6;
@@ -292,7 +292,7 @@ __device__ __forceinline__ void qx_rys_walk(const QxArgs& A_, const QxKList& kl,
     // the workgroup's share of the primitive quartets
     const int n2 = kl.ketprim > 1 ? qx_rys_prims(A_, pk0, nq) : 1;
     int mb = 0, nc = n1 * n2;
-    if (kl.psplit > 1) {
+    if (SHARE && kl.psplit > 1) {
       const long long all = nc;
       mb = (int)(all * blockIdx.z / kl.psplit);
       nc = (int)(all * (blockIdx.z + 1) / kl.psplit);
@@ -458,8 +458,10 @@ __global__ __launch_bounds__(QX_RYS_BLOCK_MAX) void qx_rk(QxArgs A_, QxKList kl)
 }
 
 // ---- integrals and derivative integrals into the pair matrix --------------------
-// (or, QX_EPI_STORE, into the class-blocked array of a single-primitive basis)
-template <int LA, int LB, int LC, int LD, bool STORE>
+// TO: 0 into the matrix; 1 added to it, where workgroups share primitive
+// quartets; 2 into the class-blocked array of a single-primitive basis.  (A
+// choice per launch: as branches of one kernel it cost (dp|dp) 20 %.)
+template <int LA, int LB, int LC, int LD, int TO>
 __global__ __launch_bounds__(QX_RYS_BLOCK) void qx_re(QxArgs A_, QxKList kl, QxPairM pm) {
   using S = QxRys<LA, LB, LC, LD, 0>;
   HIP_DYNAMIC_SHARED(double, qx_sk)
@@ -470,7 +472,7 @@ __global__ __launch_bounds__(QX_RYS_BLOCK) void qx_re(QxArgs A_, QxKList kl, QxP
   bool act = false;
   int P2 = 0;
   double I[S::NC * S::ND];
-  qx_rys_walk<S, LB, LD, double, double>(
+  qx_rys_walk<S, LB, LD, double, double, TO == 1>(
       A_, kl, b, g,
       [&](int pk0, int nq) QX_INLINE {
         act = ln.in && ln.slot < nq;
@@ -484,7 +486,7 @@ __global__ __launch_bounds__(QX_RYS_BLOCK) void qx_re(QxArgs A_, QxKList kl, QxP
       },
       [&]() QX_INLINE {
         if (act && !(A_.e.skip_single && qx_single_atom(A_, b.P1, P2))) {
-          if (STORE) {
+          if (TO == 2) {
             double* m = A_.e.out + A_.w.store_base + (long long)ln.ab * (S::NC * S::ND) * kl.nquart + kl.prefix[blockIdx.x] +
                         (P2 - b.kst);
 #pragma unroll
@@ -492,12 +494,10 @@ __global__ __launch_bounds__(QX_RYS_BLOCK) void qx_re(QxArgs A_, QxKList kl, QxP
             return;
           }
           double* m = pm.M + (pm.row0 + b.P1 - pm.rowp + (long long)ln.ab * pm.rown) * pm.ld + pm.col0 + (P2 - pm.colp);
-          if (kl.psplit > 1) {
 #pragma unroll
-            for (int k = 0; k < S::NC * S::ND; ++k) qx_atomic_add(&m[(long long)k * pm.coln], I[k]);
-          } else {
-#pragma unroll
-            for (int k = 0; k < S::NC * S::ND; ++k) m[(long long)k * pm.coln] = I[k];
+          for (int k = 0; k < S::NC * S::ND; ++k) {
+            if (TO == 1) qx_atomic_add(&m[(long long)k * pm.coln], I[k]);
+            else m[(long long)k * pm.coln] = I[k];
           }
         }
       });
@@ -857,12 +857,9 @@ static inline dim3 qx_k_grid(const QxKList& kl) {
     const bool store = a->e.epi == QX_EPI_STORE;                                                  \
     if (store ? L->kl->ketprim != 1 : !L->pm) return -1;                                          \
     const size_t sh = 4 * sizeof(double) * QxRys<LA, LB, LC, LD, 0>::LDS;                         \
-    if (store)                                                                                    \
-      hipLaunchKernelGGL((qx_re<LA, LB, LC, LD, true>), qx_k_grid(*L->kl), dim3(QX_RYS_BLOCK), sh, L->stream, *a, \
-                         *L->kl, QxPairM{});                                                      \
-    else                                                                                          \
-      hipLaunchKernelGGL((qx_re<LA, LB, LC, LD, false>), qx_k_grid(*L->kl), dim3(QX_RYS_BLOCK), sh, L->stream, *a, \
-                         *L->kl, *L->pm);                                                         \
+    auto kernel = store ? qx_re<LA, LB, LC, LD, 2> : L->kl->psplit > 1 ? qx_re<LA, LB, LC, LD, 1> : qx_re<LA, LB, LC, LD, 0>; \
+    hipLaunchKernelGGL(kernel, qx_k_grid(*L->kl), dim3(QX_RYS_BLOCK), sh, L->stream, *a, *L->kl, \
+                       store ? QxPairM{} : *L->pm);                                               \
     return (int)hipGetLastError();                                                                \
   }
 #define QX_DEFINE_RYS_D(NAME, LA, LB, LC, LD)                                                     \
