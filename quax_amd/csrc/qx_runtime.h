@@ -39,6 +39,7 @@ struct QxWorkHost {
   // ctx->d_cprefix and (fragmented contexts) first kets in ctx->d_ckstart
   long long cprefix_off;
   long long ncq;           // contracted quartets
+  int prims;               // primitive quartets of one (mean, rounded up)
   int maxket;              // most kets of one bra pair
 };
 

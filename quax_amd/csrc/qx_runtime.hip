@@ -566,6 +566,7 @@ void schwarz_and_lists(qx_ctx* c) {
       wh.w.nquart = run;
       wh.w.diag = 0;
       wh.ncq = ncq;
+      wh.prims = (int)std::max((run + ncq - 1) / std::max(ncq, 1LL), 1LL);
       allckst.push_back(0);  // one entry per prefix entry
       wh.w.store_base = c->store_total;
       const int N = ncart(c->l[c->h_pair_sa[bo]]) * ncart(c->l[c->h_pair_sb[bo]]) *
@@ -1147,13 +1148,10 @@ static void begin_pairm(qx_ctx* c, PairMatrix& m, int want, hipStream_t s) {
 #define QX_RYS_BLOCKS 1024LL  // quadrature workgroups below which they share primitive quartets
 #define QX_SUB_LANES 65536  // lanes below which contracted quartets are shared between lanes
 
-// Primitive quartets of a contracted quartet of the list (mean, rounded up).
-static long long list_prims(const QxWorkHost& wh) {
-  return std::max((wh.w.nquart + wh.ncq - 1) / std::max(wh.ncq, 1LL), 1LL);
-}
-// Lanes that share them: few contracted quartets still spread over the device.
+// Lanes that share the primitives of a contracted quartet: few quartets still
+// spread over the device.
 static int shared_lanes(const QxWorkHost& wh) {
-  return (int)std::max<long long>(1, std::min<long long>({list_prims(wh), 64, QX_SUB_LANES / std::max(wh.ncq, 1LL)}));
+  return wh.prims == 1 ? 1 : (int)std::max<long long>(1, std::min<long long>({wh.prims, 64, QX_SUB_LANES / wh.ncq}));
 }
 
 // The contracted list wh for a kernel of one lane per quartet in blocks of
@@ -1171,12 +1169,13 @@ static QxKList k_list(const qx_ctx* c, const QxWorkHost& wh, int sel, int block,
   kl.ketprim = c->class_prims[wh.ket_class];
   kl.rys = c->d_rys;
   kl.frag_atoms = c->d_frag_atoms;
-  const long long prims = list_prims(wh);
+  const long long prims = wh.prims;
   kl.sub = shared_lanes(wh);
   // a bra with few kets (a batch of small molecules) leaves lanes of its
   // workgroup idle: they share the primitives too (500 waters, minimal basis:
   // gradient 0.50 -> 0.31 ms)
-  if (block) kl.sub = (int)std::max<long long>(kl.sub, std::min<long long>({prims, 64, block * (long long)kl.nbra / std::max(wh.ncq, 1LL)}));
+  if (block && prims > kl.sub && kl.sub < 64)
+    kl.sub = (int)std::max<long long>(kl.sub, std::min<long long>({prims, 64, block * (long long)kl.nbra / wh.ncq}));
   const long long most = (wh.ncq + QX_K_BLOCKS - 1) / QX_K_BLOCKS;
   const long long per = std::max<long long>(rows ? std::max(most, std::min(4 * most, QX_K_CHUNK / prims)) : most, 1);
   // quadrature: in short lists as little as one step of each of a block's four
@@ -1188,8 +1187,11 @@ static QxKList k_list(const qx_ctx* c, const QxWorkHost& wh, int sel, int block,
   const int unit = block ? std::max(1, block / kl.sub) : per <= 16 ? std::min(step, 32) : 32;
   kl.chunk = (int)std::min<long long>((per + unit - 1) / unit * unit, 1 << 20);
   // quadrature workgroups that share a bra's primitive quartets, four or more each
-  const long long blocks = (long long)kl.nbra * ((kl.maxket + kl.chunk - 1) / std::max(kl.chunk, 1));
-  kl.psplit = block ? 1 : (int)std::max<long long>(1, std::min(prims / 4, QX_RYS_BLOCKS / std::max(blocks, 1LL)));
+  kl.psplit = 1;
+  if (!block && prims >= 8) {
+    const long long blocks = (long long)kl.nbra * ((kl.maxket + kl.chunk - 1) / kl.chunk);
+    kl.psplit = (int)std::max<long long>(1, std::min(prims / 4, QX_RYS_BLOCKS / std::max(blocks, 1LL)));
+  }
   return kl;
 }
 
