@@ -1150,13 +1150,17 @@ static void begin_pairm(qx_ctx* c, PairMatrix& m, int want, hipStream_t s) {
 
 // Lanes that share the primitives of a contracted quartet: few quartets still
 // spread over the device.
-static int shared_lanes(const QxWorkHost& wh) {
-  return wh.prims == 1 ? 1 : (int)std::max<long long>(1, std::min<long long>({wh.prims, 64, QX_SUB_LANES / wh.ncq}));
+static int shared_lanes(const QxWorkHost& wh, int most) {
+  return wh.prims == 1 ? 1 : (int)std::max<long long>(1, std::min<long long>({(long long)wh.prims, (long long)most, QX_SUB_LANES / wh.ncq}));
 }
 
 // The contracted list wh for a kernel of one lane per quartet in blocks of
-// `block` threads, or (block = 0) of the quadrature kernels; rows: a K kernel.
-static QxKList k_list(const qx_ctx* c, const QxWorkHost& wh, int sel, int block, bool rows) {
+// `block` threads, or (block = 0) of the quadrature kernels; rows: a K kernel;
+// lanes: how many may share a quartet's primitives.  (Dual numbers: 81 on as
+// many lanes take one round, not two: water's directional gradient 127 -> 114
+// us.  The values' shorter rounds lose to the wider sums: gradient of 100 waters
+// 0.11 -> 0.13 ms.)
+static QxKList k_list(const qx_ctx* c, const QxWorkHost& wh, int sel, int block, bool rows, int lanes = 64) {
   QxKList kl{};
   kl.bra0 = c->class_pair_off[wh.bra_class]; kl.ket0 = c->class_pair_off[wh.ket_class];
   kl.prefix = c->d_cprefix + wh.cprefix_off;
@@ -1170,12 +1174,13 @@ static QxKList k_list(const qx_ctx* c, const QxWorkHost& wh, int sel, int block,
   kl.rys = c->d_rys;
   kl.frag_atoms = c->d_frag_atoms;
   const long long prims = wh.prims;
-  kl.sub = shared_lanes(wh);
+  kl.sub = shared_lanes(wh, lanes);
   // a bra with few kets (a batch of small molecules) leaves lanes of its
-  // workgroup idle: they share the primitives too (500 waters, minimal basis:
-  // gradient 0.50 -> 0.31 ms)
-  if (block && prims > kl.sub && kl.sub < 64)
-    kl.sub = (int)std::max<long long>(kl.sub, std::min<long long>({prims, 64, block * (long long)kl.nbra / wh.ncq}));
+  // workgroup idle: where few share so far, they do too (500 waters, minimal
+  // basis: gradient 0.49 -> 0.30 ms; with more than eight the rounds saved are
+  // too few: 100 waters 91 -> 97 us)
+  if (block && prims > kl.sub && kl.sub <= 8)
+    kl.sub = (int)std::max<long long>(kl.sub, std::min<long long>({prims, (long long)lanes, block * (long long)kl.nbra / wh.ncq}));
   const long long most = (wh.ncq + QX_K_BLOCKS - 1) / QX_K_BLOCKS;
   const long long per = std::max<long long>(rows ? std::max(most, std::min(4 * most, QX_K_CHUNK / prims)) : most, 1);
   // quadrature: in short lists as little as one step of each of a block's four
@@ -1206,7 +1211,7 @@ static QxPairM pairm_list(const qx_ctx* c, const PairMatrix& m, const QxWorkHost
   pm.kstart = c->fragmented ? c->d_ckstart + wh.cprefix_off : nullptr;
   pm.nbra = c->class_pair_cnt[X];
   pm.nquart = wh.ncq;
-  for (pm.sub = 1; 2 * pm.sub <= shared_lanes(wh);) pm.sub *= 2;
+  for (pm.sub = 1; 2 * pm.sub <= shared_lanes(wh, 64);) pm.sub *= 2;
   return pm;
 }
 
@@ -1303,7 +1308,7 @@ static void add_grad_list(qx_ctx* c, const QxWorkHost& wh, const QxEpiDev& e, in
   if (wh.ncq <= 0 || nq <= 0) return;
   const QxClassEntry& ent = qx_class_table[wh.cls];
   const int block = c->tile[1][wh.cls];
-  const QxKList kl = k_list(c, wh, sel, (dir ? qx_rys_h : qx_rys_g)[wh.cls] ? 0 : block, false);
+  const QxKList kl = k_list(c, wh, sel, (dir ? qx_rys_h : qx_rys_g)[wh.cls] ? 0 : block, false, dir ? 128 : 64);
   const int nl = dir ? 1 : ent.ngroups;
   for (int k = 0; k < nl; ++k) {
     QxArgs a;
@@ -1327,7 +1332,7 @@ static void add_k_list(qx_ctx* c, const QxWorkHost& wh, const QxEpiDev& e, int f
   if (wh.ncq <= 0 || nq <= 0) return;
   const QxClassEntry& ent = qx_class_table[wh.cls];
   const int block = c->tile[0][wh.cls];
-  const QxKList kl = k_list(c, wh, sel, (dir ? qx_rys_h : qx_rys_k)[wh.cls] ? 0 : block, true);
+  const QxKList kl = k_list(c, wh, sel, (dir ? qx_rys_h : qx_rys_k)[wh.cls] ? 0 : block, true, dir ? 128 : 64);
   const int nl = dir ? 1 : ent.njk;
   for (int k = 0; k < nl; ++k) {
     QxArgs a;
