@@ -268,7 +268,7 @@ __device__ __forceinline__ int qx_rys_prims(const QxArgs& A_, int pk0, int nq) {
 // through LDS.  (Read by every 1D task itself, those loads kept the CU's
 // address unit busy four times longer than the arithmetic took; one step at a
 // time, (dd|ps) of a 280-function gradient took 1.22 ms against 1.08 so.)
-template <class S, int LB, int LD, typename G, typename R, bool SHARE = true, class Begin, class Step, class End>
+template <class S, int LB, int LD, typename G, typename R, bool SHARE, class Begin, class Step, class End>
 __device__ __forceinline__ void qx_rys_walk(const QxArgs& A_, const QxKList& kl, const QxKBlock& b, R* g, Begin begin, Step step,
                                             End end) {
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), waves = blockDim.x >> 6;
@@ -380,7 +380,9 @@ __device__ __forceinline__ void qx_rys_sum(const R* gq, int ox, int oy, int oz, 
 // over its quartet's lanes in LDS, one atomic per row element instead of one
 // per lane ((dd|dp) of 280 functions 457 -> 357 us, (dp|dp) 403 -> 336, with
 // larger shares of kets per workgroup 322 and 291).
-template <int LA, int LB, int LC, int LD, typename G, typename R, bool ROWS, bool STAGE>
+// SHARE: workgroups share primitive quartets (a kernel of its own: as a branch,
+// the walk's longer index arithmetic cost 1.3 % where there is one).
+template <int LA, int LB, int LC, int LD, typename G, typename R, bool ROWS, bool STAGE, bool SHARE>
 __global__ __launch_bounds__(QX_RYS_BLOCK_MAX) void qx_rk(QxArgs A_, QxKList kl) {
   using S = QxRys<LA, LB, LC, LD, 0>;
   constexpr int NA = S::NA, NB = S::NB, NC = S::NC, ND = S::ND;
@@ -395,7 +397,7 @@ __global__ __launch_bounds__(QX_RYS_BLOCK_MAX) void qx_rk(QxArgs A_, QxKList kl)
   bool act = false;
   int P2 = 0, pk = 0, nk = 0;
   G I[NC * ND];
-  qx_rys_walk<S, LB, LD, G, R>(
+  qx_rys_walk<S, LB, LD, G, R, SHARE>(
       A_, kl, b, g,
       [&](int pk0, int nq) QX_INLINE {
         pk = pk0;
@@ -513,7 +515,7 @@ __global__ __launch_bounds__(64) void qx_rs(QxArgs A_, QxKList kl) {
   const QxKBlock b{P, 0, 1, P, 0, 0};
   const QxRysLane<S, LA, LB> ln;
   double I[S::NC * S::ND] = {};
-  qx_rys_walk<S, LB, LB, double, double>(
+  qx_rys_walk<S, LB, LB, double, double, false>(
       A_, kl, b, qx_sk, [&](int, int) QX_INLINE {},
       [&](int, int) QX_INLINE {
         if (ln.slot == 0) qx_rys_sum<S, LA, LB>(qx_sk, ln.off(0), ln.off(1), ln.off(2), I);
@@ -574,7 +576,7 @@ __global__ __launch_bounds__(QX_RYS_BLOCK) void qx_rd(QxArgs A_, QxKList kl, QxP
   }
   bool act = false;
   int P2 = 0, at[4];
-  qx_rys_walk<S, LB, LD, G, G>(
+  qx_rys_walk<S, LB, LD, G, G, true>(
       A_, kl, b, g,
       [&](int pk0, int nq) QX_INLINE {
         const bool in = ln.in && ln.slot < nq;
@@ -654,7 +656,8 @@ __global__ __launch_bounds__(QX_RYS_BLOCK) void qx_rd(QxArgs A_, QxKList kl, QxP
 // ((dd|dp) of 280 functions: 1.77 ms at one wavefront per SIMD -> 0.98 at two).
 // Bound by LDS reads (busy 52-68 % of the cycles) and VALU issue (41-53 %) at two wavefronts per
 // SIMD; three (168 registers) spill and take 2.2 ms.
-template <int LA, int LB, int LC, int LD, typename G>
+// SHARE: as for K (as a branch, (dd|dd) of 280 functions took 293 us, not 280).
+template <int LA, int LB, int LC, int LD, typename G, bool SHARE>
 __global__ __launch_bounds__(QX_RYS_BLOCK, sizeof(G) == 8 && qx_ncart(LC) * qx_ncart(LD) < 36 ? 2 : 1) void qx_rg(QxArgs A_, QxKList kl) {
   using S = QxRys<LA, LB, LC, LD, 1>;
   constexpr int NC = S::NC, ND = S::ND;
@@ -685,7 +688,7 @@ __global__ __launch_bounds__(QX_RYS_BLOCK, sizeof(G) == 8 && qx_ncart(LC) * qx_n
   G v[9];
   bool act = false;
   int P2 = 0, pk = 0, nk = 0;
-  qx_rys_walk<S, LB, LD, G, G>(
+  qx_rys_walk<S, LB, LD, G, G, SHARE>(
       A_, kl, b, g,
       [&](int pk0, int nq) QX_INLINE {
         pk = pk0;
@@ -807,19 +810,22 @@ static inline dim3 qx_k_grid(const QxKList& kl) {
   template <typename G, typename R>                                                               \
   static int qx_rk_go_##NAME(const QxArgs* a, const QxLaunch* L) {                                \
     using S = QxRys<LA, LB, LC, LD, 0>;                                                           \
-    const QxKList& kl = *L->kl;                                                                   \
-    const size_t W = a->e.kcols > 0 ? a->e.kcols : a->e.nbf, rows = (S::NA + S::NB) * W * sizeof(double); \
+    QxKList kl = *L->kl;                                                                          \
+    const size_t W = a->e.kcols > 0 ? a->e.kcols : a->e.nbf, rows = (S::NA + S::NB) * W * sizeof(double);\
     const size_t wave = (size_t)S::LDS * sizeof(R);                                               \
-    /* K' rows and density rows, else K' rows, else neither; eight wavefronts in one block where two  \
+    /* K' rows and density rows, else K' rows, else neither; eight wavefronts in one block where two\
        blocks of four do not fit */                                                               \
     int n = a->e.krows ? 2 : 0;                                                                   \
     while (n > 0 && n * rows + 4 * wave > QX_K_LDS_MAX) --n;                                      \
     const size_t base = n * rows;                                                                 \
-    const int waves = 2 * (base + 4 * wave) > QX_K_LDS_MAX && base + 8 * wave <= QX_K_LDS_MAX ? 8 : 4; \
+    const int waves = 2 * (base + 4 * wave) > QX_K_LDS_MAX && base + 8 * wave <= QX_K_LDS_MAX ? 8 : 4;\
     const size_t sh = base + waves * wave;                                                        \
-    if (n == 2) hipLaunchKernelGGL((qx_rk<LA, LB, LC, LD, G, R, true, true>), qx_k_grid(kl), dim3(64 * waves), sh, L->stream, *a, kl); \
-    else if (n == 1) hipLaunchKernelGGL((qx_rk<LA, LB, LC, LD, G, R, true, false>), qx_k_grid(kl), dim3(64 * waves), sh, L->stream, *a, kl); \
-    else hipLaunchKernelGGL((qx_rk<LA, LB, LC, LD, G, R, false, false>), qx_k_grid(kl), dim3(64 * waves), sh, L->stream, *a, kl); \
+    /* values share primitives with both rows only: few workgroups means few functions */         \
+    constexpr bool DUAL = sizeof(G) > sizeof(double);                                             \
+    if (n < 2 && !DUAL) kl.psplit = 1;                                                            \
+    auto kernel = n == 1 ? qx_rk<LA, LB, LC, LD, G, R, true, false, DUAL> : qx_rk<LA, LB, LC, LD, G, R, false, false, DUAL>;\
+    if (n == 2) kernel = kl.psplit > 1 ? qx_rk<LA, LB, LC, LD, G, R, true, true, true> : qx_rk<LA, LB, LC, LD, G, R, true, true, DUAL>;\
+    hipLaunchKernelGGL(kernel, qx_k_grid(kl), dim3(64 * waves), sh, L->stream, *a, kl);           \
     return (int)hipGetLastError();                                                                \
   }
 #define QX_DEFINE_RYS_K(NAME, LA, LB, LC, LD, WITH32)                                             \
@@ -881,7 +887,9 @@ static inline dim3 qx_k_grid(const QxKList& kl) {
 template <int LA, int LB, int LC, int LD, typename G>
 static int qx_rg_go(const QxArgs* a, const QxLaunch* L) {
   const size_t sh = 4 * (size_t)QxRys<LA, LB, LC, LD, 1>::LDS * sizeof(G);
-  hipLaunchKernelGGL((qx_rg<LA, LB, LC, LD, G>), qx_k_grid(*L->kl), dim3(QX_RYS_BLOCK), sh, L->stream, *a, *L->kl);
+  constexpr bool DUAL = sizeof(G) > sizeof(double);
+  auto kernel = L->kl->psplit > 1 ? qx_rg<LA, LB, LC, LD, G, true> : qx_rg<LA, LB, LC, LD, G, DUAL>;
+  hipLaunchKernelGGL(kernel, qx_k_grid(*L->kl), dim3(QX_RYS_BLOCK), sh, L->stream, *a, *L->kl);
   return (int)hipGetLastError();
 }
 #define QX_DEFINE_RYS_G(NAME, LA, LB, LC, LD)                                                     \
